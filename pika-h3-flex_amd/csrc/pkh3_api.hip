@@ -482,7 +482,6 @@ int pkh3_qkv_proj(const pkh3_qkv_args* p, const pkh3_attn_args* a, void* stream)
   const int64_t w_blk = (int64_t)(p->K / 32) * 1024;       // bytes of one 16-row block of images over K
   const int64_t b_blk = (int64_t)(PKH3_LORA_RANK / 32) * 1024;
   const int64_t xa_blk = 3 * b_blk;                        // down-projected rows: three targets side by side
-  const int m_tiles = (int)(padded_rows(p->S) / 256);
 
   // the K epilogue max-reduces its row norms into per-head slots that must start at zero; so must the positions of
   // the projection's work queues behind them
@@ -491,7 +490,7 @@ int pkh3_qkv_proj(const pkh3_qkv_args* p, const pkh3_attn_args* a, void* stream)
   if (any_lora) {
     // x A^T for the three adapters, scaled, as the activation images of the second K segment
     GemmParams g{};
-    g.a_img = (const char*)p->x_img; g.a_blk_stride = w_blk; g.nk1 = p->K / 32; g.M = p->S; g.m_tiles = m_tiles;
+    g.a_img = (const char*)p->x_img; g.a_blk_stride = w_blk; g.nk1 = p->K / 32; g.M = p->S;
     // Three adapters whose A images lie one behind the other (8 blocks of 16 features each) with one scale are one
     // target of three heads: two workgroup tiles per 256 tokens instead of three half-empty ones.
     const char* a0 = (const char*)lin[0]->lora_a_img;
@@ -524,7 +523,7 @@ int pkh3_qkv_proj(const pkh3_qkv_args* p, const pkh3_attn_args* a, void* stream)
   }
 
   GemmParams g{};
-  g.a_img = (const char*)p->x_img; g.a_blk_stride = w_blk; g.nk1 = p->K / 32; g.M = p->S; g.m_tiles = m_tiles;
+  g.a_img = (const char*)p->x_img; g.a_blk_stride = w_blk; g.nk1 = p->K / 32; g.M = p->S;
   g.n_targets = 3;
   for (int t = 0; t < 3; ++t) {
     GemmTarget& tg = g.tg[t];
@@ -548,10 +547,7 @@ int pkh3_qkv_proj(const pkh3_qkv_args* p, const pkh3_attn_args* a, void* stream)
     GemmTarget& v = g.tg[2];
     v.epi = kEpiVImg; v.out = L.vp.out; v.out_head_stride = L.vp.out_bh_stride; v.out_blk_stride = L.vp.out_tile_stride;
   }
-  // launches of at least two rounds of workgroups take their tiles from per-XCD work queues
-  int cus = 0;
-  if ((e = device_cu_count(&cus)) != hipSuccess) return hip_fail(e, "device_cu_count");
-  if (cus > 0 && g.m_tiles * g.n_tiles >= 2 * cus) g.queue_next = (int*)(L.ws + L.w.kmax_off) + H;
+  g.queue_next = (int*)(L.ws + L.w.kmax_off) + H;
   if ((e = launch_gemm(g, st)) != hipSuccess) return hip_fail(e, "qkv projection");
   g_err[0] = 0;
   return PKH3_OK;
@@ -579,10 +575,9 @@ int pkh3_out_proj(const pkh3_out_args* p, void* stream) {
   hipError_t e;
   const int64_t w_blk = (int64_t)(p->K / 32) * 1024;
   const int64_t b_blk = (int64_t)(PKH3_LORA_RANK / 32) * 1024;
-  const int m_tiles = (int)(padded_rows(p->S) / 256);
   if (lora) {
     GemmParams g{};
-    g.a_img = (const char*)p->o_img; g.a_blk_stride = w_blk; g.nk1 = p->K / 32; g.M = p->S; g.m_tiles = m_tiles;
+    g.a_img = (const char*)p->o_img; g.a_blk_stride = w_blk; g.nk1 = p->K / 32; g.M = p->S;
     g.n_targets = 1; g.n_tiles = 1;
     GemmTarget& tg = g.tg[0];
     tg = GemmTarget{};
@@ -592,7 +587,7 @@ int pkh3_out_proj(const pkh3_out_args* p, void* stream) {
     if ((e = launch_gemm(g, st)) != hipSuccess) return hip_fail(e, "lora down-projection");
   }
   GemmParams g{};
-  g.a_img = (const char*)p->o_img; g.a_blk_stride = w_blk; g.nk1 = p->K / 32; g.M = p->S; g.m_tiles = m_tiles;
+  g.a_img = (const char*)p->o_img; g.a_blk_stride = w_blk; g.nk1 = p->K / 32; g.M = p->S;
   g.n_targets = 1;
   GemmTarget& tg = g.tg[0];
   tg = GemmTarget{};

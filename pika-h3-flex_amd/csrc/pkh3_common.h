@@ -77,10 +77,11 @@ __device__ __forceinline__ void raise_max(unsigned* slot, float v) {
 }
 
 __device__ __forceinline__ float wave_sum_groups(float x) {
-  // sum over the four lanes l % 16 == const (one per 16-lane group)
-  x += __shfl_xor(x, 16, 64);
-  x += __shfl_xor(x, 32, 64);
-  return x;
+  // sum over the four lanes l % 16 == const (one per 16-lane group): two row swaps, no trip through the LDS crossbar
+  const auto r16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = __uint_as_float(r16[0]) + __uint_as_float(r16[1]);
+  const auto r32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r32[0]) + __uint_as_float(r32[1]);
 }
 
 // ---- four lanes per row: the layout of the 16x16 operand images themselves ----
@@ -133,10 +134,11 @@ __device__ __forceinline__ void load_norm_quarter(NormQuarter& n, const RowTrans
 __device__ __forceinline__ void norm_rope_quarter(float (&x)[32], const RowTransform& t, const NormQuarter& n, const RopeQuarter& r,
                                                   bool valid, int g) {
   if (t.norm_w) {
-    float ssq = 0.f;
+    // four running sums: one would be a chain of 32 dependent instructions
+    float part[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int i = 0; i < 32; ++i) ssq += x[i] * x[i];
-    ssq = wave_sum_groups(ssq);
+    for (int i = 0; i < 32; ++i) part[i & 3] += x[i] * x[i];
+    const float ssq = wave_sum_groups((part[0] + part[1]) + (part[2] + part[3]));
     // an all-zero row with eps == 0 stays all zero instead of 0 * inf
     const float ms = ssq * (1.0f / kD) + t.eps;
     const float rs = ms > 0.f ? rsqrtf(ms) : 0.f;

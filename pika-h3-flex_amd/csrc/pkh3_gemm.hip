@@ -9,7 +9,7 @@
 // l%16, elements 8*(l/16)..+7 -- the shape of the attention kernel's K images): activations as [16-token
 // block][k-step], weights as [16-feature block][k-step] (packed once when the weights are loaded).  They move
 // HBM/L2 -> LDS -> VGPR as straight 16-byte copies, like the K/V tiles of the attention kernel: direct-to-LDS loads
-// into a 4-slot ring, three chunks ahead, one barrier per chunk.  Since the two MFMA operands have the same register
+// into a 3-slot ring, up to three chunks ahead, one barrier per chunk.  Since the two MFMA operands have the same register
 // form, one pair of images serves both orientations:
 //   C^T = W x^T  (features down the accumulator registers, one token per lane)   Q, K, row-major outputs
 //   C   = x W^T  (tokens down the registers, one feature per lane)               V images
@@ -18,10 +18,12 @@
 // token's head row: exactly what lane (g, c) of the attention kernel's K images carries, so the K epilogue stores
 // its accumulators (after norm and rotation) without any lane movement, and so do the row-major and the V epilogues.
 //
-// Work split.  Workgroup = 8 waves = 256 tokens x 256 features; wave (fh, tq) owns features fh*128..+127 (one
-// head) x tokens tq*64..+63 (one K/V tile): 32 accumulators of 16x16.  Per 32-wide k-chunk a wave reads 8 weight
-// and 4 activation images for 32 MFMAs.  LoRA is a second K segment: k-chunks beyond the hidden size take their
-// activation images from the down-projected rows (x A^T, scaled) and their weight images from B.
+// Work split.  Workgroup = 4 waves, one per SIMD = 256 features x 256, 128 or 64 tokens; wave (fh, th) owns features
+// fh*128..+127 (one head) x half of the tokens (TB = 8, 4 or 2 blocks of 16).  What bounds it: with eight waves of
+// 128 x 64 each the LDS traffic of a 32-wide k-chunk (96 KiB read, 32 KiB written) took every cycle of its MFMAs; four
+// waves of 128 x 128 read 64 KiB, whose accumulators (256 registers a lane) live in the accumulator half of the register
+// file.  LoRA is a second K segment: k-chunks beyond the hidden size take their activation images from the
+// down-projected rows (x A^T, scaled) and their weight images from B.
 #include <type_traits>
 
 #include "pkh3_common.h"
@@ -29,310 +31,431 @@
 
 namespace pkh3 {
 
-constexpr int kGemmWaves = 8;
-constexpr int kGemmTile = 256;                      // tokens and features per workgroup
-constexpr int kGemmChunkK = 32;                     // contraction elements per ring slot = one k-step
-constexpr int kGemmStageBytes = 2 * kGemmTile * kGemmChunkK * 2;  // weight part + activation part
-constexpr int kGemmRing = 4;
+constexpr int kGemmWaves = 4;                       // two 128-feature heads x two token halves
+constexpr int kGemmFeatures = 256;                  // features per workgroup
+constexpr int kGemmRing = 3;                        // ring slots: one 32-wide k-chunk of weight and activation images each
+constexpr int kGemmWPieces = kGemmFeatures / 16;    // 1 KiB weight images of a chunk
 
-__device__ __forceinline__ void gemm_dma16(const char* g, unsigned lane_off, char* l) {
-  // see lds_dma16 in pkh3_attn_fwd.hip: wave-uniform base addresses, per-lane byte offset, tracked by vmcnt
-  const unsigned lds_addr = (unsigned)(size_t)(__attribute__((address_space(3))) char*)l;
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               :
-               : "v"(lane_off), "s"(g), "s"(lds_addr)
-               : "memory", "m0");
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<N, I + 1>(f);
+  }
 }
 
-template <int EPI>
-__device__ __forceinline__ void gemm_tile(const GemmParams& p, const GemmTarget& tg, int m_tile, int n_tile_in_target,
-                                          char* lds_raw) {
-  constexpr int WAVES = kGemmWaves;
-  constexpr int PP = 32 / WAVES;                     // 1 KiB pieces of a chunk each wave copies
+// The two halves of a direct-to-LDS copy (see lds_dma16 in pkh3_attn_fwd.hip: wave-uniform base address, per-lane byte
+// offset, tracked by vmcnt): where the next one goes, and the copy.  `lanes`: all or none -- past the last chunk
+// the copies are still issued, so that the waits count the same, but move nothing.
+__device__ __forceinline__ void dma_to(unsigned lds_addr) { asm volatile("s_mov_b32 m0, %0" ::"s"(lds_addr) : "m0"); }
+__device__ __forceinline__ void dma_from(const char* g, unsigned lane_off, unsigned long long lanes) {
+  asm volatile("s_mov_b64 exec, %2\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1"
+               :
+               : "v"(lane_off), "s"(g), "s"(lanes)
+               : "memory");
+}
+// One 1 KiB image from LDS.  As an instruction of its own so that it stays between the MFMAs it is written between; the
+// wait for it is the one at the top of the next chunk.
+template <int OFF>
+__device__ __forceinline__ void lds_image(bf16x8& v, unsigned addr) {
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
+}
+
+// c += a b.  Written as an instruction because the compiler, left to place 256 accumulator registers itself, moves them
+// between the two halves of the register file inside the loop (456 moves per 128 MFMAs).  AGPR: the accumulators fill the
+// accumulator half (TB = 8); the smaller forms keep them in the vector half, where the epilogue reads them in place.
+template <bool AGPR>
+__device__ __forceinline__ void mfma_acc(f32x4& c, const bf16x8& a, const bf16x8& b) {
+  if constexpr (AGPR) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+  else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+}
+
+// A 16-token block's accumulators in vector registers.  From the accumulator half by instructions that stay where they are
+// written: the compiler would move all blocks first and spill.
+template <bool AGPR>
+__device__ __forceinline__ float acc_value(float a) {
+  if constexpr (!AGPR) return a;
+  float v;
+  asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(a));
+  return v;
+}
+template <bool AGPR>
+__device__ __forceinline__ void acc_block(float (&x)[32], const f32x4 (&a)[8]) {
+  static_for<8>([&](auto fc) {
+    constexpr int fb = decltype(fc)::value;
+    const f32x4 q = a[fb];
+    x[4 * fb] = acc_value<AGPR>(q[0]), x[4 * fb + 1] = acc_value<AGPR>(q[1]);
+    x[4 * fb + 2] = acc_value<AGPR>(q[2]), x[4 * fb + 3] = acc_value<AGPR>(q[3]);
+  });
+}
+
+// Main loop: acc[t][fb] = the wave's 16-token block t x 16-feature block fb.  SWAP: tokens down the registers (V images).
+template <int TB, bool SWAP>
+__device__ __forceinline__ void gemm_loop(const GemmParams& p, const GemmTarget& tg, int m_tile, int n_tile_in_target, bool head_live,
+                                          char* lds_raw, f32x4 (&acc)[TB][8]) {
+  constexpr int kStage = (kGemmWPieces + 2 * TB) * 1024;
+  constexpr int kXPieces = TB / 2;                   // activation pieces of a chunk each wave copies (and 4 weight pieces)
+  constexpr int PP = 4 + kXPieces;
+  constexpr int R = kGemmRing;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int g = lane >> 4, c = lane & 15;
-  const int fh = wave & 1, tq = wave >> 1;           // feature half (one head), 64-token slice
-  const int head = n_tile_in_target * 2 + fh;        // 128-feature head inside the target
-  const bool head_live = head * 128 < tg.n;
-  const int nk1 = p.nk1, nk = p.nk1 + tg.nk2;
-  const unsigned lane_off = lane * 16;
+  const int fh = wave & 1, th = wave >> 1;
+  const int nk1 = p.nk1, nk = __builtin_amdgcn_readfirstlane(p.nk1 + tg.nk2);
 
-  // this wave's 1 KiB pieces of every chunk: pieces PP*wave.. of [16 weight blocks | 16 token blocks]
-  const int piece0 = wave * PP;
-  const bool w_side = piece0 < 16;
-  const int blk0 = piece0 & 15;                      // first of the 16-row blocks this wave copies
-  const char* seg1 = w_side ? tg.w_img + (int64_t)(n_tile_in_target * 16 + blk0) * tg.w_blk_stride
-                            : p.a_img + (int64_t)(m_tile * 16 + blk0) * p.a_blk_stride;
-  const int64_t seg1_step = w_side ? tg.w_blk_stride : p.a_blk_stride;
-  const char* seg2 = w_side ? tg.w2_img + (int64_t)(n_tile_in_target * 16 + blk0) * tg.w2_blk_stride
-                            : tg.a2_img + (int64_t)(m_tile * 16 + blk0) * tg.a2_blk_stride;
-  const int64_t seg2_step = w_side ? tg.w2_blk_stride : tg.a2_blk_stride;
-  // this wave's copies of one chunk: the chunk's image of PP consecutive blocks, `step` bytes apart, into ring slot `slot`
-  auto dma_from = [&](const char* gp, int64_t step, int slot) {
-    char* d = lds_raw + slot * kGemmStageBytes + piece0 * 1024;
+  // sources of this wave's pieces of the next chunk to copy: running pointers inside the current K segment, per-lane
+  // offsets of the pieces behind them (consecutive 16-row blocks)
+  const char* w_next = tg.w_img + (int64_t)(n_tile_in_target * kGemmWPieces + wave * 4) * tg.w_blk_stride;
+  const char* x_next = p.a_img + (int64_t)(m_tile * 2 * TB + wave * kXPieces) * p.a_blk_stride;
+  unsigned w_off[4], x_off[kXPieces];
 #pragma unroll
-    for (int b = 0; b < PP; ++b) gemm_dma16(gp + b * step, lane_off, d + b * 1024);
+  for (int i = 0; i < 4; ++i) w_off[i] = lane * 16 + i * (unsigned)tg.w_blk_stride;
+#pragma unroll
+  for (int i = 0; i < kXPieces; ++i) x_off[i] = lane * 16 + i * (unsigned)p.a_blk_stride;
+  int left = nk1;                                    // chunks not yet copied of the segment the pointers walk
+  const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) char*)lds_raw;
+  unsigned long long lanes = ~0ull;                  // all lanes while chunks are left, then none
+  int total_left = nk;
+  // this wave's piece I of the next chunk, into ring slot `slot`; the last piece moves on to the chunk after it
+  auto piece_to = [&](auto ic, int slot) {
+    constexpr int i = decltype(ic)::value;
+    dma_to(lds0 + slot * kStage + (i < 4 ? wave * 4 + i : kGemmWPieces + wave * kXPieces + i - 4) * 1024);
   };
-  auto dma = [&](int kc, int slot) {
-    const bool first = kc < nk1;
-    dma_from(first ? seg1 + (int64_t)kc * 1024 : seg2 + (int64_t)(kc - nk1) * 1024, first ? seg1_step : seg2_step, slot);
-  };
-  // waits until at most `chunks` of this wave's newest chunk copies are still in flight
-  auto wait_dma = [&](int chunks) {
-    if (chunks >= 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PP) : "memory");
-    else if (chunks == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PP) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  };
-
-  f32x4 acc[4][8];                                   // (16-token block of the wave's 64, 16-feature block of the head)
+  auto piece_from = [&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    if constexpr (i < 4) dma_from(w_next, w_off[i], lanes);
+    else dma_from(x_next, x_off[i - 4], lanes);
+    if constexpr (i == PP - 1) {
+      w_next += 1024;
+      x_next += 1024;
+      --total_left;
+      asm volatile("s_cmp_gt_i32 %1, 0\n\ts_cselect_b64 %0, -1, 0" : "=s"(lanes) : "s"(total_left) : "scc");
+      if (--left == 0) {                             // on to the second segment (past the end: not read any more)
+        w_next = tg.w2_img + (int64_t)(n_tile_in_target * kGemmWPieces + wave * 4) * tg.w2_blk_stride;
+        x_next = tg.a2_img + (int64_t)(m_tile * 2 * TB + wave * kXPieces) * tg.a2_blk_stride;
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
+        for (int j = 0; j < 4; ++j) w_off[j] = lane * 16 + j * (unsigned)tg.w2_blk_stride;
 #pragma unroll
-    for (int fb = 0; fb < 8; ++fb) acc[t][fb] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  // Ring of four chunks.  Entering iteration kc: chunk kc is in LDS for every wave and its token images and first four
-  // weight images are already on their way to this wave's registers; chunks kc+1 and kc+2 are in flight.  The barrier at
-  // the top makes chunk kc+1 visible and frees the slot of chunk kc-1 for chunk kc+3, so the first images of the next
-  // chunk can be read at the tail of this iteration and no wave starts a chunk by waiting for LDS.
-  const int n_pre = nk < 3 ? nk : 3;
-  for (int cc = 0; cc < n_pre; ++cc) dma(cc, cc);
-  wait_dma(n_pre - 1);
-  __syncthreads();
-  const int w_off = (fh * 8) * 1024 + lane * 16;            // weight blocks fh*8..+7 of a slot
-  const int a_off = 16384 + (tq * 4) * 1024 + lane * 16;    // this wave's token blocks
-  bf16x8 wa[4], wb[4], xc[4], xn[4];                        // weight blocks 0..3 / 4..7, token images of this / the next chunk
-  auto read_w = [&](int slot, int half, bf16x8 (&w4)[4]) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) w4[i] = *(const bf16x8*)(lds_raw + slot * kGemmStageBytes + w_off + (half * 4 + i) * 1024);
-  };
-  auto read_x = [&](int slot, bf16x8 (&x4)[4]) {
-#pragma unroll
-    for (int t = 0; t < 4; ++t) x4[t] = *(const bf16x8*)(lds_raw + slot * kGemmStageBytes + a_off + t * 1024);
-  };
-  auto mfmas = [&](int half, const bf16x8 (&w4)[4], const bf16x8 (&x4)[4]) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        if constexpr (EPI == kEpiVImg) acc[t][half * 4 + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x4[t], w4[i], acc[t][half * 4 + i], 0, 0, 0);
-        else acc[t][half * 4 + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w4[i], x4[t], acc[t][half * 4 + i], 0, 0, 0);
-      }
-  };
-  if (head_live) {
-    read_x(0, xc);
-    read_w(0, 0, wa);
-  }
-  int slot = 0;
-  // source of the next chunk to copy (chunk kc + 3 in the steady loop): a running pointer inside its K segment
-  const char* g_next = nullptr;
-  int64_t step_next = seg1_step;
-  int left_next = 0;  // chunks left in the segment g_next walks, this one included
-  if (nk > 3) {
-    const bool first = 3 < nk1;
-    g_next = first ? seg1 + 3 * 1024 : seg2 + (int64_t)(3 - nk1) * 1024;
-    step_next = first ? seg1_step : seg2_step;
-    left_next = first ? nk1 - 3 : nk - 3;
-  }
-  // One chunk.  MORE1/2/3: chunks kc+1 / kc+2 / kc+3 exist (compile-time, so the steady loop carries no tests).
-  auto chunk = [&](auto more1, auto more2, auto more3) {
-    if constexpr (more1()) {
-      // chunk kc+1 has landed (this wave's pieces; the barrier covers the others'); only chunk kc+2's copies may be pending
-      if constexpr (more2()) wait_dma(1);
-      else wait_dma(0);
-      __syncthreads();
-    }
-    const int next = (slot + 1) & 3;
-    if (head_live) {  // wave-uniform: a head past the end of the target only copies and synchronises
-      read_w(slot, 1, wb);
-      mfmas(0, wa, xc);
-    }
-    // the copies of chunk kc+3 are issued under the first half's MFMAs, not in front of them: their address
-    // arithmetic is a scalar chain every wave of the workgroup would otherwise run at the same time, right after
-    // the barrier, with the MFMA pipe idle
-    __builtin_amdgcn_sched_barrier(0);
-    if constexpr (more3()) {
-      dma_from(g_next, step_next, (slot + 3) & 3);
-      g_next += 1024;
-      if (--left_next == 0) {
-        g_next = seg2;
-        step_next = seg2_step;
+        for (int j = 0; j < kXPieces; ++j) x_off[j] = lane * 16 + j * (unsigned)tg.a2_blk_stride;
       }
     }
-    __builtin_amdgcn_sched_barrier(0);
-    if (head_live) {
-      if constexpr (more1()) {
-        read_x(next, xn);
-        read_w(next, 0, wa);
-      }
-      mfmas(1, wb, xc);
-      if constexpr (more1()) {
-#pragma unroll
-        for (int t = 0; t < 4; ++t) xc[t] = xn[t];
-      }
-    }
-    slot = next;
   };
-  constexpr std::true_type yes{};
-  constexpr std::false_type no{};
-  int kc = 0;
-  for (; kc + 3 < nk; ++kc) chunk(yes, yes, yes);
-  if (kc + 2 < nk) { chunk(yes, yes, no); ++kc; }
-  if (kc + 1 < nk) { chunk(yes, no, no); ++kc; }
-  chunk(no, no, no);
-  // let the last MFMA retire before anything the compiler places after the loop reads the accumulators
-#pragma unroll
-  for (int t = 0; t < 4; ++t)
-    asm volatile("s_nop 15\n\ts_nop 15"
-                 : "+v"(acc[t][0]), "+v"(acc[t][1]), "+v"(acc[t][2]), "+v"(acc[t][3]), "+v"(acc[t][4]), "+v"(acc[t][5]),
-                   "+v"(acc[t][6]), "+v"(acc[t][7])::"memory");
-  if (!head_live) return;
+  auto copy_chunk = [&](int slot) {
+    static_for<PP>([&](auto ic) {
+      piece_to(ic, slot);
+      asm volatile("s_nop 0");
+      piece_from(ic);
+    });
+  };
 
-  const float* bias = tg.bias ? tg.bias + head * 128 : nullptr;
-  const int tok0 = m_tile * kGemmTile + tq * 64;     // the wave's 64 tokens: one K/V tile
-  const int tile = m_tile * 4 + tq;
-  if (tok0 >= p.M) return;                           // a tile past the last token: nothing to write
-
-  if constexpr (EPI == kEpiVImg) {
-    // lane (g, c) = feature 16*fb + c of the head, registers = tokens 4*g + i of a 16-token block: the V image
-    // (half, db = fb) wants, in that same lane, the tokens 16*(j/4) + 4*g + j%4 of its 32: blocks 2*half and 2*half + 1
-    char* rec = tg.out + (int64_t)head * tg.out_head_stride + (int64_t)tile * tg.out_blk_stride;
-#pragma unroll
-    for (int half = 0; half < 2; ++half)
-#pragma unroll
-      for (int fb = 0; fb < 8; ++fb) {
-        const float bv = bias ? bias[16 * fb + c] : 0.f;
-        bf16x8 img;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int token = tok0 + 32 * half + v_image_key(g, j);
-          img[j] = token < p.M ? (__bf16)(acc[2 * half + (j >> 2)][fb][j & 3] + bv) : (__bf16)0.0f;
-        }
-        *(bf16x8*)(rec + ((half * 8 + fb) * 64 + lane) * 16) = img;
-      }
-  } else {
-    // lane (g, c) = token 16*t + c; its accumulators (t, fb) are elements 32*ks + 8*g + j of the head row with
-    // fb = 2*ks + j/4, i = j%4 (the weight-row permutation, see pack_rows_kernel): x[8*ks + j]
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int token = tok0 + 16 * t + c;
-      const bool valid = token < p.M;
-      float x[32];
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) x[ks * 8 + j] = valid ? acc[t][2 * ks + (j >> 2)][j & 3] * tg.out_scale : 0.f;
-      if (bias) {
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-          const f32x4 b0 = *(const f32x4*)(bias + 32 * ks + 8 * g), b1 = *(const f32x4*)(bias + 32 * ks + 8 * g + 4);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            x[ks * 8 + j] += valid ? b0[j] : 0.f;
-            x[ks * 8 + 4 + j] += valid ? b1[j] : 0.f;
-          }
-        }
-      }
-      if constexpr (EPI == kEpiKImg) {
-        const RowTransform tf{tg.norm_w, tg.norm_eps, tg.rope_mode, tg.cos_t, tg.sin_t};
-        norm_rope_quarter(x, tf, valid ? token : 0, valid, g);
-        // kept for the tile-wide reductions below
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-          for (int j = 0; j < 8; ++j) acc[t][2 * ks + (j >> 2)][j & 3] = x[ks * 8 + j];
-      } else if constexpr (EPI == kEpiAImg) {
-        // operand images of these GEMMs: [16-token block][k-step], this lane's piece ks at its own place in image ks
-        char* rec = tg.out + (int64_t)head * tg.out_head_stride + (int64_t)(m_tile * 16 + tq * 4 + t) * tg.out_blk_stride;
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-          bf16x8 v;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) v[j] = (__bf16)x[ks * 8 + j];
-          *(bf16x8*)(rec + (ks * 64 + lane) * 16) = v;
-        }
+  // the bias is what the sums start from (launches with a bias have out_scale 1)
+  static_for<8>([&](auto fc) {
+    constexpr int fb = decltype(fc)::value;
+    f32x4 start = {0.f, 0.f, 0.f, 0.f};
+    if (tg.bias && head_live) {
+      const float* bias = tg.bias + (n_tile_in_target * 2 + fh) * 128;
+      const int g = lane >> 4, c = lane & 15;
+      if constexpr (SWAP) {
+        const float b = bias[16 * fb + c];
+        start = f32x4{b, b, b, b};
       } else {
-        // row-major bf16 rows: y = residual + gate[row_index] * (acc*scale + bias); 16-byte pieces per lane
-        if (!valid) continue;
-        __bf16* orow = (__bf16*)tg.out + (int64_t)token * tg.out_row_stride + (int64_t)head * tg.out_head_elems;
-        const __bf16* res = tg.residual ? (const __bf16*)tg.residual + (int64_t)token * tg.res_row_stride + head * 128 : nullptr;
-        const __bf16* gate = tg.gate ? (const __bf16*)tg.gate + (int64_t)(tg.row_index ? tg.row_index[token] : 0) * tg.gate_row_stride + head * 128
-                                     : nullptr;
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-          const int d0 = 32 * ks + 8 * g;
-          bf16x8 o, gv, rv;
-          if (gate) gv = *(const bf16x8*)(gate + d0);
-          if (res) rv = *(const bf16x8*)(res + d0);
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            float v = x[ks * 8 + j];
-            if (gate) v *= (float)gv[j];
-            if (res) v += (float)rv[j];
-            o[j] = (__bf16)v;
-          }
-          *(bf16x8*)(orow + d0) = o;
-        }
+        start = *(const f32x4*)(bias + 32 * (fb >> 1) + 8 * g + 4 * (fb & 1));
       }
     }
-    if constexpr (EPI == kEpiKImg) {
-      // the wave's 64 tokens are one K tile: largest row norm, fp8 scale, then every piece at its place in the tile
-      float nmax = 0.f, amax = 0.f;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        float ssq = 0.f;
-#pragma unroll
-        for (int fb = 0; fb < 8; ++fb)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            ssq += acc[t][fb][i] * acc[t][fb][i];
-            amax = fmaxf(amax, fabsf(acc[t][fb][i]));
-          }
-        nmax = fmaxf(nmax, wave_sum_groups(ssq));
+    static_for<TB>([&](auto tc) { acc[decltype(tc)::value][fb] = start; });
+  });
+
+  bf16x8 wa[8], wb[8], xa[TB], xb[TB];               // operand images of this and of the next chunk, in turn
+  const unsigned w_lds = lds0 + lane * 16 + fh * 8 * 1024, x_lds = lds0 + lane * 16 + (kGemmWPieces + th * TB) * 1024;
+  constexpr int kReads = 8 + TB;
+  auto read_image = [&](auto ic, unsigned w_at, unsigned x_at, bf16x8 (&w)[8], bf16x8 (&x)[TB]) {
+    constexpr int i = decltype(ic)::value;
+    if constexpr (i < TB) lds_image<i * 1024>(x[i], x_at);
+    else lds_image<(i - TB) * 1024>(w[i - TB], w_at);
+  };
+  // One chunk: the MFMAs on w, x with, between them, the reads of the next chunk's images (w2, x2) and the copies of the
+  // chunk R ahead, which goes into the slot this chunk came from (its images are in every wave's registers).  A wave is
+  // alone on its SIMD, so the pipe idles whenever something else takes longer to issue than the 12 cycles an MFMA leaves
+  // free: at most one such instruction follows an MFMA.  15,342 tokens x 9,216 features, K 3,072: everything at the head
+  // of the chunk 1.18 PFLOP/s, three or four at the head of each feature block 1.40, one at a time 1.51.
+  auto chunk = [&](int read_slot, int dma_slot, bf16x8 (&w)[8], bf16x8 (&x)[TB], bf16x8 (&w2)[8], bf16x8 (&x2)[TB]) {
+    const unsigned w_at = w_lds + read_slot * kStage, x_at = x_lds + read_slot * kStage;
+    constexpr int kEvery = TB > 4 ? 8 : 4;           // MFMAs from copy to copy
+    // this wave's pieces of the next chunk have landed, and so have the images it read for this one
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((R - 2) * PP) : "memory");
+    __builtin_amdgcn_s_barrier();
+    static_for<8 * TB>([&](auto kc) {
+      constexpr int k = decltype(kc)::value, fb = k / TB, t = k % TB;
+      if constexpr (SWAP) mfma_acc<TB == 8>(acc[t][fb], x[t], w[fb]);
+      else mfma_acc<TB == 8>(acc[t][fb], w[fb], x[t]);
+      if constexpr (TB > 2) {
+        // reads after MFMAs 0, 2, 4 ..; a copy's target after 1 + i*kEvery, the copy itself two later
+        static_assert(2 * kReads <= 8 * TB && kEvery * (PP - 1) + 3 < 8 * TB, "all of them fit between the MFMAs");
+        if constexpr (k % 2 == 0 && k / 2 < kReads) read_image(std::integral_constant<int, k / 2>{}, w_at, x_at, w2, x2);
+        if constexpr (k % kEvery == 1 && k / kEvery < PP) piece_to(std::integral_constant<int, k / kEvery>{}, dma_slot);
+        if constexpr (k % kEvery == 3 && k / kEvery < PP) piece_from(std::integral_constant<int, k / kEvery>{});
+      } else {
+        static_assert(kReads + PP <= 16, "all of them fit between the MFMAs");
+        if constexpr (k < kReads) {
+          read_image(std::integral_constant<int, k>{}, w_at, x_at, w2, x2);
+        } else if constexpr (k - kReads < PP) {
+          piece_to(std::integral_constant<int, k - kReads>{}, dma_slot);
+          piece_from(std::integral_constant<int, k - kReads>{});
+        }
       }
-      if (tg.norm_max) {
-        nmax = sqrtf(wave_max(nmax));
-        if (lane == 0) raise_max(tg.norm_max + head, nmax);
-      }
-      char* rec = tg.out + (int64_t)head * tg.out_head_stride + (int64_t)tile * tg.out_blk_stride;
-      if (!tg.fp8) {
-        // K tile image (half, ks, kb2) of 16-token block t = 2*half + kb2: this lane's piece ks at its own place
+    });
+  };
+  auto next = [](int slot) { return slot == R - 1 ? 0 : slot + 1; };
+
+  // Ring: entering chunk kc, its images are in this wave's registers and chunks kc+1 .. kc+R-1 are on their way to LDS.
+  // The barrier at its top makes chunk kc+1 visible (each wave has waited for its own pieces) and tells that every wave
+  // holds chunk kc in registers, so its slot can be refilled.
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
+  for (int i = 0; i < R; ++i) copy_chunk(i);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((R - 1) * PP) : "memory");
+  __syncthreads();
+  int slot = 0, kc = 0;
+  if (!head_live) {
+    // a head past the end of the target: this wave only copies and synchronises
+    for (; kc < nk; ++kc) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((R - 2) * PP) : "memory");
+      __builtin_amdgcn_s_barrier();
+      copy_chunk(slot);
+      slot = next(slot);
+    }
+    return;
+  }
+  static_for<kReads>([&](auto ic) { read_image(ic, w_lds, x_lds, wa, xa); });
+  for (; kc + 2 <= nk; kc += 2) {
+    const int s1 = next(slot), s2 = next(s1);
+    chunk(s1, slot, wa, xa, wb, xb);
+    chunk(s2, s1, wb, xb, wa, xa);
+    slot = s2;
+  }
+  if (kc < nk) chunk(next(slot), slot, wa, xa, wb, xb);
+  // the compiler does not know the instructions above for MFMAs: let the last one retire before anything reads the accumulators
+  static_for<TB>([&](auto tc) {
+    f32x4(&a)[8] = acc[decltype(tc)::value];
+    if constexpr (TB == 8)
+      asm volatile("s_nop 15\n\ts_nop 15"
+                   : "+a"(a[0]), "+a"(a[1]), "+a"(a[2]), "+a"(a[3]), "+a"(a[4]), "+a"(a[5]),
+                     "+a"(a[6]), "+a"(a[7])::"memory");
+    else
+      asm volatile("s_nop 15\n\ts_nop 15"
+                   : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]),
+                     "+v"(a[6]), "+v"(a[7])::"memory");
+  });
+}
+
+// Lane (g, c) = feature 16*fb + c of the head, registers = tokens 4*g + i of a 16-token block: the V image (half, db = fb)
+// wants, in that same lane, the tokens 16*(j/4) + 4*g + j%4 of its 32: blocks 2*half and 2*half + 1.
+template <int TB>
+__device__ __forceinline__ void epilogue_v(const GemmParams& p, const GemmTarget& tg, int head, int tok0, const f32x4 (&acc)[TB][8]) {
+  const int lane = threadIdx.x & 63, g = lane >> 4;
+  static_for<TB / 2>([&](auto tc) {
+    constexpr int t2 = decltype(tc)::value;
+    const int tok = tok0 + 32 * t2;
+    if ((tok & ~63) >= p.M) return;                  // a tile past the last token has no record
+    char* rec = tg.out + (int64_t)head * tg.out_head_stride + (int64_t)(tok >> 6) * tg.out_blk_stride + ((tok >> 5) & 1) * 8192;
+    float x[2][32];
+    acc_block<TB == 8>(x[0], acc[2 * t2]);
+    acc_block<TB == 8>(x[1], acc[2 * t2 + 1]);
+    bool live[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) live[j] = tok + v_image_key(g, j) < p.M;
+#pragma unroll
+    for (int fb = 0; fb < 8; ++fb) {
+      bf16x8 img;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) img[j] = live[j] ? (__bf16)x[j >> 2][4 * fb + (j & 3)] : (__bf16)0.0f;
+      *(bf16x8*)(rec + (fb * 64 + lane) * 16) = img;
+    }
+  });
+}
+
+// In the other orientation lane (g, c) = token 16*t + c; its accumulators (t, fb) are elements 32*ks + 8*g + j of the head
+// row with fb = 2*ks + j/4, i = j%4 (the weight-row permutation, see pack_rows_kernel), so acc_block() leaves piece ks of
+// the row in x[8*ks .. 8*ks + 7].
+
+// K tiles of the attention kernel: norm, rotation, largest row norm, (fp8) one scale per 64-token tile.  With fp8 the rows
+// are formed twice, before and after the tile's scale is known: they do not fit the registers beside the accumulators.
+template <int TB, int ROPE>
+__device__ __forceinline__ void epilogue_k(const GemmParams& p, const GemmTarget& tg, int head, bool head_live, int tok0,
+                                           const f32x4 (&acc)[TB][8]) {
+  constexpr int kTilesHere = TB >= 4 ? TB / 4 : 1;   // 64-token tiles of this wave (TB == 2: half a tile)
+  constexpr int kTBlk = TB >= 4 ? 4 : 2;             // 16-token blocks of each
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+  const int wave = threadIdx.x >> 6;
+  const RowTransform tf{tg.norm_w, tg.norm_eps, ROPE, tg.cos_t, tg.sin_t};
+  const bool full = tok0 + 16 * TB <= p.M;           // (wave-uniform) no row of this wave lies past the end
+  NormQuarter norm;
+  // tables of the next blocks to form, asked for one or two blocks ahead (what the registers allow): one after the other,
+  // every block would wait for a trip to memory
+  constexpr int kAhead = TB == 4 ? 1 : 2;
+  RopeQuarter rope[kAhead];
+  auto fetch_rope = [&](int t, RopeQuarter& r) {
+    if constexpr (ROPE != 0) load_rope_quarter(r, tf, min(tok0 + 16 * t + c, p.M - 1), g);
+  };
+  auto form_row = [&](float (&x)[32], auto tc, int t_next) {   // t_next: block kAhead later in the order they are formed in
+    constexpr int t = decltype(tc)::value;
+    acc_block<TB == 8>(x, acc[t]);
+    if (!full) {
+      const bool valid = tok0 + 16 * t + c < p.M;
+#pragma unroll
+      for (int i = 0; i < 32; ++i) x[i] = valid ? x[i] : 0.f;   // zero through norm and rotation as well
+    }
+    norm_rope_quarter(x, tf, norm, rope[t % kAhead], true, g);
+    fetch_rope(t_next, rope[t % kAhead]);
+  };
+  if (tf.norm_w) load_norm_quarter(norm, tf, g);
+#pragma unroll
+  for (int i = 0; i < kAhead; ++i) fetch_rope(i, rope[i]);
+  static_for<kTilesHere>([&](auto hc) {
+    constexpr int half = decltype(hc)::value;
+    const int tile0 = tok0 + 64 * half;
+    const bool live = head_live && (tile0 & ~63) < p.M;   // (wave-uniform) a tile past the last token has no record
+    char* rec = tg.out + (int64_t)head * tg.out_head_stride + (int64_t)(tile0 >> 6) * tg.out_blk_stride;
+    constexpr int t0 = half * kTBlk;                 // its first 16-token block in the wave ...
+    const int tb0 = (tile0 & 63) >> 4;               // ... and in the tile
+    float nmax = 0.f, amax = 0.f;
+    if (live) {
+      static_for<kTBlk>([&](auto tc) {
+        constexpr int tt = decltype(tc)::value;
+        float x[32];
+        const int again = t0 + (tt + kAhead) % kTBlk;   // with fp8 the tile's blocks come a second time
+        form_row(x, std::integral_constant<int, t0 + tt>{}, tt + kAhead >= kTBlk && tg.fp8 ? again : min(t0 + tt + kAhead, TB - 1));
+        float ssq[4] = {0.f, 0.f, 0.f, 0.f};         // four running sums: one would be a chain of dependent instructions
+        if (!tg.fp8) {
+          // K tile image (half, ks, kb2) of 16-token block tb = 2*half + kb2: this lane's piece ks at its own place
+          const int tb = tb0 + tt;
 #pragma unroll
           for (int ks = 0; ks < 4; ++ks) {
             bf16x8 v;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = (__bf16)acc[t][2 * ks + (j >> 2)][j & 3];
-            *(bf16x8*)(rec + ((((t >> 1) * 4 + ks) * 2 + (t & 1)) * 64 + lane) * 16) = v;
+            for (int j = 0; j < 8; ++j) v[j] = (__bf16)x[ks * 8 + j];
+            // the row norm of the rounded values, two at a time
+#pragma unroll
+            for (int j = 0; j < 8; j += 2) ssq[j / 2] = __builtin_amdgcn_fdot2_f32_bf16(bf16x2{v[j], v[j + 1]}, bf16x2{v[j], v[j + 1]}, ssq[j / 2], false);
+            *(bf16x8*)(rec + ((((tb >> 1) * 4 + ks) * 2 + (tb & 1)) * 64 + lane) * 16) = v;
           }
-      } else {
-        amax = wave_max(amax);
-        const float scale = fp8_block_scale(amax, tg.fp8_pow2 != 0);
-        const float inv = 1.0f / scale;
-        if (lane == 0) tg.scale_out[(int64_t)head * tg.scale_head_stride + tile] = scale;
-        // fp8 K tile: key block t is 2 KiB, chunk c2 of a lane holds its pieces ks = 2*c2 and 2*c2 + 1
+        } else {
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
+          for (int i = 0; i < 32; ++i) ssq[i & 3] += x[i] * x[i];
 #pragma unroll
-          for (int c2 = 0; c2 < 2; ++c2) {
-            float lo[8], hi[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-              lo[j] = acc[t][4 * c2 + (j >> 2)][j & 3];
-              hi[j] = acc[t][4 * c2 + 2 + (j >> 2)][j & 3];
-            }
-            const i32x2 q0 = quant_fp8_piece(lo, inv), q1 = quant_fp8_piece(hi, inv);
-            *(i32x4*)(rec + ((t * 2 + c2) * 64 + lane) * 16) = i32x4{q0[0], q0[1], q1[0], q1[1]};
-          }
+          for (int i = 0; i < 32; ++i) amax = fmaxf(amax, fabsf(x[i]));
+          asm volatile("" : "+v"(amax));   // here, not where it is used: the rows of all blocks would have to live until then
+        }
+        nmax = fmaxf(nmax, wave_sum_groups((ssq[0] + ssq[1]) + (ssq[2] + ssq[3])));
+      });
+      if (tg.norm_max) {
+        nmax = sqrtf(wave_max(nmax));
+        if (lane == 0) raise_max(tg.norm_max + head, nmax);
       }
     }
-  }
+    if (!tg.fp8) return;
+    amax = wave_max(amax);
+    if constexpr (TB == 2) {
+      // two waves hold half a tile each: the scale is that of the larger of their magnitudes
+      __shared__ float half_amax[kGemmWaves];
+      if (lane == 0) half_amax[wave] = amax;
+      __syncthreads();
+      amax = fmaxf(amax, half_amax[wave ^ 2]);
+    }
+    if (!live) return;
+    const float scale = fp8_block_scale(amax, tg.fp8_pow2 != 0);
+    const float inv = 1.0f / scale;
+    if (lane == 0 && tb0 == 0) tg.scale_out[(int64_t)head * tg.scale_head_stride + (tile0 >> 6)] = scale;
+    // fp8 K tile: key block tb is 2 KiB, chunk c2 of a lane holds its pieces ks = 2*c2 and 2*c2 + 1
+    static_for<kTBlk>([&](auto tc) {
+      constexpr int tt = decltype(tc)::value;
+      float x[32];
+      form_row(x, std::integral_constant<int, t0 + tt>{}, min(t0 + tt + kAhead, TB - 1));
+#pragma unroll
+      for (int c2 = 0; c2 < 2; ++c2) {
+        const i32x2 q0 = quant_fp8_piece(x + 16 * c2, inv), q1 = quant_fp8_piece(x + 16 * c2 + 8, inv);
+        *(i32x4*)(rec + (((tb0 + tt) * 2 + c2) * 64 + lane) * 16) = i32x4{q0[0], q0[1], q1[0], q1[1]};
+      }
+    });
+  });
 }
 
-template <int WAVES>
-__global__ __launch_bounds__(64 * WAVES, 1) void gemm_kernel(GemmParams p) {
-  __shared__ __attribute__((aligned(1024))) char lds_raw[kGemmRing * kGemmStageBytes];
+// operand images of these GEMMs: [16-token block][k-step], this lane's piece ks at its own place in image ks
+template <int TB>
+__device__ __forceinline__ void epilogue_a(const GemmParams& p, const GemmTarget& tg, int head, int tok0, const f32x4 (&acc)[TB][8]) {
+  const int lane = threadIdx.x & 63, c = lane & 15;
+  static_for<TB>([&](auto tc) {
+    constexpr int t = decltype(tc)::value;
+    const int blk = tok0 + 16 * t;
+    float x[32];
+    acc_block<TB == 8>(x, acc[t]);
+    const float scale = blk + c < p.M ? tg.out_scale : 0.f;
+    char* rec = tg.out + (int64_t)head * tg.out_head_stride + (int64_t)(blk >> 4) * tg.out_blk_stride;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      bf16x8 v;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = (__bf16)(x[ks * 8 + j] * scale);
+      *(bf16x8*)(rec + (ks * 64 + lane) * 16) = v;
+    }
+  });
+}
+
+// row-major bf16 rows: y = residual + gate[row_index] * acc (the bias is in it); 16-byte pieces per lane.  The table rows
+// of all blocks are asked for first and the gate and residual pieces one or two blocks ahead (what the registers allow):
+// one after the other, each block would wait for two trips to memory.
+template <int TB, bool GATE, bool RES>
+__device__ __forceinline__ void epilogue_rows(const GemmParams& p, const GemmTarget& tg, int head, int tok0, const f32x4 (&acc)[TB][8]) {
+  constexpr int kAhead = TB == 4 ? 1 : 2;
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+  const int last = p.M - 1;                          // rows past the end read the last one and write nothing
+  int rows[(TB + 3) / 4];                            // table rows of the wave's tokens, 64 to a register
+  if constexpr (GATE) {
+#pragma unroll
+    for (int i = 0; i < (TB + 3) / 4; ++i) rows[i] = tg.row_index ? tg.row_index[min(tok0 + 64 * i + lane, last)] : 0;
+  }
+  struct Pieces { bf16x8 gate[4], res[4]; } even, odd;
+  auto fetch = [&](int t, Pieces& f) {
+    if constexpr (RES) {
+      const __bf16* res = (const __bf16*)tg.residual + (int64_t)min(tok0 + 16 * t + c, last) * tg.res_row_stride + head * 128 + 8 * g;
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) f.res[ks] = *(const bf16x8*)(res + 32 * ks);
+    }
+    if constexpr (GATE) {
+      const int row = __shfl(rows[t / 4], 16 * (t & 3) + c, 64);
+      const __bf16* gate = (const __bf16*)tg.gate + (int64_t)row * tg.gate_row_stride + head * 128 + 8 * g;
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) f.gate[ks] = *(const bf16x8*)(gate + 32 * ks);
+    }
+  };
+  auto block = [&](auto tc, Pieces& f) {
+    constexpr int t = decltype(tc)::value;
+    float x[32];
+    acc_block<TB == 8>(x, acc[t]);
+    const int token = tok0 + 16 * t + c;
+    bf16x8 o[4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        float v = x[ks * 8 + j];
+        if constexpr (GATE) v *= (float)f.gate[ks][j];
+        if constexpr (RES) v += (float)f.res[ks][j];
+        o[ks][j] = (__bf16)v;
+      }
+    if (t + kAhead < TB) fetch(t + kAhead, f);
+    __bf16* orow = (__bf16*)tg.out + (int64_t)token * tg.out_row_stride + (int64_t)head * tg.out_head_elems + 8 * g;
+    if (token < p.M) {
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) *(bf16x8*)(orow + 32 * ks) = o[ks];
+    }
+  };
+  fetch(0, even);
+  if constexpr (kAhead == 2) fetch(1, odd);
+  static_for<TB>([&](auto tc) { block(tc, kAhead == 2 && (decltype(tc)::value & 1) ? odd : even); });
+}
+
+template <int TB>
+__global__ __launch_bounds__(64 * kGemmWaves, TB == 8 ? 1 : 2) void gemm_kernel(GemmParams p) {
+  __shared__ __attribute__((aligned(1024))) char lds_raw[kGemmRing * (kGemmWPieces + 2 * TB) * 1024];
   // Workgroups go to the 8 XCDs round-robin; each XCD takes one contiguous run of the tile order below, in which 32
   // consecutive tiles (the workgroups the 32 CUs behind one L2 run together) form a block of 4 token tiles x 8
   // feature tiles: every activation panel is then shared by 8 and every weight panel by 4 of them.
@@ -364,20 +487,71 @@ __global__ __launch_bounds__(64 * WAVES, 1) void gemm_kernel(GemmParams p) {
   int t = 0;
   while (t + 1 < p.n_targets && n_tile >= p.tg[t].n_tiles) { n_tile -= p.tg[t].n_tiles; ++t; }
   const GemmTarget& tg = p.tg[t];
-  switch (tg.epi) {
-    case kEpiRows: gemm_tile<kEpiRows>(p, tg, m_tile, n_tile, lds_raw); break;
-    case kEpiKImg: gemm_tile<kEpiKImg>(p, tg, m_tile, n_tile, lds_raw); break;
-    case kEpiAImg: gemm_tile<kEpiAImg>(p, tg, m_tile, n_tile, lds_raw); break;
-    default: gemm_tile<kEpiVImg>(p, tg, m_tile, n_tile, lds_raw); break;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int head = n_tile * 2 + (wave & 1);             // 128-feature head inside the target
+  const bool head_live = head * 128 < tg.n;
+  const int tok0 = (m_tile * 2 + (wave >> 1)) * (16 * TB);   // first of the wave's tokens
+  f32x4 acc[TB][8];
+  if (tg.epi == kEpiVImg) {
+    gemm_loop<TB, true>(p, tg, m_tile, n_tile, head_live, lds_raw, acc);
+    if (head_live && tok0 < p.M) epilogue_v<TB>(p, tg, head, tok0, acc);
+    return;
   }
+  gemm_loop<TB, false>(p, tg, m_tile, n_tile, head_live, lds_raw, acc);
+  if (tg.epi == kEpiKImg) {
+    if (tg.rope_mode == 1) epilogue_k<TB, 1>(p, tg, head, head_live, tok0, acc);
+    else if (tg.rope_mode == 2) epilogue_k<TB, 2>(p, tg, head, head_live, tok0, acc);
+    else epilogue_k<TB, 0>(p, tg, head, head_live, tok0, acc);
+    return;
+  }
+  if (!head_live || tok0 >= p.M) return;
+  if (tg.epi == kEpiAImg) epilogue_a<TB>(p, tg, head, tok0, acc);
+  else if (tg.gate && tg.residual) epilogue_rows<TB, true, true>(p, tg, head, tok0, acc);
+  else if (tg.gate) epilogue_rows<TB, true, false>(p, tg, head, tok0, acc);
+  else if (tg.residual) epilogue_rows<TB, false, true>(p, tg, head, tok0, acc);
+  else epilogue_rows<TB, false, false>(p, tg, head, tok0, acc);
+}
+
+// Tokens per workgroup of a launch (16 * 2 * TB).  Time of a CU's share of the launch, in units of 100 us for K = 3,072 with an
+// adapter, from the workgroups it runs: one alone on the CU, and two (side by side for the smaller forms, one after the
+// other for TB = 8).  Measured at 1,085, 15,342 and 48,360 tokens x 9,216 and 3,072 features: TB = 8 67 us alone, 79 - 84 us
+// each in a long launch; TB = 4 40 us alone, 80 us for two; TB = 2 34 and 61 us.  What sets them: a form's LDS traffic per
+// MFMA (64, 72 and 90 KiB per 512 MFMAs read) against how evenly its tiles fill the CUs.
+static int gemm_token_blocks(int tokens, int n_tiles, int cus) {
+  static const struct { int tb; float one, two; } kForms[3] = {{8, 0.67f, 1.55f}, {4, 0.40f, 0.80f}, {2, 0.34f, 0.61f}};
+  int best = 8;
+  float best_cost = 0.f;
+  for (const auto& f : kForms) {
+    const int tiles = (tokens + 32 * f.tb - 1) / (32 * f.tb) * n_tiles;
+    const int per_cu = (tiles + cus - 1) / cus;
+    const float cost = (per_cu / 2) * f.two + (per_cu & 1) * f.one;
+    if (f.tb == 8 || cost < best_cost) best = f.tb, best_cost = cost;
+  }
+  return best;
+}
+
+template <int TB>
+static hipError_t launch_gemm_tb(GemmParams p, int cus, hipStream_t st) {
+  p.m_tiles = (p.M + 32 * TB - 1) / (32 * TB);
+  const int total = p.m_tiles * p.n_tiles;
+  // launches of at least two rounds of workgroups take their tiles from per-XCD work queues, with an eighth more
+  // workgroups than tiles, the spare ones for the XCDs that finish early
+  if (total < 2 * cus * (TB == 8 ? 1 : 2)) p.queue_next = nullptr;
+  const int wgs = p.queue_next ? total + (total / 8 > kQueues ? total / 8 : kQueues) : total;
+  hipLaunchKernelGGL(gemm_kernel<TB>, dim3((wgs + 7) / 8 * 8), dim3(64 * kGemmWaves), 0, st, p);
+  return hipGetLastError();
 }
 
 hipError_t launch_gemm(const GemmParams& p, hipStream_t st) {
-  const int total = p.m_tiles * p.n_tiles;
-  // with work queues: an eighth more workgroups than tiles, the spare ones for the XCDs that finish early
-  const int wgs = p.queue_next ? total + (total / 8 > kQueues ? total / 8 : kQueues) : total;
-  hipLaunchKernelGGL(gemm_kernel<kGemmWaves>, dim3((wgs + 7) / 8 * 8), dim3(64 * kGemmWaves), 0, st, p);
-  return hipGetLastError();
+  int cus = 0;
+  hipError_t e = device_cu_count(&cus);
+  if (e != hipSuccess) return e;
+  if (cus <= 0) cus = 1;
+  switch (gemm_token_blocks(p.M, p.n_tiles, cus)) {
+    case 8: return launch_gemm_tb<8>(p, cus, st);
+    case 4: return launch_gemm_tb<4>(p, cus, st);
+    default: return launch_gemm_tb<2>(p, cus, st);
+  }
 }
 
 // ------------------------------------------------------------------------------------------------

@@ -155,10 +155,11 @@ struct GemmParams {
   int64_t a_blk_stride;    // bytes between consecutive 16-token blocks
   int nk1;                 // 32-wide k-chunks of the first segment
   int M;                   // tokens
-  int m_tiles, n_tiles;    // 256 x 256 workgroup tiles
+  int n_tiles;             // 256-feature workgroup tiles
+  int m_tiles;             // workgroup tiles along the tokens (set by launch_gemm, which chooses their height)
   int n_targets;
   GemmTarget tg[3];
-  int* queue_next;         // [kQueues] zeroed positions of the per-XCD work queues the tiles are taken from, or null: fixed map
+  int* queue_next;         // [kQueues] zeroed positions of the per-XCD work queues long launches take their tiles from, or null: fixed map
 };
 
 // rows (activations or weights) -> operand images, optionally normalised and modulated

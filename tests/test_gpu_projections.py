@@ -196,6 +196,71 @@ def test_out_projection_with_gate_and_residual(S, N, K, lora, extras):
     assert err <= 2e-2 * max(1.0, float(ref.abs().max())) and cos >= 0.9999
 
 
+# The GEMM's three workgroup heights (64, 128, 256 tokens; chosen by tokens x feature tiles) on both sides of their edges,
+# an odd number of k-chunks (K = 96 + the adapter's 128) and an even one.
+@pytest.mark.parametrize("S,H,K,fp8,mode", [
+    (31, 1, 96, False, 1), (129, 2, 128, True, 2), (449, 3, 96, True, 1),          # 64 tokens
+    (3585, 24, 96, False, 1), (3713, 24, 128, True, 2), (3600, 23, 96, "pow2", 1),  # 128 tokens
+    (1025, 24, 96, False, 2), (1279, 24, 128, True, 1), (1088, 23, 96, False, 0),   # 256 tokens
+])
+def test_gemm_forms_of_the_qkv_projection(S, H, K, fp8, mode):
+    """Q against float32 torch, and the attention output against the same kernel fed with torch's K and V through the
+    separate K/V pass: every token and head, so a wrong 16-token block of any epilogue shows."""
+    import pika_h3_flex_amd as pk
+    from oracle import attention_oracle as AO
+    from pika_h3_flex_amd import projections as P
+
+    x = _r(S, K, seed=1).to(torch.bfloat16).cuda()
+    lin = {n: _linear(H * D, K, 20 + 10 * i, bias=(n != "k")) for i, n in enumerate(("q", "k", "v"))}
+    opts = dict(q_norm_weight=(1 + 0.1 * _r(D, seed=2)).cuda(), k_norm_weight=(1 + 0.1 * _r(D, seed=3)).cuda(), fp8_qk=fp8)
+    if mode:
+        opts.update(rope_mode=mode, rope_q=pk.rope_tables(pk.video_position_ids(1, 1, S).cuda()))
+    out, q = P.qkv_attention(P.pack_rows(x), S, _packed(lin["q"]), _packed(lin["k"]), _packed(lin["v"], head_perm=False),
+                             heads=H, return_q=True, **opts)
+
+    def layer(d):
+        y = x.float() @ d["weight"].cuda().float().t() + d["lora_scale"] * (x.float() @ d["lora_a"].cuda().float().t()) @ d["lora_b"].cuda().float().t()
+        return (y + d["bias"].cuda() if "bias" in d else y).view(1, S, H, D)
+
+    ref = {n: layer(d) for n, d in lin.items()}
+    want = pk.attention(*(ref[n].to(torch.bfloat16) for n in ("q", "k", "v")), **opts)
+    torch.cuda.synchronize()
+    err, cos = AO.max_abs_and_cosine(q.cpu(), ref["q"].cpu())
+    # per row and head: bf16 rounding of Q, K, V and P moves a row's direction by less than 1e-3 (fp8: another K rounding
+    # flips e4m3 steps, relative 2^-4 each, on a share of the 128 products)
+    rows = torch.nn.functional.cosine_similarity(out.float(), want.float(), dim=-1).min().item()
+    print(f"S={S} H={H} K={K} fp8={fp8} mode={mode}: Q max_abs={err:.3e} cos={cos:.8f}; O worst row cos={rows:.6f}", flush=True)
+    assert err <= 2e-2 * max(1.0, float(ref["q"].abs().max())) and cos >= 0.9999
+    assert rows >= (0.99 if fp8 else 0.999)
+
+
+@pytest.mark.parametrize("S,N", [(65, 256), (1471, 3072), (1537, 2944), (3583, 3072), (3649, 2944)])
+@pytest.mark.parametrize("gate,residual", [(True, True), (True, False), (False, True), (False, False)])
+def test_gemm_forms_of_the_out_projection(S, N, gate, residual):
+    """The three workgroup heights of the row-major epilogue with each of its four combinations, every row."""
+    from pika_h3_flex_amd import projections as P
+
+    K = 96
+    o = _r(S, K, seed=5).to(torch.bfloat16).cuda()
+    lin = _linear(N, K, 6)
+    g = _r(3, N, seed=7, std=0.5).to(torch.bfloat16).cuda()
+    idx = (torch.arange(S) * 3 // S).to(torch.int32).cuda()
+    res = _r(S, N, seed=8).to(torch.bfloat16).cuda()
+    y = P.out_proj(o, _packed(lin), **(dict(gate=g, row_index=idx) if gate else {}), **(dict(residual=res) if residual else {}))
+    w = {n: t.cuda().float() for n, t in lin.items() if torch.is_tensor(t)}
+    ref = o.float() @ w["weight"].t() + w["bias"] + lin["lora_scale"] * (o.float() @ w["lora_a"].t()) @ w["lora_b"].t()
+    if gate:
+        ref = ref * g.float()[idx.long()]
+    if residual:
+        ref = ref + res.float()
+    torch.cuda.synchronize()
+    # one bf16 rounding of the result (at most 2^-8 of its size), and that of the 128 down-projected values (size 0.5,
+    # rounding 2^-9 of it each, through weights of 0.05 and a gate of at most 2.5: spread 8e-4, times six)
+    err = (y.float() - ref).abs()
+    print(f"out_proj S={S} N={N} gate={gate} residual={residual}: max_abs={err.max().item():.3e}", flush=True)
+    assert bool((err <= ref.abs() / 256 + 5e-3).all())
+
+
 @pytest.mark.parametrize("S,H", [(300, 2), (1000, 3), (257, 1)])
 def test_adapters_in_one_buffer_give_the_same_bits(S, H):
     """``PackedLinear.share_adapter_buffer`` lays the three down-projection images one behind the other, and
