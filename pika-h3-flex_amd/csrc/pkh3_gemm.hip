@@ -232,6 +232,13 @@ __device__ __forceinline__ void gemm_loop(const GemmParams& p, const GemmTarget&
     slot = s2;
   }
   if (kc < nk) chunk(next(slot), slot, wa, xa, wb, xb);
+  // The last chunk's reads ahead have no reader, so their registers would be free to hold something else while they are
+  // still on their way: held until they have landed.
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < 8; ++i) asm volatile("" ::"v"(wa[i]), "v"(wb[i]));
+#pragma unroll
+  for (int i = 0; i < TB; ++i) asm volatile("" ::"v"(xa[i]), "v"(xb[i]));
   // the compiler does not know the instructions above for MFMAs: let the last one retire before anything reads the accumulators
   static_for<TB>([&](auto tc) {
     f32x4(&a)[8] = acc[decltype(tc)::value];
