@@ -165,7 +165,6 @@ void build(const pkh3_attn_args* a, void* workspace, Launch& L, bool part_scratc
   v.B = a->B; v.H = a->H; v.S = a->Sk; v.nKt = L.w.nKt;
   v.gather_idx = L.idx; v.row_cnt = L.cnt;
   v.out = ws + L.w.kv_off + kBytes; v.out_bh_stride = k.out_bh_stride; v.out_tile_stride = L.w.kvTileBytes;
-  v.zero_init = (unsigned*)(ws + L.w.kmax_off);
 
   FwdParams& f = L.f;
   f = FwdParams{};
@@ -199,12 +198,13 @@ int hip_fail(hipError_t e, const char* what) {
 // The K/V side of a call: key-mask compaction, then V and K into the workspace in the attention kernel's layout.
 int run_kv_side(const pkh3_attn_args* a, const Launch& L, hipStream_t st) {
   hipError_t e;
+  // the K/V pass max-reduces its row norms into per-head slots that must start at zero
   if (a->key_mask) {
-    if ((e = launch_mask_compact(a->key_mask, a->B, a->Sk, L.idx, L.cnt, st)) != hipSuccess) return hip_fail(e, "mask_compact");
+    if ((e = launch_mask_compact(a->key_mask, a->B, a->Sk, L.idx, L.cnt, L.kp.norm_max, a->H, st)) != hipSuccess) return hip_fail(e, "mask_compact");
+  } else if ((e = launch_fill_zero(L.kp.norm_max, a->B * a->H, st)) != hipSuccess) {
+    return hip_fail(e, "fill_zero");
   }
-  // V first: it also clears the per-head slots the K pass max-reduces its row norms into
-  if ((e = launch_v_prologue(L.vp, st)) != hipSuccess) return hip_fail(e, "v prologue");
-  if ((e = launch_qk_prologue(L.kp, st)) != hipSuccess) return hip_fail(e, "k prologue");
+  if ((e = launch_kv_prologue(L.kp, L.vp, st)) != hipSuccess) return hip_fail(e, "k/v pass");
   return PKH3_OK;
 }
 

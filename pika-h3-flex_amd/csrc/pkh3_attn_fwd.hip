@@ -106,14 +106,6 @@ __device__ __forceinline__ float load_device(const float* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// maximum over the four lanes l % 16 == const (one per 16-lane group): two row swaps, no LDS crossbar
-__device__ __forceinline__ float max_across_groups(float x) {
-  const auto r16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  x = fmaxf(__uint_as_float(r16[0]), __uint_as_float(r16[1]));
-  const auto r32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r32[0]), __uint_as_float(r32[1]));
-}
-
 // Per-wave state.  Lane (c = l % 16, g = l / 16) works for the two queries 16*qb + c, qb = 0, 1, of the wave's 32.
 template <bool FP8>
 struct WaveState {

@@ -84,6 +84,14 @@ __device__ __forceinline__ float wave_sum_groups(float x) {
   return __uint_as_float(r32[0]) + __uint_as_float(r32[1]);
 }
 
+// maximum over the four lanes l % 16 == const (one per 16-lane group): two row swaps, no LDS crossbar
+__device__ __forceinline__ float max_across_groups(float x) {
+  const auto r16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = fmaxf(__uint_as_float(r16[0]), __uint_as_float(r16[1]));
+  const auto r32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r32[0]), __uint_as_float(r32[1]));
+}
+
 // ---- four lanes per row: the layout of the 16x16 operand images themselves ----
 // Lane (c = l % 16, g = l / 16) holds the pieces p8 = 4*ks + g of row c of a 16-row block, i.e. elements
 // d = 32*ks + 8*g + j at x[8*ks + j]; the three other lane groups (lanes l ^ 16, l ^ 32, l ^ 48) hold the rest of the

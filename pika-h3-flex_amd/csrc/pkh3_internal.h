@@ -50,7 +50,7 @@ struct QkPrologueParams {
   float* scale_out;         // fp8: [B*H, nBlk64] dequantisation scales, else null
   int fp8;
   int fp8_pow2;             // fp8: block scales rounded up to a power of two
-  unsigned* norm_max;       // [B*H] float bits: max row norm after norm+rotation (atomic max), or null
+  unsigned* norm_max;       // [B*H] float bits: max row norm after norm+rotation (atomic max)
 };
 
 struct VPrologueParams {
@@ -62,7 +62,6 @@ struct VPrologueParams {
   char* out;                // points at the V part of tile 0
   int64_t out_bh_stride;
   int out_tile_stride;
-  unsigned* zero_init;      // [B*H] words this launch clears (the K launch after it max-reduces into them)
 };
 
 struct FwdParams {
@@ -183,9 +182,9 @@ hipError_t launch_gemm(const GemmParams& p, hipStream_t st);
 hipError_t launch_pack_rows(const PackParams& p, hipStream_t st);
 hipError_t launch_fill_zero(unsigned* p, int n, hipStream_t st);
 
-hipError_t launch_mask_compact(const uint8_t* mask, int B, int Sk, int* idx, int* cnt, hipStream_t st);
-hipError_t launch_qk_prologue(const QkPrologueParams& p, hipStream_t st);
-hipError_t launch_v_prologue(const VPrologueParams& p, hipStream_t st);
+// `zero_init`: [B*H] words the launch clears (the K/V pass after it max-reduces into them)
+hipError_t launch_mask_compact(const uint8_t* mask, int B, int Sk, int* idx, int* cnt, unsigned* zero_init, int H, hipStream_t st);
+hipError_t launch_kv_prologue(const QkPrologueParams& k, const VPrologueParams& v, hipStream_t st);
 hipError_t launch_attn_fwd(const FwdParams& p, hipStream_t st);
 hipError_t device_cu_count(int* out);  // CUs of the current device (cached per device after the first call)
 hipError_t launch_sparse_plan(const int* row_ptr, const int* col_idx, int nRow64, int nQ64, int nKt, int* plan,

@@ -110,6 +110,15 @@ def test_rectangular_with_rope_and_separate_tables(Sq, Sk, mode, fp8):
     _run_and_check(1, Sq, Sk, 2, seed=7 * Sq + Sk + mode, rope_mode=mode, weight_random=True, fp8=fp8)
 
 
+@pytest.mark.parametrize("B,H,Sk,mode,fp8,masked", [(1, 7, 17901, 1, False, False), (1, 7, 17901, 2, True, False), (2, 5, 17900, 0, False, True)])
+def test_kv_pass_walks_several_heads(B, H, Sk, mode, fp8, masked):
+    """Key sets long enough that a workgroup of the K/V pass takes several heads one after the other (here 3, the last
+    group with fewer), with a partial last tile, and through a scattered key mask."""
+    gen = torch.Generator().manual_seed(Sk + mode)
+    mask = (torch.rand((B, Sk), generator=gen) < 0.4) if masked else None
+    _run_and_check(B, 40, Sk, H, seed=31 + mode, rope_mode=mode, weight_random=True, fp8=fp8, mask=mask)
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("scale", [0.05, 0.2])
 def test_softmax_scale_other_than_default(scale, fp8):
