@@ -24,14 +24,17 @@
 // scalar: no cross-lane traffic in the rescale, none between the two GEMMs.  O leaves through LDS, turned
 // around into whole 256-byte rows.
 //
-// Other forms of the dense kernel (see attn_fwd_body): the short-key form (at most 16 key tiles: 4 waves per
-// workgroup, 32-key half tiles, three workgroups per CU), and the long form with the key tiles of a unit shared out
+// Other forms of the dense kernel (see attn_fwd_body): the short-key form (few key tiles, or few queries: 4 waves per
+// workgroup, 32-key half tiles, three workgroups per CU), the narrow form (fewer queries still: one 32-query block per
+// workgroup, its waves share the keys out; attn_fwd_narrow_kernel), and the long form with the key tiles of a unit shared out
 // among several workgroups that merge through global scratch, for a thinly filled last round of a long call.
 //
 // Block-sparse variant.  A workgroup covers 4 query row-blocks (64 queries each, a wave pair per row-block).
 // Phase 1 walks the key tiles all four row-blocks keep, exactly like the dense kernel.  Phase 2 walks the
 // remaining tiles per row-block: every iteration gives each wave pair one 32-key half of a tile of its own
 // list in its own LDS area, so all 8 waves stay busy.  The lists are built on the device by a plan kernel.
+#include <limits.h>
+
 #include <atomic>
 
 #include "pkh3_common.h"
@@ -384,6 +387,9 @@ __device__ __forceinline__ void softmax_pv_half(WaveState<FP8>& w, float c, int 
 // writes the output.
 constexpr int kMergeBytes = kPartialBytes;  // one wave's partial result in fp32
 
+// workgroups of `blocks` 32-query blocks a (batch, head) needs
+__host__ __device__ constexpr int units_per_head(int Sq, int blocks) { return ((Sq + 31) / 32 + blocks - 1) / blocks; }
+
 // bytes of LDS a form of the kernel needs
 template <bool FP8, bool SPARSE, int WAVES>
 constexpr int fwd_lds_bytes() {
@@ -441,7 +447,7 @@ __device__ __forceinline__ void attn_fwd_body(const FwdParams& p, int blk, int u
   const int part = lin / units, ul = lin % units;
   const int unit = unit0 + ul;
   const int wq = wave;                                    // which 32-query block of the unit
-  const int nQt = (p.nQ64 * 2 + WAVES - 1) / WAVES;       // units per (batch, head)
+  const int nQt = SPARSE ? p.nQ64 / kSparseRows : units_per_head(p.Sq, WAVES);  // units per (batch, head)
   const int bh = unit / nQt, qt = unit % nQt;
   const int q32 = qt * WAVES + wq;
   const int b = bh / p.H, h = bh % p.H;
@@ -902,6 +908,271 @@ __global__ __launch_bounds__(64 * kDenseWaves, 1) void attn_fwd_dense_kernel(Fwd
   attn_fwd_body<FP8, false, kDenseWaves, POW2>(p, blk, unit0, units, parts, part_base, cnt_base, lds_raw, fetched);
 }
 
+// The narrow form, for calls whose 32-query blocks hardly outnumber the CUs: a workgroup is one block of 32 queries, and its
+// 4 waves share the keys out in runs of 32-key half tiles.  No two waves of a workgroup read the same images, and an image
+// is exactly what a lane of the MFMA wants, so they go from the L2 straight into registers: no LDS ring and no barrier in
+// the loop, the next K images on their way under the softmax, the V images under S^T.  The partial results meet in LDS,
+// where every wave adds up its share of the 16-row blocks of O^T, in the order of the key shares.
+// Bound by the CU's 64 bytes per clock of vector loads (16 KiB for 32 MFMAs: twice what the matrix units need for them) and,
+// for few keys, by the start and the merge of a workgroup; two workgroups of 4 waves share a CU, so that those of one run
+// under the loads of the other (one of 8 waves: the same up to 256 blocks, 8 x 2000 rows 28.0 against 23.9 us).  Kernel times
+// against the form that took these calls before: 4 heads x 1,024 rows 23.4 -> 10.4 us, 2 x 3,000 88 -> 18.5,
+// 24 x 256 rows and 2,048 keys 61 -> 14.7, 8 x 2,000 62 -> 24 (fp8 57 -> 21), 1 x 15,000 404 -> 138.
+constexpr int kNarrowWaves = 4;
+
+// The tiles a query block walks: all of them, or (block-sparse) the two lists of the plan it belongs to.
+template <bool SPARSE>
+struct TileWalk {
+  const int* shared;   // tiles its whole plan entry keeps ...
+  int n_shared;
+  const int* own;      // ... and those its row-block keeps besides
+  __device__ __forceinline__ int operator()(int e) const {
+    if constexpr (!SPARSE) return e;
+    else return e < n_shared ? uniform_load(shared, e) : uniform_load(own, e - n_shared);
+  }
+};
+
+template <bool FP8, bool POW2, bool SPARSE, bool STATIC>
+__device__ __forceinline__ void narrow_loop(WaveState<FP8>& w, i32x4 (&kf)[FP8 ? 4 : 8], const char* kv, int tile_stride, const float* kscale,
+                                            const TileWalk<SPARSE>& walk, int h0, int h1, int sk, float c, int lane) {
+  constexpr int kKBytes = FP8 ? kK8TileBytes : kKTileBytes;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  int tile = h0 < h1 ? walk(h0 >> 1) : 0;
+#pragma unroll 1
+  for (int i = h0; i < h1; ++i) {
+    // (the last iteration asks for its own K images again: the loads need no branch)
+    const int n = min(i + 1, h1 - 1);
+    const int tile_next = walk(n >> 1);
+    const char* v = kv + (int64_t)tile * tile_stride + kKBytes + (i & 1) * (kVTileBytes / 2);
+    const float ks = FP8 ? uniform_load(kscale, tile) : 1.0f;
+    const int lim = sk - 64 * tile - 32 * (i & 1);
+    const bool live = !SPARSE || lim > 0;   // (wave-uniform) the second half of a short last tile holds nothing
+    if (live) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) w.vf[j] = *(const bf16x8*)(v + (j * 64 + lane) * 16);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (!FP8) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+#pragma unroll
+          for (int qb = 0; qb < 2; ++qb)
+            w.s[j & 1][qb] = PKH3_MFMA16(__builtin_bit_cast(bf16x8, kf[j]), w.qf[qb][j >> 1], j < 2 ? zero : w.s[j & 1][qb]);
+      } else {
+        const int ke = e8m0_of(ks);
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+          const i32x4 a0 = kf[2 * kb], a1 = kf[2 * kb + 1];
+          const i32x8 a = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
+#pragma unroll
+          for (int qb = 0; qb < 2; ++qb)
+            w.s[kb][qb] = POW2 ? PKH3_MFMA16_F8S(a, w.q8[qb], zero, ke, w.qe) : PKH3_MFMA16_F8(a, w.q8[qb], zero);
+        }
+      }
+    }
+    const char* k = kv + (int64_t)tile_next * tile_stride + (n & 1) * (kKBytes / 2);
+#pragma unroll
+    for (int j = 0; j < (FP8 ? 4 : 8); ++j) kf[j] = *(const i32x4*)(k + (j * 64 + lane) * 16);
+    __builtin_amdgcn_sched_barrier(0);
+    if (live) softmax_pv_half<FP8, STATIC, false, false, POW2>(w, (FP8 && !POW2) ? c * ks : c, lim, lane);
+    tile = tile_next;
+  }
+  PKH3_MFMA_DRAIN(w);
+}
+
+template <bool FP8, bool POW2, bool SPARSE>
+__global__ __launch_bounds__(64 * kNarrowWaves, 2) void attn_fwd_narrow_kernel(FwdParams p) {
+  constexpr int NW = kNarrowWaves;
+  constexpr int kKBytes = FP8 ? kK8TileBytes : kKTileBytes;
+  constexpr int kSlot = 64 * 64 * 4;                       // one wave's O^T in fp32
+  __shared__ __attribute__((aligned(1024))) char part[NW * kSlot];
+  __shared__ __attribute__((aligned(1024))) char rows[32 * kD * 2];   // the Q images, later the output rows
+  __shared__ float part_l[NW][2][16], part_m[NW][2][16];
+  __shared__ float s_n2[2], s_amax[4];
+  const int lane = threadIdx.x & 63, c16 = lane & 15, g4 = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int per_xcd = (p.sec_units[0] + 7) / 8;            // a contiguous run of (batch, head, query block) per XCD
+  const int lin = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per_xcd || lin >= p.sec_units[0]) return;
+  const int nq = units_per_head(p.Sq, 1);
+  const int bh = lin / nq, q32 = lin % nq;
+  const int b = bh / p.H, h = bh % p.H;
+  const int sk = p.row_cnt ? p.row_cnt[b] : p.Sk;
+  TileWalk<SPARSE> walk{};
+  int n_half = (sk + 31) / 32;
+  if constexpr (SPARSE) {
+    // plan entry of this block's 256 queries, row-block of its 64 (the lists of attn_fwd_body, walked in the same order)
+    const int entry = q32 / (2 * kSparseRows), r = (q32 / 2) % kSparseRows;
+    walk.shared = p.plan + (int64_t)entry * p.plan_stride;
+    walk.own = walk.shared + (1 + r) * p.nKt;
+    walk.n_shared = uniform_load(p.plan_cnt + entry * kSparseLists, 0);
+    const int n = walk.n_shared + uniform_load(p.plan_cnt + entry * kSparseLists, 1 + r);
+    // a last tile of at most 32 keys has one half tile: a full map is shared out as the dense call is
+    const bool short_end = n > 0 && (n_half & 1) && walk(n - 1) == p.nKt - 1;
+    n_half = 2 * n - (short_end ? 1 : 0);
+  }
+  const int h0 = wave * n_half / NW, h1 = (wave + 1) * n_half / NW;
+  const char* kv = p.kv + (int64_t)bh * p.kv_bh_stride;
+
+  WaveState<FP8> w;
+  i32x4 kf[FP8 ? 4 : 8];
+  if (h0 < h1) {
+    const char* k = kv + (int64_t)walk(h0 >> 1) * p.kv_tile_stride + (h0 & 1) * (kKBytes / 2);
+#pragma unroll
+    for (int j = 0; j < (FP8 ? 4 : 8); ++j) kf[j] = *(const i32x4*)(k + (j * 64 + lane) * 16);
+  }
+  // The queries, a 16-row block per wave for all waves (layout and arithmetic of attn_fwd_body's Q load).  fp8: one scale
+  // per 64 queries, so four waves look at the four blocks this block's 64 queries consist of, and two of them are it.
+  const int mine = FP8 ? wave - 2 * (q32 & 1) : wave;      // which of the two 16-query blocks, if 0 or 1
+  const bool prepares = (unsigned)mine < 2u;
+  float x[32];
+  float qscale = 1.0f;
+  if (FP8 || prepares) {
+    const RowTransform tf{p.q_norm_w, p.q_eps, p.q_rope_mode, p.q_cos, p.q_sin};
+    const int qrow = q32 * 32 + 16 * mine + c16;
+    const bool valid = qrow < p.Sq;
+    const __bf16* row = (const __bf16*)p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)(valid ? qrow : 0) * p.q_ss + 8 * g4;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      const bf16x8 raw = *(const bf16x8*)(row + 32 * ks);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[ks * 8 + j] = valid ? (float)raw[j] : 0.f;
+    }
+    norm_rope_quarter(x, tf, qrow, valid, g4);
+    // softmax_scale * log2(e) rides in Q' (bf16, and fp8 with power-of-two scales)
+    if constexpr (!FP8 || POW2) {
+#pragma unroll
+      for (int i = 0; i < 32; ++i) x[i] *= p.c;
+    }
+    if constexpr (FP8) {
+      float amax = 0.f;
+#pragma unroll
+      for (int i = 0; i < 32; ++i) amax = fmaxf(amax, fabsf(x[i]));
+      amax = wave_max(amax);
+      if (lane == 0) s_amax[wave] = amax;
+    }
+  }
+  if constexpr (FP8) {
+    __syncthreads();
+    qscale = fp8_block_scale(fmaxf(fmaxf(s_amax[0], s_amax[1]), fmaxf(s_amax[2], s_amax[3])), POW2);
+    w.qe = e8m0_of(qscale);
+  }
+  if (prepares) {
+    float n2 = 0.f;
+    if constexpr (!FP8) {
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        bf16x8 t;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          t[j] = (__bf16)x[ks * 8 + j];
+          n2 = fmaf(x[ks * 8 + j], x[ks * 8 + j], n2);
+        }
+        *(bf16x8*)(rows + ((mine * 4 + ks) * 64 + lane) * 16) = t;
+      }
+    } else {
+      const float inv = 1.0f / qscale;
+#pragma unroll
+      for (int c2 = 0; c2 < 2; ++c2) {
+        const i32x2 q0 = quant_fp8_piece(x + 16 * c2, inv), q1 = quant_fp8_piece(x + 16 * c2 + 8, inv);
+        const i32x4 q = {q0[0], q0[1], q1[0], q1[1]};
+#pragma unroll
+        for (int wd = 0; wd < 4; ++wd) {
+          const auto lo = __builtin_amdgcn_cvt_pk_f32_fp8(q[wd], false);
+          const auto hi = __builtin_amdgcn_cvt_pk_f32_fp8(q[wd], true);
+          n2 += lo[0] * lo[0] + lo[1] * lo[1] + hi[0] * hi[0] + hi[1] * hi[1];
+        }
+        *(i32x4*)(rows + ((mine * 2 + c2) * 64 + lane) * 16) = q;
+      }
+      n2 *= qscale * qscale;
+    }
+    n2 = wave_max(fmaxf(wave_sum_groups(n2), 0.f));
+    if (lane == 0) s_n2[mine] = n2;
+  }
+#pragma unroll
+  for (int db = 0; db < 8; ++db)
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb) w.o[db][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  w.m[0] = w.m[1] = -INFINITY;
+  w.l[0] = w.l[1] = 0.f;
+  __syncthreads();
+#pragma unroll
+  for (int qb = 0; qb < 2; ++qb) {
+    if constexpr (!FP8) {
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) w.qf[qb][ks] = *(const bf16x8*)(rows + ((qb * 4 + ks) * 64 + lane) * 16);
+    } else {
+      const i32x4 a0 = *(const i32x4*)(rows + ((qb * 2) * 64 + lane) * 16), a1 = *(const i32x4*)(rows + ((qb * 2 + 1) * 64 + lane) * 16);
+      w.q8[qb] = i32x8{a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
+    }
+  }
+  // the bound of attn_fwd_body: small enough, and no running maximum is needed
+  const float margin = FP8 ? (POW2 ? 1.08f : p.c * 1.08f) : 1.01f;
+  const bool static_max = n_half > 0 && __all(sqrtf(fmaxf(s_n2[0], s_n2[1])) * uniform_load(p.kmax, bh) * margin <= kStaticMaxLimit);
+  const float* kscale = FP8 ? p.kscale + (int64_t)bh * p.nKt : nullptr;
+  const float c = POW2 ? 1.0f : p.c * qscale;   // what the softmax still multiplies the logits by (fp8 absmax form only)
+  if (static_max) narrow_loop<FP8, POW2, SPARSE, true>(w, kf, kv, p.kv_tile_stride, kscale, walk, h0, h1, sk, c, lane);
+  else narrow_loop<FP8, POW2, SPARSE, false>(w, kf, kv, p.kv_tile_stride, kscale, walk, h0, h1, sk, c, lane);
+
+#pragma unroll
+  for (int db = 0; db < 8; ++db)
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb) *(f32x4*)(part + wave * kSlot + ((db * 2 + qb) * 64 + lane) * 16) = w.o[db][qb];
+#pragma unroll
+  for (int qb = 0; qb < 2; ++qb) {
+    const float l = wave_sum_groups(w.l[qb]);
+    if (g4 == 0) part_l[wave][qb][c16] = l, part_m[wave][qb][c16] = w.m[qb];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int qb = 0; qb < 2; ++qb) {
+    float top = -INFINITY, l = 0.f, a[NW];
+    if (!static_max) {
+#pragma unroll
+      for (int j = 0; j < NW; ++j) top = fmaxf(top, part_m[j][qb][c16]);
+    }
+#pragma unroll
+    for (int j = 0; j < NW; ++j) {
+      a[j] = static_max ? 1.0f : top == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(part_m[j][qb][c16] - top);
+      l += a[j] * part_l[j][qb][c16];
+    }
+    const float inv = l > 0.f ? 1.0f / l : 0.f;
+#pragma unroll
+    for (int i = 0; i < 8 / NW; ++i) {
+      const int db = wave + i * NW;
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < NW; ++j) {
+        const f32x4 t = *(const f32x4*)(part + j * kSlot + ((db * 2 + qb) * 64 + lane) * 16);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[r] += a[j] * t[r];
+      }
+      bf16x4 o;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] = (__bf16)(acc[r] * inv);
+      // elements d = 16*db + 4*g .. +3 of row 16*qb + c, chunks XOR-swizzled by the row as in attn_fwd_body
+      *(bf16x4*)(rows + (16 * qb + c16) * 256 + (((2 * db + (g4 >> 1)) ^ c16) * 16) + 8 * (g4 & 1)) = o;
+    }
+  }
+  __syncthreads();
+  if (p.o_images) {
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) {
+      const int ks = wave, r = 16 * rb + c16;
+      bf16x8 v = *(const bf16x8*)(rows + r * 256 + (((4 * ks + g4) ^ c16) * 16));
+      if (q32 * 32 + r >= p.Sq) v = bf16x8{};
+      *(bf16x8*)((char*)p.o + (int64_t)(q32 * 2 + rb) * p.o_img_blk_stride + ((int64_t)h * (kD / 32) + ks) * 1024 + lane * 16) = v;
+    }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 32 / (4 * NW); ++i) {
+    const int row = (threadIdx.x >> 4) + i * 4 * NW;
+    const bf16x8 v = *(const bf16x8*)(rows + row * 256 + ((c16 ^ (row & 15)) * 16));
+    if (q32 * 32 + row < p.Sq)
+      *(bf16x8*)((__bf16*)p.o + (int64_t)b * p.o_sb + (int64_t)h * p.o_sh + (int64_t)(q32 * 32 + row) * p.o_ss + 8 * c16) = v;
+  }
+}
+
 static int blocks_of(int workgroups) { return (workgroups + 7) / 8 * 8; }
 
 // How a long dense call ends.  One 12-wave workgroup per CU at a time: the call runs in rounds of `cus` workgroups, and
@@ -936,11 +1207,29 @@ static TailPlan plan_tail(int rest, int cus, int n_tiles, int64_t max_workgroups
 
 template <bool FP8, bool POW2 = false>
 static hipError_t launch_fp(FwdParams p, int cus, hipStream_t st) {
-  const int nQ32 = p.nQ64 * 2;
-  auto units = [&](int blocks) { return p.B * p.H * ((nQ32 + blocks - 1) / blocks); };
+  auto units = [&](int blocks) { return p.B * p.H * units_per_head(p.Sq, blocks); };
   for (int i = 0; i < kSections; ++i) p.sec_units[i] = p.sec_blocks[i] = 0, p.sec_parts[i] = 1;
+  // Calls of at most two short-key workgroups per CU leave a long form's chip half empty, whatever the number of keys.  They
+  // take the narrow form where it is estimated shorter, else the short-key form.  The estimates are straight lines through
+  // kernel times in microseconds (bf16; fp8 lies within a tenth of them): the narrow form, a start and a merge and 0.135 per half tile
+  // for every 32-query block a CU gets; the short-key form, a half tile per 0.60 with one workgroup on a CU and per 0.87
+  // with two.  Measured (narrow / short-key / long): 240 blocks x 10 half tiles 7.9 / 11.1 / 17.2, 504 x 63 23.9 / 41.9 / 62.9,
+  // 768 x 64 34.8 / 43.4 / 63.7, 1,256 x 157 115 / 128 / 144; on the other side of the line 456 x 4 7.9 / 7.7 / 12.6,
+  // 816 x 34 27.3 / 26.3 / 38.5, 1,504 x 94 86 / 81 / 90, 1,896 x 79 95 / 73 / 78.  With three short-key workgroups per CU the
+  // long form is ahead as long as its own workgroups are no more than the CUs (2,256 x 94: 114 / 94), and behind when a few
+  // are left over for a second round (3,000 x 125: 165 / 218).
+  const int n4 = units(kShortWaves), n32 = units(1), n_half = (p.Sk + 31) / 32;
+  const int per_cu = cus > 0 ? (n4 + cus - 1) / cus : INT_MAX;
+  if (per_cu <= 2 && !p.long_key_kernel &&
+      3.2f + (n32 + cus - 1) / cus * (0.135f * n_half + 2.7f) < 5.0f + (per_cu == 1 ? 0.60f : 0.87f) * n_half) {
+    p.queue_next = nullptr;
+    p.sec_units[0] = n32;
+    if (p.plan) hipLaunchKernelGGL((attn_fwd_narrow_kernel<FP8, POW2, true>), dim3(blocks_of(n32)), dim3(64 * kNarrowWaves), 0, st, p);
+    else hipLaunchKernelGGL((attn_fwd_narrow_kernel<FP8, POW2, false>), dim3(blocks_of(n32)), dim3(64 * kNarrowWaves), 0, st, p);
+    return hipGetLastError();
+  }
   if (p.plan) {
-    const int n = units(kSparseWaves);
+    const int n = p.B * p.H * (p.nQ64 / kSparseRows);
     p.sec_units[0] = n;
     int wgs = n;
     if (p.queue_next && cus > 0 && n >= cus) {
@@ -954,9 +1243,10 @@ static hipError_t launch_fp(FwdParams p, int cus, hipStream_t st) {
     hipLaunchKernelGGL((attn_fwd_kernel<FP8, true, kSparseWaves, POW2>), dim3(blocks_of(wgs)), dim3(64 * kSparseWaves), 0, st, p);
     return hipGetLastError();
   }
-  if (p.nKt <= kShortMaxTiles && !p.long_key_kernel) {
+  const bool few = per_cu <= 2 || (per_cu == 3 && units(kDenseWaves) > cus);
+  if ((few || p.nKt <= kShortMaxTiles) && !p.long_key_kernel) {
     p.queue_next = nullptr;
-    p.sec_units[0] = units(kShortWaves);
+    p.sec_units[0] = n4;
     hipLaunchKernelGGL((attn_fwd_kernel<FP8, false, kShortWaves, POW2>), dim3(blocks_of(p.sec_units[0])), dim3(64 * kShortWaves), 0, st, p);
     return hipGetLastError();
   }

@@ -20,7 +20,7 @@ constexpr int kPartialBytes = 64 * 64 * 4 + 4 * 64 * 4;
 constexpr int kMaxPartWorkgroups = 512;
 constexpr int kSections = 3;     // sections of a long dense launch
 constexpr int kQueueSlots = 64;  // ints set aside for their positions, in front of the arrival counters
-constexpr int kShortMaxTiles = 16;  // dense calls with at most this many key tiles run the short-key kernel
+constexpr int kShortMaxTiles = 16;  // dense calls with at most this many key tiles never run the long-key kernel by themselves
 
 // Where each intermediate lives inside the caller's workspace (byte offsets, 256-aligned).
 struct WsPlan {

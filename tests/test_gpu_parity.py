@@ -101,6 +101,29 @@ def test_rectangular(Sq, Sk):
     _run_and_check(1, Sq, Sk, 3, seed=Sq + Sk)
 
 
+@pytest.mark.parametrize("fp8", [False, "pow2", True])
+@pytest.mark.parametrize("B,Sq,Sk,H", [(1, 1, 97, 1), (1, 31, 129, 3), (2, 33, 255, 2), (1, 64, 1025, 2), (1, 65, 96, 5), (1, 97, 3000, 3),
+                                       (1, 641, 1089, 24)])
+def test_few_query_blocks(B, Sq, Sk, H, fp8):
+    """Calls whose 32-query blocks hardly outnumber the CUs: key counts around whole half tiles (some of the four waves with
+    one half tile more than others, the last one partial), a lone query, halves of a 64-query fp8 scale block beyond the end, and
+    the short-key form on more than 16 key tiles (the last).  Bounded and running-maximum softmax."""
+    _run_and_check(B, Sq, Sk, H, seed=Sq + Sk, weight_random=True, fp8=fp8)
+    if not fp8:
+        _run_and_check(B, Sq, Sk, H, seed=Sq + Sk, weight_scale=4.0, bf16_operands=True)
+
+
+@pytest.mark.parametrize("valid", [0, 1, 33, 64, 230])
+def test_few_query_blocks_masked(valid):
+    """Fewer valid keys than the waves of a workgroup have shares for, none among them, and running-maximum softmax with
+    empty shares."""
+    mask = torch.zeros((2, 300), dtype=torch.bool)
+    mask[0, 300 - valid:] = True
+    mask[1, ::2] = True
+    _run_and_check(2, 77, 300, 2, seed=valid, mask=mask, weight_random=True)
+    _run_and_check(2, 77, 300, 2, seed=valid, mask=mask, weight_scale=4.0, bf16_operands=True)
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("mode", [1, 2])
 @pytest.mark.parametrize("Sq,Sk", [(5, 300), (300, 5), (513, 129), (200, 2100)])
