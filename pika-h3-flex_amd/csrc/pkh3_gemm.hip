@@ -519,6 +519,94 @@ __global__ __launch_bounds__(64 * kGemmWaves, TB == 8 ? 1 : 2) void gemm_kernel(
   else epilogue_rows<TB, false, false>(p, tg, head, tok0, acc);
 }
 
+// The down-projections (x A^T: 128 features per adapter) of few tokens.  gemm_kernel gives them a workgroup per 64 tokens x 256
+// features, which walks all of K while most CUs have none (1,085 tokens: 17 or 34 workgroups).  Here a workgroup is
+// 32 tokens x 64 features and its eight waves share K out: no two of them read the same images, so the images go from the L2
+// straight into the registers of the MFMAs, four chunks ahead, without LDS or barrier; the partial sums meet in LDS, in the
+// order of the shares.  Bound by the CU's 64 bytes per clock of vector loads (6 KiB per 8 MFMAs), which is why the rule in
+// launch_gemm leaves larger calls to the form that shares its copies.
+// A block's two launches of them together (K 3,072; whole block before and after): 500 tokens 149 -> 116 us, 1,085 198 -> 164,
+// 2,340 324 -> 307, 4,000 552 -> 530.
+constexpr int kThinWaves = 8, kThinTokens = 32, kThinFeatures = 64;
+
+__global__ __launch_bounds__(64 * kThinWaves, 2) void gemm_thin_kernel(GemmParams p, int n_tiles) {
+  constexpr int kGroup = 4;                              // chunks asked for together
+  __shared__ __attribute__((aligned(16))) char part[kThinWaves * 8 * 1024];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int total = (p.M + kThinTokens - 1) / kThinTokens * n_tiles;
+  const int per_xcd = (total + 7) / 8;                   // a contiguous run of token tiles per XCD
+  const int lin = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per_xcd || lin >= total) return;
+  const int m_tile = lin / n_tiles;
+  int n_tile = lin % n_tiles, t = 0;
+  while (t + 1 < p.n_targets && n_tile >= p.tg[t].n / kThinFeatures) n_tile -= p.tg[t].n / kThinFeatures, ++t;
+  const GemmTarget& tg = p.tg[t];
+  const char* x0 = p.a_img + (int64_t)(m_tile * 2) * p.a_blk_stride;
+  const char* w0 = tg.w_img + (int64_t)(n_tile * 4) * tg.w_blk_stride;
+  const int k0 = wave * p.nk1 / kThinWaves, k1 = (wave + 1) * p.nk1 / kThinWaves;
+  struct Images { bf16x8 x[kGroup][2], w[kGroup][4]; };
+  auto fetch = [&](Images& im, int kc) {                 // chunks past the share: its last one again, not used
+#pragma unroll
+    for (int u = 0; u < kGroup; ++u) {
+      const int64_t at = (int64_t)min(kc + u, k1 - 1) * 1024 + lane * 16;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) im.x[u][i] = *(const bf16x8*)(x0 + i * p.a_blk_stride + at);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) im.w[u][i] = *(const bf16x8*)(w0 + i * tg.w_blk_stride + at);
+    }
+  };
+  f32x4 acc[2][4];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int fb = 0; fb < 4; ++fb) acc[i][fb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto use = [&](const Images& im, int kc) {
+#pragma unroll
+    for (int u = 0; u < kGroup; ++u) {
+      if (kc + u >= k1) break;
+#pragma unroll
+      for (int fb = 0; fb < 4; ++fb)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) acc[i][fb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(im.w[u][fb], im.x[u][i], acc[i][fb], 0, 0, 0);
+    }
+  };
+  if (k0 < k1) {
+    Images a, b;
+    fetch(a, k0);
+#pragma unroll 1
+    for (int kc = k0; kc < k1; kc += 2 * kGroup) {
+      fetch(b, kc + kGroup);
+      __builtin_amdgcn_sched_barrier(0);
+      use(a, kc);
+      __builtin_amdgcn_sched_barrier(0);
+      if (kc + kGroup < k1) {
+        fetch(a, kc + 2 * kGroup);
+        __builtin_amdgcn_sched_barrier(0);
+        use(b, kc + kGroup);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int fb = 0; fb < 4; ++fb) *(f32x4*)(part + wave * 8192 + ((i * 4 + fb) * 64 + lane) * 16) = acc[i][fb];
+  __syncthreads();
+  // wave (i, fb) adds up token block i, feature block fb: lane (g, c) = token c, elements 32*ks + 8*g + 4*(fb%2) .. +3 of the
+  // head, ks = fb/2 of its 64-feature half: half of this lane's piece of image ks (see epilogue_a)
+  f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < kThinWaves; ++j) sum += *(const f32x4*)(part + j * 8192 + (wave * 64 + lane) * 16);
+  const int i = wave >> 2, fb = (n_tile & 1) * 4 + (wave & 3), blk = m_tile * 2 + i;
+  const float scale = blk * 16 + (lane & 15) < p.M ? tg.out_scale : 0.f;
+  bf16x4 o;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) o[r] = (__bf16)(sum[r] * scale);
+  char* rec = tg.out + (int64_t)(n_tile >> 1) * tg.out_head_stride + (int64_t)blk * tg.out_blk_stride;
+  *(bf16x4*)(rec + ((fb >> 1) * 64 + lane) * 16 + 8 * (fb & 1)) = o;
+}
+
 // Tokens per workgroup of a launch (16 * 2 * TB).  Time of a CU's share of the launch, in units of 100 us for K = 3,072 with an
 // adapter, from the workgroups it runs: one alone on the CU, and two (side by side for the smaller forms, one after the
 // other for TB = 8).  Measured at 1,085, 15,342 and 48,360 tokens x 9,216 and 3,072 features: TB = 8 67 us alone, 79 - 84 us
@@ -554,6 +642,22 @@ hipError_t launch_gemm(const GemmParams& p, hipStream_t st) {
   hipError_t e = device_cu_count(&cus);
   if (e != hipSuccess) return e;
   if (cus <= 0) cus = 1;
+  // Thin tiles for launches of down-projections only, up to three of them per CU: measured against the other form (whole block)
+  // two 64-feature tiles a 32-token tile gain 15 us at 1,085 tokens, 22 at 4,000, 5 at 9,360 and nothing at 11,700; six gain 15 at
+  // 1,085, nothing at 4,000 and lose 10 at 9,360.
+  int thin_tiles = 0;
+  for (int t = 0; t < p.n_targets; ++t) {
+    const GemmTarget& tg = p.tg[t];
+    if (tg.epi != kEpiAImg || tg.nk2 || tg.bias || tg.n % 128) { thin_tiles = -1; break; }
+    thin_tiles += tg.n / kThinFeatures;
+  }
+  if (thin_tiles > 0) {
+    const int64_t total = (int64_t)((p.M + kThinTokens - 1) / kThinTokens) * thin_tiles;
+    if (total <= 3 * cus) {
+      hipLaunchKernelGGL(gemm_thin_kernel, dim3((unsigned)(total + 7) / 8 * 8), dim3(64 * kThinWaves), 0, st, p, thin_tiles);
+      return hipGetLastError();
+    }
+  }
   switch (gemm_token_blocks(p.M, p.n_tiles, cus)) {
     case 8: return launch_gemm_tb<8>(p, cus, st);
     case 4: return launch_gemm_tb<4>(p, cus, st);

@@ -261,6 +261,28 @@ def test_gemm_forms_of_the_out_projection(S, N, gate, residual):
     assert bool((err <= ref.abs() / 256 + 5e-3).all())
 
 
+@pytest.mark.parametrize("S,K", [(1, 32), (31, 96), (33, 256), (65, 288), (300, 2080), (1085, 3072), (12289, 64)])
+def test_forms_of_the_down_projection(S, K):
+    """The adapter's path alone (the layer's own weight is zero): fewer k-chunks than the eight waves that share them, shares of
+    unequal length, shares that are not whole groups of four, a lone row; the last case takes the large-call form."""
+    from pika_h3_flex_amd import projections as P
+
+    o = _r(S, K, seed=11).to(torch.bfloat16).cuda()
+    lin = _linear(128, K, 12, bias=False)
+    lin["weight"] = torch.zeros_like(lin["weight"])
+    y = P.out_proj(o, _packed(lin))
+    xa = lin["lora_scale"] * (o.float() @ lin["lora_a"].cuda().float().t())
+    b = lin["lora_b"].cuda().float()
+    ref = xa @ b.t()
+    torch.cuda.synchronize()
+    # the bf16 rounding of the result (2^-8 of its size at most) and of the 128 down-projected values, at most 2^-8 of each:
+    # six times the spread of their sum
+    bound = ref.abs() / 256 + 6.0 / 256 * ((xa * xa) @ (b * b).t()).sqrt()
+    err = (y.float() - ref).abs()
+    print(f"down-projection S={S} K={K}: worst {(err / bound).max().item():.3f} of the bound", flush=True)
+    assert bool((err <= bound).all())
+
+
 @pytest.mark.parametrize("S,H", [(300, 2), (1000, 3), (257, 1)])
 def test_adapters_in_one_buffer_give_the_same_bits(S, H):
     """``PackedLinear.share_adapter_buffer`` lays the three down-projection images one behind the other, and
