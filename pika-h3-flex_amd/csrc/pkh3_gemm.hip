@@ -501,7 +501,9 @@ __global__ __launch_bounds__(64 * kGemmWaves, TB == 8 ? 1 : 2) void gemm_kernel(
   f32x4 acc[TB][8];
   if (tg.epi == kEpiVImg) {
     gemm_loop<TB, true>(p, tg, m_tile, n_tile, head_live, lds_raw, acc);
-    if (head_live && tok0 < p.M) epilogue_v<TB>(p, tg, head, tok0, acc);
+    // by the 64-token record, not by the wave's own tokens: with TB == 2 a wave holds half a record, and a half without tokens
+    // is written as zeros (kernels that walk whole 64-key tiles multiply it by probabilities of 0)
+    if (head_live && (tok0 & ~63) < p.M) epilogue_v<TB>(p, tg, head, tok0, acc);
     return;
   }
   gemm_loop<TB, false>(p, tg, m_tile, n_tile, head_live, lds_raw, acc);

@@ -234,6 +234,40 @@ def test_gemm_forms_of_the_qkv_projection(S, H, K, fp8, mode):
     assert rows >= (0.99 if fp8 else 0.999)
 
 
+@pytest.mark.parametrize("S,H,variant", [(1, 1, "dense"), (31, 3, "dense"), (129, 2, "dense"), (449, 3, "dense"), (129, 2, "fp8"),
+                                         (31, 32, "sparse"), (31, 2, "sparse"), (257, 32, "sparse"), (449, 2, "sparse_pow2"),
+                                         (641, 24, "dense"), (3585, 24, "dense"), (1025, 24, "sparse")])
+def test_qkv_projection_writes_whole_key_tiles(S, H, variant):
+    """S % 64 in 1 .. 32: the second half of the last K/V record holds no key.  The kernels that walk whole 64-key tiles still
+    multiply its V images (by probabilities of 0), so the projection has to write it whatever the workspace held before: here
+    NaN in every byte pair.  All three workgroup heights of the GEMM; the long-key and the 8-wave block-sparse kernels."""
+    import pika_h3_flex_amd as pk
+    from pika_h3_flex_amd import projections as P
+
+    K = 96
+    x = _r(S, K, seed=1).to(torch.bfloat16).cuda()
+    packed = [_packed(_linear(H * D, K, 20 + 10 * i, bias=False), head_perm=i < 2) for i in range(3)]
+    opts = dict(q_norm_weight=torch.ones(D).cuda(), k_norm_weight=torch.ones(D).cuda(), long_key_kernel=True)
+    if variant.startswith("sparse"):
+        n = (S + 63) // 64
+        keep = (torch.rand((n, n), generator=torch.Generator().manual_seed(2)) < 0.5) | torch.eye(n, dtype=torch.bool)
+        keep[:, n - 1] = True
+        opts["block_mask"] = pk.BlockMask.from_dense(keep, device="cuda")
+    opts["fp8_qk"] = {"fp8": True, "sparse_pow2": "pow2"}.get(variant, False)
+    outs = []
+    for fill in (0x00, 0xFF):
+        made = []
+
+        def workspace(device, nbytes):
+            made.append(torch.full((nbytes,), fill, dtype=torch.uint8, device=device))
+            return made[0]
+
+        outs.append(P.qkv_attention(P.pack_rows(x), S, *packed, heads=H, workspace=workspace, **opts))
+    torch.cuda.synchronize()
+    print(f"S={S} H={H} {variant}: {int(torch.isnan(outs[1].float()).sum())} NaN", flush=True)
+    assert torch.isfinite(outs[1].float()).all() and torch.equal(outs[0], outs[1])
+
+
 @pytest.mark.parametrize("S,N", [(65, 256), (1471, 3072), (1537, 2944), (3583, 3072), (3649, 2944)])
 @pytest.mark.parametrize("gate,residual", [(True, True), (True, False), (False, True), (False, False)])
 def test_gemm_forms_of_the_out_projection(S, N, gate, residual):
