@@ -394,13 +394,13 @@ __device__ __forceinline__ void epilogue_a(const GemmParams& p, const GemmTarget
     const int blk = tok0 + 16 * t;
     float x[32];
     acc_block<TB == 8>(x, acc[t]);
-    const float scale = blk + c < p.M ? tg.out_scale : 0.f;
+    const bool valid = blk + c < p.M;                  // rows past the end are zeros, whatever their activations held
     char* rec = tg.out + (int64_t)head * tg.out_head_stride + (int64_t)(blk >> 4) * tg.out_blk_stride;
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
       bf16x8 v;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = (__bf16)(x[ks * 8 + j] * scale);
+      for (int j = 0; j < 8; ++j) v[j] = valid ? (__bf16)(x[ks * 8 + j] * tg.out_scale) : (__bf16)0.0f;
       *(bf16x8*)(rec + (ks * 64 + lane) * 16) = v;
     }
   });
@@ -601,10 +601,10 @@ __global__ __launch_bounds__(64 * kThinWaves, 2) void gemm_thin_kernel(GemmParam
 #pragma unroll
   for (int j = 0; j < kThinWaves; ++j) sum += *(const f32x4*)(part + j * 8192 + (wave * 64 + lane) * 16);
   const int i = wave >> 2, fb = (n_tile & 1) * 4 + (wave & 3), blk = m_tile * 2 + i;
-  const float scale = blk * 16 + (lane & 15) < p.M ? tg.out_scale : 0.f;
+  const bool valid = blk * 16 + (lane & 15) < p.M;       // rows past the end are zeros, whatever their activations held
   bf16x4 o;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) o[r] = (__bf16)(sum[r] * scale);
+  for (int r = 0; r < 4; ++r) o[r] = valid ? (__bf16)(sum[r] * tg.out_scale) : (__bf16)0.0f;
   char* rec = tg.out + (int64_t)(n_tile >> 1) * tg.out_head_stride + (int64_t)blk * tg.out_blk_stride;
   *(bf16x4*)(rec + ((fb >> 1) * 64 + lane) * 16 + 8 * (fb & 1)) = o;
 }

@@ -317,6 +317,35 @@ def test_forms_of_the_down_projection(S, K):
     assert bool((err <= bound).all())
 
 
+@pytest.mark.parametrize("S", [1, 17, 40, 300, 12290])
+def test_down_projected_rows_past_the_end_are_zero(S):
+    """Image rows past S are unwritten memory when the attention kernel left the activations (here NaN): the down-projected rows
+    they give are zeros all the same, in the thin and in the large-call form (the last size)."""
+    import ctypes as C
+
+    from pika_h3_flex_amd import _lib
+    from pika_h3_flex_amd import projections as P
+
+    K = 96
+    lin = _packed(_linear(128, K, 12))
+    img = P.pack_rows(_r(S, K, seed=11).to(torch.bfloat16).cuda())
+    cells = img.view(torch.bfloat16).view(-1, K // 32, 4, 16, 8)               # [16-row block, k-step, g, row, j]
+    rows = torch.arange(cells.shape[0] * 16, device="cuda").view(-1, 1, 1, 16, 1)
+    cells.masked_fill_(rows >= S, float("nan"))
+    scratch = torch.full((P.packed_bytes(S, 128),), 0xFF, dtype=torch.uint8, device="cuda")
+    y = torch.empty((S, 128), dtype=torch.bfloat16, device="cuda")
+    a = _lib.OutArgs()
+    a.o_img, a.S, a.K, a.N = img.data_ptr(), S, K, 128
+    a.proj = lin.c_struct()
+    a.y, a.y_stride = y.data_ptr(), 128
+    a.lora_workspace, a.lora_workspace_bytes = scratch.data_ptr(), scratch.numel()
+    _lib.check(_lib.load().pkh3_out_proj(C.byref(a), C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    torch.cuda.synchronize()
+    assert torch.isfinite(y.float()).all()
+    tail = _unpack(scratch, (S + 15) // 16 * 16, 128)[S:]
+    assert torch.count_nonzero(tail) == 0 and torch.isfinite(tail.float()).all()
+
+
 @pytest.mark.parametrize("S,H", [(300, 2), (1000, 3), (257, 1)])
 def test_adapters_in_one_buffer_give_the_same_bits(S, H):
     """``PackedLinear.share_adapter_buffer`` lays the three down-projection images one behind the other, and
