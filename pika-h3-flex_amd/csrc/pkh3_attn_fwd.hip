@@ -33,6 +33,7 @@
 // Phase 1 walks the key tiles all four row-blocks keep, exactly like the dense kernel.  Phase 2 walks the
 // remaining tiles per row-block: every iteration gives each wave pair one 32-key half of a tile of its own
 // list in its own LDS area, so all 8 waves stay busy.  The lists are built on the device by a plan kernel.
+#include <float.h>
 #include <limits.h>
 
 #include <atomic>
@@ -49,6 +50,9 @@ constexpr int kMinPartTiles = 24;  // ... and fewest key tiles such a workgroup 
 constexpr int kSparseWaves = 2 * kSparseRows;  // block-sparse: a wave pair per row-block; two such workgroups share a CU
 constexpr int kRing = 3;               // LDS ring depth (tiles)
 constexpr float kRescaleSlack = 8.0f;  // the running max is only raised when exceeded by 2^8
+// The running max before the first key.  Finite: keys whose logits are all -inf then weigh exp2(-inf - max) = 0, wherever
+// among a wave's keys they lie, and two shares without a key meet as exp2(0) times a row sum of 0.
+constexpr float kNoMax = -FLT_MAX;
 constexpr float kStaticMaxLimit = 48.0f;  // rows whose |logit| bound is below this skip the running max (terms 2^-48 .. 2^48)
 
 #define PKH3_SGB(mask, n) __builtin_amdgcn_sched_group_barrier(mask, n, 0)
@@ -597,7 +601,7 @@ __device__ __forceinline__ void attn_fwd_body(const FwdParams& p, int blk, int u
     for (int qb = 0; qb < 2; ++qb)
 #pragma unroll
       for (int i = 0; i < 4; ++i) w.o[db][qb][i] = 0.f;
-  w.m[0] = w.m[1] = -INFINITY;
+  w.m[0] = w.m[1] = kNoMax;
   w.l[0] = w.l[1] = 0.f;
   const float c = POW2 ? 1.0f : p.c * qscale;  // what the softmax still multiplies the logits by (fp8 absmax form only)
   const float* kscale = FP8 ? p.kscale + (int64_t)bh * p.nKt : nullptr;
@@ -798,8 +802,8 @@ __device__ __forceinline__ void attn_fwd_body(const FwdParams& p, int blk, int u
           float a1 = src == 0 ? 0.0f : 1.0f, a2 = 1.0f;
           if (!static_max && src != 0) {
             const float mn = fmaxf(w.m[qb], m2);
-            a1 = mn == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(w.m[qb] - mn);
-            a2 = mn == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m2 - mn);
+            a1 = __builtin_amdgcn_exp2f(w.m[qb] - mn);
+            a2 = __builtin_amdgcn_exp2f(m2 - mn);
             w.m[qb] = mn;
           } else if (src == 0) {
             w.m[qb] = m2;
@@ -1092,7 +1096,7 @@ __global__ __launch_bounds__(64 * kNarrowWaves, 2) void attn_fwd_narrow_kernel(F
   for (int db = 0; db < 8; ++db)
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) w.o[db][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  w.m[0] = w.m[1] = -INFINITY;
+  w.m[0] = w.m[1] = kNoMax;
   w.l[0] = w.l[1] = 0.f;
   __syncthreads();
 #pragma unroll
@@ -1125,14 +1129,14 @@ __global__ __launch_bounds__(64 * kNarrowWaves, 2) void attn_fwd_narrow_kernel(F
   __syncthreads();
 #pragma unroll
   for (int qb = 0; qb < 2; ++qb) {
-    float top = -INFINITY, l = 0.f, a[NW];
+    float top = kNoMax, l = 0.f, a[NW];
     if (!static_max) {
 #pragma unroll
       for (int j = 0; j < NW; ++j) top = fmaxf(top, part_m[j][qb][c16]);
     }
 #pragma unroll
     for (int j = 0; j < NW; ++j) {
-      a[j] = static_max ? 1.0f : top == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(part_m[j][qb][c16] - top);
+      a[j] = static_max ? 1.0f : __builtin_amdgcn_exp2f(part_m[j][qb][c16] - top);
       l += a[j] * part_l[j][qb][c16];
     }
     const float inv = l > 0.f ? 1.0f / l : 0.f;

@@ -124,6 +124,33 @@ def test_few_query_blocks_masked(valid):
     _run_and_check(2, 77, 300, 2, seed=valid, mask=mask, weight_scale=4.0, bf16_operands=True)
 
 
+@pytest.mark.parametrize("first,last", [(128, 192), (0, 64), (96, 160), (384, 512)])
+@pytest.mark.parametrize("sparse", [False, True])
+@pytest.mark.parametrize("H", [1, 180])
+def test_runs_of_keys_with_logits_of_minus_infinity(first, last, sparse, H):
+    """Keys first .. last - 1 have an element of -inf against positive query elements: their logits are -inf and they weigh
+    nothing, also where they are the first keys, or all the keys, that one of the waves sharing the keys out walks (one head:
+    a wave takes 128 of the 512 keys; 180 heads: one wave walks them all)."""
+    import pika_h3_flex_amd as pk
+
+    O = _oracle()
+    gen = torch.Generator().manual_seed(first + H)
+    q, k, v = _rand((1, 80, H, 128), gen), _rand((1, 512, H, 128), gen), _rand((1, 512, H, 128), gen)
+    q[..., 0] = q[..., 0].abs() + 0.5
+    k[:, first:last, :, 0] = -math.inf
+    opts = dict(block_mask=pk.BlockMask.from_dense(torch.ones((2, 8), dtype=torch.bool), device="cuda")) if sparse else {}
+    mask = torch.ones((1, 512), dtype=torch.bool)
+    mask[:, first:last] = False
+    ref = O.reference_layer(q, torch.nan_to_num(k, neginf=0.0), v, key_mask=mask)
+    for long_form in (False, True):
+        out = pk.attention(q.cuda(), k.cuda(), v.cuda(), long_key_kernel=long_form, **opts)
+        torch.cuda.synchronize()
+        assert torch.isfinite(out.float()).all(), long_form
+        err, cos = O.max_abs_and_cosine(out.cpu(), ref)
+        print(f"-inf keys {first}..{last - 1} sparse={sparse} H={H} long_form={long_form}: max_abs={err:.3e} cos={cos:.7f}", flush=True)
+        assert err <= MAX_ABS and cos >= MIN_COS
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("mode", [1, 2])
 @pytest.mark.parametrize("Sq,Sk", [(5, 300), (300, 5), (513, 129), (200, 2100)])
