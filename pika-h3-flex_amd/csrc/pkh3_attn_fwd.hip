@@ -949,35 +949,33 @@ __device__ __forceinline__ void narrow_loop(WaveState<FP8>& w, i32x4 (&kf)[FP8 ?
     const int tile_next = walk(n >> 1);
     const char* v = kv + (int64_t)tile * tile_stride + kKBytes + (i & 1) * (kVTileBytes / 2);
     const float ks = FP8 ? uniform_load(kscale, tile) : 1.0f;
+    // (a sparse list may go on behind the short last tile, whose second half then holds no key: lim <= 0, probabilities of 0)
     const int lim = sk - 64 * tile - 32 * (i & 1);
-    const bool live = !SPARSE || lim > 0;   // (wave-uniform) the second half of a short last tile holds nothing
-    if (live) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) w.vf[j] = *(const bf16x8*)(v + (j * 64 + lane) * 16);
-      __builtin_amdgcn_sched_barrier(0);
-      if constexpr (!FP8) {
+    for (int j = 0; j < 8; ++j) w.vf[j] = *(const bf16x8*)(v + (j * 64 + lane) * 16);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (!FP8) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
+      for (int j = 0; j < 8; ++j)
 #pragma unroll
-          for (int qb = 0; qb < 2; ++qb)
-            w.s[j & 1][qb] = PKH3_MFMA16(__builtin_bit_cast(bf16x8, kf[j]), w.qf[qb][j >> 1], j < 2 ? zero : w.s[j & 1][qb]);
-      } else {
-        const int ke = e8m0_of(ks);
+        for (int qb = 0; qb < 2; ++qb)
+          w.s[j & 1][qb] = PKH3_MFMA16(__builtin_bit_cast(bf16x8, kf[j]), w.qf[qb][j >> 1], j < 2 ? zero : w.s[j & 1][qb]);
+    } else {
+      const int ke = e8m0_of(ks);
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-          const i32x4 a0 = kf[2 * kb], a1 = kf[2 * kb + 1];
-          const i32x8 a = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
+      for (int kb = 0; kb < 2; ++kb) {
+        const i32x4 a0 = kf[2 * kb], a1 = kf[2 * kb + 1];
+        const i32x8 a = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
 #pragma unroll
-          for (int qb = 0; qb < 2; ++qb)
-            w.s[kb][qb] = POW2 ? PKH3_MFMA16_F8S(a, w.q8[qb], zero, ke, w.qe) : PKH3_MFMA16_F8(a, w.q8[qb], zero);
-        }
+        for (int qb = 0; qb < 2; ++qb)
+          w.s[kb][qb] = POW2 ? PKH3_MFMA16_F8S(a, w.q8[qb], zero, ke, w.qe) : PKH3_MFMA16_F8(a, w.q8[qb], zero);
       }
     }
     const char* k = kv + (int64_t)tile_next * tile_stride + (n & 1) * (kKBytes / 2);
 #pragma unroll
     for (int j = 0; j < (FP8 ? 4 : 8); ++j) kf[j] = *(const i32x4*)(k + (j * 64 + lane) * 16);
     __builtin_amdgcn_sched_barrier(0);
-    if (live) softmax_pv_half<FP8, STATIC, false, false, POW2>(w, (FP8 && !POW2) ? c * ks : c, lim, lane);
+    softmax_pv_half<FP8, STATIC, false, false, POW2>(w, (FP8 && !POW2) ? c * ks : c, lim, lane);
     tile = tile_next;
   }
   PKH3_MFMA_DRAIN(w);

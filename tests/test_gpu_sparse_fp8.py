@@ -93,6 +93,29 @@ def test_block_sparse_full_map_equals_dense():
     assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("long_form", [False, True])
+@pytest.mark.parametrize("fp8", [False, True, "pow2"])
+@pytest.mark.parametrize("last", [1, 20, 32, 33])
+def test_block_sparse_list_goes_on_behind_a_short_last_tile(last, fp8, long_form):
+    """All row-blocks keep the last key tile, which holds ``last`` keys, and each one more of its own: the tiles kept by all are
+    walked first, so the half tile without keys (``last`` <= 32) lies in the middle of a wave's walk.  Bounded and
+    running-max softmax."""
+    import pika_h3_flex_amd as pk
+    from oracle import attention_oracle as O
+
+    q, k, v, gen = _inputs(1, 250, 256 + last, 2, seed=last)
+    tm = torch.eye(4, 5, dtype=torch.bool)
+    tm[:, 4] = True
+    for scale in (1.0, 4.0):
+        w = torch.full((D,), scale)
+        ref = O.reference_layer(q, k, v, q_norm_weight=w, k_norm_weight=torch.ones(D), tile_map=tm, fp8_qk=fp8, bf16_operands=scale > 1 and not fp8)
+        out = _call(q, k, v, q_norm_weight=w.cuda(), k_norm_weight=_ones(), fp8_qk=fp8, long_key_kernel=long_form,
+                    block_mask=pk.BlockMask.from_dense(tm, device="cuda"))
+        err, cos = O.max_abs_and_cosine(out, ref)
+        print(f"last tile of {last} keys fp8={fp8} weight {scale} long_form={long_form}: max_abs={err:.3e} cos={cos:.7f}", flush=True)
+        assert cos >= (0.995 if fp8 else 0.9999) and (fp8 or err <= 2e-2)
+
+
 def test_block_sparse_empty_rows_are_zero():
     import pika_h3_flex_amd as pk
 
