@@ -164,13 +164,14 @@ def load() -> C.CDLL:
 
 
 BENCH_LIB_PATH = os.path.join(os.path.dirname(LIB_PATH), "libpkh3attn_bench.so")
-BENCH_EXPORTS = ("pkh3_attn_time_kernel",)   # include/pkh3_attn_bench.h
+BENCH_EXPORTS = ("pkh3_attn_time_kernel", "pkh3_attn_form")   # include/pkh3_attn_bench.h
+FORM_LONG, FORM_SHORT, FORM_NARROW, FORM_SPARSE = 0, 1, 2, 3    # results of pkh3_attn_form
 _bench = None
 
 
 def load_bench() -> C.CDLL:
-    """The measurement library (``libpkh3attn_bench.so``, the one call that synchronises with the device): for
-    benchmark harnesses only, never loaded by the product path.  It links against the product library, which is
+    """The measurement library (``libpkh3attn_bench.so``, with the one call that synchronises with the device): for
+    benchmark harnesses and tests only, never loaded by the product path.  It links against the product library, which is
     loaded first so that both share one copy of it."""
     global _bench
     if _bench is not None:
@@ -181,6 +182,8 @@ def load_bench() -> C.CDLL:
     lib = C.CDLL(BENCH_LIB_PATH)
     lib.pkh3_attn_time_kernel.argtypes = [C.POINTER(AttnArgs), C.c_void_p, C.c_int, C.POINTER(C.c_float)]
     lib.pkh3_attn_time_kernel.restype = C.c_int
+    lib.pkh3_attn_form.argtypes = [C.POINTER(AttnArgs), C.c_int]
+    lib.pkh3_attn_form.restype = C.c_int
     _bench = lib
     return lib
 

@@ -303,6 +303,18 @@ int prepare_call(const pkh3_attn_args* a, hipStream_t st, FwdParams* out) {
   return PKH3_OK;
 }
 
+// The parameters of the call's attention launch without launching anything, from shapes and options alone (pointers are only
+// looked at for NULL).  For the measurement library as well.
+int call_params(const pkh3_attn_args* a, FwdParams* out) {
+  int rc = validate(a, false);
+  if (rc) return rc;
+  Launch L;
+  build(a, nullptr, L);
+  *out = L.f;
+  g_err[0] = 0;
+  return PKH3_OK;
+}
+
 int report_error(int code, const char* text) { return fail(code, "%s", text); }
 
 }  // namespace pkh3

@@ -34,7 +34,6 @@
 // remaining tiles per row-block: every iteration gives each wave pair one 32-key half of a tile of its own
 // list in its own LDS area, so all 8 waves stay busy.  The lists are built on the device by a plan kernel.
 #include <float.h>
-#include <limits.h>
 
 #include <atomic>
 
@@ -1207,11 +1206,22 @@ static TailPlan plan_tail(int rest, int cus, int n_tiles, int64_t max_workgroups
   return best;
 }
 
-template <bool FP8, bool POW2 = false>
-static hipError_t launch_fp(FwdParams p, int cus, hipStream_t st) {
+// Which form of the kernel a call takes.
+AttnForm attn_form(const FwdParams& p, int cus) {
+  if (p.long_key_kernel) return p.plan ? kFormSparse : kFormLong;
+  cus = max(cus, 1);
   auto units = [&](int blocks) { return p.B * p.H * units_per_head(p.Sq, blocks); };
-  for (int i = 0; i < kSections; ++i) p.sec_units[i] = p.sec_blocks[i] = 0, p.sec_parts[i] = 1;
-  // Calls of at most two short-key workgroups per CU leave a long form's chip half empty, whatever the number of keys.  They
+  const int n4 = units(kShortWaves), n32 = units(1), n_half = (p.Sk + 31) / 32;
+  const int per_cu = (n4 + cus - 1) / cus;
+  // Block-sparse calls of at most four 32-query blocks per CU take the narrow form, whatever their maps (the kept tiles are
+  // known on the device only).  Narrow / 8-wave form, 24 heads, us, at densities 0.03, 0.1, 0.3 and 1: 641 rows (504 blocks) 8.1 / 12.6,
+  // 9.4 / 19.8, 10.6 / 22.3, 13.5 / 21.4; 900 rows (696) 13.1 / 16.6, 14.2 / 18.5, 16.3 / 27.4, 22.9 / 27.0; 1,300 rows (984)
+  // 14.4 / 15.9, 16.2 / 22.6, 21.6 / 32.6, 33.4 / 34.3 (fp8 15.8 / 15.9, 17.3 / 21.9, 21.2 / 30.7, 30.7 / 33.1).  From five blocks per CU
+  // on it is behind on some maps: 1,500 rows (1,128) 17.6 / 18.6, 20.7 / 24.0, 26.6 / 40.8, 45.2 / 39.2; 1,700 (1,296) 19.5 / 15.9,
+  // 22.5 / 22.7, 29.1 / 39.5, 55.4 / 41.9.  fp8 calls of many keys take it up to five blocks per CU: 10 heads x 4,000 rows (1,250),
+  // densities 0.06, 0.2, 0.5, 0.8 and 1: 26.3 / 29.0, 38.6 / 49.8, 60 / 68, 80 / 83, 88 / 84.
+  if (p.plan) return n32 <= (p.fp8 && n_half >= 96 ? 5 : 4) * cus ? kFormNarrow : kFormSparse;
+  // Dense calls of at most two short-key workgroups per CU leave a long form's chip half empty, whatever the number of keys.  They
   // take the narrow form where it is estimated shorter, else the short-key form.  The estimates are straight lines through
   // kernel times in microseconds (bf16; fp8 lies within a tenth of them): the narrow form, a start and a merge and 0.135 per half tile
   // for every 32-query block a CU gets; the short-key form, a half tile per 0.60 with one workgroup on a CU and per 0.87
@@ -1220,17 +1230,25 @@ static hipError_t launch_fp(FwdParams p, int cus, hipStream_t st) {
   // 816 x 34 27.3 / 26.3 / 38.5, 1,504 x 94 86 / 81 / 90, 1,896 x 79 95 / 73 / 78.  With three short-key workgroups per CU the
   // long form is ahead as long as its own workgroups are no more than the CUs (2,256 x 94: 114 / 94), and behind when a few
   // are left over for a second round (3,000 x 125: 165 / 218).
-  const int n4 = units(kShortWaves), n32 = units(1), n_half = (p.Sk + 31) / 32;
-  const int per_cu = cus > 0 ? (n4 + cus - 1) / cus : INT_MAX;
-  if (per_cu <= 2 && !p.long_key_kernel &&
-      3.2f + (n32 + cus - 1) / cus * (0.135f * n_half + 2.7f) < 5.0f + (per_cu == 1 ? 0.60f : 0.87f) * n_half) {
+  if (per_cu <= 2 && 3.2f + (n32 + cus - 1) / cus * (0.135f * n_half + 2.7f) < 5.0f + (per_cu == 1 ? 0.60f : 0.87f) * n_half) return kFormNarrow;
+  const bool few = per_cu <= 2 || (per_cu == 3 && units(kDenseWaves) > cus);
+  return few || p.nKt <= kShortMaxTiles ? kFormShort : kFormLong;
+}
+
+template <bool FP8, bool POW2 = false>
+static hipError_t launch_fp(FwdParams p, int cus, hipStream_t st) {
+  auto units = [&](int blocks) { return p.B * p.H * units_per_head(p.Sq, blocks); };
+  for (int i = 0; i < kSections; ++i) p.sec_units[i] = p.sec_blocks[i] = 0, p.sec_parts[i] = 1;
+  const AttnForm form = attn_form(p, cus);
+  if (form == kFormNarrow) {
+    const int n = units(1);
     p.queue_next = nullptr;
-    p.sec_units[0] = n32;
-    if (p.plan) hipLaunchKernelGGL((attn_fwd_narrow_kernel<FP8, POW2, true>), dim3(blocks_of(n32)), dim3(64 * kNarrowWaves), 0, st, p);
-    else hipLaunchKernelGGL((attn_fwd_narrow_kernel<FP8, POW2, false>), dim3(blocks_of(n32)), dim3(64 * kNarrowWaves), 0, st, p);
+    p.sec_units[0] = n;
+    if (p.plan) hipLaunchKernelGGL((attn_fwd_narrow_kernel<FP8, POW2, true>), dim3(blocks_of(n)), dim3(64 * kNarrowWaves), 0, st, p);
+    else hipLaunchKernelGGL((attn_fwd_narrow_kernel<FP8, POW2, false>), dim3(blocks_of(n)), dim3(64 * kNarrowWaves), 0, st, p);
     return hipGetLastError();
   }
-  if (p.plan) {
+  if (form == kFormSparse) {
     const int n = p.B * p.H * (p.nQ64 / kSparseRows);
     p.sec_units[0] = n;
     int wgs = n;
@@ -1245,10 +1263,9 @@ static hipError_t launch_fp(FwdParams p, int cus, hipStream_t st) {
     hipLaunchKernelGGL((attn_fwd_kernel<FP8, true, kSparseWaves, POW2>), dim3(blocks_of(wgs)), dim3(64 * kSparseWaves), 0, st, p);
     return hipGetLastError();
   }
-  const bool few = per_cu <= 2 || (per_cu == 3 && units(kDenseWaves) > cus);
-  if ((few || p.nKt <= kShortMaxTiles) && !p.long_key_kernel) {
+  if (form == kFormShort) {
     p.queue_next = nullptr;
-    p.sec_units[0] = n4;
+    p.sec_units[0] = units(kShortWaves);
     hipLaunchKernelGGL((attn_fwd_kernel<FP8, false, kShortWaves, POW2>), dim3(blocks_of(p.sec_units[0])), dim3(64 * kShortWaves), 0, st, p);
     return hipGetLastError();
   }

@@ -1,11 +1,12 @@
-// libpkh3attn_bench.so: the measurement hook of include/pkh3_attn_bench.h, kept out of the product library because
-// it synchronises with the device.  Links against libpkh3attn.so and launches its attention kernel.
+// libpkh3attn_bench.so: the measurement and test hooks of include/pkh3_attn_bench.h, kept out of the product library because
+// one of them synchronises with the device.  Links against libpkh3attn.so and launches its attention kernel.
 #include "../../include/pkh3_attn_bench.h"
 
 #include "pkh3_internal.h"
 
 namespace pkh3 {
 int prepare_call(const pkh3_attn_args* a, hipStream_t st, FwdParams* out);  // pkh3_api.hip
+int call_params(const pkh3_attn_args* a, FwdParams* out);
 int report_error(int code, const char* text);                                // sets pkh3_last_error()
 }  // namespace pkh3
 
@@ -39,4 +40,10 @@ extern "C" int pkh3_attn_time_kernel(const pkh3_attn_args* a, void* stream, int 
   if (es != hipSuccess) return report_error(PKH3_EHIP, hipGetErrorString(es));
   *ms_out = ms / iters;
   return PKH3_OK;
+}
+
+extern "C" int pkh3_attn_form(const pkh3_attn_args* a, int cus) {
+  FwdParams f;
+  const int rc = call_params(a, &f);
+  return rc ? rc : (int)attn_form(f, cus);
 }

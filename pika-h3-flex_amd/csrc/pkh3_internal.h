@@ -186,6 +186,8 @@ hipError_t launch_fill_zero(unsigned* p, int n, hipStream_t st);
 hipError_t launch_mask_compact(const uint8_t* mask, int B, int Sk, int* idx, int* cnt, unsigned* zero_init, int H, hipStream_t st);
 hipError_t launch_kv_prologue(const QkPrologueParams& k, const VPrologueParams& v, hipStream_t st);
 hipError_t launch_attn_fwd(const FwdParams& p, hipStream_t st);
+enum AttnForm { kFormLong = 0, kFormShort = 1, kFormNarrow = 2, kFormSparse = 3 };
+AttnForm attn_form(const FwdParams& p, int cus);  // the form launch_attn_fwd takes on a device of `cus` CUs
 hipError_t device_cu_count(int* out);  // CUs of the current device (cached per device after the first call)
 hipError_t launch_sparse_plan(const int* row_ptr, const int* col_idx, int nRow64, int nQ64, int nKt, int* plan,
                               int plan_stride, int* plan_cnt, hipStream_t st);
