@@ -34,6 +34,8 @@
 // remaining tiles per row-block: every iteration gives each wave pair one 32-key half of a tile of its own
 // list in its own LDS area, so all 8 waves stay busy.  The lists are built on the device by a plan kernel.
 #include <float.h>
+#include <limits.h>
+#include <math.h>
 
 #include <atomic>
 
@@ -980,8 +982,13 @@ __device__ __forceinline__ void narrow_loop(WaveState<FP8>& w, i32x4 (&kf)[FP8 ?
   PKH3_MFMA_DRAIN(w);
 }
 
-template <bool FP8, bool POW2, bool SPARSE>
+// MASKED (key mask: how many keys are valid is known on the device only).  The start and the merge of every block of 32 queries are
+// worth it for long walks alone.  The launch holds the workgroups of both forms, and where fewer than p.few_halves half tiles are
+// valid it is the short-key ones (128 queries each, in front) that do the work.  24 heads x 1,558 rows, 23 of
+// 2,526 keys valid: 16.1 -> 8.9 us; 4 x 24 heads x 87 rows, 29 of 446: 7.2 -> 6.0.
+template <bool FP8, bool POW2, bool SPARSE, bool MASKED = false>
 __global__ __launch_bounds__(64 * kNarrowWaves, 2) void attn_fwd_narrow_kernel(FwdParams p) {
+  static_assert(!MASKED || (!FP8 && !SPARSE), "key masks are taken by dense bf16 calls only");
   constexpr int NW = kNarrowWaves;
   constexpr int kKBytes = FP8 ? kK8TileBytes : kKTileBytes;
   constexpr int kSlot = 64 * 64 * 4;                       // one wave's O^T in fp32
@@ -991,15 +998,28 @@ __global__ __launch_bounds__(64 * kNarrowWaves, 2) void attn_fwd_narrow_kernel(F
   __shared__ float s_n2[2], s_amax[4];
   const int lane = threadIdx.x & 63, c16 = lane & 15, g4 = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int nth = blockIdx.x >> 3;                               // of the workgroups of this XCD
+  if constexpr (MASKED) {
+    static_assert(kNarrowWaves == kShortWaves && fwd_lds_bytes<false, false, kShortWaves>() <= (int)sizeof(part), "a workgroup of the short-key form");
+    const int per_xcd4 = (p.sec_units[1] + 7) / 8;
+    if (nth < per_xcd4) {
+      const int unit = (blockIdx.x & 7) * per_xcd4 + nth;
+      if (unit >= p.sec_units[1] || (p.row_cnt[unit / units_per_head(p.Sq, kShortWaves) / p.H] + 31) / 32 >= p.few_halves) return;
+      attn_fwd_body<false, false, kShortWaves, false>(p, 0, 0, p.sec_units[1], 1, 0, 0, part, unit);
+      return;
+    }
+    nth -= per_xcd4;
+  }
   const int per_xcd = (p.sec_units[0] + 7) / 8;            // a contiguous run of (batch, head, query block) per XCD
-  const int lin = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  if ((int)(blockIdx.x >> 3) >= per_xcd || lin >= p.sec_units[0]) return;
+  const int lin = (blockIdx.x & 7) * per_xcd + nth;
+  if (nth >= per_xcd || lin >= p.sec_units[0]) return;
   const int nq = units_per_head(p.Sq, 1);
   const int bh = lin / nq, q32 = lin % nq;
   const int b = bh / p.H, h = bh % p.H;
   const int sk = p.row_cnt ? p.row_cnt[b] : p.Sk;
   TileWalk<SPARSE> walk{};
   int n_half = (sk + 31) / 32;
+  if (MASKED && n_half < p.few_halves) return;
   if constexpr (SPARSE) {
     // plan entry of this block's 256 queries, row-block of its 64 (the lists of attn_fwd_body, walked in the same order)
     const int entry = q32 / (2 * kSparseRows), r = (q32 / 2) % kSparseRows;
@@ -1235,6 +1255,20 @@ AttnForm attn_form(const FwdParams& p, int cus) {
   return few || p.nKt <= kShortMaxTiles ? kFormShort : kFormLong;
 }
 
+// Half tiles of valid keys from which a masked call of `n32` blocks of 32 queries (`n4` of 128) is better off in the narrow form: where
+// straight lines through kernel times in us meet.  Narrow: 5.9 while every CU has one block, then 2.6 and 4.2 for every round of two
+// blocks per CU, and 0.125 per half tile for every block a CU gets; short-key: 5.5 and 0.585 per half tile with one
+// workgroup on a CU, 8.0 and 0.80 with two.  Measured (narrow / short-key): 40 blocks x 1 half tile 6.0 / 5.9, x 2 6.1 / 6.4; 288 x 1
+// 7.1 / 6.0, x 4 7.5 / 7.8; 504 x 1 7.4 / 6.3, x 4 7.9 / 8.1; 656 x 1 10.8 / 6.4, x 16 16.4 / 15.3, x 32 22.0 / 24.3; 1,056 x 1
+// 15.4 / 8.6, x 16 22.9 / 21.0, x 32 33.2 / 33.2, x 75 59.4 / 64.7.
+static int narrow_from(int n32, int n4, int cus) {
+  const int per_cu = (n32 + cus - 1) / cus, rounds = (n32 + 2 * cus - 1) / (2 * cus);
+  const bool one = n4 <= cus;
+  const float start = (per_cu == 1 ? 5.9f : 2.6f + 4.2f * rounds) - (one ? 5.5f : 8.0f);
+  const float gain = (one ? 0.585f : 0.80f) - 0.125f * per_cu;   // per half tile
+  return gain > 0.f ? (int)ceilf(start / gain) : INT_MAX;
+}
+
 template <bool FP8, bool POW2 = false>
 static hipError_t launch_fp(FwdParams p, int cus, hipStream_t st) {
   auto units = [&](int blocks) { return p.B * p.H * units_per_head(p.Sq, blocks); };
@@ -1244,8 +1278,16 @@ static hipError_t launch_fp(FwdParams p, int cus, hipStream_t st) {
     const int n = units(1);
     p.queue_next = nullptr;
     p.sec_units[0] = n;
-    if (p.plan) hipLaunchKernelGGL((attn_fwd_narrow_kernel<FP8, POW2, true>), dim3(blocks_of(n)), dim3(64 * kNarrowWaves), 0, st, p);
-    else hipLaunchKernelGGL((attn_fwd_narrow_kernel<FP8, POW2, false>), dim3(blocks_of(n)), dim3(64 * kNarrowWaves), 0, st, p);
+    const dim3 grid(blocks_of(n)), block(64 * kNarrowWaves);
+    if (p.plan) {
+      hipLaunchKernelGGL((attn_fwd_narrow_kernel<FP8, POW2, true>), grid, block, 0, st, p);
+    } else if (!FP8 && p.row_cnt) {
+      p.sec_units[1] = units(kShortWaves);
+      p.few_halves = narrow_from(n, p.sec_units[1], cus);
+      hipLaunchKernelGGL((attn_fwd_narrow_kernel<false, false, false, true>), dim3(blocks_of(p.sec_units[1]) + blocks_of(n)), block, 0, st, p);
+    } else {
+      hipLaunchKernelGGL((attn_fwd_narrow_kernel<FP8, POW2, false>), grid, block, 0, st, p);
+    }
     return hipGetLastError();
   }
   if (form == kFormSparse) {

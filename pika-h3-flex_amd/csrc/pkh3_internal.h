@@ -97,6 +97,7 @@ struct FwdParams {
   size_t split_scratch_bytes;
   int* split_cnt;           // arrival counters; the kQueueSlots ints in front of them belong to the work queues
   int* queue_next;          // [kQueues] next unit of each work queue (= split_cnt - kQueueSlots), or null: fixed map
+  int few_halves;           // filled per launch (narrow form with a key mask): fewer half tiles of valid keys are walked as the short-key form does
   // filled per launch: the sections of the launch.  A unit is one workgroup's block of queries; section i covers
   // sec_units[i] units after those of the sections before it, sec_parts[i] workgroups per unit, in sec_blocks[i]
   // workgroup indices (a multiple of 8)

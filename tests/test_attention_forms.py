@@ -36,6 +36,12 @@ def test_block_sparse_calls_go_by_their_query_blocks(B, H, Sq, Sk, want, fp8):
     assert form(B, H, Sq, Sk, sparse=True, fp8=fp8, long_key_kernel=True) == SPARSE
 
 
+def test_masked_calls_go_by_the_padded_keys():
+    """(The valid ones are counted on the device: test_masked_calls_of_few_and_many_valid_keys in the GPU tests runs these.)"""
+    assert form(3, 24, 200, 400, masked=True) == form(3, 24, 500, 2040, masked=True) == NARROW
+    assert form(3, 8, 777, 777, masked=True) == SHORT and form(1, 24, 49640, 512, masked=True) == SHORT
+
+
 def test_form_of_a_bad_call_is_an_error():
     with pytest.raises(_lib.Pkh3Error):
         form(0, 1, 1, 1)

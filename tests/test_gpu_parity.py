@@ -124,6 +124,18 @@ def test_few_query_blocks_masked(valid):
     _run_and_check(2, 77, 300, 2, seed=valid, mask=mask, weight_scale=4.0, bf16_operands=True)
 
 
+@pytest.mark.parametrize("H,Sq,Sk,valid", [(24, 200, 400, (96, 97, 0)), (24, 200, 400, (1, 32, 33)), (24, 500, 2040, (1312, 1345, 1)),
+                                           (24, 500, 2040, (2040, 1311, 1313))])
+def test_masked_calls_of_few_and_many_valid_keys(H, Sq, Sk, valid):
+    """Batch entries on both sides of the number of valid keys below which a masked call of few query blocks is walked like the
+    short-key form (4 half tiles at the first size, 42 at the second), each by its own count, in one launch."""
+    mask = torch.zeros((3, Sk), dtype=torch.bool)
+    gen = torch.Generator().manual_seed(sum(valid))
+    for b, n in enumerate(valid):
+        mask[b, torch.randperm(Sk, generator=gen)[:n]] = True
+    _run_and_check(3, Sq, Sk, H, seed=sum(valid), mask=mask, weight_random=True)
+
+
 @pytest.mark.parametrize("first,last", [(128, 192), (0, 64), (96, 160), (384, 512)])
 @pytest.mark.parametrize("sparse", [False, True])
 @pytest.mark.parametrize("H", [1, 180])
