@@ -54,12 +54,8 @@ __device__ __forceinline__ void dma_from(const char* g, unsigned lane_off, unsig
                : "v"(lane_off), "s"(g), "s"(lanes)
                : "memory");
 }
-// One 1 KiB image from LDS.  As an instruction of its own so that it stays between the MFMAs it is written between; the
-// wait for it is the one at the top of the next chunk.
-template <int OFF>
-__device__ __forceinline__ void lds_image(bf16x8& v, unsigned addr) {
-  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
-}
+// operand of s_waitcnt: at most `vm` copies and `lgkm` LDS reads still on their way
+constexpr int waitcnt_vm_lgkm(int vm, int lgkm) { return (vm & 15) | ((vm >> 4) << 14) | (7 << 4) | (lgkm << 8); }
 
 // c += a b.  Written as an instruction because the compiler, left to place 256 accumulator registers itself, moves them
 // between the two halves of the register file inside the loop (456 moves per 128 MFMAs).  AGPR: the accumulators fill the
@@ -165,12 +161,14 @@ __device__ __forceinline__ void gemm_loop(const GemmParams& p, const GemmTarget&
   });
 
   bf16x8 wa[8], wb[8], xa[TB], xb[TB];               // operand images of this and of the next chunk, in turn
-  const unsigned w_lds = lds0 + lane * 16 + fh * 8 * 1024, x_lds = lds0 + lane * 16 + (kGemmWPieces + th * TB) * 1024;
+  const char* w_lds = lds_raw + lane * 16 + fh * 8 * 1024;
+  const char* x_lds = lds_raw + lane * 16 + (kGemmWPieces + th * TB) * 1024;
   constexpr int kReads = 8 + TB;
-  auto read_image = [&](auto ic, unsigned w_at, unsigned x_at, bf16x8 (&w)[8], bf16x8 (&x)[TB]) {
+  // (a plain load: it stays between the MFMAs it is written between, whose statements the compiler takes for accesses to memory)
+  auto read_image = [&](auto ic, const char* w_at, const char* x_at, bf16x8 (&w)[8], bf16x8 (&x)[TB]) {
     constexpr int i = decltype(ic)::value;
-    if constexpr (i < TB) lds_image<i * 1024>(x[i], x_at);
-    else lds_image<(i - TB) * 1024>(w[i - TB], w_at);
+    if constexpr (i < TB) x[i] = *(const bf16x8*)(x_at + i * 1024);
+    else w[i - TB] = *(const bf16x8*)(w_at + (i - TB) * 1024);
   };
   // One chunk: the MFMAs on w, x with, between them, the reads of the next chunk's images (w2, x2) and the copies of the
   // chunk R ahead, which goes into the slot this chunk came from (its images are in every wave's registers).  A wave is
@@ -178,11 +176,13 @@ __device__ __forceinline__ void gemm_loop(const GemmParams& p, const GemmTarget&
   // free: at most one such instruction follows an MFMA.  15,342 tokens x 9,216 features, K 3,072: everything at the head
   // of the chunk 1.18 PFLOP/s, three or four at the head of each feature block 1.40, one at a time 1.51.
   auto chunk = [&](int read_slot, int dma_slot, bf16x8 (&w)[8], bf16x8 (&x)[TB], bf16x8 (&w2)[8], bf16x8 (&x2)[TB]) {
-    const unsigned w_at = w_lds + read_slot * kStage, x_at = x_lds + read_slot * kStage;
+    const char *w_at = w_lds + read_slot * kStage, *x_at = x_lds + read_slot * kStage;
     constexpr int kEvery = TB > 4 ? 8 : 4;           // MFMAs from copy to copy
     // this wave's pieces of the next chunk have landed, and so have the images it read for this one
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((R - 2) * PP) : "memory");
+    // (the builtin, which the compiler counts the images' arrival by: it then adds no waits of its own)
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm((R - 2) * PP, 0));
     __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
     static_for<8 * TB>([&](auto kc) {
       constexpr int k = decltype(kc)::value, fb = k / TB, t = k % TB;
       if constexpr (SWAP) mfma_acc<TB == 8>(acc[t][fb], x[t], w[fb]);
@@ -232,13 +232,6 @@ __device__ __forceinline__ void gemm_loop(const GemmParams& p, const GemmTarget&
     slot = s2;
   }
   if (kc < nk) chunk(next(slot), slot, wa, xa, wb, xb);
-  // The last chunk's reads ahead have no reader, so their registers would be free to hold something else while they are
-  // still on their way: held until they have landed.
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-  for (int i = 0; i < 8; ++i) asm volatile("" ::"v"(wa[i]), "v"(wb[i]));
-#pragma unroll
-  for (int i = 0; i < TB; ++i) asm volatile("" ::"v"(xa[i]), "v"(xb[i]));
   // the compiler does not know the instructions above for MFMAs: let the last one retire before anything reads the accumulators
   static_for<TB>([&](auto tc) {
     f32x4(&a)[8] = acc[decltype(tc)::value];

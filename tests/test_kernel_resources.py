@@ -43,3 +43,18 @@ def test_no_kernel_spills_registers(tmp_path):
             spills[name] = int(re.search(r"\.vgpr_spill_count:\s+(\d+)", kernel).group(1)) + int(re.search(r"\.private_segment_fixed_size:\s+(\d+)", kernel).group(1))
     assert any("attn_fwd_narrow_kernel" in n for n in spills) and any("gemm_kernel" in n for n in spills), sorted(spills)
     assert not {n: s for n, s in spills.items() if s}
+
+
+def test_no_load_into_registers_is_inline_assembly():
+    """The compiler takes the output of an assembly statement for written at once, so a load in flight could land in a register
+    that holds something else by then: such loads are left to the compiler, which waits for them.  (Copies from memory
+    to LDS have no register output.)"""
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "pika-h3-flex_amd", "csrc")
+    found = []
+    for name in sorted(os.listdir(csrc)):
+        if name.endswith((".hip", ".h")):
+            text = open(os.path.join(csrc, name)).read()
+            for m in re.finditer(r"\basm\b[^;]*;", text):
+                loads = re.findall(r"\b(?:ds_read|ds_load|global_load|buffer_load|flat_load|scratch_load|s_load)_\w+", m.group(0))
+                found += [(name, op) for op in loads if not op.startswith("global_load_lds")]
+    assert not found
