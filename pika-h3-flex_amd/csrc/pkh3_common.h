@@ -230,6 +230,9 @@ constexpr int kQueues = 8;       // work queues of a launch: one per XCD
 // and, when that is empty, of the queue with the most units left; the launch holds an eighth more workgroups than
 // units, so an XCD that is through early keeps getting workgroups, which take units off the slower ones.  A workgroup
 // that finds every queue empty exits.  Returns the unit (index inside the section) or -1.
+// STRIDE: ints between the queues' positions.  The accesses of all XCDs to one stretch of 32 bytes are served one after the
+// other, which is the rate of a launch of short workgroups whose positions share one (see gemm_kernel).
+template <int STRIDE = 1>
 __device__ __forceinline__ int fetch_unit(int* queue_next, int home, int units) {
   const int per = (units + kQueues - 1) / kQueues;
   int q = home;
@@ -239,13 +242,13 @@ __device__ __forceinline__ int fetch_unit(int* queue_next, int home, int units) 
   for (;;) {
     const int size = max(0, min(per, units - q * per));
     // a look first: a queue that is empty stays empty, no need to count it further up
-    if (__hip_atomic_load(queue_next + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < size) {
-      const int i = __hip_atomic_fetch_add(queue_next + q, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__hip_atomic_load(queue_next + q * STRIDE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < size) {
+      const int i = __hip_atomic_fetch_add(queue_next + q * STRIDE, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (i < size) return q * per + i;
     }
     int best = -1, most = 0;
     for (int j = 0; j < kQueues; ++j) {
-      const int left = max(0, min(per, units - j * per)) - __hip_atomic_load(queue_next + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const int left = max(0, min(per, units - j * per)) - __hip_atomic_load(queue_next + j * STRIDE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (left > most) most = left, best = j;
     }
     if (best < 0) return -1;

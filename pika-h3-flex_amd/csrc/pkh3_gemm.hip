@@ -467,7 +467,7 @@ __global__ __launch_bounds__(64 * kGemmWaves, TB == 8 ? 1 : 2) void gemm_kernel(
     // tiles from per-XCD work queues (see fetch_unit): the launch holds spare workgroups, and an XCD that is through
     // with its run early takes tiles off the slower ones
     __shared__ int fetched_tile;
-    if (threadIdx.x == 0) fetched_tile = fetch_unit(p.queue_next, blockIdx.x & (kQueues - 1), total);
+    if (threadIdx.x == 0) fetched_tile = fetch_unit<kGemmQueueStride>(p.queue_next, blockIdx.x & (kQueues - 1), total);
     __syncthreads();
     lin = __builtin_amdgcn_readfirstlane(fetched_tile);
     if (lin < 0) return;
@@ -769,14 +769,15 @@ hipError_t launch_pack_rows(const PackParams& p, hipStream_t st) {
   return hipGetLastError();
 }
 
-// clears `n` 32-bit words (used for the per-head K row-norm maxima before the K epilogue max-reduces into them)
-__global__ void fill_zero_kernel(unsigned* p, int n) {
+// clears `n` 32-bit words, and `n2` others (the per-head K row-norm maxima before the K epilogue max-reduces into them, queue positions)
+__global__ void fill_zero_kernel(unsigned* p, int n, unsigned* p2, int n2) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0u;
+  else if (i - n < n2) p2[i - n] = 0u;
 }
 
-hipError_t launch_fill_zero(unsigned* p, int n, hipStream_t st) {
-  hipLaunchKernelGGL(fill_zero_kernel, dim3((n + 255) / 256), dim3(256), 0, st, p, n);
+hipError_t launch_fill_zero(unsigned* p, int n, hipStream_t st, unsigned* p2, int n2) {
+  hipLaunchKernelGGL(fill_zero_kernel, dim3((n + n2 + 255) / 256), dim3(256), 0, st, p, n, p2, n2);
   return hipGetLastError();
 }
 

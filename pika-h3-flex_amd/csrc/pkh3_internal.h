@@ -20,6 +20,7 @@ constexpr int kPartialBytes = 64 * 64 * 4 + 4 * 64 * 4;
 constexpr int kMaxPartWorkgroups = 512;
 constexpr int kSections = 3;     // sections of a long dense launch
 constexpr int kQueueSlots = 64;  // ints set aside for their positions, in front of the arrival counters
+constexpr int kGemmQueueStride = kQueueSlots / kQueues;  // ints between the queue positions of the fused q/k/v projection, which runs before the attention call and keeps them there
 constexpr int kShortMaxTiles = 16;  // dense calls with at most this many key tiles never run the long-key kernel by themselves
 
 // Where each intermediate lives inside the caller's workspace (byte offsets, 256-aligned).
@@ -96,7 +97,7 @@ struct FwdParams {
   float* split_scratch;
   size_t split_scratch_bytes;
   int* split_cnt;           // arrival counters; the kQueueSlots ints in front of them belong to the work queues
-  int* queue_next;          // [kQueues] next unit of each work queue (= split_cnt - kQueueSlots), or null: fixed map
+  int* queue_next;          // [kSections][kQueues] next unit of each work queue (= split_cnt - kQueueSlots), or null: fixed map
   int few_halves;           // filled per launch (narrow form with a key mask): fewer half tiles of valid keys are walked as the short-key form does
   // filled per launch: the sections of the launch.  A unit is one workgroup's block of queries; section i covers
   // sec_units[i] units after those of the sections before it, sec_parts[i] workgroups per unit, in sec_blocks[i]
@@ -159,7 +160,7 @@ struct GemmParams {
   int m_tiles;             // workgroup tiles along the tokens (set by launch_gemm, which chooses their height)
   int n_targets;
   GemmTarget tg[3];
-  int* queue_next;         // [kQueues] zeroed positions of the per-XCD work queues long launches take their tiles from, or null: fixed map
+  int* queue_next;         // [kQueueSlots] zeroed: positions of the per-XCD work queues long launches take their tiles from, kGemmQueueStride apart, or null: fixed map
 };
 
 // rows (activations or weights) -> operand images, optionally normalised and modulated
@@ -181,7 +182,7 @@ struct PackParams {
 
 hipError_t launch_gemm(const GemmParams& p, hipStream_t st);
 hipError_t launch_pack_rows(const PackParams& p, hipStream_t st);
-hipError_t launch_fill_zero(unsigned* p, int n, hipStream_t st);
+hipError_t launch_fill_zero(unsigned* p, int n, hipStream_t st, unsigned* p2 = nullptr, int n2 = 0);
 
 // `zero_init`: [B*H] words the launch clears (the K/V pass after it max-reduces into them)
 hipError_t launch_mask_compact(const uint8_t* mask, int B, int Sk, int* idx, int* cnt, unsigned* zero_init, int H, hipStream_t st);
