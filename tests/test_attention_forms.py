@@ -5,6 +5,11 @@ import pytest
 
 from pika_h3_flex_amd import _lib
 
+# Dense calls of the short-key form (B, H, Sq, Sk, key mask), with one, two and three of its workgroups on a CU, on at most and on more than
+# 16 key tiles; the GPU tests run them against the oracle.
+SHORT_KEY_CALLS = [(1, 64, 250, 97, False), (1, 200, 127, 700, False), (1, 200, 128, 1089, False), (1, 150, 250, 1100, False),
+                   (1, 260, 129, 1057, False), (2, 130, 100, 700, True), (2, 130, 97, 1100, True)]
+
 LONG, SHORT, NARROW, SPARSE = _lib.FORM_LONG, _lib.FORM_SHORT, _lib.FORM_NARROW, _lib.FORM_SPARSE
 
 
@@ -40,6 +45,22 @@ def test_masked_calls_go_by_the_padded_keys():
     """(The valid ones are counted on the device: test_masked_calls_of_few_and_many_valid_keys in the GPU tests runs these.)"""
     assert form(3, 24, 200, 400, masked=True) == form(3, 24, 500, 2040, masked=True) == NARROW
     assert form(3, 8, 777, 777, masked=True) == SHORT and form(1, 24, 49640, 512, masked=True) == SHORT
+
+
+@pytest.mark.parametrize("B,H,Sq,Sk,masked", SHORT_KEY_CALLS)
+def test_calls_of_the_short_key_form(B, H, Sq, Sk, masked):
+    for fp8 in (False,) if masked else (False, True, "pow2"):
+        assert form(B, H, Sq, Sk, masked=masked, fp8=fp8) == SHORT
+        assert form(B, H, Sq, Sk, masked=masked, fp8=fp8, long_key_kernel=True) == LONG
+
+
+@pytest.mark.parametrize("B,H,Sq,Sk,want", [
+    (1, 4, 1024, 1024, NARROW), (1, 24, 641, 1089, NARROW), (1, 24, 1085, 1085, SHORT),   # a small call; the attention of one image
+    (1, 24, 3008, 3008, LONG), (1, 24, 4000, 4000, SHORT),   # three short-key workgroups per CU; long ones: 192 and 264 on 256 CUs
+    (1, 24, 49640, 512, SHORT), (1, 24, 14830, 1024, SHORT), (1, 24, 14830, 1025, LONG), (1, 24, 48360, 48360, LONG),
+])
+def test_dense_calls_go_by_their_workgroups_and_keys(B, H, Sq, Sk, want):
+    assert form(B, H, Sq, Sk) == want
 
 
 def test_form_of_a_bad_call_is_an_error():

@@ -332,7 +332,7 @@ def test_golden_vectors():
             opts.update(block_mask=pk.BlockMask.from_dense(case["tile_map"], device="cuda"))
         if case.get("fp8"):
             opts.update(fp8_qk=True)
-        for long_form in (False, True):  # both forms of the dense kernel (the flag is ignored by the sparse one)
+        for long_form in (False, True):  # the forms these sizes take by themselves, and the long-key or 8-wave one
             out = pk.attention(case["q"].cuda(), case["k"].cuda(), case["v"].cuda(), long_key_kernel=long_form, **opts)
             torch.cuda.synchronize()
             err, cos = O.max_abs_and_cosine(out.cpu(), case["out"])

@@ -6,6 +6,8 @@ import math
 import pytest
 import torch
 
+from tests import test_attention_forms as forms
+
 pytestmark = pytest.mark.gpu
 
 MAX_ABS = 2e-2
@@ -20,6 +22,11 @@ def _oracle():
 
 def _rand(shape, gen, std=1.0):
     return (torch.randn(shape, generator=gen, dtype=torch.float32) * std).to(torch.bfloat16)
+
+
+def _form(*call, **opts):
+    """The form of the attention kernel the call takes on this part."""
+    return forms.form(*call, cus=torch.cuda.get_device_properties(0).multi_processor_count, **opts)
 
 
 def _run_and_check(B, Sq, Sk, H, *, seed=0, norm=True, rope_mode=0, mask=None, std=1.0, min_cos=MIN_COS,
@@ -55,13 +62,12 @@ def _run_and_check(B, Sq, Sk, H, *, seed=0, norm=True, rope_mode=0, mask=None, s
     opts = dict(q_norm_weight=f32(qw), k_norm_weight=f32(kw), norm_eps=1e-6, rope_mode=rope_mode, fp8_qk=fp8,
                 softmax_scale=scale)
     if fp8:
-        min_cos, max_abs = 0.9995, 2e-2
+        min_cos = 0.9995
     if rope_mode:
         opts.update(rope_q=(f32(rope_q[0]), f32(rope_q[1])), rope_k=(f32(rope_k[0]), f32(rope_k[1])))
     if mask is not None:
         opts.update(key_mask=mask.to(dev))
-    # calls with at most 16 key tiles normally take the short-key form of the kernel: check the long-key form
-    # on the same inputs too, so both forms see every small case
+    # small calls take the narrow or the short-key form of the kernel: check the long-key form on the same inputs too
     def on_device(t):
         """[B, S, H, D] on the card; with batch_pad as a view into a wider buffer, so the batch stride is S*H*D + pad"""
         if not batch_pad:
@@ -107,10 +113,27 @@ def test_rectangular(Sq, Sk):
 def test_few_query_blocks(B, Sq, Sk, H, fp8):
     """Calls whose 32-query blocks hardly outnumber the CUs: key counts around whole half tiles (some of the four waves with
     one half tile more than others, the last one partial), a lone query, halves of a 64-query fp8 scale block beyond the end, and
-    the short-key form on more than 16 key tiles (the last).  Bounded and running-maximum softmax."""
+    two blocks per CU (the last).  All of them in the narrow form.  Bounded and running-maximum softmax."""
+    assert _form(B, H, Sq, Sk, fp8=fp8) == forms.NARROW
     _run_and_check(B, Sq, Sk, H, seed=Sq + Sk, weight_random=True, fp8=fp8)
     if not fp8:
         _run_and_check(B, Sq, Sk, H, seed=Sq + Sk, weight_scale=4.0, bf16_operands=True)
+
+
+@pytest.mark.parametrize("B,H,Sq,Sk,masked,fp8", [(*call, fp8) for call in forms.SHORT_KEY_CALLS for fp8 in ((False,) if call[4] else (False, "pow2", True))])
+def test_short_key_form(B, H, Sq, Sk, masked, fp8):
+    """Ragged ends of queries and keys, one to three workgroups per CU, up to and beyond 16 key tiles; scattered key masks with a batch
+    entry that has no key at all.  Bounded and running-maximum softmax."""
+    assert _form(B, H, Sq, Sk, masked=masked, fp8=fp8) == forms.SHORT
+    mask = None
+    if masked:
+        mask = torch.rand((B, Sk), generator=torch.Generator().manual_seed(Sk)) < 0.6
+        mask[1] = False
+    _run_and_check(B, Sq, Sk, H, seed=Sq + Sk, mask=mask, weight_random=True, fp8=fp8, rope_mode=1 + Sk % 2)
+    # fp8 at weight 4: an element that float32 and float64 round to neighbouring e4m3 values (1/8 apart at most; |q'| <= 16, |k'| <= 4)
+    # moves a logit by up to 0.088 * 16 * 4 / 8 = 0.7, a probability by up to a quarter of that, and an output by that much of
+    # the distance of two values of V (<= 8): 1.4 at most, 0.35 for one of twice the usual size (q' 8, k' 2)
+    _run_and_check(B, Sq, Sk, H, seed=Sq + Sk, mask=mask, weight_scale=4.0, bf16_operands=not fp8, fp8=fp8, max_abs=0.35 if fp8 else MAX_ABS)
 
 
 @pytest.mark.parametrize("valid", [0, 1, 33, 64, 230])

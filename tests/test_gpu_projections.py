@@ -7,6 +7,8 @@ documented index formula, written out here independently of the kernels."""
 import pytest
 import torch
 
+from tests import test_attention_forms as forms
+
 pytestmark = pytest.mark.gpu
 
 D = 128
@@ -626,29 +628,35 @@ def test_document_kwargs_drive_the_fused_block():
     assert torch.equal(pos[vi[:60], 1:], pos[vi[60:120], 1:]) and float(pos[vi[:60], 0].abs().sum()) == 0.0
 
 
-@pytest.mark.parametrize("S,H,variant", [(300, 2, "dense"), (1000, 3, "fp8"), (777, 2, "sparse"), (130, 1, "short"),
+@pytest.mark.parametrize("S,H,variant", [(300, 2, "dense"), (1000, 3, "fp8"), (777, 2, "sparse"), (777, 2, "sparse_long"),
+                                         (130, 1, "narrow"), (1085, 24, "short"), (1085, 24, "short_fp8"),
                                          (4200, 24, "shared"), (4200, 24, "shared_fp8")])
 def test_attention_writes_the_out_projection_images(S, H, variant):
     """With PKH3_FLAG_O_IMAGES the attention epilogue writes what pkh3_pack_rows would make of its row-major output:
-    the same bytes for every image row that exists, in every form of the kernel (long, short-key, shared last round, block-sparse)."""
+    the same bytes for every image row that exists, in every form of the kernel (long, short-key, narrow, shared last round, block-sparse in both)."""
     import pika_h3_flex_amd as pk
     from pika_h3_flex_amd import projections as P
+
+    sparse, fp8, long_form = "sparse" in variant, "fp8" in variant, variant in ("dense", "sparse_long")
+    want_form = {"sparse": forms.NARROW, "sparse_long": forms.SPARSE, "narrow": forms.NARROW, "fp8": forms.NARROW, "short": forms.SHORT,
+                 "short_fp8": forms.SHORT}.get(variant, forms.LONG)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert forms.form(1, H, S, S, sparse=sparse, fp8=fp8, long_key_kernel=long_form, cus=cus) == want_form
 
     g = torch.Generator().manual_seed(21)
     q, k, v = (torch.randn((1, S, H, 128), generator=g).to(torch.bfloat16).cuda() for _ in range(3))
     w = (1.0 + 0.1 * torch.randn(128, generator=g)).cuda()
     pos = (torch.rand((S, 3), generator=g, dtype=torch.float64) * 20).cuda()
     opts = dict(q_norm_weight=w, k_norm_weight=w, rope_mode=pk.ROPE_INTERLEAVED, rope_q=pk.rope_tables(pos))
-    if variant in ("fp8", "shared_fp8"):
+    if fp8:
         opts["fp8_qk"] = True
     # "shared": 264 query tiles on a 256-CU part: whole rounds, then the last 8 tiles shared out two ways
-    if variant == "sparse":
+    if sparse:
         nt = (S + 63) // 64
         keep = torch.rand((nt, nt), generator=g) < 0.5
         keep |= torch.eye(nt, dtype=torch.bool)
         opts["block_mask"] = pk.BlockMask.from_dense(keep.cuda())
-    if variant != "short":
-        opts["long_key_kernel"] = variant == "dense"
+    opts["long_key_kernel"] = long_form
     rows = pk.attention(q, k, v, **opts)
     want = P.pack_rows(rows.view(S, H * 128))
     img = torch.full((P.packed_bytes(S, H * 128),), 0xAB, dtype=torch.uint8, device="cuda")

@@ -1,4 +1,5 @@
-"""GPU parity of the block-sparse and fp8-QK^T paths against the oracle's expanded-mask /
+"""GPU parity of the block-sparse and fp8-QK^T paths (``long_form``: the 8-wave block-sparse kernel, which small calls leave to
+the narrow one otherwise, and the long-key dense kernel) against the oracle's expanded-mask /
 fake-quant emulation.  The reference has no such paths, so the contract's cosine >= 0.995 is
 checked against the oracle; the bf16 block-sparse path is additionally held to the bf16 bar
 (max-abs <= 2e-2, cosine >= 0.9999)."""
@@ -39,8 +40,9 @@ def _ones():
     return torch.ones(D, dtype=torch.float32, device="cuda")
 
 
+@pytest.mark.parametrize("long_form", [False, True])
 @pytest.mark.parametrize("Sq,Sk,density", [(256, 256, 0.5), (700, 700, 0.3), (1000, 1333, 0.2), (65, 4000, 0.1)])
-def test_block_sparse_bf16(Sq, Sk, density):
+def test_block_sparse_bf16(Sq, Sk, density, long_form):
     import pika_h3_flex_amd as pk
     from oracle import attention_oracle as O
 
@@ -48,14 +50,16 @@ def test_block_sparse_bf16(Sq, Sk, density):
     tm = _tile_map((Sq + 63) // 64, (Sk + 63) // 64, density, gen)
     w = torch.ones(D)
     ref = O.reference_layer(q, k, v, q_norm_weight=w, k_norm_weight=w, tile_map=tm)
-    out = _call(q, k, v, q_norm_weight=_ones(), k_norm_weight=_ones(), block_mask=pk.BlockMask.from_dense(tm, device="cuda"))
+    out = _call(q, k, v, q_norm_weight=_ones(), k_norm_weight=_ones(), block_mask=pk.BlockMask.from_dense(tm, device="cuda"),
+                long_key_kernel=long_form)
     err, cos = O.max_abs_and_cosine(out, ref)
-    print(f"sparse Sq={Sq} Sk={Sk} density={tm.float().mean():.2f}: max_abs={err:.3e} cos={cos:.7f}", flush=True)
+    print(f"sparse Sq={Sq} Sk={Sk} density={tm.float().mean():.2f} long_form={long_form}: max_abs={err:.3e} cos={cos:.7f}", flush=True)
     assert err <= 2e-2 and cos >= 0.9999
 
 
-def test_block_sparse_one_row_private_tile_every_query_block():
-    """One workgroup (256 queries, 1 head) whose first row-block keeps one tile the others do not: the shared walk is
+@pytest.mark.parametrize("long_form", [False, True])
+def test_block_sparse_one_row_private_tile_every_query_block(long_form):
+    """One workgroup of the 8-wave kernel (256 queries, 1 head) whose first row-block keeps one tile the others do not: the shared walk is
     a single tile and the row-private walk a single tile of one wave pair.  This is the shape on which a stale 32-row
     block of the output accumulators was once returned (reads of the accumulators placed right behind the last MFMA
     of a tile loop, before its result was written back); every 32-query block is therefore checked on its own."""
@@ -67,7 +71,7 @@ def test_block_sparse_one_row_private_tile_every_query_block():
     tm = torch.tensor([[1, 0, 0, 1], [1, 0, 0, 0], [1, 0, 0, 0], [1, 0, 0, 0]], dtype=torch.bool)
     ref = O.reference_layer(q, k, v, tile_map=tm)
     bm = pk.BlockMask.from_dense(tm, device="cuda")
-    outs = [_call(q, k, v, block_mask=bm) for _ in range(3)]
+    outs = [_call(q, k, v, block_mask=bm, long_key_kernel=long_form) for _ in range(3)]
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[1], outs[2])
     err = (outs[0].double() - ref).abs()[0, :, 0]
     per_block = [float(err[i * 32:(i + 1) * 32].max()) for i in range(8)]
@@ -75,7 +79,7 @@ def test_block_sparse_one_row_private_tile_every_query_block():
     assert max(per_block) <= 2e-2
     for fp8 in (False, True):   # the same map through the fp8 instantiation and with the running-max softmax
         w = torch.full((D,), 4.0)
-        out = _call(q, k, v, block_mask=bm, fp8_qk=fp8, q_norm_weight=w.cuda(), k_norm_weight=_ones())
+        out = _call(q, k, v, block_mask=bm, fp8_qk=fp8, q_norm_weight=w.cuda(), k_norm_weight=_ones(), long_key_kernel=long_form)
         r = O.reference_layer(q, k, v, tile_map=tm, fp8_qk=fp8, q_norm_weight=w, k_norm_weight=torch.ones(D), bf16_operands=not fp8)
         e = (out.double() - r)[0, :, 0]
         cos = [float(torch.nn.functional.cosine_similarity(out.double()[0, i * 32:(i + 1) * 32, 0].flatten(),
@@ -83,13 +87,14 @@ def test_block_sparse_one_row_private_tile_every_query_block():
         assert min(cos) >= (0.995 if fp8 else 0.9999), cos
 
 
-def test_block_sparse_full_map_equals_dense():
+@pytest.mark.parametrize("long_form", [False, True])
+def test_block_sparse_full_map_equals_dense(long_form):
     import pika_h3_flex_amd as pk
 
     q, k, v, gen = _inputs(2, 300, 450, 2, seed=8)
     tm = torch.ones((5, 8), dtype=torch.bool)
-    a = _call(q, k, v)
-    b = _call(q, k, v, block_mask=pk.BlockMask.from_dense(tm, device="cuda"))
+    a = _call(q, k, v, long_key_kernel=long_form)
+    b = _call(q, k, v, block_mask=pk.BlockMask.from_dense(tm, device="cuda"), long_key_kernel=long_form)
     assert torch.equal(a, b)
 
 
@@ -116,13 +121,14 @@ def test_block_sparse_list_goes_on_behind_a_short_last_tile(last, fp8, long_form
         assert cos >= (0.995 if fp8 else 0.9999) and (fp8 or err <= 2e-2)
 
 
-def test_block_sparse_empty_rows_are_zero():
+@pytest.mark.parametrize("long_form", [False, True])
+def test_block_sparse_empty_rows_are_zero(long_form):
     import pika_h3_flex_amd as pk
 
     q, k, v, gen = _inputs(1, 320, 320, 2, seed=9)
     tm = torch.zeros((5, 5), dtype=torch.bool)
     tm[0, 0] = tm[2, 4] = tm[4, 1] = True
-    out = _call(q, k, v, block_mask=pk.BlockMask.from_dense(tm, device="cuda"))
+    out = _call(q, k, v, block_mask=pk.BlockMask.from_dense(tm, device="cuda"), long_key_kernel=long_form)
     assert torch.count_nonzero(out[:, 64:128]) == 0 and torch.count_nonzero(out[:, 192:256]) == 0
     assert torch.count_nonzero(out[:, 0:64]) > 0 and torch.count_nonzero(out[:, 128:192]) > 0
 
@@ -150,7 +156,8 @@ def test_fp8_qk(S, rope, long_form):
     assert cos8 >= 0.9995 and err8 <= 2e-2  # the emulation is followed much more tightly than the contract asks
 
 
-def test_fp8_block_sparse():
+@pytest.mark.parametrize("long_form", [False, True])
+def test_fp8_block_sparse(long_form):
     import pika_h3_flex_amd as pk
     from oracle import attention_oracle as O
 
@@ -158,14 +165,15 @@ def test_fp8_block_sparse():
     tm = _tile_map(15, 15, 0.3, gen)
     w = torch.ones(D)
     ref8 = O.reference_layer(q, k, v, q_norm_weight=w, k_norm_weight=w, fp8_qk=True, tile_map=tm)
-    out = _call(q, k, v, q_norm_weight=_ones(), k_norm_weight=_ones(), fp8_qk=True,
+    out = _call(q, k, v, q_norm_weight=_ones(), k_norm_weight=_ones(), fp8_qk=True, long_key_kernel=long_form,
                 block_mask=pk.BlockMask.from_dense(tm, device="cuda"))
     err8, cos8 = O.max_abs_and_cosine(out, ref8)
     print(f"fp8+sparse: max_abs={err8:.3e} cos={cos8:.6f}", flush=True)
     assert cos8 >= 0.995
 
 
-def test_sparse_and_fp8_with_large_logits():
+@pytest.mark.parametrize("long_form", [False, True])
+def test_sparse_and_fp8_with_large_logits(long_form):
     """Norm weight x4 lifts the logit bound above the limit, so these run the running-max softmax path."""
     import pika_h3_flex_amd as pk
     from oracle import attention_oracle as O
@@ -174,11 +182,12 @@ def test_sparse_and_fp8_with_large_logits():
     tm = _tile_map(10, 10, 0.4, gen)
     w4 = torch.full((D,), 4.0)
     ref = O.reference_layer(q, k, v, q_norm_weight=w4, k_norm_weight=torch.ones(D), tile_map=tm, bf16_operands=True)
-    out = _call(q, k, v, q_norm_weight=w4.cuda(), k_norm_weight=_ones(), block_mask=pk.BlockMask.from_dense(tm, device="cuda"))
+    out = _call(q, k, v, q_norm_weight=w4.cuda(), k_norm_weight=_ones(), block_mask=pk.BlockMask.from_dense(tm, device="cuda"),
+                long_key_kernel=long_form)
     err, cos = O.max_abs_and_cosine(out, ref)
     assert err <= 2e-2 and cos >= 0.9999
     ref8 = O.reference_layer(q, k, v, q_norm_weight=w4, k_norm_weight=torch.ones(D), fp8_qk=True)
-    out8 = _call(q, k, v, q_norm_weight=w4.cuda(), k_norm_weight=_ones(), fp8_qk=True)
+    out8 = _call(q, k, v, q_norm_weight=w4.cuda(), k_norm_weight=_ones(), fp8_qk=True, long_key_kernel=long_form)
     err8, cos8 = O.max_abs_and_cosine(out8, ref8)
     print(f"fp8 large logits: max_abs={err8:.3e} cos={cos8:.6f}", flush=True)
     assert cos8 >= 0.995
@@ -188,7 +197,7 @@ def test_sparse_and_fp8_with_large_logits():
 @pytest.mark.parametrize("Sq,Sk,rope,scale", [(256, 256, 0, None), (1000, 1000, 1, None), (777, 1500, 2, 0.2), (300, 5000, 1, 0.05)])
 def test_fp8_pow2_scales(Sq, Sk, rope, scale, long_form):
     """fp8_qk="pow2" (power-of-two block scales inside the scaled MFMA, softmax scale folded into Q before the
-    quantisation) against the oracle with the same rule: the short-key and the long-key forms, rectangular calls
+    quantisation) against the oracle with the same rule: the narrow and the long-key forms, rectangular calls
     with their own key tables, other softmax scales."""
     from oracle import attention_oracle as O
 
@@ -215,7 +224,8 @@ def test_fp8_pow2_scales(Sq, Sk, rope, scale, long_form):
     assert cos >= 0.995
 
 
-def test_fp8_pow2_block_sparse_large_logits_and_zero_rows():
+@pytest.mark.parametrize("long_form", [False, True])
+def test_fp8_pow2_block_sparse_large_logits_and_zero_rows(long_form):
     """The same rule through the block-sparse kernel, through the running-max softmax (norm weight 4), and on
     all-zero Q and K blocks (scale 1, exponent byte 127: finite outputs, zero logits)."""
     import pika_h3_flex_amd as pk
@@ -225,7 +235,7 @@ def test_fp8_pow2_block_sparse_large_logits_and_zero_rows():
     tm = _tile_map(15, 15, 0.3, gen)
     w = torch.ones(D)
     ref8 = O.reference_layer(q, k, v, q_norm_weight=w, k_norm_weight=w, fp8_qk="pow2", tile_map=tm)
-    out = _call(q, k, v, q_norm_weight=_ones(), k_norm_weight=_ones(), fp8_qk="pow2",
+    out = _call(q, k, v, q_norm_weight=_ones(), k_norm_weight=_ones(), fp8_qk="pow2", long_key_kernel=long_form,
                 block_mask=pk.BlockMask.from_dense(tm, device="cuda"))
     err8, cos8 = O.max_abs_and_cosine(out, ref8)
     print(f"fp8 pow2 + sparse: max_abs={err8:.3e} cos={cos8:.6f}", flush=True)
@@ -234,7 +244,7 @@ def test_fp8_pow2_block_sparse_large_logits_and_zero_rows():
     w4 = torch.full((D,), 4.0)
     for extra, rex in ((dict(), dict()), (dict(block_mask=pk.BlockMask.from_dense(tm, device="cuda")), dict(tile_map=tm))):
         ref = O.reference_layer(q, k, v, q_norm_weight=w4, k_norm_weight=w, fp8_qk="pow2", **rex)
-        out = _call(q, k, v, q_norm_weight=w4.cuda(), k_norm_weight=_ones(), fp8_qk="pow2", **extra)
+        out = _call(q, k, v, q_norm_weight=w4.cuda(), k_norm_weight=_ones(), fp8_qk="pow2", long_key_kernel=long_form, **extra)
         err, cos = O.max_abs_and_cosine(out, ref)
         print(f"fp8 pow2 large logits {list(extra)}: max_abs={err:.3e} cos={cos:.6f}", flush=True)
         assert cos >= 0.995
@@ -243,7 +253,7 @@ def test_fp8_pow2_block_sparse_large_logits_and_zero_rows():
     qz[:, 64:128] = 0
     kz[:, 128:192] = 0
     ref = O.reference_layer(qz, kz, v, fp8_qk="pow2")
-    out = _call(qz, kz, v, fp8_qk="pow2")
+    out = _call(qz, kz, v, fp8_qk="pow2", long_key_kernel=long_form)
     assert torch.isfinite(out.float()).all()
     err, cos = O.max_abs_and_cosine(out, ref)
     assert cos >= 0.9995 and err <= 2e-2
