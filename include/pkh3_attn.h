@@ -85,12 +85,14 @@ enum {
                                  pkh3_qkv_proj and the calls on their keys must agree on it.  At most one binade of
                                  the e4m3 range is given up; the error stays that of an e4m3 rounding (relative step
                                  2^-4) */
-  PKH3_FLAG_LONG_KEY_KERNEL = 1u << 1 /* dense calls with at most 16 key tiles (Sk <= 1024) normally run a
-                                 short-key form of the kernel (small workgroups, three per CU), and long dense
-                                 calls share the query tiles of a thinly filled last round of workgroups out
-                                 among several workgroups each; this flag selects the plain long-key form,
-                                 one workgroup per query tile, for all of them.  Same results to the tolerance
-                                 of the path; meant for tests and measurements */
+  PKH3_FLAG_LONG_KEY_KERNEL = 1u << 1 /* calls of few queries or keys normally run smaller forms of the kernel (short-key:
+                                 small workgroups, three per CU, for dense calls of few key tiles or of too few
+                                 queries to fill the part; narrow: 32 queries per workgroup whose waves share the
+                                 keys out, dense and block-sparse), and long dense calls share the query tiles of
+                                 a thinly filled last round of workgroups out among several workgroups each; this
+                                 flag selects the plain long-key form, one workgroup per query tile, for dense
+                                 calls and the 8-wave form for block-sparse ones, whatever their sizes.  Same
+                                 results to the tolerance of the path; meant for tests and measurements */
 };
 
 typedef struct pkh3_attn_args {

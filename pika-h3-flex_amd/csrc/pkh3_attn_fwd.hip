@@ -921,7 +921,7 @@ __global__ __launch_bounds__(64 * kDenseWaves, 1) void attn_fwd_dense_kernel(Fwd
 // Bound by the CU's 64 bytes per clock of vector loads (16 KiB for 32 MFMAs: twice what the matrix units need for them) and,
 // for few keys, by the start and the merge of a workgroup; two workgroups of 4 waves share a CU, so that those of one run
 // under the loads of the other (one of 8 waves: the same up to 256 blocks, 8 x 2000 rows 28.0 against 23.9 us).  Kernel times
-// against the form that took these calls before: 4 heads x 1,024 rows 23.4 -> 10.4 us, 2 x 3,000 88 -> 18.5,
+// (launches back to back) against the form that took these calls before: 4 heads x 1,024 rows 23.2 -> 10.3 us, 2 x 3,000 88 -> 18.5,
 // 24 x 256 rows and 2,048 keys 61 -> 14.7, 8 x 2,000 62 -> 24 (fp8 57 -> 21), 1 x 15,000 404 -> 138.
 constexpr int kNarrowWaves = 4;
 

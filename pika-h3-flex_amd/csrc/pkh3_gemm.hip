@@ -19,10 +19,13 @@
 // its accumulators (after norm and rotation) without any lane movement, and so do the row-major and the V epilogues.
 //
 // Work split.  Workgroup = 4 waves, one per SIMD = 256 features x 256, 128 or 64 tokens; wave (fh, th) owns features
-// fh*128..+127 (one head) x half of the tokens (TB = 8, 4 or 2 blocks of 16).  What bounds it: with eight waves of
-// 128 x 64 each the LDS traffic of a 32-wide k-chunk (96 KiB read, 32 KiB written) took every cycle of its MFMAs; four
-// waves of 128 x 128 read 64 KiB, whose accumulators (256 registers a lane) live in the accumulator half of the register
-// file.  LoRA is a second K segment: k-chunks beyond the hidden size take their activation images from the
+// fh*128..+127 (one head) x half of the tokens (TB = 8, 4 or 2 blocks of 16).  Eight waves of
+// 128 x 64 read 96 KiB of LDS for a 32-wide k-chunk; four of 128 x 128 read 64 KiB and need no second wave to cover their
+// issue, but accumulators of 256 registers a lane, which live in the accumulator half of the register file.  What bounds it
+// (counters, to_q/to_k/to_v, hidden size 3,072): in long launches the MFMAs, at the clock the part holds under them: pipe busy
+// 68 % at 1.98 GHz at 48,360 tokens (eight waves: 63 % at 1.82), 75 % at 1.69 GHz at 15,342 (TB = 4), LDS busy 17 and 28 %; in
+// short ones the CUs without a workgroup and, with one workgroup of TB = 2 alone on a CU, the wait for its copies at
+// every chunk's barrier (MFMA 30 %, waiting 36 % of the time, LDS 19 %).  LoRA is a second K segment: k-chunks beyond the hidden size take their activation images from the
 // down-projected rows (x A^T, scaled) and their weight images from B.
 #include <type_traits>
 
@@ -605,8 +608,9 @@ __global__ __launch_bounds__(64 * kThinWaves, 2) void gemm_thin_kernel(GemmParam
 // Tokens per workgroup of a launch (16 * 2 * TB).  Time of a CU's share of the launch, in units of 100 us for K = 3,072 with an
 // adapter, from the workgroups it runs: one alone on the CU, and two (side by side for the smaller forms, one after the
 // other for TB = 8).  Measured at 1,085, 15,342 and 48,360 tokens x 9,216 and 3,072 features: TB = 8 67 us alone, 79 - 84 us
-// each in a long launch; TB = 4 40 us alone, 80 us for two; TB = 2 34 and 61 us.  What sets them: a form's LDS traffic per
-// MFMA (64, 72 and 90 KiB per 512 MFMAs read) against how evenly its tiles fill the CUs.
+// each in a long launch; TB = 4 40 us alone, 80 us for two; TB = 2 34 and 61 us.  What sets them: the smaller forms copy and
+// read more for the same MFMAs (a chunk: 64, 48 and 40 KiB read and 32, 24 and 20 KiB copied for 256, 128 and 64 MFMAs) and have
+// fewer of them between two barriers to cover a copy's way with, against how evenly their tiles fill the CUs.
 static int gemm_token_blocks(int tokens, int n_tiles, int cus) {
   static const struct { int tb; float one, two; } kForms[3] = {{8, 0.67f, 1.55f}, {4, 0.40f, 0.80f}, {2, 0.34f, 0.61f}};
   int best = 8;
@@ -668,7 +672,7 @@ hipError_t launch_gemm(const GemmParams& p, hipStream_t st) {
 // belongs to image (16-row block r/16, k-step pc/4), lane 16*(pc%4) + r%16: byte ((r/16)*(K/32) + pc/4)*1024 +
 // (16*(pc%4) + r%16)*16.
 // `head_perm`: the rows are weight rows (output features) and are stored permuted inside each 128-row head
-// (see gemm_tile): image row 16*fb + 4*g + i takes source row 32*(fb/2) + 8*g + 4*(fb%2) + i.
+// (see acc_block and epilogue_k): image row 16*fb + 4*g + i takes source row 32*(fb/2) + 8*g + 4*(fb%2) + i.
 constexpr int kPackMaxPieces = 8;  // 16-byte pieces per lane: rows of up to 64 * 8 * 8 = 4096 elements
 
 constexpr int kPackRows = 8;                                        // rows (waves) of a workgroup

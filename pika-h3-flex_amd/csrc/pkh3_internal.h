@@ -37,7 +37,7 @@ struct QkPrologueParams {
   const void* x;            // bf16 [B,S,H,D] strided
   int64_t sb, ss, sh;
   int B, H, S;
-  int nBlk64;               // 64-row blocks to write (>= ceil(S/64); rows past the end are zero)
+  int nBlk64;               // 64-row blocks to write (>= ceil(S/64); rows past the end are zero, blocks without a valid key are left as they are)
   const float* norm_w;      // [D] or null
   float eps;
   int rope_mode;
@@ -91,7 +91,7 @@ struct FwdParams {
   const float* kmax;        // [B*H] largest K' row norm
   int fp8;
   int fp8_pow2;         // fp8: the block scales are powers of two and ride in the scaled MFMA's operands
-  int long_key_kernel;  // only the plain long-key form (no short-key form, no shared last round)
+  int long_key_kernel;  // only the plain long-key form (no short-key or narrow form, no shared last round), block-sparse: only the 8-wave form
   // scratch of the long dense form's shared units (see launch_fp): partial results, and arrival counters (one per
   // wave of a unit of the call's last round)
   float* split_scratch;
