@@ -96,7 +96,8 @@ enum {
 };
 
 typedef struct pkh3_attn_args {
-  /* bf16 tensors, logical shape [B, S, H, D], addressed as base + b*sb + s*ss + h*sh + d */
+  /* bf16 tensors, logical shape [B, S, H, D], addressed as base + b*sb + s*ss + h*sh + d.  `o` may be `q` with q's
+     strides (the output then takes the queries' place); it must not overlap them otherwise */
   const void* q;
   const void* k;
   const void* v;

@@ -173,6 +173,7 @@ void build(const pkh3_attn_args* a, void* workspace, Launch& L, bool part_scratc
   f.kv = ws + L.w.kv_off; f.kv_bh_stride = k.out_bh_stride; f.kv_tile_stride = L.w.kvTileBytes;
   f.row_cnt = L.cnt;
   f.o = a->o; f.o_sb = a->o_sb; f.o_ss = a->o_ss; f.o_sh = a->o_sh;
+  f.in_place = a->q && a->o == a->q;
   // output as the operand images of the out-projection GEMM: [16-row block][(H*128)/32 k-steps] of 1 KiB
   f.o_images = (a->flags & PKH3_FLAG_O_IMAGES) ? 1 : 0;
   f.o_img_blk_stride = (int64_t)a->H * (kD / 32) * 1024;

@@ -1233,6 +1233,9 @@ AttnForm attn_form(const FwdParams& p, int cus) {
   auto units = [&](int blocks) { return p.B * p.H * units_per_head(p.Sq, blocks); };
   const int n4 = units(kShortWaves), n32 = units(1), n_half = (p.Sk + 31) / 32;
   const int per_cu = (n4 + cus - 1) / cus;
+  // A narrow workgroup of an fp8 call reads the 64 queries its scale is of and writes 32 of them: with the output in the queries' place it
+  // could read rows its neighbour has written.  The other forms read no query but those they write.
+  const bool narrow = !(p.fp8 && p.in_place);
   // Block-sparse calls of at most four 32-query blocks per CU take the narrow form, whatever their maps (the kept tiles are
   // known on the device only).  Narrow / 8-wave form, 24 heads, us, at densities 0.03, 0.1, 0.3 and 1: 641 rows (504 blocks) 8.1 / 12.6,
   // 9.4 / 19.8, 10.6 / 22.3, 13.5 / 21.4; 900 rows (696) 13.1 / 16.6, 14.2 / 18.5, 16.3 / 27.4, 22.9 / 27.0; 1,300 rows (984)
@@ -1240,7 +1243,7 @@ AttnForm attn_form(const FwdParams& p, int cus) {
   // on it is behind on some maps: 1,500 rows (1,128) 17.6 / 18.6, 20.7 / 24.0, 26.6 / 40.8, 45.2 / 39.2; 1,700 (1,296) 19.5 / 15.9,
   // 22.5 / 22.7, 29.1 / 39.5, 55.4 / 41.9.  fp8 calls of many keys take it up to five blocks per CU: 10 heads x 4,000 rows (1,250),
   // densities 0.06, 0.2, 0.5, 0.8 and 1: 26.3 / 29.0, 38.6 / 49.8, 60 / 68, 80 / 83, 88 / 84.
-  if (p.plan) return n32 <= (p.fp8 && n_half >= 96 ? 5 : 4) * cus ? kFormNarrow : kFormSparse;
+  if (p.plan) return narrow && n32 <= (p.fp8 && n_half >= 96 ? 5 : 4) * cus ? kFormNarrow : kFormSparse;
   // Dense calls of at most two short-key workgroups per CU leave a long form's chip half empty, whatever the number of keys.  They
   // take the narrow form where it is estimated shorter, else the short-key form.  The estimates are straight lines through
   // kernel times in microseconds (bf16; fp8 lies within a tenth of them): the narrow form, a start and a merge and 0.135 per half tile
@@ -1250,7 +1253,7 @@ AttnForm attn_form(const FwdParams& p, int cus) {
   // 816 x 34 27.3 / 26.3 / 38.5, 1,504 x 94 86 / 81 / 90, 1,896 x 79 95 / 73 / 78.  With three short-key workgroups per CU the
   // long form is ahead as long as its own workgroups are no more than the CUs (2,256 x 94: 114 / 94), and behind when a few
   // are left over for a second round (3,000 x 125: 165 / 218).
-  if (per_cu <= 2 && 3.2f + (n32 + cus - 1) / cus * (0.135f * n_half + 2.7f) < 5.0f + (per_cu == 1 ? 0.60f : 0.87f) * n_half) return kFormNarrow;
+  if (narrow && per_cu <= 2 && 3.2f + (n32 + cus - 1) / cus * (0.135f * n_half + 2.7f) < 5.0f + (per_cu == 1 ? 0.60f : 0.87f) * n_half) return kFormNarrow;
   const bool few = per_cu <= 2 || (per_cu == 3 && units(kDenseWaves) > cus);
   return few || p.nKt <= kShortMaxTiles ? kFormShort : kFormLong;
 }

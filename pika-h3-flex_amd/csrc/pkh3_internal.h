@@ -79,6 +79,7 @@ struct FwdParams {
   const int* row_cnt;       // [B] valid keys after compaction, or null (= Sk)
   void* o;
   int64_t o_sb, o_ss, o_sh;
+  int in_place;             // o is q: a workgroup's output takes the place of its own queries
   int o_images;             // write O as 16-row operand images [row block][H*4 k-steps] instead of [B, Sq, H, D] rows
   int64_t o_img_blk_stride; // bytes between consecutive 16-row blocks of those images
   int B, H, Sq, Sk;

@@ -13,11 +13,13 @@ SHORT_KEY_CALLS = [(1, 64, 250, 97, False), (1, 200, 127, 700, False), (1, 200, 
 LONG, SHORT, NARROW, SPARSE = _lib.FORM_LONG, _lib.FORM_SHORT, _lib.FORM_NARROW, _lib.FORM_SPARSE
 
 
-def form(B, H, Sq, Sk, *, sparse=False, masked=False, fp8=False, long_key_kernel=False, cus=256):
+def form(B, H, Sq, Sk, *, sparse=False, masked=False, fp8=False, long_key_kernel=False, in_place=False, cus=256):
     a = _lib.AttnArgs()
     a.B, a.H, a.Sq, a.Sk, a.D = B, H, Sq, Sk, 128
     a.flags = ((_lib.FLAG_FP8_QK if fp8 else 0) | (_lib.FLAG_FP8_POW2_SCALES if fp8 == "pow2" else 0)
                | (_lib.FLAG_LONG_KEY_KERNEL if long_key_kernel else 0))
+    if in_place:
+        a.q = a.o = 0x10000   # (as the rest, never dereferenced here)
     if sparse:
         a.blk_row_ptr = a.blk_col_idx = 0x10000   # never dereferenced here
     if masked:
@@ -61,6 +63,15 @@ def test_calls_of_the_short_key_form(B, H, Sq, Sk, masked):
 ])
 def test_dense_calls_go_by_their_workgroups_and_keys(B, H, Sq, Sk, want):
     assert form(B, H, Sq, Sk) == want
+
+
+@pytest.mark.parametrize("Sq", [33, 64, 1000])
+@pytest.mark.parametrize("fp8", [True, "pow2"])
+def test_fp8_calls_in_place_are_not_narrow(Sq, fp8):
+    """A narrow workgroup reads 64 queries for their scale and writes 32: out = q would be a race between neighbours."""
+    assert form(1, 4, Sq, Sq, fp8=fp8) == form(1, 4, Sq, Sq, sparse=True, fp8=fp8) == form(1, 4, Sq, Sq, in_place=True) == NARROW
+    assert form(1, 4, Sq, Sq, fp8=fp8, in_place=True) == SHORT
+    assert form(1, 4, Sq, Sq, sparse=True, fp8=fp8, in_place=True) == SPARSE
 
 
 def test_form_of_a_bad_call_is_an_error():

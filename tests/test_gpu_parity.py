@@ -217,6 +217,30 @@ def test_softmax_scale_on_the_running_max_path():
     _run_and_check(1, 333, 333, 2, seed=21, rope_mode=2, scale=0.2, weight_scale=4.0, bf16_operands=True)
 
 
+@pytest.mark.parametrize("fp8", [False, True, "pow2"])
+@pytest.mark.parametrize("H,S,sparse", [(4, 1000, False), (2, 777, True), (200, 127, False), (24, 1500, True), (24, 4200, False)])
+def test_output_in_the_place_of_the_queries(H, S, sparse, fp8):
+    """out = q gives what a buffer of its own gives, in every form (narrow, short-key, long with a shared last round, 8-wave)."""
+    import pika_h3_flex_amd as pk
+
+    gen = torch.Generator().manual_seed(S)
+    q, k, v = (_rand((1, S, H, 128), gen).cuda() for _ in range(3))
+    w = (1.0 + 0.2 * torch.randn(128, generator=gen)).cuda()
+    opts = dict(q_norm_weight=w, k_norm_weight=w, fp8_qk=fp8)
+    if sparse:
+        n = (S + 63) // 64
+        opts["block_mask"] = pk.BlockMask.from_dense((torch.rand((n, n), generator=gen) < 0.5) | torch.eye(n, dtype=torch.bool), device="cuda")
+    want = pk.attention(q, k, v, **opts)
+    got = q.clone()
+    assert pk.attention(got, k, v, out=got, **opts) is got
+    torch.cuda.synchronize()
+    same = _form(1, H, S, S, sparse=sparse, fp8=fp8) == _form(1, H, S, S, sparse=sparse, fp8=fp8, in_place=True)
+    err, cos = _oracle().max_abs_and_cosine(got.cpu(), want.cpu())
+    print(f"out = q: H={H} S={S} sparse={sparse} fp8={fp8}: same form {same}, max_abs={err:.3e} cos={cos:.7f}", flush=True)
+    # another form adds the same products in another order: a bf16 step of the output at most
+    assert torch.equal(got, want) if same else err <= 2.0 ** -6 * max(1.0, float(want.float().abs().max())) and cos >= 0.99999
+
+
 def test_batch_stride_is_not_the_dense_one():
     """B = 3 with 264 stray elements between batch entries of q, k, v and the output (batch stride != S*H*D)."""
     _run_and_check(3, 130, 200, 2, seed=19, rope_mode=1, batch_pad=264)
