@@ -1126,9 +1126,11 @@ __global__ __launch_bounds__(64 * kNarrowWaves, 2) void attn_fwd_narrow_kernel(F
       w.q8[qb] = i32x8{a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
     }
   }
-  // the bound of attn_fwd_body: small enough, and no running maximum is needed
+  // The bound of attn_fwd_body: small enough, and no running maximum is needed.  As there, block-sparse rows without a tile that all of their
+  // plan entry keeps run the maximum all the same: their largest weights are then 1 and carry no rounding.
   const float margin = FP8 ? (POW2 ? 1.08f : p.c * 1.08f) : 1.01f;
-  const bool static_max = n_half > 0 && __all(sqrtf(fmaxf(s_n2[0], s_n2[1])) * uniform_load(p.kmax, bh) * margin <= kStaticMaxLimit);
+  const bool static_max = (SPARSE ? walk.n_shared : n_half) > 0 &&
+                          __all(sqrtf(fmaxf(s_n2[0], s_n2[1])) * uniform_load(p.kmax, bh) * margin <= kStaticMaxLimit);
   const float* kscale = FP8 ? p.kscale + (int64_t)bh * p.nKt : nullptr;
   const float c = POW2 ? 1.0f : p.c * qscale;   // what the softmax still multiplies the logits by (fp8 absmax form only)
   if (static_max) narrow_loop<FP8, POW2, SPARSE, true>(w, kf, kv, p.kv_tile_stride, kscale, walk, h0, h1, sk, c, lane);
@@ -1237,12 +1239,13 @@ AttnForm attn_form(const FwdParams& p, int cus) {
   // could read rows its neighbour has written.  The other forms read no query but those they write.
   const bool narrow = !(p.fp8 && p.in_place);
   // Block-sparse calls of at most four 32-query blocks per CU take the narrow form, whatever their maps (the kept tiles are
-  // known on the device only).  Narrow / 8-wave form, 24 heads, us, at densities 0.03, 0.1, 0.3 and 1: 641 rows (504 blocks) 8.1 / 12.6,
-  // 9.4 / 19.8, 10.6 / 22.3, 13.5 / 21.4; 900 rows (696) 13.1 / 16.6, 14.2 / 18.5, 16.3 / 27.4, 22.9 / 27.0; 1,300 rows (984)
-  // 14.4 / 15.9, 16.2 / 22.6, 21.6 / 32.6, 33.4 / 34.3 (fp8 15.8 / 15.9, 17.3 / 21.9, 21.2 / 30.7, 30.7 / 33.1).  From five blocks per CU
-  // on it is behind on some maps: 1,500 rows (1,128) 17.6 / 18.6, 20.7 / 24.0, 26.6 / 40.8, 45.2 / 39.2; 1,700 (1,296) 19.5 / 15.9,
-  // 22.5 / 22.7, 29.1 / 39.5, 55.4 / 41.9.  fp8 calls of many keys take it up to five blocks per CU: 10 heads x 4,000 rows (1,250),
-  // densities 0.06, 0.2, 0.5, 0.8 and 1: 26.3 / 29.0, 38.6 / 49.8, 60 / 68, 80 / 83, 88 / 84.
+  // known on the device only).  Narrow / 8-wave form, 24 heads, us, at densities 0.03, 0.1, 0.3 and 1 (with the diagonal): 641 rows (504
+  // blocks) 8.5 / 12.6, 10.2 / 18.2, 11.0 / 19.2, 13.7 / 21.5; 900 rows (696) 13.4 / 14.1, 15.6 / 17.3, 17.2 / 27.1, 22.0 / 26.2; 1,300 rows
+  // (984) 16.0 / 17.5, 17.7 / 21.3, 21.3 / 30.7, 32.5 / 33.4 (fp8 17.1 / 17.4, 18.7 / 20.7, 21.0 / 28.7, 28.9 / 32.1).  Behind on maps of one
+  // tile a row-block alone, from three blocks per CU on: 15.0 / 11.5 at 1,300 rows.  From five blocks per CU on it is behind on more of
+  // them: 1,500 rows (1,128) 17.6 / 18.6, 20.7 / 24.0, 26.6 / 40.8, 45.2 / 39.2; 1,700 (1,296) 19.5 / 15.9, 22.5 / 22.7, 29.1 / 39.5,
+  // 55.4 / 41.9.  fp8 calls of many keys take it up to five blocks per CU: 10 heads x 4,000 rows (1,250), densities 0.03, 0.1,
+  // 0.3, 0.6 and 1: 24.1 / 23.9, 30.1 / 36.5, 44.4 / 62.2, 58.2 / 75.7, 82.1 / 76.7.
   if (p.plan) return narrow && n32 <= (p.fp8 && n_half >= 96 ? 5 : 4) * cus ? kFormNarrow : kFormSparse;
   // Dense calls of at most two short-key workgroups per CU leave a long form's chip half empty, whatever the number of keys.  They
   // take the narrow form where it is estimated shorter, else the short-key form.  The estimates are straight lines through
