@@ -126,6 +126,21 @@ struct WaveState {
   int qe;                               // fp8 with power-of-two scales: exponent byte (E8M0) of the Q block's scale
 };
 
+// One 16-row block of raw queries with its rotation tables, as a lane group of norm_rope_quarter holds them.  Rows past the end read
+// row 0, whose place is in bounds.
+struct QRows {
+  bf16x8 raw[4];
+  RopeQuarter rope;
+};
+template <typename Params>
+__device__ __forceinline__ void load_q_rows(QRows& r, const Params& p, const RowTransform& tf, int b, int h, int qrow, int g) {
+  const int src = qrow < p.Sq ? qrow : 0;
+  const __bf16* row = (const __bf16*)p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)src * p.q_ss + 8 * g;
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) r.raw[ks] = *(const bf16x8*)(row + 32 * ks);
+  if (p.q_rope_mode != 0) load_rope_quarter(r.rope, tf, src, g);
+}
+
 #define PKH3_MFMA16(A, B, C) __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, C, 0, 0, 0)
 // format codes 0/0 = e4m3 x e4m3; scale operands 0 select the unscaled form of the instruction
 #define PKH3_MFMA16_F8(A, B, C) __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(A, B, C, 0, 0, 0, 0, 0, 0)
@@ -417,8 +432,9 @@ constexpr int fwd_lds_bytes() {
 // One workgroup's work.  `blk`: index of the workgroup inside its section of the launch; the section covers the
 // units [unit0, unit0 + units), a unit being one workgroup's block of queries (`parts` workgroups per unit; their
 // partial results start at slot `part_base` of the scratch, their counters at unit slot `cnt_base`).
-template <bool FP8, bool SPARSE, int WAVES, bool POW2>
-__device__ __forceinline__ void attn_fwd_body(const FwdParams& p, int blk, int unit0, int units, int parts, int part_base,
+// Block-sparse with work queues: returns the next position of the home queue, taken (thread 0) while the output is stored.
+template <bool FP8, bool SPARSE, int WAVES, bool POW2, typename Params>
+__device__ __forceinline__ int attn_fwd_body(const Params& p, int blk, int unit0, int units, int parts, int part_base,
                                               int cnt_base, char* lds_raw, int fetched = -1) {
   static_assert(!SPARSE || WAVES == kSparseWaves, "block-sparse layout: a wave pair per row-block of the plan");
   static_assert(FP8 || !POW2, "power-of-two scales belong to the fp8 form");
@@ -446,7 +462,7 @@ __device__ __forceinline__ void attn_fwd_body(const FwdParams& p, int blk, int u
   const int total = units * parts;
   const int per_xcd = (total + 7) / 8;
   const int lin = fetched >= 0 ? fetched : (blk & 7) * per_xcd + (blk >> 3);
-  if (lin >= total) return;
+  if (lin >= total) return 0;
   // unit inside the section, and which share of its keys: share-major, so that the workgroups an XCD runs at the
   // same time walk the same key tiles of (mostly) the same head, as the whole units before them do
   const int part = lin / units, ul = lin % units;
@@ -457,7 +473,18 @@ __device__ __forceinline__ void attn_fwd_body(const FwdParams& p, int blk, int u
   const int q32 = qt * WAVES + wq;
   const int b = bh / p.H, h = bh % p.H;
 
-  const int sk = p.row_cnt ? p.row_cnt[b] : p.Sk;
+  QRows q_rows[2];
+  NormQuarter q_norm;
+  const RowTransform q_tf{p.q_norm_w, p.q_eps, p.q_rope_mode, p.q_cos, p.q_sin};
+  auto load_q = [&](int qb) { load_q_rows(q_rows[qb], p, q_tf, b, h, q32 * 32 + 16 * qb + (lane & 15), lane >> 4); };
+  // The block-sparse form has one workgroup per CU and nothing to run beside this: rows, tables and weights are asked for before
+  // anything else of the unit is known, so that they cost one trip to memory between them and the plan's look-ups and the first
+  // key copies run beside it (14,907 rows, fp8: the call 691 -> 679 us; 48,360, bf16: 6,880 -> 6,800).  Where other workgroups or
+  // a third wave per SIMD run beside it, it gave nothing.
+  if constexpr (SPARSE) load_q(0), load_q(1);
+  if (p.q_norm_w) load_norm_quarter(q_norm, q_tf, lane >> 4);
+
+  const int sk = p.row_cnt ? uniform_load(p.row_cnt, b) : p.Sk;
   const int nkt = (sk + kTileKeys - 1) / kTileKeys;
   // sparse: [tiles every row-block of this workgroup keeps | tiles only row-block 0 keeps | ... 1 | ...]
   const int* plan = SPARSE ? p.plan + (int64_t)qt * p.plan_stride : nullptr;
@@ -512,33 +539,23 @@ __device__ __forceinline__ void attn_fwd_body(const FwdParams& p, int blk, int u
     dma(entry(t_begin), 0);
     if (kAhead > 1 && t_end > t_begin + 1) dma(entry(t_begin + 1), 1);
   }
-  // Q load, fused with QK-RMSNorm, rotation and (fp8) quantisation, in the layout of the MFMA B images themselves:
-  // lane (c, g) reads, for each of the wave's two 16-query blocks qb, the 32 elements d = 32*ks + 8*g + j of query
+  // Q, fused with QK-RMSNorm, rotation and (fp8) quantisation, in the layout of the MFMA B images themselves:
+  // lane (c, g) has read, for each of the wave's two 16-query blocks qb, the 32 elements d = 32*ks + 8*g + j of query
   // row q32*32 + 16*qb + c (four lanes per row, norm_rope_quarter), so the operand images are formed in the lane
   // that uses them and Q' never exists in memory.
   float qscale = 1.0f;
   float qn2 = 0.f;  // largest squared norm of this lane's Q' rows (bf16: before the rounding; fp8: dequantised)
   {
-    const int c16 = lane & 15, g4 = lane >> 4;
-    const RowTransform tf{p.q_norm_w, p.q_eps, p.q_rope_mode, p.q_cos, p.q_sin};
-    NormQuarter norm;
-    if (p.q_norm_w) load_norm_quarter(norm, tf, g4);
     float x[2][32];
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
-      const int qrow = q32 * 32 + 16 * qb + c16;
-      const bool valid = qrow < p.Sq;
-      const __bf16* row = (const __bf16*)p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)(valid ? qrow : 0) * p.q_ss + 8 * g4;
-      bf16x8 raw[4];
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) raw[ks] = *(const bf16x8*)(row + 32 * ks);
-      RopeQuarter rope;
-      if (p.q_rope_mode != 0 && valid) load_rope_quarter(rope, tf, qrow, g4);
+      const bool valid = q32 * 32 + 16 * qb + (lane & 15) < p.Sq;
+      if constexpr (!SPARSE) load_q(qb);
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) x[qb][ks * 8 + j] = valid ? (float)raw[ks][j] : 0.f;
-      norm_rope_quarter(x[qb], tf, norm, rope, valid, g4);
+        for (int j = 0; j < 8; ++j) x[qb][ks * 8 + j] = valid ? (float)q_rows[qb].raw[ks][j] : 0.f;
+      norm_rope_quarter(x[qb], q_tf, q_norm, q_rows[qb].rope, valid, lane >> 4);
     }
     if constexpr (!FP8) {
 #pragma unroll
@@ -760,6 +777,11 @@ __device__ __forceinline__ void attn_fwd_body(const FwdParams& p, int blk, int u
 #undef PKH3_HALF_LOOP
   }
 
+  int next_pos = 0;
+  if constexpr (SPARSE) {
+    if (p.queue_next && threadIdx.x == 0) next_pos = take_position(p.queue_next + (blockIdx.x & (kQueues - 1)));
+  }
+
   // Epilogue: O = O^T / l in bf16.  A lane holds 4 consecutive d of a query per accumulator, which would make 8-byte
   // stores scattered over 16 rows; instead each wave turns its 32 x 128 block around in its own 8 KiB of LDS
   // (16-byte chunks XOR-swizzled by the row so both directions are conflict-free) and stores whole 256-byte rows,
@@ -789,7 +811,7 @@ __device__ __forceinline__ void attn_fwd_body(const FwdParams& p, int blk, int u
       if (lane == 0)
         arrived = __hip_atomic_fetch_add(p.split_cnt + (cnt_base + ul) * WAVES + wave, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       arrived = __builtin_amdgcn_readfirstlane(arrived);
-      if (arrived != parts - 1) return;
+      if (arrived != parts - 1) return 0;
       // The partials are added up in the order of the shares, whichever wave does it (its own comes back from the
       // scratch like the others), so the result does not depend on which workgroup finished last.
 #pragma unroll 1
@@ -845,7 +867,7 @@ __device__ __forceinline__ void attn_fwd_body(const FwdParams& p, int blk, int u
   if (p.o_images) {
     // operand images of the out-projection GEMM: image (16-row block, k-step h*4 + ks) holds, in lane (c = l % 16,
     // g = l / 16), elements 32*ks + 8*g .. +7 of this head for row c of the block -- one 1 KiB store per image
-    if (q32 * 32 >= p.Sq) return;  // a block without rows: the buffer may end before it
+    if (q32 * 32 >= p.Sq) return next_pos;  // a block without rows: the buffer may end before it
     const int c16 = lane & 15, g4 = lane >> 4;
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
@@ -859,7 +881,7 @@ __device__ __forceinline__ void attn_fwd_body(const FwdParams& p, int blk, int u
         *(bf16x8*)(img + (ks * 64 + lane) * 16) = v;
       }
     }
-    return;
+    return next_pos;
   }
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
@@ -868,22 +890,44 @@ __device__ __forceinline__ void attn_fwd_body(const FwdParams& p, int blk, int u
     const int q = q32 * 32 + row;
     if (q < p.Sq) *(bf16x8*)(ob + (int64_t)q * p.o_ss + 8 * c) = v;
   }
+  return next_pos;
 }
 
 // The block-sparse kernel and the short-key dense kernel (the block-sparse one takes its units from the work queues
-// when the launch has them: its workgroups differ in length with the tile lists on top of the XCDs' clocks).
+// when the launch has them: they differ in length with the tile lists on top of the XCDs' clocks).
 template <bool FP8, bool SPARSE, int WAVES, bool POW2>
 __global__ __launch_bounds__(64 * WAVES, (SPARSE ? 8 / WAVES : 3)) void attn_fwd_kernel(FwdParams p) {
   __shared__ __attribute__((aligned(1024))) char lds_raw[fwd_lds_bytes<FP8, SPARSE, WAVES>()];
-  __shared__ int fetched_unit;
-  int fetched = -1;
-  if (p.queue_next) {   // wave-uniform
-    if (threadIdx.x == 0) fetched_unit = fetch_unit(p.queue_next, blockIdx.x & (kQueues - 1), p.sec_units[0]);
-    __syncthreads();
-    fetched = __builtin_amdgcn_readfirstlane(fetched_unit);
-    if (fetched < 0) return;
+  if constexpr (!SPARSE) {
+    attn_fwd_body<FP8, SPARSE, WAVES, POW2>(p, blockIdx.x, 0, p.sec_units[0], 1, 0, 0, lds_raw);
+  } else {
+    __shared__ int fetched_unit;
+    int next_pos = 0;
+    if (p.queue_next && threadIdx.x == 0) next_pos = take_position(p.queue_next + (blockIdx.x & (kQueues - 1)));
+    // A workgroup per CU takes units until the queues are empty (each pass takes a position, so the loop ends); without queues it
+    // does the unit of its index.  A workgroup per unit, dealt out by the hardware, left CUs idle for 15 us between two units and
+    // up to a quarter of them while a few long units ran on others (rows that keep every tile last four times as long): with
+    // 14,907 rows (fp8, density 0.28) 117 of 787 us a CU, now 40.  The call 727 -> 688 us; at 48,360 rows the same.  Handing out
+    // the longest units first gave nothing on top of this (689).
+#pragma unroll 1
+    do {
+      int fetched = -1;
+      if (p.queue_next) {   // wave-uniform
+        // (every wave has left the last unit's LDS when it comes to this barrier)
+        if (threadIdx.x == 0) fetched_unit = fetch_unit(p.queue_next, blockIdx.x & (kQueues - 1), p.sec_units[0], next_pos);
+        __syncthreads();
+        fetched = __builtin_amdgcn_readfirstlane(fetched_unit);
+        if (fetched < 0) return;
+      }
+      // The arguments are read again for every unit, from where the kernel got them: kept across the loop, what is made of them
+      // does not fit the scalar registers.
+      unsigned at = 0;
+      asm volatile("" : "+s"(at));
+      typedef const __attribute__((address_space(4))) char* KernargBytes;
+      const auto& again = *(const __attribute__((address_space(4))) FwdParams*)((KernargBytes)__builtin_amdgcn_kernarg_segment_ptr() + at);
+      next_pos = attn_fwd_body<FP8, SPARSE, WAVES, POW2>(again, blockIdx.x, 0, again.sec_units[0], 1, 0, 0, lds_raw, fetched);
+    } while (p.queue_next);
   }
-  attn_fwd_body<FP8, SPARSE, WAVES, POW2>(p, blockIdx.x, 0, p.sec_units[0], 1, 0, 0, lds_raw, fetched);
 }
 
 // The long dense kernel: a launch of up to kSections sections, handed out in this order as CUs fall free.  Section 0
@@ -1301,10 +1345,10 @@ static hipError_t launch_fp(FwdParams p, int cus, hipStream_t st) {
     p.sec_units[0] = n;
     int wgs = n;
     if (p.queue_next && cus > 0 && n >= cus) {
-      // at least a round of workgroups: units from the work queues, an eighth more workgroups than units
+      // at least a round of workgroups: one per CU (the LDS of the form holds no second), units from the work queues
       hipError_t e = launch_fill_zero((unsigned*)p.queue_next, kQueues, st);
       if (e != hipSuccess) return e;
-      wgs += max(kQueues, n / 8);
+      wgs = cus;
     } else {
       p.queue_next = nullptr;
     }

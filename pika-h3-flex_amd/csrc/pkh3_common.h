@@ -230,12 +230,16 @@ constexpr int kQueues = 8;       // work queues of a launch: one per XCD
 // and, when that is empty, of the queue with the most units left; the launch holds an eighth more workgroups than
 // units, so an XCD that is through early keeps getting workgroups, which take units off the slower ones.  A workgroup
 // that finds every queue empty exits.  Returns the unit (index inside the section) or -1.
+// `taken`: a position of the home queue that the caller has taken ahead (take_position), or -1.
 // STRIDE: ints between the queues' positions.  The accesses of all XCDs to one stretch of 32 bytes are served one after the
 // other, which is the rate of a launch of short workgroups whose positions share one (see gemm_kernel).
+__device__ __forceinline__ int take_position(int* next) { return __hip_atomic_fetch_add(next, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
 template <int STRIDE = 1>
-__device__ __forceinline__ int fetch_unit(int* queue_next, int home, int units) {
+__device__ __forceinline__ int fetch_unit(int* queue_next, int home, int units, int taken = -1) {
   const int per = (units + kQueues - 1) / kQueues;
   int q = home;
+  if (taken >= 0 && taken < min(per, units - home * per)) return home * per + taken;
   // Every pass either takes a unit, or finds all queues empty, or lost a unit to another workgroup (which is
   // progress of the launch as a whole: the positions only grow), so the loop ends.
 #pragma unroll 1
@@ -243,7 +247,7 @@ __device__ __forceinline__ int fetch_unit(int* queue_next, int home, int units) 
     const int size = max(0, min(per, units - q * per));
     // a look first: a queue that is empty stays empty, no need to count it further up
     if (__hip_atomic_load(queue_next + q * STRIDE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < size) {
-      const int i = __hip_atomic_fetch_add(queue_next + q * STRIDE, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const int i = take_position(queue_next + q * STRIDE);
       if (i < size) return q * per + i;
     }
     int best = -1, most = 0;
