@@ -108,7 +108,9 @@ WsPlan plan(const pkh3_attn_args* a, bool part_scratch = true) {
   w.kscale_off = off; if (fp8) off = align_up(off + bh * w.nKt * sizeof(float), 256);
   w.cnt_off = off;    if (a->key_mask) off = align_up(off + (size_t)a->B * sizeof(int), 256);
   w.idx_off = off;    if (a->key_mask) off = align_up(off + (size_t)a->B * a->Sk * sizeof(int), 256);
-  w.kmax_off = off;   off = align_up(off + bh * sizeof(float), 256);
+  w.knorm_stride = (2 * w.nKt + 3) / 4 * 4;
+  w.knorm_bytes = align_up(bh * w.knorm_stride * sizeof(float), 256);
+  w.knorm_off = off;  off += w.knorm_bytes;
   // everything above is the K/V side and depends on B, H, Sk and the K-side options only (pkh3_kv_prepare);
   // what follows depends on the queries of the call
   w.plan_off = off;   if (a->blk_row_ptr) off = align_up(off + (size_t)(w.nQ64 / kSparseRows) * kSparseLists * w.nKt * sizeof(int), 256);
@@ -156,7 +158,7 @@ void build(const pkh3_attn_args* a, void* workspace, Launch& L, bool part_scratc
   k.out = ws + L.w.kv_off; k.out_bh_stride = (int64_t)L.w.nKt * L.w.kvTileBytes; k.out_blk_stride = L.w.kvTileBytes;
   k.scale_out = fp8 ? (float*)(ws + L.w.kscale_off) : nullptr; k.fp8 = fp8;
   k.fp8_pow2 = (a->flags & PKH3_FLAG_FP8_POW2_SCALES) ? 1 : 0;
-  k.norm_max = (unsigned*)(ws + L.w.kmax_off);
+  k.norm_out = (float*)(ws + L.w.knorm_off); k.norm_stride = L.w.knorm_stride;
 
   VPrologueParams& v = L.vp;
   v = VPrologueParams{};
@@ -184,7 +186,7 @@ void build(const pkh3_attn_args* a, void* workspace, Launch& L, bool part_scratc
   f.plan_cnt = a->blk_row_ptr ? (const int*)(ws + L.w.plan_cnt_off) : nullptr;
   f.plan_stride = kSparseLists * L.w.nKt;
   f.kscale = k.scale_out; f.fp8 = fp8; f.fp8_pow2 = k.fp8_pow2; f.long_key_kernel = (a->flags & PKH3_FLAG_LONG_KEY_KERNEL) ? 1 : 0;
-  f.kmax = (const float*)(ws + L.w.kmax_off);
+  f.knorm = k.norm_out; f.knorm_stride = k.norm_stride;
   f.split_scratch = L.w.split_bytes ? (float*)(ws + L.w.split_off) : nullptr;
   f.split_scratch_bytes = L.w.split_bytes;
   f.split_cnt = (int*)(ws + L.w.split_cnt_off) + kQueueSlots;
@@ -198,12 +200,7 @@ int hip_fail(hipError_t e, const char* what) {
 // The K/V side of a call: key-mask compaction, then V and K into the workspace in the attention kernel's layout.
 int run_kv_side(const pkh3_attn_args* a, const Launch& L, hipStream_t st) {
   hipError_t e;
-  // the K/V pass max-reduces its row norms into per-head slots that must start at zero
-  if (a->key_mask) {
-    if ((e = launch_mask_compact(a->key_mask, a->B, a->Sk, L.idx, L.cnt, L.kp.norm_max, a->H, st)) != hipSuccess) return hip_fail(e, "mask_compact");
-  } else if ((e = launch_fill_zero(L.kp.norm_max, a->B * a->H, st)) != hipSuccess) {
-    return hip_fail(e, "fill_zero");
-  }
+  if (a->key_mask && (e = launch_mask_compact(a->key_mask, a->B, a->Sk, L.idx, L.cnt, st)) != hipSuccess) return hip_fail(e, "mask_compact");
   if ((e = launch_kv_prologue(L.kp, L.vp, st)) != hipSuccess) return hip_fail(e, "k/v pass");
   return PKH3_OK;
 }
@@ -260,7 +257,14 @@ int check_linear(const char* name, const pkh3_linear* l) {
 // Scratch of pkh3_attn_fwd_noalloc: one array per GPU the library is loaded on, held until the process ends.
 // In host code the array's name is only a handle; each device's copy has its own address, looked up once per
 // device (with that device current) and used from then on wherever the memory itself is meant.
-static __device__ __align__(256) unsigned char scratch[PKH3_NOALLOC_SCRATCH_BYTES];
+// The row norms of the keys (2 floats per 64-key tile, whose record takes at least 24 KiB) don't count against the
+// advertised size but for one float a head: the array holds them besides.
+constexpr size_t kNormRoom = 65536;
+static __device__ __align__(256) unsigned char scratch[PKH3_NOALLOC_SCRATCH_BYTES + kNormRoom];
+
+size_t counted_bytes(const pkh3_attn_args* a, const WsPlan& w) {
+  return w.total - w.knorm_bytes + align_up((size_t)a->B * a->H * sizeof(float), 256);
+}
 
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
@@ -391,8 +395,8 @@ int pkh3_attn_fwd_noalloc(const pkh3_attn_args* a, void* stream) {
   if (a->flags & PKH3_FLAG_KV_PREPARED)
     return fail(PKH3_EUNSUPPORTED, "pkh3_attn_fwd_noalloc: prepared K/V live in a caller workspace, which this call does not take");
   // the scratch of the shared last round (a matter of speed only) is left out when the built-in buffer cannot hold it
-  const bool part_scratch = plan(a, true).total <= (size_t)PKH3_NOALLOC_SCRATCH_BYTES;
-  const size_t need = plan(a, part_scratch).total;
+  const bool part_scratch = counted_bytes(a, plan(a, true)) <= (size_t)PKH3_NOALLOC_SCRATCH_BYTES;
+  const size_t need = counted_bytes(a, plan(a, part_scratch));
   if (need > (size_t)PKH3_NOALLOC_SCRATCH_BYTES)
     return fail(PKH3_EWORKSPACE,
                 "pkh3_attn_fwd_noalloc: this call needs %zu bytes of scratch, the built-in buffer holds %zu; use "
@@ -495,11 +499,6 @@ int pkh3_qkv_proj(const pkh3_qkv_args* p, const pkh3_attn_args* a, void* stream)
   const int64_t b_blk = (int64_t)(PKH3_LORA_RANK / 32) * 1024;
   const int64_t xa_blk = 3 * b_blk;                        // down-projected rows: three targets side by side
 
-  // the K epilogue max-reduces its row norms into per-head slots that must start at zero; so must the positions of
-  // the projection's work queues
-  int* const queues = (int*)(L.ws + L.w.split_cnt_off);
-  if ((e = launch_fill_zero((unsigned*)(L.ws + L.w.kmax_off), H, st, (unsigned*)queues, kQueueSlots)) != hipSuccess) return hip_fail(e, "fill_zero");
-
   if (any_lora) {
     // x A^T for the three adapters, scaled, as the activation images of the second K segment
     GemmParams g{};
@@ -556,11 +555,11 @@ int pkh3_qkv_proj(const pkh3_qkv_args* p, const pkh3_attn_args* a, void* stream)
     GemmTarget& k = g.tg[1];
     k.epi = kEpiKImg; k.out = L.kp.out; k.out_head_stride = L.kp.out_bh_stride; k.out_blk_stride = L.kp.out_blk_stride;
     k.norm_w = a->k_norm_w; k.norm_eps = a->norm_eps; k.rope_mode = a->rope_mode; k.cos_t = a->k_rope_cos; k.sin_t = a->k_rope_sin;
-    k.norm_max = L.kp.norm_max; k.fp8 = fp8; k.fp8_pow2 = L.kp.fp8_pow2; k.scale_out = L.kp.scale_out; k.scale_head_stride = L.w.nKt;
+    k.norm_out = L.kp.norm_out; k.norm_stride = L.kp.norm_stride; k.fp8 = fp8; k.fp8_pow2 = L.kp.fp8_pow2; k.scale_out = L.kp.scale_out; k.scale_head_stride = L.w.nKt;
     GemmTarget& v = g.tg[2];
     v.epi = kEpiVImg; v.out = L.vp.out; v.out_head_stride = L.vp.out_bh_stride; v.out_blk_stride = L.vp.out_tile_stride;
   }
-  g.queue_next = queues;
+  g.queue_next = (int*)(L.ws + L.w.split_cnt_off);
   if ((e = launch_gemm(g, st)) != hipSuccess) return hip_fail(e, "qkv projection");
   g_err[0] = 0;
   return PKH3_OK;

@@ -396,6 +396,25 @@ __device__ __forceinline__ void softmax_pv_half(WaveState<FP8>& w, float c, int 
   }
 }
 
+// The largest K' row norm of a (batch, head) over its `n` 32-key halves, in two parts: the first 256 halves are asked for ahead of
+// time (`first`), the wave's lanes meet where the number is needed.
+template <typename Params>
+__device__ __forceinline__ f32x4 ask_key_norms(const Params& p, int bh, int lane) {
+  return *(const f32x4*)(p.knorm + (int64_t)bh * p.knorm_stride + min(4 * lane, p.knorm_stride - 4));
+}
+template <typename Params>
+__device__ __forceinline__ float largest_key_norm(const Params& p, int bh, int n, f32x4 first, int lane) {
+  const float* norms = p.knorm + (int64_t)bh * p.knorm_stride;
+  float top = 0.f;
+  auto take = [&](const f32x4& v, int at) {   // places past the valid keys may never have been written
+#pragma unroll
+    for (int j = 0; j < 4; ++j) top = at + j < n ? fmaxf(top, v[j]) : top;
+  };
+  take(first, 4 * lane);
+  for (int at = 4 * lane + 256; at < n; at += 256) take(*(const f32x4*)(norms + at), at);
+  return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(wave_max(top))));
+}
+
 // WAVES == kShortWaves selects the short-key form of the dense kernel: 4 waves (one per SIMD, <= 168 VGPRs) and a
 // ring of 32-key half tiles in 48 KiB of LDS, so three workgroups share a CU and the Q load and O store of one
 // run under the tiles of the others.  With few key tiles that overlap is worth more than the three-fold K/V
@@ -476,6 +495,7 @@ __device__ __forceinline__ int attn_fwd_body(const Params& p, int blk, int unit0
   QRows q_rows[2];
   NormQuarter q_norm;
   const RowTransform q_tf{p.q_norm_w, p.q_eps, p.q_rope_mode, p.q_cos, p.q_sin};
+  const f32x4 first_norms = ask_key_norms(p, bh, lane);
   auto load_q = [&](int qb) { load_q_rows(q_rows[qb], p, q_tf, b, h, q32 * 32 + 16 * qb + (lane & 15), lane >> 4); };
   // The block-sparse form has one workgroup per CU and nothing to run beside this: rows, tables and weights are asked for before
   // anything else of the unit is known, so that they cost one trip to memory between them and the plan's look-ups and the first
@@ -632,7 +652,7 @@ __device__ __forceinline__ int attn_fwd_body(const Params& p, int blk, int unit0
   if (HALFMODE ? n_half > 0 : nt > 0) {
     // margins: Q' and K' are rounded to bf16 (relative step 2^-9 each; fp8: K' to e4m3, relative step 2^-4) after
     // their norms were taken
-    const float bound = sqrtf(qn2) * uniform_load(p.kmax, bh) * (FP8 ? (POW2 ? 1.08f : p.c * 1.08f) : 1.01f);
+    const float bound = sqrtf(qn2) * largest_key_norm(p, bh, n_half, first_norms, lane) * (FP8 ? (POW2 ? 1.08f : p.c * 1.08f) : 1.01f);
     static_max = __all(bound <= kStaticMaxLimit);
   }
 
@@ -1085,6 +1105,7 @@ __global__ __launch_bounds__(64 * kNarrowWaves, 2) void attn_fwd_narrow_kernel(F
 #pragma unroll
     for (int j = 0; j < (FP8 ? 4 : 8); ++j) kf[j] = *(const i32x4*)(k + (j * 64 + lane) * 16);
   }
+  const f32x4 first_norms = ask_key_norms(p, bh, lane);
   // The queries, a 16-row block per wave for all waves (layout and arithmetic of attn_fwd_body's Q load).  fp8: one scale
   // per 64 queries, so four waves look at the four blocks this block's 64 queries consist of, and two of them are it.
   const int mine = FP8 ? wave - 2 * (q32 & 1) : wave;      // which of the two 16-query blocks, if 0 or 1
@@ -1174,7 +1195,7 @@ __global__ __launch_bounds__(64 * kNarrowWaves, 2) void attn_fwd_narrow_kernel(F
   // plan entry keeps run the maximum all the same: their largest weights are then 1 and carry no rounding.
   const float margin = FP8 ? (POW2 ? 1.08f : p.c * 1.08f) : 1.01f;
   const bool static_max = (SPARSE ? walk.n_shared : n_half) > 0 &&
-                          __all(sqrtf(fmaxf(s_n2[0], s_n2[1])) * uniform_load(p.kmax, bh) * margin <= kStaticMaxLimit);
+                          __all(sqrtf(fmaxf(s_n2[0], s_n2[1])) * largest_key_norm(p, bh, (sk + 31) / 32, first_norms, lane) * margin <= kStaticMaxLimit);
   const float* kscale = FP8 ? p.kscale + (int64_t)bh * p.nKt : nullptr;
   const float c = POW2 ? 1.0f : p.c * qscale;   // what the softmax still multiplies the logits by (fp8 absmax form only)
   if (static_max) narrow_loop<FP8, POW2, SPARSE, true>(w, kf, kv, p.kv_tile_stride, kscale, walk, h0, h1, sk, c, lane);

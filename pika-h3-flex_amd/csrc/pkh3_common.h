@@ -38,6 +38,7 @@ typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(8))) int i32x8;
 typedef __attribute__((ext_vector_type(4))) int i32x4;
 typedef __attribute__((ext_vector_type(2))) int i32x2;
@@ -66,15 +67,6 @@ struct RowTransform {
   const float* cos_t;   // [rows, D/2]
   const float* sin_t;
 };
-
-// *slot = max(*slot, v) for non-negative floats kept as their bit patterns (they order like unsigned integers).
-// Thousands of waves raise the same few words: atomics on one address are served one after the other, so the word is
-// read first and the atomic only issued by a wave that would raise it (the value only grows, so a wave that sees an
-// older, smaller one merely issues an atomic it did not need).
-__device__ __forceinline__ void raise_max(unsigned* slot, float v) {
-  const unsigned bits = __float_as_uint(v);
-  if (bits > __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(slot, bits);
-}
 
 __device__ __forceinline__ float wave_sum_groups(float x) {
   // sum over the four lanes l % 16 == const (one per 16-lane group): two row swaps, no trip through the LDS crossbar

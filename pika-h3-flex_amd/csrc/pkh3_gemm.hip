@@ -349,10 +349,9 @@ __device__ __forceinline__ void epilogue_k(const GemmParams& p, const GemmTarget
         }
         nmax = fmaxf(nmax, wave_sum_groups((ssq[0] + ssq[1]) + (ssq[2] + ssq[3])));
       });
-      if (tg.norm_max) {
-        nmax = sqrtf(wave_max(nmax));
-        if (lane == 0) raise_max(tg.norm_max + head, nmax);
-      }
+      nmax = sqrtf(wave_max(nmax));
+      float* norms = tg.norm_out + (int64_t)head * tg.norm_stride + (tile0 >> 5);
+      if (lane < kTBlk / 2) norms[lane] = nmax;      // the places of the 32-token halves this wave holds
     }
     if (!tg.fp8) return;
     amax = wave_max(amax);
@@ -631,6 +630,10 @@ static hipError_t launch_gemm_tb(GemmParams p, int cus, hipStream_t st) {
   // launches of at least two rounds of workgroups take their tiles from per-XCD work queues, with an eighth more
   // workgroups than tiles, the spare ones for the XCDs that finish early
   if (total < 2 * cus * (TB == 8 ? 1 : 2)) p.queue_next = nullptr;
+  if (p.queue_next) {
+    hipError_t e = launch_fill_zero((unsigned*)p.queue_next, kQueueSlots, st);
+    if (e != hipSuccess) return e;
+  }
   const int wgs = p.queue_next ? total + (total / 8 > kQueues ? total / 8 : kQueues) : total;
   hipLaunchKernelGGL(gemm_kernel<TB>, dim3((wgs + 7) / 8 * 8), dim3(64 * kGemmWaves), 0, st, p);
   return hipGetLastError();
@@ -773,15 +776,14 @@ hipError_t launch_pack_rows(const PackParams& p, hipStream_t st) {
   return hipGetLastError();
 }
 
-// clears `n` 32-bit words, and `n2` others (the per-head K row-norm maxima before the K epilogue max-reduces into them, queue positions)
-__global__ void fill_zero_kernel(unsigned* p, int n, unsigned* p2, int n2) {
+// clears `n` 32-bit words (queue positions, arrival counters)
+__global__ void fill_zero_kernel(unsigned* p, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0u;
-  else if (i - n < n2) p2[i - n] = 0u;
 }
 
-hipError_t launch_fill_zero(unsigned* p, int n, hipStream_t st, unsigned* p2, int n2) {
-  hipLaunchKernelGGL(fill_zero_kernel, dim3((n + n2 + 255) / 256), dim3(256), 0, st, p, n, p2, n2);
+hipError_t launch_fill_zero(unsigned* p, int n, hipStream_t st) {
+  hipLaunchKernelGGL(fill_zero_kernel, dim3((n + 255) / 256), dim3(256), 0, st, p, n);
   return hipGetLastError();
 }
 

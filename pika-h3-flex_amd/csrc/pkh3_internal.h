@@ -28,7 +28,9 @@ struct WsPlan {
   int nQ64;      // 64-query blocks, padded to a multiple of 4 (one workgroup = 4 waves x 64 queries)
   int nKt;       // 64-key tiles
   int kvTileBytes;  // bytes of one [K tile | V tile] record
-  size_t kv_off, kscale_off, cnt_off, idx_off, plan_off, plan_cnt_off, kmax_off, split_off, split_cnt_off, total;
+  size_t kv_off, kscale_off, cnt_off, idx_off, plan_off, plan_cnt_off, knorm_off, split_off, split_cnt_off, total;
+  int knorm_stride;    // floats between consecutive (b,h) at knorm_off
+  size_t knorm_bytes;
   size_t split_bytes;  // bytes at split_off: partial results of the long dense form's paired workgroups
 };
 
@@ -51,7 +53,8 @@ struct QkPrologueParams {
   float* scale_out;         // fp8: [B*H, nBlk64] dequantisation scales, else null
   int fp8;
   int fp8_pow2;             // fp8: block scales rounded up to a power of two
-  unsigned* norm_max;       // [B*H] float bits: max row norm after norm+rotation (atomic max)
+  float* norm_out;          // [B*H][norm_stride]: largest row norm (after norm and rotation) of every 32 rows written
+  int norm_stride;
 };
 
 struct VPrologueParams {
@@ -89,7 +92,8 @@ struct FwdParams {
   const int* plan_cnt;      // [nQ64/kSparseRows][kSparseLists] entries per list
   int plan_stride;          // ints between consecutive workgroups' lists (kSparseLists * nKt)
   const float* kscale;      // [B*H, nKt] fp8 dequantisation scales of the K tiles
-  const float* kmax;        // [B*H] largest K' row norm
+  const float* knorm;       // [B*H][knorm_stride] largest K' row norm of every 32 keys (written for every tile that holds one)
+  int knorm_stride;         // a multiple of 4
   int fp8;
   int fp8_pow2;         // fp8: the block scales are powers of two and ride in the scaled MFMA's operands
   int long_key_kernel;  // only the plain long-key form (no short-key or narrow form, no shared last round), block-sparse: only the 8-wave form
@@ -139,7 +143,8 @@ struct GemmTarget {
   int rope_mode;
   const float* cos_t;
   const float* sin_t;
-  unsigned* norm_max;      // [heads] float bits, atomic max of the row norms, or null
+  float* norm_out;         // [heads][norm_stride] largest row norm of every 32 tokens
+  int norm_stride;
   int fp8;
   int fp8_pow2;            // fp8: block scales rounded up to a power of two
   float* scale_out;        // fp8: [heads][scale_head_stride] dequantisation scales
@@ -161,7 +166,7 @@ struct GemmParams {
   int m_tiles;             // workgroup tiles along the tokens (set by launch_gemm, which chooses their height)
   int n_targets;
   GemmTarget tg[3];
-  int* queue_next;         // [kQueueSlots] zeroed: positions of the per-XCD work queues long launches take their tiles from, kGemmQueueStride apart, or null: fixed map
+  int* queue_next;         // [kQueueSlots] positions of the per-XCD work queues long launches take their tiles from, kGemmQueueStride apart (cleared by the launch), or null: fixed map
 };
 
 // rows (activations or weights) -> operand images, optionally normalised and modulated
@@ -183,10 +188,9 @@ struct PackParams {
 
 hipError_t launch_gemm(const GemmParams& p, hipStream_t st);
 hipError_t launch_pack_rows(const PackParams& p, hipStream_t st);
-hipError_t launch_fill_zero(unsigned* p, int n, hipStream_t st, unsigned* p2 = nullptr, int n2 = 0);
+hipError_t launch_fill_zero(unsigned* p, int n, hipStream_t st);
 
-// `zero_init`: [B*H] words the launch clears (the K/V pass after it max-reduces into them)
-hipError_t launch_mask_compact(const uint8_t* mask, int B, int Sk, int* idx, int* cnt, unsigned* zero_init, int H, hipStream_t st);
+hipError_t launch_mask_compact(const uint8_t* mask, int B, int Sk, int* idx, int* cnt, hipStream_t st);
 hipError_t launch_kv_prologue(const QkPrologueParams& k, const VPrologueParams& v, hipStream_t st);
 hipError_t launch_attn_fwd(const FwdParams& p, hipStream_t st);
 enum AttnForm { kFormLong = 0, kFormShort = 1, kFormNarrow = 2, kFormSparse = 3 };

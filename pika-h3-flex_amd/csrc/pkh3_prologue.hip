@@ -14,16 +14,13 @@ namespace pkh3 {
 // Key-mask compaction: idx[b][slot] = key index of the slot-th valid key, cnt[b] = number of valid keys.
 // One workgroup of 1024 threads per batch walks the mask in chunks, carrying the running count.
 __global__ __launch_bounds__(1024) void mask_compact_kernel(const uint8_t* __restrict__ mask, int Sk,
-                                                            int* __restrict__ idx, int* __restrict__ cnt,
-                                                            unsigned* __restrict__ zero_init, int H) {
+                                                            int* __restrict__ idx, int* __restrict__ cnt) {
   __shared__ int wave_tot[16];
   __shared__ int carry;
   const int b = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const uint8_t* m = mask + (int64_t)b * Sk;
   int* out = idx + (int64_t)b * Sk;
-  // the K/V pass after this launch max-reduces its row norms into these words
-  for (int h = tid; h < H; h += 1024) zero_init[b * H + h] = 0u;
   if (tid == 0) carry = 0;
   __syncthreads();
   for (int base = 0; base < Sk; base += 1024) {
@@ -47,8 +44,8 @@ __global__ __launch_bounds__(1024) void mask_compact_kernel(const uint8_t* __res
   if (tid == 0) cnt[b] = carry;
 }
 
-hipError_t launch_mask_compact(const uint8_t* mask, int B, int Sk, int* idx, int* cnt, unsigned* zero_init, int H, hipStream_t st) {
-  hipLaunchKernelGGL(mask_compact_kernel, dim3(B), dim3(1024), 0, st, mask, Sk, idx, cnt, zero_init, H);
+hipError_t launch_mask_compact(const uint8_t* mask, int B, int Sk, int* idx, int* cnt, hipStream_t st) {
+  hipLaunchKernelGGL(mask_compact_kernel, dim3(B), dim3(1024), 0, st, mask, Sk, idx, cnt);
   return hipGetLastError();
 }
 
@@ -133,11 +130,16 @@ __device__ __forceinline__ void k_tile(const QkPrologueParams& p, int tile, int 
       }
     }
   }
-  // largest row norm of each head after norm and rotation: an upper bound for every logit is |q_i| * max_j |k_j|, which
-  // lets the attention kernel drop the running max when the bound is small
+  // largest row norm of the tile in each head, after norm and rotation: an upper bound for every logit is |q_i| * max_j |k_j|,
+  // which lets the attention kernel drop the running max when the bound is small.  Every tile has places of its own (one
+  // for each 32 rows, as the projection's K epilogue fills them): one word a head, raised by all its tiles, was what a call of few
+  // heads and tiles waited for -- atomics of eight XCDs on one line, 3 x 8 heads x 13 tiles 15.4 us against 8.0 (with
+  // rotation 17.5 against 11.8), and a launch to clear the words besides.
   __syncthreads();
-  if ((int)threadIdx.x < n_heads)
-    raise_max(p.norm_max + b * p.H + h0 + threadIdx.x, sqrtf(__uint_as_float(s_norm[threadIdx.x])));
+  if ((int)threadIdx.x < n_heads) {
+    const float top = sqrtf(__uint_as_float(s_norm[threadIdx.x]));
+    *(f32x2*)(p.norm_out + (int64_t)(b * p.H + h0 + threadIdx.x) * p.norm_stride + 2 * tile) = f32x2{top, top};
+  }
 }
 
 // V: wave (half, odd) takes 32 keys of the even or odd heads.  Whole 16-byte pieces of rows go through 8 KiB of LDS of

@@ -217,6 +217,29 @@ def test_softmax_scale_on_the_running_max_path():
     _run_and_check(1, 333, 333, 2, seed=21, rope_mode=2, scale=0.2, weight_scale=4.0, bf16_operands=True)
 
 
+@pytest.mark.parametrize("H,Sq,Sk,at,sparse,long_key,fp8", [
+    (1, 64, 70, 69, False, False, False), (2, 40, 9000, 8999, False, False, False), (1, 64, 8193, 8192, False, False, "pow2"),   # narrow form
+    (24, 1085, 1085, 1084, False, False, False), (24, 1085, 1085, 33, False, False, True),   # short-key form
+    (1, 400, 9000, 8193, False, True, False), (1, 64, 16500, 16499, False, True, True),      # long form
+    (2, 300, 9000, 8999, True, True, False), (1, 64, 130, 129, True, False, False),          # block-sparse, 8 waves and narrow
+])
+def test_one_key_of_a_large_norm_wherever_it_lies(H, Sq, Sk, at, sparse, long_key, fp8):
+    """The softmax runs without a maximum where the largest key norm allows it: a key of a logit of 260 (base 2) anywhere, in
+    a short last half tile or behind the first 256 halves, has to be seen.  Every query then attends to it alone."""
+    import pika_h3_flex_amd as pk
+
+    gen = torch.Generator().manual_seed(Sk + at)
+    q = (1.0 + 0.01 * torch.randn((1, Sq, H, 128), generator=gen)).to("cuda", torch.bfloat16)
+    k = (0.01 * torch.randn((1, Sk, H, 128), generator=gen)).to("cuda", torch.bfloat16)
+    v = torch.randn((1, Sk, H, 128), generator=gen).to("cuda", torch.bfloat16)
+    k[:, at] = 16.0
+    opts = {"long_key_kernel": long_key, "fp8_qk": fp8}
+    if sparse:
+        opts["block_mask"] = pk.BlockMask.from_dense(torch.ones((-(-Sq // 64), -(-Sk // 64)), dtype=torch.bool), device="cuda")
+    out = pk.attention(q, k, v, **opts)
+    assert torch.equal(out, v[:, at:at + 1].expand_as(out))   # the other weights are below 2^-200 of this one
+
+
 @pytest.mark.parametrize("fp8", [False, True, "pow2"])
 @pytest.mark.parametrize("H,S,sparse", [(4, 1000, False), (2, 777, True), (200, 127, False), (24, 1500, True), (24, 4200, False)])
 def test_output_in_the_place_of_the_queries(H, S, sparse, fp8):
