@@ -154,7 +154,7 @@ void build(const pkh3_attn_args* a, void* workspace, Launch& L, bool part_scratc
   k.B = a->B; k.H = a->H; k.S = a->Sk; k.nBlk64 = L.w.nKt;
   k.norm_w = a->k_norm_w; k.eps = a->norm_eps; k.rope_mode = a->rope_mode;
   k.cos_t = a->k_rope_cos; k.sin_t = a->k_rope_sin;
-  k.gather_idx = L.idx; k.row_cnt = L.cnt;
+  k.mask = a->Sk <= kOwnMaskKeys ? a->key_mask : nullptr; k.gather_idx = L.idx; k.row_cnt = L.cnt;
   k.out = ws + L.w.kv_off; k.out_bh_stride = (int64_t)L.w.nKt * L.w.kvTileBytes; k.out_blk_stride = L.w.kvTileBytes;
   k.scale_out = fp8 ? (float*)(ws + L.w.kscale_off) : nullptr; k.fp8 = fp8;
   k.fp8_pow2 = (a->flags & PKH3_FLAG_FP8_POW2_SCALES) ? 1 : 0;
@@ -164,7 +164,6 @@ void build(const pkh3_attn_args* a, void* workspace, Launch& L, bool part_scratc
   v = VPrologueParams{};
   v.v = a->v; v.sb = a->v_sb; v.ss = a->v_ss; v.sh = a->v_sh;
   v.B = a->B; v.H = a->H; v.S = a->Sk; v.nKt = L.w.nKt;
-  v.gather_idx = L.idx; v.row_cnt = L.cnt;
   v.out = ws + L.w.kv_off + kBytes; v.out_bh_stride = k.out_bh_stride; v.out_tile_stride = L.w.kvTileBytes;
 
   FwdParams& f = L.f;
@@ -200,7 +199,7 @@ int hip_fail(hipError_t e, const char* what) {
 // The K/V side of a call: key-mask compaction, then V and K into the workspace in the attention kernel's layout.
 int run_kv_side(const pkh3_attn_args* a, const Launch& L, hipStream_t st) {
   hipError_t e;
-  if (a->key_mask && (e = launch_mask_compact(a->key_mask, a->B, a->Sk, L.idx, L.cnt, st)) != hipSuccess) return hip_fail(e, "mask_compact");
+  if (a->key_mask && !L.kp.mask && (e = launch_mask_compact(a->key_mask, a->B, a->Sk, L.idx, L.cnt, st)) != hipSuccess) return hip_fail(e, "mask_compact");
   if ((e = launch_kv_prologue(L.kp, L.vp, st)) != hipSuccess) return hip_fail(e, "k/v pass");
   return PKH3_OK;
 }

@@ -21,6 +21,7 @@ constexpr int kMaxPartWorkgroups = 512;
 constexpr int kSections = 3;     // sections of a long dense launch
 constexpr int kQueueSlots = 64;  // ints set aside for their positions, in front of the arrival counters
 constexpr int kGemmQueueStride = kQueueSlots / kQueues;  // ints between the queue positions of the fused q/k/v projection, which runs before the attention call and keeps them there
+constexpr int kOwnMaskKeys = 4096;  // key masks of at most this many keys are compacted by the K/V pass itself
 constexpr int kShortMaxTiles = 16;  // dense calls with at most this many key tiles never run the long-key kernel by themselves
 
 // Where each intermediate lives inside the caller's workspace (byte offsets, 256-aligned).
@@ -45,8 +46,9 @@ struct QkPrologueParams {
   int rope_mode;
   const float* cos_t;       // [S, D/2] or null
   const float* sin_t;
-  const int* gather_idx;    // [B, S] compacted row -> source row, or null
-  const int* row_cnt;       // [B] rows that exist after compaction, or null (= S)
+  const uint8_t* mask;      // [B, S] key mask that the pass compacts itself, writing row_cnt, or null
+  const int* gather_idx;    // [B, S] compacted row -> source row, or null (read where `mask` is null)
+  int* row_cnt;             // [B] rows that exist after compaction, or null (= S)
   char* out;                // images
   int64_t out_bh_stride;    // bytes between consecutive (b,h)
   int out_blk_stride;       // bytes between consecutive 64-row blocks
@@ -61,9 +63,7 @@ struct VPrologueParams {
   const void* v;
   int64_t sb, ss, sh;
   int B, H, S, nKt;
-  const int* gather_idx;
-  const int* row_cnt;
-  char* out;                // points at the V part of tile 0
+  char* out;                // points at the V part of tile 0 (key mask: as for K)
   int64_t out_bh_stride;
   int out_tile_stride;
 };

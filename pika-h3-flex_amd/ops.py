@@ -143,7 +143,8 @@ def fill_args(
         if tuple(key_mask.shape) != (B, Sk):
             raise ValueError(f"key_mask must be [B, Sk] = {(B, Sk)}, got {tuple(key_mask.shape)}")
         _on_device("key_mask", key_mask, dev)
-        km = key_mask.to(torch.uint8).contiguous() if key_mask.dtype != torch.uint8 else key_mask.contiguous()
+        # (a bool is a byte of 0 or 1: read in place, no conversion)
+        km = key_mask.contiguous().view(torch.uint8) if key_mask.dtype == torch.bool else key_mask.to(torch.uint8).contiguous()
         a.key_mask = km.data_ptr()
         keep.append(km)
     if block_mask is not None:

@@ -331,6 +331,31 @@ def test_key_mask_suffix_and_scattered():
     _run_and_check(B, 200, Sk, 2, seed=6, mask=mask)
 
 
+@pytest.mark.parametrize("dtype", [torch.bool, torch.uint8, torch.int64])
+@pytest.mark.parametrize("Sk", [1, 64, 255, 257, 4096, 4097])
+def test_key_masks_compacted_by_the_kv_pass_and_before_it(Sk, dtype):
+    """Up to 4,096 keys the K/V pass finds the valid ones itself.  What lies in masked keys and values is never read as a number, and
+    the valid ones are taken in order: the same bits as the call on them alone."""
+    import pika_h3_flex_amd as pk
+
+    gen = torch.Generator().manual_seed(Sk)
+    q, k, v = (_rand((2, n, 3, 128), gen).cuda() for n in (70, Sk, Sk))
+    keep = torch.rand((2, Sk), generator=gen) < 0.6
+    keep[:, -1] = True
+    n = int(keep.sum(1).min())
+    for b in range(2):   # as many in both entries, so that one unmasked call has them all
+        extra = keep[b].nonzero()[:-1, 0]
+        keep[b, extra[torch.randperm(len(extra), generator=gen)[:int(keep[b].sum()) - n]]] = False
+    keep = keep.cuda()
+    ks, vs = (torch.stack([x[b, keep[b]] for b in range(2)]) for x in (k, v))
+    k[~keep], v[~keep] = float("nan"), float("inf")
+    mask = keep if dtype == torch.bool else keep.to(dtype) * 3
+    got = pk.attention(q, k, v, key_mask=mask, long_key_kernel=True)
+    assert torch.equal(got, pk.attention(q, ks, vs, long_key_kernel=True))
+    other = pk.attention(q, k, v, key_mask=mask)
+    assert (other.float() - got.float()).abs().max() <= 2 ** -7 * got.float().abs().max()   # sums in another order, rounded to bf16
+
+
 def test_key_mask_all_valid_equals_no_mask():
     import pika_h3_flex_amd as pk
 
