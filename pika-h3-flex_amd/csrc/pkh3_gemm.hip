@@ -18,8 +18,8 @@
 // token's head row: exactly what lane (g, c) of the attention kernel's K images carries, so the K epilogue stores
 // its accumulators (after norm and rotation) without any lane movement, and so do the row-major and the V epilogues.
 //
-// Work split.  Workgroup = 4 waves, one per SIMD = 256 features x 256, 128 or 64 tokens; wave (fh, th) owns features
-// fh*128..+127 (one head) x half of the tokens (TB = 8, 4 or 2 blocks of 16).  Eight waves of
+// Work split.  Workgroup = 4 waves, one per SIMD = 256 features x 256, 192, 128 or 64 tokens; wave (fh, th) owns features
+// fh*128..+127 (one head) x half of the tokens (TB = 8, 6, 4 or 2 blocks of 16).  Eight waves of
 // 128 x 64 read 96 KiB of LDS for a 32-wide k-chunk; four of 128 x 128 read 64 KiB and need no second wave to cover their
 // issue, but accumulators of 256 registers a lane, which live in the accumulator half of the register file.  What bounds it
 // (counters, to_q/to_k/to_v, hidden size 3,072): in long launches the MFMAs, at the clock the part holds under them: pipe busy
@@ -61,11 +61,14 @@ __device__ __forceinline__ void dma_from(const char* g, unsigned lane_off, unsig
 constexpr int waitcnt_vm_lgkm(int vm, int lgkm) { return (vm & 15) | ((vm >> 4) << 14) | (7 << 4) | (lgkm << 8); }
 
 // c += a b.  Written as an instruction because the compiler, left to place 256 accumulator registers itself, moves them
-// between the two halves of the register file inside the loop (456 moves per 128 MFMAs).  AGPR: the accumulators fill the
-// accumulator half (TB = 8); the smaller forms keep them in the vector half, where the epilogue reads them in place.
-template <bool AGPR>
+// between the two halves of the register file inside the loop (456 moves per 128 MFMAs).  AGPR: the accumulators lie in the
+// accumulator half (TB = 8 and 6); the smaller forms keep them in the vector half, where the epilogue reads them in place.
+// WAIT: the last of a chunk with 192 accumulators.  The compiler does not know these instructions for MFMAs; where two paths join it
+// copied such an accumulator (it has registers to copy into) right behind its MFMA, before the result was there.
+template <bool AGPR, bool WAIT>
 __device__ __forceinline__ void mfma_acc(f32x4& c, const bf16x8& a, const bf16x8& b) {
-  if constexpr (AGPR) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+  if constexpr (AGPR && WAIT) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\ts_nop 13" : "+a"(c) : "v"(a), "v"(b));
+  else if constexpr (AGPR) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
   else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
 }
 
@@ -93,9 +96,9 @@ template <int TB, bool SWAP>
 __device__ __forceinline__ void gemm_loop(const GemmParams& p, const GemmTarget& tg, int m_tile, int n_tile_in_target, bool head_live,
                                           char* lds_raw, f32x4 (&acc)[TB][8]) {
   constexpr int kStage = (kGemmWPieces + 2 * TB) * 1024;
+  constexpr int R = kGemmRing;
   constexpr int kXPieces = TB / 2;                   // activation pieces of a chunk each wave copies (and 4 weight pieces)
   constexpr int PP = 4 + kXPieces;
-  constexpr int R = kGemmRing;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int fh = wave & 1, th = wave >> 1;
@@ -104,12 +107,15 @@ __device__ __forceinline__ void gemm_loop(const GemmParams& p, const GemmTarget&
   // sources of this wave's pieces of the next chunk to copy: running pointers inside the current K segment, per-lane
   // offsets of the pieces behind them (consecutive 16-row blocks)
   const char* w_next = tg.w_img + (int64_t)(n_tile_in_target * kGemmWPieces + wave * 4) * tg.w_blk_stride;
-  const char* x_next = p.a_img + (int64_t)(m_tile * 2 * TB + wave * kXPieces) * p.a_blk_stride;
+  // (a tile of 192 tokens may reach past the blocks the images are padded to: those past the last token's are read as that one)
+  const int x_blk = m_tile * 2 * TB + wave * kXPieces, x_last = (p.M - 1) / 16;
+  auto x_at = [&](int i) { return TB == 6 ? min(x_blk + i, x_last) : x_blk + i; };
+  const char* x_next = p.a_img + (int64_t)x_at(0) * p.a_blk_stride;
   unsigned w_off[4], x_off[kXPieces];
 #pragma unroll
   for (int i = 0; i < 4; ++i) w_off[i] = lane * 16 + i * (unsigned)tg.w_blk_stride;
 #pragma unroll
-  for (int i = 0; i < kXPieces; ++i) x_off[i] = lane * 16 + i * (unsigned)p.a_blk_stride;
+  for (int i = 0; i < kXPieces; ++i) x_off[i] = lane * 16 + (x_at(i) - x_at(0)) * (unsigned)p.a_blk_stride;
   int left = nk1;                                    // chunks not yet copied of the segment the pointers walk
   const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) char*)lds_raw;
   unsigned long long lanes = ~0ull;                  // all lanes while chunks are left, then none
@@ -130,11 +136,11 @@ __device__ __forceinline__ void gemm_loop(const GemmParams& p, const GemmTarget&
       asm volatile("s_cmp_gt_i32 %1, 0\n\ts_cselect_b64 %0, -1, 0" : "=s"(lanes) : "s"(total_left) : "scc");
       if (--left == 0) {                             // on to the second segment (past the end: not read any more)
         w_next = tg.w2_img + (int64_t)(n_tile_in_target * kGemmWPieces + wave * 4) * tg.w2_blk_stride;
-        x_next = tg.a2_img + (int64_t)(m_tile * 2 * TB + wave * kXPieces) * tg.a2_blk_stride;
+        x_next = tg.a2_img + (int64_t)x_at(0) * tg.a2_blk_stride;
 #pragma unroll
         for (int j = 0; j < 4; ++j) w_off[j] = lane * 16 + j * (unsigned)tg.w2_blk_stride;
 #pragma unroll
-        for (int j = 0; j < kXPieces; ++j) x_off[j] = lane * 16 + j * (unsigned)tg.a2_blk_stride;
+        for (int j = 0; j < kXPieces; ++j) x_off[j] = lane * 16 + (x_at(j) - x_at(0)) * (unsigned)tg.a2_blk_stride;
       }
     }
   };
@@ -180,7 +186,7 @@ __device__ __forceinline__ void gemm_loop(const GemmParams& p, const GemmTarget&
   // of the chunk 1.18 PFLOP/s, three or four at the head of each feature block 1.40, one at a time 1.51.
   auto chunk = [&](int read_slot, int dma_slot, bf16x8 (&w)[8], bf16x8 (&x)[TB], bf16x8 (&w2)[8], bf16x8 (&x2)[TB]) {
     const char *w_at = w_lds + read_slot * kStage, *x_at = x_lds + read_slot * kStage;
-    constexpr int kEvery = TB > 4 ? 8 : 4;           // MFMAs from copy to copy
+    constexpr int kEvery = TB > 4 ? TB : 4;          // MFMAs from copy to copy
     // this wave's pieces of the next chunk have landed, and so have the images it read for this one
     // (the builtin, which the compiler counts the images' arrival by: it then adds no waits of its own)
     __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm((R - 2) * PP, 0));
@@ -188,8 +194,8 @@ __device__ __forceinline__ void gemm_loop(const GemmParams& p, const GemmTarget&
     asm volatile("" ::: "memory");
     static_for<8 * TB>([&](auto kc) {
       constexpr int k = decltype(kc)::value, fb = k / TB, t = k % TB;
-      if constexpr (SWAP) mfma_acc<TB == 8>(acc[t][fb], x[t], w[fb]);
-      else mfma_acc<TB == 8>(acc[t][fb], w[fb], x[t]);
+      if constexpr (SWAP) mfma_acc<(TB > 4), TB == 6 && k == 8 * TB - 1>(acc[t][fb], x[t], w[fb]);
+      else mfma_acc<(TB > 4), TB == 6 && k == 8 * TB - 1>(acc[t][fb], w[fb], x[t]);
       if constexpr (TB > 2) {
         // reads after MFMAs 0, 2, 4 ..; a copy's target after 1 + i*kEvery, the copy itself two later
         static_assert(2 * kReads <= 8 * TB && kEvery * (PP - 1) + 3 < 8 * TB, "all of them fit between the MFMAs");
@@ -238,7 +244,7 @@ __device__ __forceinline__ void gemm_loop(const GemmParams& p, const GemmTarget&
   // the compiler does not know the instructions above for MFMAs: let the last one retire before anything reads the accumulators
   static_for<TB>([&](auto tc) {
     f32x4(&a)[8] = acc[decltype(tc)::value];
-    if constexpr (TB == 8)
+    if constexpr (TB > 4)
       asm volatile("s_nop 15\n\ts_nop 15"
                    : "+a"(a[0]), "+a"(a[1]), "+a"(a[2]), "+a"(a[3]), "+a"(a[4]), "+a"(a[5]),
                      "+a"(a[6]), "+a"(a[7])::"memory");
@@ -260,8 +266,8 @@ __device__ __forceinline__ void epilogue_v(const GemmParams& p, const GemmTarget
     if ((tok & ~63) >= p.M) return;                  // a tile past the last token has no record
     char* rec = tg.out + (int64_t)head * tg.out_head_stride + (int64_t)(tok >> 6) * tg.out_blk_stride + ((tok >> 5) & 1) * 8192;
     float x[2][32];
-    acc_block<TB == 8>(x[0], acc[2 * t2]);
-    acc_block<TB == 8>(x[1], acc[2 * t2 + 1]);
+    acc_block<(TB > 4)>(x[0], acc[2 * t2]);
+    acc_block<(TB > 4)>(x[1], acc[2 * t2 + 1]);
     bool live[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) live[j] = tok + v_image_key(g, j) < p.M;
@@ -284,8 +290,9 @@ __device__ __forceinline__ void epilogue_v(const GemmParams& p, const GemmTarget
 template <int TB, int ROPE>
 __device__ __forceinline__ void epilogue_k(const GemmParams& p, const GemmTarget& tg, int head, bool head_live, int tok0,
                                            const f32x4 (&acc)[TB][8]) {
-  constexpr int kTilesHere = TB >= 4 ? TB / 4 : 1;   // 64-token tiles of this wave (TB == 2: half a tile)
-  constexpr int kTBlk = TB >= 4 ? 4 : 2;             // 16-token blocks of each
+  // parts of the wave's tokens: whole 64-token tiles, or (TB == 2 and 6) the 32-token halves of tiles it may share with another wave
+  constexpr int kTBlk = TB % 4 ? 2 : 4;              // 16-token blocks of a part
+  constexpr int kParts = TB / kTBlk;
   const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
   const int wave = threadIdx.x >> 6;
   const RowTransform tf{tg.norm_w, tg.norm_eps, ROPE, tg.cos_t, tg.sin_t};
@@ -300,7 +307,7 @@ __device__ __forceinline__ void epilogue_k(const GemmParams& p, const GemmTarget
   };
   auto form_row = [&](float (&x)[32], auto tc, int t_next) {   // t_next: block kAhead later in the order they are formed in
     constexpr int t = decltype(tc)::value;
-    acc_block<TB == 8>(x, acc[t]);
+    acc_block<(TB > 4)>(x, acc[t]);
     if (!full) {
       const bool valid = tok0 + 16 * t + c < p.M;
 #pragma unroll
@@ -312,69 +319,88 @@ __device__ __forceinline__ void epilogue_k(const GemmParams& p, const GemmTarget
   if (tf.norm_w) load_norm_quarter(norm, tf, g);
 #pragma unroll
   for (int i = 0; i < kAhead; ++i) fetch_rope(i, rope[i]);
-  static_for<kTilesHere>([&](auto hc) {
-    constexpr int half = decltype(hc)::value;
-    const int tile0 = tok0 + 64 * half;
-    const bool live = head_live && (tile0 & ~63) < p.M;   // (wave-uniform) a tile past the last token has no record
-    char* rec = tg.out + (int64_t)head * tg.out_head_stride + (int64_t)(tile0 >> 6) * tg.out_blk_stride;
-    constexpr int t0 = half * kTBlk;                 // its first 16-token block in the wave ...
-    const int tb0 = (tile0 & 63) >> 4;               // ... and in the tile
-    float nmax = 0.f, amax = 0.f;
-    if (live) {
-      static_for<kTBlk>([&](auto tc) {
-        constexpr int tt = decltype(tc)::value;
-        float x[32];
-        const int again = t0 + (tt + kAhead) % kTBlk;   // with fp8 the tile's blocks come a second time
-        form_row(x, std::integral_constant<int, t0 + tt>{}, tt + kAhead >= kTBlk && tg.fp8 ? again : min(t0 + tt + kAhead, TB - 1));
-        float ssq[4] = {0.f, 0.f, 0.f, 0.f};         // four running sums: one would be a chain of dependent instructions
-        if (!tg.fp8) {
-          // K tile image (half, ks, kb2) of 16-token block tb = 2*half + kb2: this lane's piece ks at its own place
-          const int tb = tb0 + tt;
+  float amax[kParts];
+  auto part_live = [&](int part) { return head_live && ((tok0 + 16 * kTBlk * part) & ~63) < p.M; };   // (wave-uniform) a tile past the last token has no record
+  auto record = [&](int part) { return tg.out + (int64_t)head * tg.out_head_stride + (int64_t)((tok0 + 16 * kTBlk * part) >> 6) * tg.out_blk_stride; };
+  int n_live = 0;                                    // 16-token blocks of the parts that are formed, which come first
 #pragma unroll
-          for (int ks = 0; ks < 4; ++ks) {
-            bf16x8 v;
+  for (int i = 0; i < kParts; ++i) n_live += part_live(i) ? kTBlk : 0;
+  static_for<kParts>([&](auto hc) {
+    constexpr int part = decltype(hc)::value;
+    const int first = tok0 + 16 * kTBlk * part;
+    amax[part] = 0.f;
+    if (!part_live(part)) return;
+    char* rec = record(part);
+    float nmax = 0.f;
+    static_for<kTBlk>([&](auto tc) {
+      constexpr int t = part * kTBlk + decltype(tc)::value;
+      float x[32];
+      // with fp8 the blocks of the parts that are formed come a second time
+      form_row(x, std::integral_constant<int, t>{}, t + kAhead < n_live || !tg.fp8 ? min(t + kAhead, TB - 1) : t + kAhead - n_live);
+      float ssq[4] = {0.f, 0.f, 0.f, 0.f};           // four running sums: one would be a chain of dependent instructions
+      if (!tg.fp8) {
+        // K tile image (half, ks, kb2) of 16-token block tb = 2*half + kb2: this lane's piece ks at its own place
+        const int tb = ((first & 63) >> 4) + decltype(tc)::value;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = (__bf16)x[ks * 8 + j];
-            // the row norm of the rounded values, two at a time
+        for (int ks = 0; ks < 4; ++ks) {
+          bf16x8 v;
 #pragma unroll
-            for (int j = 0; j < 8; j += 2) ssq[j / 2] = __builtin_amdgcn_fdot2_f32_bf16(bf16x2{v[j], v[j + 1]}, bf16x2{v[j], v[j + 1]}, ssq[j / 2], false);
-            *(bf16x8*)(rec + ((((tb >> 1) * 4 + ks) * 2 + (tb & 1)) * 64 + lane) * 16) = v;
-          }
-        } else {
+          for (int j = 0; j < 8; ++j) v[j] = (__bf16)x[ks * 8 + j];
+          // the row norm of the rounded values, two at a time
 #pragma unroll
-          for (int i = 0; i < 32; ++i) ssq[i & 3] += x[i] * x[i];
-#pragma unroll
-          for (int i = 0; i < 32; ++i) amax = fmaxf(amax, fabsf(x[i]));
-          asm volatile("" : "+v"(amax));   // here, not where it is used: the rows of all blocks would have to live until then
+          for (int j = 0; j < 8; j += 2) ssq[j / 2] = __builtin_amdgcn_fdot2_f32_bf16(bf16x2{v[j], v[j + 1]}, bf16x2{v[j], v[j + 1]}, ssq[j / 2], false);
+          *(bf16x8*)(rec + ((((tb >> 1) * 4 + ks) * 2 + (tb & 1)) * 64 + lane) * 16) = v;
         }
-        nmax = fmaxf(nmax, wave_sum_groups((ssq[0] + ssq[1]) + (ssq[2] + ssq[3])));
-      });
-      nmax = sqrtf(wave_max(nmax));
-      float* norms = tg.norm_out + (int64_t)head * tg.norm_stride + (tile0 >> 5);
-      if (lane < kTBlk / 2) norms[lane] = nmax;      // the places of the 32-token halves this wave holds
+      } else {
+#pragma unroll
+        for (int i = 0; i < 32; ++i) ssq[i & 3] += x[i] * x[i];
+#pragma unroll
+        for (int i = 0; i < 32; ++i) amax[part] = fmaxf(amax[part], fabsf(x[i]));
+        asm volatile("" : "+v"(amax[part]));   // here, not where it is used: the rows of all blocks would have to live until then
+      }
+      nmax = fmaxf(nmax, wave_sum_groups((ssq[0] + ssq[1]) + (ssq[2] + ssq[3])));
+    });
+    nmax = sqrtf(wave_max(nmax));
+    float* norms = tg.norm_out + (int64_t)head * tg.norm_stride + (first >> 5);
+    if (lane < kTBlk / 2) norms[lane] = nmax;        // the places of the part's 32-token halves
+  });
+  if (!tg.fp8) return;
+#pragma unroll
+  for (int i = 0; i < kParts; ++i) amax[i] = wave_max(amax[i]);
+  if constexpr (kTBlk == 2) {
+    // the scale of a tile is that of the larger magnitude of its halves, this wave's next one or the other wave's of this head
+    __shared__ float half_amax[kGemmWaves][kParts];
+    if (lane < kParts) {
+      float mine = amax[0];
+#pragma unroll
+      for (int i = 1; i < kParts; ++i) mine = lane == i ? amax[i] : mine;
+      half_amax[wave][lane] = mine;
     }
-    if (!tg.fp8) return;
-    amax = wave_max(amax);
-    if constexpr (TB == 2) {
-      // two waves hold half a tile each: the scale is that of the larger of their magnitudes
-      __shared__ float half_amax[kGemmWaves];
-      if (lane == 0) half_amax[wave] = amax;
-      __syncthreads();
-      amax = fmaxf(amax, half_amax[wave ^ 2]);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kParts; ++i) {
+      const int half = (wave >> 1) * kParts + i, other = half ^ 1;   // halves of the workgroup's tokens, a whole number of tiles
+      amax[i] = fmaxf(amax[i], half_amax[(wave & 1) + 2 * (other / kParts)][other % kParts]);
     }
-    if (!live) return;
-    const float scale = fp8_block_scale(amax, tg.fp8_pow2 != 0);
+  }
+  static_for<kParts>([&](auto hc) {
+    constexpr int part = decltype(hc)::value;
+    const int first = tok0 + 16 * kTBlk * part;
+    if (!part_live(part)) return;
+    char* rec = record(part);
+    const float scale = fp8_block_scale(amax[part], tg.fp8_pow2 != 0);
     const float inv = 1.0f / scale;
-    if (lane == 0 && tb0 == 0) tg.scale_out[(int64_t)head * tg.scale_head_stride + (tile0 >> 6)] = scale;
+    if (lane == 0 && (first & 63) == 0) tg.scale_out[(int64_t)head * tg.scale_head_stride + (first >> 6)] = scale;
     // fp8 K tile: key block tb is 2 KiB, chunk c2 of a lane holds its pieces ks = 2*c2 and 2*c2 + 1
     static_for<kTBlk>([&](auto tc) {
-      constexpr int tt = decltype(tc)::value;
+      constexpr int t = part * kTBlk + decltype(tc)::value;
+      const int tb = ((first & 63) >> 4) + decltype(tc)::value;
       float x[32];
-      form_row(x, std::integral_constant<int, t0 + tt>{}, min(t0 + tt + kAhead, TB - 1));
+      form_row(x, std::integral_constant<int, t>{}, min(t + kAhead, TB - 1));
 #pragma unroll
       for (int c2 = 0; c2 < 2; ++c2) {
         const i32x2 q0 = quant_fp8_piece(x + 16 * c2, inv), q1 = quant_fp8_piece(x + 16 * c2 + 8, inv);
-        *(i32x4*)(rec + (((tb0 + tt) * 2 + c2) * 64 + lane) * 16) = i32x4{q0[0], q0[1], q1[0], q1[1]};
+        *(i32x4*)(rec + ((tb * 2 + c2) * 64 + lane) * 16) = i32x4{q0[0], q0[1], q1[0], q1[1]};
       }
     });
   });
@@ -388,7 +414,7 @@ __device__ __forceinline__ void epilogue_a(const GemmParams& p, const GemmTarget
     constexpr int t = decltype(tc)::value;
     const int blk = tok0 + 16 * t;
     float x[32];
-    acc_block<TB == 8>(x, acc[t]);
+    acc_block<(TB > 4)>(x, acc[t]);
     const bool valid = blk + c < p.M;                  // rows past the end are zeros, whatever their activations held
     char* rec = tg.out + (int64_t)head * tg.out_head_stride + (int64_t)(blk >> 4) * tg.out_blk_stride;
 #pragma unroll
@@ -431,7 +457,7 @@ __device__ __forceinline__ void epilogue_rows(const GemmParams& p, const GemmTar
   auto block = [&](auto tc, Pieces& f) {
     constexpr int t = decltype(tc)::value;
     float x[32];
-    acc_block<TB == 8>(x, acc[t]);
+    acc_block<(TB > 4)>(x, acc[t]);
     const int token = tok0 + 16 * t + c;
     bf16x8 o[4];
 #pragma unroll
@@ -456,7 +482,7 @@ __device__ __forceinline__ void epilogue_rows(const GemmParams& p, const GemmTar
 }
 
 template <int TB>
-__global__ __launch_bounds__(64 * kGemmWaves, TB == 8 ? 1 : 2) void gemm_kernel(GemmParams p) {
+__global__ __launch_bounds__(64 * kGemmWaves, TB > 4 ? 1 : 2) void gemm_kernel(GemmParams p) {
   __shared__ __attribute__((aligned(1024))) char lds_raw[kGemmRing * (kGemmWPieces + 2 * TB) * 1024];
   // Workgroups go to the 8 XCDs round-robin; each XCD takes one contiguous run of the tile order below, in which 32
   // consecutive tiles (the workgroups the 32 CUs behind one L2 run together) form a block of 4 token tiles x 8
@@ -607,16 +633,20 @@ __global__ __launch_bounds__(64 * kThinWaves, 2) void gemm_thin_kernel(GemmParam
 // Tokens per workgroup of a launch (16 * 2 * TB).  Time of a CU's share of the launch, in units of 100 us for K = 3,072 with an
 // adapter, from the workgroups it runs: one alone on the CU, and two (side by side for the smaller forms, one after the
 // other for TB = 8).  Measured at 1,085, 15,342 and 48,360 tokens x 9,216 and 3,072 features: TB = 8 67 us alone, 79 - 84 us
-// each in a long launch; TB = 4 40 us alone, 80 us for two; TB = 2 34 and 61 us.  What sets them: the smaller forms copy and
+// each in a long launch; TB = 6 53 and 104 us; TB = 4 40 us alone, 80 us for two; TB = 2 34 and 61 us.  What sets them: the smaller forms copy and
 // read more for the same MFMAs (a chunk: 64, 48 and 40 KiB read and 32, 24 and 20 KiB copied for 256, 128 and 64 MFMAs) and have
 // fewer of them between two barriers to cover a copy's way with, against how evenly their tiles fill the CUs.
+// TB = 6 is for launches of one tile a CU, where 192 tokens fill them better than 256 or 128 (us, 256 / 192 / 128 tokens: 1,085 x 9,216
+// 64.7 / 54.7 / 65.4, 3,000 x 3,072 63.9 / 52.9 / 64.8); in longer ones it is behind one of the others or the same (6,000 x 9,216 272 / 270 /
+// 251, 6,000 x 3,072 131 / 104 / 104).
 static int gemm_token_blocks(int tokens, int n_tiles, int cus) {
-  static const struct { int tb; float one, two; } kForms[3] = {{8, 0.67f, 1.55f}, {4, 0.40f, 0.80f}, {2, 0.34f, 0.61f}};
+  static const struct { int tb; float one, two; } kForms[4] = {{8, 0.67f, 1.55f}, {6, 0.53f, 0.f}, {4, 0.40f, 0.80f}, {2, 0.34f, 0.61f}};
   int best = 8;
   float best_cost = 0.f;
   for (const auto& f : kForms) {
     const int tiles = (tokens + 32 * f.tb - 1) / (32 * f.tb) * n_tiles;
     const int per_cu = (tiles + cus - 1) / cus;
+    if (f.tb == 6 && per_cu > 1) continue;
     const float cost = (per_cu / 2) * f.two + (per_cu & 1) * f.one;
     if (f.tb == 8 || cost < best_cost) best = f.tb, best_cost = cost;
   }
@@ -629,7 +659,7 @@ static hipError_t launch_gemm_tb(GemmParams p, int cus, hipStream_t st) {
   const int total = p.m_tiles * p.n_tiles;
   // launches of at least two rounds of workgroups take their tiles from per-XCD work queues, with an eighth more
   // workgroups than tiles, the spare ones for the XCDs that finish early
-  if (total < 2 * cus * (TB == 8 ? 1 : 2)) p.queue_next = nullptr;
+  if (total < 2 * cus * (TB > 4 ? 1 : 2)) p.queue_next = nullptr;
   if (p.queue_next) {
     hipError_t e = launch_fill_zero((unsigned*)p.queue_next, kQueueSlots, st);
     if (e != hipSuccess) return e;
@@ -662,6 +692,7 @@ hipError_t launch_gemm(const GemmParams& p, hipStream_t st) {
   }
   switch (gemm_token_blocks(p.M, p.n_tiles, cus)) {
     case 8: return launch_gemm_tb<8>(p, cus, st);
+    case 6: return launch_gemm_tb<6>(p, cus, st);
     case 4: return launch_gemm_tb<4>(p, cus, st);
     default: return launch_gemm_tb<2>(p, cus, st);
   }

@@ -198,12 +198,14 @@ def test_out_projection_with_gate_and_residual(S, N, K, lora, extras):
     assert err <= 2e-2 * max(1.0, float(ref.abs().max())) and cos >= 0.9999
 
 
-# The GEMM's three workgroup heights (64, 128, 256 tokens; chosen by tokens x feature tiles) on both sides of their edges,
+# The GEMM's four workgroup heights (64, 128, 192, 256 tokens; chosen by tokens x feature tiles) on both sides of their edges,
 # an odd number of k-chunks (K = 96 + the adapter's 128) and an even one.
 @pytest.mark.parametrize("S,H,K,fp8,mode", [
     (31, 1, 96, False, 1), (129, 2, 128, True, 2), (449, 3, 96, True, 1),          # 64 tokens
     (3585, 24, 96, False, 1), (3713, 24, 128, True, 2), (3600, 23, 96, "pow2", 1),  # 128 tokens
-    (1025, 24, 96, False, 2), (1279, 24, 128, True, 1), (1088, 23, 96, False, 0),   # 256 tokens
+    (1025, 24, 96, False, 2), (1279, 24, 128, True, 1), (1088, 23, 96, False, 0),   # 192 tokens
+    (1153, 24, 96, True, 1), (1121, 23, 128, "pow2", 2), (1152, 24, 128, False, 1),   # (key tiles of one wave and shared by two)
+    (1345, 24, 96, False, 2), (1536, 24, 128, True, 1), (1409, 23, 96, "pow2", 0),   # 256 tokens
 ])
 def test_gemm_forms_of_the_qkv_projection(S, H, K, fp8, mode):
     """Q against float32 torch, and the attention output against the same kernel fed with torch's K and V through the
@@ -238,11 +240,12 @@ def test_gemm_forms_of_the_qkv_projection(S, H, K, fp8, mode):
 
 @pytest.mark.parametrize("S,H,variant", [(1, 1, "dense"), (31, 3, "dense"), (129, 2, "dense"), (449, 3, "dense"), (129, 2, "fp8"),
                                          (31, 32, "sparse"), (31, 2, "sparse"), (257, 32, "sparse"), (449, 2, "sparse_pow2"),
-                                         (641, 24, "dense"), (3585, 24, "dense"), (1025, 24, "sparse")])
+                                         (641, 24, "dense"), (3585, 24, "dense"), (1025, 24, "sparse"), (1089, 24, "dense"),
+                                         (1345, 24, "sparse")])
 def test_qkv_projection_writes_whole_key_tiles(S, H, variant):
     """S % 64 in 1 .. 32: the second half of the last K/V record holds no key.  The kernels that walk whole 64-key tiles still
     multiply its V images (by probabilities of 0), so the projection has to write it whatever the workspace held before: here
-    NaN in every byte pair.  All three workgroup heights of the GEMM; the long-key and the 8-wave block-sparse kernels."""
+    NaN in every byte pair.  All workgroup heights of the GEMM; the long-key and the 8-wave block-sparse kernels."""
     import pika_h3_flex_amd as pk
     from pika_h3_flex_amd import projections as P
 
@@ -270,7 +273,7 @@ def test_qkv_projection_writes_whole_key_tiles(S, H, variant):
     assert torch.isfinite(outs[1].float()).all() and torch.equal(outs[0], outs[1])
 
 
-@pytest.mark.parametrize("S,N", [(65, 256), (1471, 3072), (1537, 2944), (3583, 3072), (3649, 2944)])
+@pytest.mark.parametrize("S,N", [(65, 256), (1471, 3072), (1537, 2944), (3583, 3072), (3649, 2944), (2881, 3072), (3263, 2944)])
 @pytest.mark.parametrize("gate,residual", [(True, True), (True, False), (False, True), (False, False)])
 def test_gemm_forms_of_the_out_projection(S, N, gate, residual):
     """The three workgroup heights of the row-major epilogue with each of its four combinations, every row."""
