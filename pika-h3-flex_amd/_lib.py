@@ -6,6 +6,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import struct
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # PKH3_LIB_PATH selects another build of the same library (e.g. an experimental one); default: next to this file
@@ -72,6 +73,11 @@ class AttnArgs(C.Structure):
         ("flags", C.c_uint32),
         ("workspace", C.c_void_p), ("workspace_bytes", C.c_size_t),
     ]
+
+
+# the same fields for struct.pack: pointers, strides, sizes in the order of AttnArgs
+ATTN_ARGS_FORMAT = struct.Struct("@4P12q5if2Pfi4P3PIPN")
+assert ATTN_ARGS_FORMAT.size == C.sizeof(AttnArgs)
 
 
 class Linear(C.Structure):

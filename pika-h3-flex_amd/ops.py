@@ -41,15 +41,18 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
-def _check_bshd(name: str, t: torch.Tensor) -> None:
+def _check_bshd(name: str, t: torch.Tensor) -> Tuple[int, int, int, int]:
+    """Raises unless the kernels can read (or write) ``t`` as [B, S, H, D]; its strides."""
     if t.dim() != 4:
         raise ValueError(f"{name} must be [B, S, H, D], got shape {tuple(t.shape)}")
     if t.dtype != torch.bfloat16:
         raise TypeError(f"{name} must be bfloat16, got {t.dtype}")
-    if t.stride(3) != 1:
-        raise ValueError(f"{name}: head-dim stride must be 1, got {t.stride(3)}")
+    strides = t.stride()
+    if strides[3] != 1:
+        raise ValueError(f"{name}: head-dim stride must be 1, got {strides[3]}")
     if not t.is_cuda:
         raise ValueError(f"{name} must live in device memory (got {t.device}); the HIP library is the only compute path")
+    return strides
 
 
 def _on_device(name: str, t: torch.Tensor, device) -> None:
@@ -61,7 +64,7 @@ def _on_device(name: str, t: torch.Tensor, device) -> None:
 def _f32(name: str, t: Optional[torch.Tensor], shape, device) -> Optional[torch.Tensor]:
     if t is None:
         return None
-    if t.dtype != torch.float32 or not t.is_contiguous() or tuple(t.shape) != tuple(shape):
+    if t.dtype != torch.float32 or not t.is_contiguous() or t.shape != shape:
         raise ValueError(f"{name} must be contiguous float32 {tuple(shape)}, got {t.dtype} {tuple(t.shape)}")
     _on_device(name, t, device)
     return t
@@ -95,39 +98,33 @@ def fill_args(
     H*D)`` bytes) instead of a ``[B, Sq, H, D]`` tensor, and B must be 1."""
     if kv_prepared != (k is None) or (k is None) != (v is None):
         raise ValueError("k and v are None exactly when kv_prepared is set")
-    for n, t in (("q", q), ("k", k), ("v", v)) + (() if out_images else (("out", out),)):
-        if t is not None:
-            _check_bshd(n, t)
-    B, Sq, H, D = q.shape
+    q_st = _check_bshd("q", q)
+    k_st = v_st = o_st = (0, 0, 0)
+    if k is not None:
+        k_st, v_st = _check_bshd("k", k), _check_bshd("v", v)
+    if not out_images:
+        o_st = _check_bshd("out", out)
+    q_shape = q.shape
+    B, Sq, H, D = q_shape
     Sk = (Sq if prepared_keys is None else int(prepared_keys)) if k is None else k.shape[1]
-    if k is not None and (tuple(k.shape) != (B, Sk, H, D) or tuple(v.shape) != (B, Sk, H, D)):
-        raise ValueError(f"k/v shapes {tuple(k.shape)}/{tuple(v.shape)} do not match q {tuple(q.shape)}")
+    if k is not None and (k.shape != (B, Sk, H, D) or v.shape != (B, Sk, H, D)):
+        raise ValueError(f"k/v shapes {tuple(k.shape)}/{tuple(v.shape)} do not match q {tuple(q_shape)}")
     if out_images:
         need = ((Sq + 255) // 256 * 256) * H * D * 2
         if out.dtype != torch.uint8 or not out.is_contiguous() or out.numel() < need or B != 1:
             raise ValueError(f"out_images: out must be a contiguous uint8 buffer of at least {need} bytes and B must be 1")
-    elif tuple(out.shape) != (B, Sq, H, D):
+    elif out.shape != q_shape:
         raise ValueError(f"out shape {tuple(out.shape)} != {(B, Sq, H, D)}")
     dev = q.device
-    for n, t in (("k", k), ("v", v), ("out", out)):
-        if t is not None:
-            _on_device(n, t, dev)
-    keep = [q, k, v, out]
-    a = _lib.AttnArgs()
-    a.q, a.o = q.data_ptr(), out.data_ptr()
-    a.q_sb, a.q_ss, a.q_sh = q.stride(0), q.stride(1), q.stride(2)
     if k is not None:
-        a.k, a.v = k.data_ptr(), v.data_ptr()
-        a.k_sb, a.k_ss, a.k_sh = k.stride(0), k.stride(1), k.stride(2)
-        a.v_sb, a.v_ss, a.v_sh = v.stride(0), v.stride(1), v.stride(2)
-    if not out_images:
-        a.o_sb, a.o_ss, a.o_sh = out.stride(0), out.stride(1), out.stride(2)
-    a.B, a.H, a.Sq, a.Sk, a.D = B, H, Sq, Sk, D
-    a.softmax_scale = float(softmax_scale) if softmax_scale is not None else 0.0
+        _on_device("k", k, dev)
+        _on_device("v", v, dev)
+    _on_device("out", out, dev)
+    keep = [q, k, v, out]
     qw = _f32("q_norm_weight", q_norm_weight, (D,), dev)
     kw = _f32("k_norm_weight", k_norm_weight, (D,), dev)
-    a.q_norm_w, a.k_norm_w, a.norm_eps = _ptr(qw), _ptr(kw), float(norm_eps)
-    a.rope_mode = int(rope_mode)
+    rope_mode = int(rope_mode)
+    tables = (0, 0, 0, 0)
     if rope_mode != _lib.ROPE_NONE:
         if rope_q is None:
             raise ValueError("rope_mode set but rope_q tables missing")
@@ -137,15 +134,16 @@ def fill_args(
             rope_k = rope_q
         qc, qs = _f32("rope_q cos", rope_q[0], (Sq, D // 2), dev), _f32("rope_q sin", rope_q[1], (Sq, D // 2), dev)
         kc, ks = _f32("rope_k cos", rope_k[0], (Sk, D // 2), dev), _f32("rope_k sin", rope_k[1], (Sk, D // 2), dev)
-        a.q_rope_cos, a.q_rope_sin, a.k_rope_cos, a.k_rope_sin = qc.data_ptr(), qs.data_ptr(), kc.data_ptr(), ks.data_ptr()
+        tables = (qc.data_ptr(), qs.data_ptr(), kc.data_ptr(), ks.data_ptr())
         keep += [qc, qs, kc, ks]
+    mask_ptr = row_ptr = col_idx = 0
     if key_mask is not None:
-        if tuple(key_mask.shape) != (B, Sk):
+        if key_mask.shape != (B, Sk):
             raise ValueError(f"key_mask must be [B, Sk] = {(B, Sk)}, got {tuple(key_mask.shape)}")
         _on_device("key_mask", key_mask, dev)
         # (a bool is a byte of 0 or 1: read in place, no conversion)
         km = key_mask.contiguous().view(torch.uint8) if key_mask.dtype == torch.bool else key_mask.to(torch.uint8).contiguous()
-        a.key_mask = km.data_ptr()
+        mask_ptr = km.data_ptr()
         keep.append(km)
     if block_mask is not None:
         nrow = (Sq + 63) // 64
@@ -159,13 +157,20 @@ def fill_args(
         _on_device("block mask col_idx", block_mask.col_idx, dev)
         if not (block_mask.row_ptr.is_contiguous() and block_mask.col_idx.is_contiguous()):
             raise ValueError("block mask CSR arrays must be contiguous")
-        a.blk_row_ptr, a.blk_col_idx = block_mask.row_ptr.data_ptr(), block_mask.col_idx.data_ptr()
+        row_ptr, col_idx = block_mask.row_ptr.data_ptr(), block_mask.col_idx.data_ptr()
         keep += [block_mask.row_ptr, block_mask.col_idx]
     fp8_qk = fp8_mode(fp8_qk)
-    a.flags = ((_lib.FLAG_FP8_QK if fp8_qk else 0) | (_lib.FLAG_FP8_POW2_SCALES if fp8_qk == FP8_POW2 else 0)
-               | (_lib.FLAG_LONG_KEY_KERNEL if long_key_kernel else 0)
-               | (_lib.FLAG_KV_PREPARED if kv_prepared else 0) | (_lib.FLAG_O_IMAGES if out_images else 0))
+    flags = ((_lib.FLAG_FP8_QK if fp8_qk else 0) | (_lib.FLAG_FP8_POW2_SCALES if fp8_qk == FP8_POW2 else 0)
+             | (_lib.FLAG_LONG_KEY_KERNEL if long_key_kernel else 0)
+             | (_lib.FLAG_KV_PREPARED if kv_prepared else 0) | (_lib.FLAG_O_IMAGES if out_images else 0))
     keep += [qw, kw]
+    # all fields at once: a small call waits for the host, and a ctypes structure set field by field is a good part of that
+    a = _lib.AttnArgs.from_buffer_copy(_lib.ATTN_ARGS_FORMAT.pack(
+        q.data_ptr(), 0 if k is None else k.data_ptr(), 0 if v is None else v.data_ptr(), out.data_ptr(),
+        q_st[0], q_st[1], q_st[2], k_st[0], k_st[1], k_st[2], v_st[0], v_st[1], v_st[2], o_st[0], o_st[1], o_st[2],
+        B, H, Sq, Sk, D, 0.0 if softmax_scale is None else C.c_float(softmax_scale).value,
+        0 if qw is None else qw.data_ptr(), 0 if kw is None else kw.data_ptr(), C.c_float(norm_eps).value, rope_mode, *tables,
+        mask_ptr, row_ptr, col_idx, flags, 0, 0))
     return a, keep
 
 
@@ -174,6 +179,18 @@ def workspace_bytes(args: _lib.AttnArgs) -> int:
     if n == 0:
         raise _lib.Pkh3Error(_lib.PKH3_EARG, _lib.load().pkh3_last_error().decode())
     return int(n)
+
+
+def _attn_fwd(lib, args: _lib.AttnArgs, device, workspace: Optional[torch.Tensor]) -> None:
+    """Enqueues the call on the device's current stream.  ``workspace``: one that may belong to another stream than this: it must
+    outlive the kernels, so it is tied to the stream.  (Memory allocated here belongs to this stream already.)"""
+    if device.index == torch.cuda.current_device():
+        _lib.check(lib.pkh3_attn_fwd(C.byref(args), torch._C._cuda_getCurrentRawStream(device.index)))
+    else:
+        with torch.cuda.device(device):
+            _lib.check(lib.pkh3_attn_fwd(C.byref(args), torch._C._cuda_getCurrentRawStream(device.index)))
+    if workspace is not None:
+        workspace.record_stream(torch.cuda.current_stream(device))
 
 
 def attention(
@@ -191,7 +208,7 @@ def attention(
     if out is None:
         if opts.get("out_images"):
             raise ValueError("out_images needs the image buffer as out")
-        out = torch.empty((q.shape[0], q.shape[1], q.shape[2], q.shape[3]), dtype=torch.bfloat16, device=q.device)
+        out = torch.empty(q.shape, dtype=torch.bfloat16, device=q.device)
     args, keep = fill_args(q, k, v, out, **opts)
     if static_scratch:
         with torch.cuda.device(q.device):
@@ -200,17 +217,14 @@ def attention(
     need = workspace_bytes(args)
     if callable(workspace):
         workspace = workspace(q.device, need)
-    if workspace is None or workspace.numel() * workspace.element_size() < need:
+    own = workspace is None or workspace.numel() * workspace.element_size() < need
+    if own:
         workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
-    args.workspace = workspace.data_ptr()
-    args.workspace_bytes = workspace.numel() * workspace.element_size()
-    if workspace.device != q.device:
+    elif workspace.device != q.device:
         raise ValueError(f"workspace must live on {q.device} (got {workspace.device})")
-    with torch.cuda.device(q.device):
-        stream = torch.cuda.current_stream()
-        _lib.check(lib.pkh3_attn_fwd(C.byref(args), C.c_void_p(stream.cuda_stream)))
-        # the workspace must outlive the kernels: tie it to the stream, not to this Python frame
-        workspace.record_stream(stream)
+    args.workspace = workspace.data_ptr()
+    args.workspace_bytes = need if own else workspace.numel() * workspace.element_size()
+    _attn_fwd(lib, args, q.device, None if own else workspace)
     return out
 
 
@@ -289,10 +303,7 @@ def attention_prepared(q: torch.Tensor, kv: PreparedKV, *, out: Optional[torch.T
     if kv.workspace.numel() < need:
         raise ValueError(f"the prepared workspace holds {kv.workspace.numel()} bytes, this call needs {need} (give prepare_kv q_rows)")
     args.workspace, args.workspace_bytes = kv.workspace.data_ptr(), kv.workspace.numel()
-    with torch.cuda.device(q.device):
-        stream = torch.cuda.current_stream()
-        _lib.check(lib.pkh3_attn_fwd(C.byref(args), C.c_void_p(stream.cuda_stream)))
-        kv.workspace.record_stream(stream)
+    _attn_fwd(lib, args, q.device, kv.workspace)
     return out
 
 

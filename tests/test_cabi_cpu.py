@@ -407,3 +407,9 @@ def test_headers_compile_as_c_and_a_c_program_links(tmp_path):
     assert int(out[0]) == _lib.load().pkh3_version()
     assert int(out[1]) == 0            # invalid arguments: no size
     assert int(out[2]) < 0 and out[3].strip()
+
+
+def test_argument_struct_is_packed_in_the_order_of_its_fields():
+    values = tuple(float(i) if t is C.c_float else i for i, (_, t) in enumerate(_lib.AttnArgs._fields_, 1))
+    a = _lib.AttnArgs.from_buffer_copy(_lib.ATTN_ARGS_FORMAT.pack(*values))
+    assert tuple(getattr(a, n) for n, _ in _lib.AttnArgs._fields_) == values
