@@ -38,6 +38,7 @@
 #include <math.h>
 
 #include <atomic>
+#include <type_traits>
 
 #include "pkh3_common.h"
 #include "pkh3_internal.h"
@@ -50,6 +51,7 @@ constexpr int kMaxParts = 8;     // long dense form: most workgroups a unit's ke
 constexpr int kMinPartTiles = 24;  // ... and fewest key tiles such a workgroup is worth starting for
 constexpr int kSparseWaves = 2 * kSparseRows;  // block-sparse: a wave pair per row-block; two such workgroups share a CU
 constexpr int kRing = 3;               // LDS ring depth (tiles)
+constexpr int kPipeRing = 4;           // ... of the pipelined short-key form (32-key halves)
 constexpr float kRescaleSlack = 8.0f;  // the running max is only raised when exceeded by 2^8
 // The running max before the first key.  Finite: keys whose logits are all -inf then weigh exp2(-inf - max) = 0, wherever
 // among a wave's keys they lie, and two shares without a key meet as exp2(0) times a row sum of 0.
@@ -227,14 +229,14 @@ __device__ __forceinline__ float softmax_numerator(float s, float c, float m) {
   else return __builtin_amdgcn_exp2f(STATIC ? s : s - m);
 }
 
-// Softmax numerators of NKB key blocks of w.s (a whole tile: 4, a 32-key half: 2) into the P^T operands of
+// Softmax numerators of NKB key blocks of w.s (a whole tile: 4, a 32-key half: 2), from block AT on, into the P^T operands of
 // the P.V MFMAs: operand (half, qb) takes, for lane group g, the keys v_image_key(g, j) of its half, i.e. registers
 // 0..3 of key block 2*half and of key block 2*half + 1 -- P never leaves its lane.  Also the running max / rescale
 // of the online path and the row sums.  `lim` = keys of these blocks that exist (only read when MASKED).
 // STATIC: w.m is not used: every logit is bounded (|q_i| * max_j |k_j| * c), small enough that exp2(logit) is a
 // normal number; the running max, its exchange across the lane groups and the O^T rescale are then not needed at
 // all, and the numerators of the first 32 keys do not wait for the second half of S^T.
-template <bool FP8, bool STATIC, bool MASKED, int NKB, bool POW2 = false>
+template <bool FP8, bool STATIC, bool MASKED, int NKB, bool POW2 = false, int AT = 0>
 __device__ __forceinline__ void softmax_blocks(WaveState<FP8>& w, bf16x8 (&pf)[NKB / 2][2], float c, int lim, int lane) {
   constexpr bool MUL = FP8 && !POW2;  // the logits still need their dequantisation scales
   const int g = lane >> 4;
@@ -244,19 +246,19 @@ __device__ __forceinline__ void softmax_blocks(WaveState<FP8>& w, bf16x8 (&pf)[N
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         if (16 * kb + 4 * g + i >= lim) {
-          w.s[kb][0][i] = -INFINITY;
-          w.s[kb][1][i] = -INFINITY;
+          w.s[AT + kb][0][i] = -INFINITY;
+          w.s[AT + kb][1][i] = -INFINITY;
         }
   }
   float m_new[2] = {w.m[0], w.m[1]}, alpha[2] = {1.0f, 1.0f};
   if constexpr (!STATIC) {
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
-      float mx = w.s[0][qb][0];
+      float mx = w.s[AT][qb][0];
 #pragma unroll
       for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) mx = fmaxf(mx, w.s[kb][qb][i]);
+        for (int i = 0; i < 4; ++i) mx = fmaxf(mx, w.s[AT + kb][qb][i]);
       mx = max_across_groups(mx) * (MUL ? c : 1.0f);
       m_new[qb] = (mx > w.m[qb] + kRescaleSlack) ? mx : w.m[qb];
       alpha[qb] = __builtin_amdgcn_exp2f(w.m[qb] - m_new[qb]);
@@ -280,7 +282,7 @@ __device__ __forceinline__ void softmax_blocks(WaveState<FP8>& w, bf16x8 (&pf)[N
       bf16x8 pk;
 #pragma unroll
       for (int j = 0; j < 8; ++j)
-        pk[j] = (__bf16)softmax_numerator<MUL, STATIC>(w.s[2 * half + (j >> 2)][qb][j & 3], c, m_new[qb]);
+        pk[j] = (__bf16)softmax_numerator<MUL, STATIC>(w.s[AT + 2 * half + (j >> 2)][qb][j & 3], c, m_new[qb]);
       // row sum over the bf16-rounded values, the same numbers the P.V MFMA consumes
 #pragma unroll
       for (int j = 0; j < 8; j += 2) {
@@ -322,10 +324,10 @@ __device__ __forceinline__ void softmax_pv_tile(WaveState<FP8>& w, const char* v
 }
 
 // ---- 32-key half tiles: the short-key form of the dense kernel, phase 2 of the block-sparse one ----
-// S^T (32 keys x 32 queries) into w.s[0..1]; kbuf/vbuf point at this half's K images (8 bf16 / 4 fp8 chunks)
+// S^T (32 keys x 32 queries) into w.s[AT..AT + 1]; kbuf/vbuf point at this half's K images (8 bf16 / 4 fp8 chunks)
 // and V images (8).
 // LEAN (three waves per SIMD): the K reads run 4 images ahead and only the fp8 path prefetches V (4 images).
-template <bool FP8, bool LEAN = false, bool POW2 = false>
+template <bool FP8, bool LEAN = false, bool POW2 = false, int AT = 0>
 __device__ __forceinline__ void qk_half(WaveState<FP8>& w, const char* kbuf, const char* vbuf, int lane, int ke = 0) {
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   if constexpr (!FP8 && LEAN) {
@@ -335,7 +337,7 @@ __device__ __forceinline__ void qk_half(WaveState<FP8>& w, const char* kbuf, con
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
 #pragma unroll
-      for (int qb = 0; qb < 2; ++qb) w.s[i & 1][qb] = PKH3_MFMA16(kf[i], w.qf[qb][i >> 1], i < 2 ? zero : w.s[i & 1][qb]);
+      for (int qb = 0; qb < 2; ++qb) w.s[AT + (i & 1)][qb] = PKH3_MFMA16(kf[i], w.qf[qb][i >> 1], i < 2 ? zero : w.s[AT + (i & 1)][qb]);
       if (i + 4 < 8) kf[i + 4] = *(const bf16x8*)(kbuf + ((i + 4) * 64 + lane) * 16);
     }
   } else if constexpr (!FP8) {
@@ -345,7 +347,7 @@ __device__ __forceinline__ void qk_half(WaveState<FP8>& w, const char* kbuf, con
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
 #pragma unroll
-      for (int qb = 0; qb < 2; ++qb) w.s[i & 1][qb] = PKH3_MFMA16(kf[i], w.qf[qb][i >> 1], i < 2 ? zero : w.s[i & 1][qb]);
+      for (int qb = 0; qb < 2; ++qb) w.s[AT + (i & 1)][qb] = PKH3_MFMA16(kf[i], w.qf[qb][i >> 1], i < 2 ? zero : w.s[AT + (i & 1)][qb]);
       w.vf[i] = *(const bf16x8*)(vbuf + (i * 64 + lane) * 16);
     }
   } else {
@@ -358,7 +360,7 @@ __device__ __forceinline__ void qk_half(WaveState<FP8>& w, const char* kbuf, con
       const i32x8 a = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
 #pragma unroll
       for (int qb = 0; qb < 2; ++qb)
-        w.s[kb][qb] = POW2 ? PKH3_MFMA16_F8S(a, w.q8[qb], zero, ke, w.qe) : PKH3_MFMA16_F8(a, w.q8[qb], zero);
+        w.s[AT + kb][qb] = POW2 ? PKH3_MFMA16_F8S(a, w.q8[qb], zero, ke, w.qe) : PKH3_MFMA16_F8(a, w.q8[qb], zero);
 #pragma unroll
       for (int i = 0; i < (LEAN ? 2 : 4); ++i) {
         const int v = (LEAN ? 2 : 4) * kb + i;
@@ -368,16 +370,16 @@ __device__ __forceinline__ void qk_half(WaveState<FP8>& w, const char* kbuf, con
   }
 }
 
-// Softmax numerators of w.s[0..1] and O^T += V^T P^T for one half tile (V images already in w.vf).
+// Softmax numerators of w.s[AT..AT + 1] and O^T += V^T P^T for one half tile (V images already in w.vf).
 // `lim` = keys of this half that exist (<= 0: none; only read when < 32).
 // LEAN: the V images (beyond the 4 the fp8 path prefetched) are read here, 4 ahead of their MFMAs, from vbuf.
 // FULL: the caller guarantees lim == 32, no masking code at all.
-template <bool FP8, bool STATIC, bool LEAN = false, bool FULL = false, bool POW2 = false>
+template <bool FP8, bool STATIC, bool LEAN = false, bool FULL = false, bool POW2 = false, int AT = 0>
 __device__ __forceinline__ void softmax_pv_half(WaveState<FP8>& w, float c, int lim, int lane, const char* vbuf = nullptr) {
   bf16x8 pf[1][2];
   // the running-max form always takes the masking copy (two copies of it do not fit the registers of some variants)
-  if (!FULL && (!STATIC || lim < 32)) softmax_blocks<FP8, STATIC, true, 2, POW2>(w, pf, c, lim, lane);
-  else softmax_blocks<FP8, STATIC, false, 2, POW2>(w, pf, c, lim, lane);
+  if (!FULL && (!STATIC || lim < 32)) softmax_blocks<FP8, STATIC, true, 2, POW2, AT>(w, pf, c, lim, lane);
+  else softmax_blocks<FP8, STATIC, false, 2, POW2, AT>(w, pf, c, lim, lane);
   if constexpr (LEAN) {
     bf16x8 vg[8];
 #pragma unroll
@@ -415,6 +417,57 @@ __device__ __forceinline__ float largest_key_norm(const Params& p, int bh, int n
   return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(wave_max(top))));
 }
 
+// The loop of the pipelined short-key form.  A pass runs S^T of the next half beside the softmax of this one, for waves that
+// have their SIMD to themselves or share it with one other.  A half takes 0.48 us with one
+// workgroup on a CU and 0.41 with two, of which 512 cycles are MFMAs.  (Measured, the same: P.V of half i, softmax of i + 1 and
+// S^T of i + 2 in one pass; six passes of lookahead instead of two.)  K of half i + 1 and V of half i are used,
+// half i + 2 is on its way and half i + 3 takes the slot of half i - 1 (past the end: the last half once more, into a slot that is
+// not read again, which leaves the pass without a branch).
+template <bool FP8, bool STATIC, bool POW2, typename Copy>
+__device__ __forceinline__ void pipe_loop(WaveState<FP8>& w, char* ring, int n, int sk, const float* kscale, float c, int lane, const Copy& copy) {
+  constexpr int kKHalf = (FP8 ? kK8TileBytes : kKTileBytes) / 2, kHalf = kKHalf + kVTileBytes / 2;
+  constexpr int kCopies = kHalf / 1024 / kShortWaves;    // of a half, by each wave
+  static_assert(kPipeRing == 4, "slots by the low bits of the half");
+  auto slot = [&](int i) { return ring + (i & 3) * kHalf; };
+  auto scale = [&](int i) { return FP8 ? uniform_load(kscale, min(i, n - 1) >> 1) : 1.0f; };
+  auto arrived = [&]() {                                 // all halves but the newest, for every wave
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kCopies) : "memory");
+    __syncthreads();
+  };
+  if (n == 0) return;
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kCopies) : "memory");
+  __syncthreads();
+  float ks = scale(0);
+  qk_half<FP8, false, POW2>(w, slot(0), slot(0) + kKHalf, lane, e8m0_of(ks));
+  auto pass = [&](auto at, auto full, int i) {
+    constexpr int AT = decltype(at)::value;
+    constexpr bool FULL = decltype(full)::value;
+    arrived();
+    const float ks_next = scale(i + 1);
+    qk_half<FP8, false, POW2, 2 - AT>(w, slot(i + 1), slot(i) + kKHalf, lane, e8m0_of(ks_next));
+    copy(min(i + 3, n - 1), (i + 3) & 3);
+    softmax_pv_half<FP8, STATIC, false, FULL, POW2, AT>(w, (FP8 && !POW2) ? c * ks : c, sk - 32 * i, lane);
+    ks = ks_next;
+  };
+  // the last half has no next one, and is the one that may be partial: its pass computes S^T of nothing that is used
+  const std::integral_constant<int, 0> even;
+  const std::integral_constant<int, 2> odd;
+  int i = 0;
+#pragma unroll 1
+  for (; i + 2 < n; i += 2) {
+    pass(even, std::true_type{}, i);
+    pass(odd, std::true_type{}, i + 1);
+  }
+  if (i + 1 < n) {
+    pass(even, std::true_type{}, i);
+    pass(odd, std::false_type{}, i + 1);
+  } else {
+    pass(even, std::false_type{}, i);
+  }
+  PKH3_MFMA_DRAIN(w);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the spare copies: the epilogue uses the LDS
+}
+
 // WAVES == kShortWaves selects the short-key form of the dense kernel: 4 waves (one per SIMD, <= 168 VGPRs) and a
 // ring of 32-key half tiles in 48 KiB of LDS, so three workgroups share a CU and the Q load and O store of one
 // run under the tiles of the others.  With few key tiles that overlap is worth more than the three-fold K/V
@@ -430,7 +483,7 @@ constexpr int kMergeBytes = kPartialBytes;  // one wave's partial result in fp32
 __host__ __device__ constexpr int units_per_head(int Sq, int blocks) { return ((Sq + 31) / 32 + blocks - 1) / blocks; }
 
 // bytes of LDS a form of the kernel needs
-template <bool FP8, bool SPARSE, int WAVES>
+template <bool FP8, bool SPARSE, int WAVES, bool PIPE = false>
 constexpr int fwd_lds_bytes() {
   constexpr bool HALFMODE = !SPARSE && WAVES == kShortWaves;
   constexpr int kRingT = (SPARSE && !FP8 && WAVES < 8) ? 2 : kRing;
@@ -440,7 +493,7 @@ constexpr int fwd_lds_bytes() {
   constexpr int kStageBytes = 32 * kD * 2;    // one wave's 32 x 128 bf16 output block, staged for the row-wise store
   // dense / phase 1: ring of kRingT whole tiles; sparse phase 2: kStages2 stages of row-private half tiles
   constexpr int kPhase2Bytes = SPARSE ? kStages2 * kSparseRows * kHalfBytes : 0;
-  constexpr int kRingBytes = HALFMODE ? kRing * kHalfBytes
+  constexpr int kRingBytes = HALFMODE ? (PIPE ? kPipeRing : kRing) * kHalfBytes
                              : (kPhase2Bytes > kRingT * kTileBytes ? kPhase2Bytes : kRingT * kTileBytes);
   constexpr int kAfterBytes = WAVES * kStageBytes;  // LDS use after the loops
   return kRingBytes > kAfterBytes ? kRingBytes : kAfterBytes;
@@ -452,7 +505,7 @@ constexpr int fwd_lds_bytes() {
 // units [unit0, unit0 + units), a unit being one workgroup's block of queries (`parts` workgroups per unit; their
 // partial results start at slot `part_base` of the scratch, their counters at unit slot `cnt_base`).
 // Block-sparse with work queues: returns the next position of the home queue, taken (thread 0) while the output is stored.
-template <bool FP8, bool SPARSE, int WAVES, bool POW2, typename Params>
+template <bool FP8, bool SPARSE, int WAVES, bool POW2, bool PIPE = false, typename Params>
 __device__ __forceinline__ int attn_fwd_body(const Params& p, int blk, int unit0, int units, int parts, int part_base,
                                               int cnt_base, char* lds_raw, int fetched = -1) {
   static_assert(!SPARSE || WAVES == kSparseWaves, "block-sparse layout: a wave pair per row-block of the plan");
@@ -552,7 +605,12 @@ __device__ __forceinline__ int attn_fwd_body(const Params& p, int blk, int unit0
   };
 
   WaveState<FP8> w;
-  if constexpr (HALFMODE) {
+  if constexpr (PIPE) {
+    if (n_half > 0) {
+#pragma unroll
+      for (int i = 0; i < kPipeRing - 1; ++i) dma_short(min(i, n_half - 1), i);
+    }
+  } else if constexpr (HALFMODE) {
     if (n_mine > 0) dma_short(h_begin, 0);
     if (n_mine > 1) dma_short(h_begin + 1, 1);
   } else if (t_end > t_begin) {
@@ -706,7 +764,11 @@ __device__ __forceinline__ int attn_fwd_body(const Params& p, int blk, int unit0
       softmax_pv_half<FP8, STATIC, true, FULL, POW2>(w, ct, sk - 32 * half, lane, hbuf + kKHalfB);      \
     }                                                                                                   \
   }
-  if constexpr (HALFMODE) {
+  if constexpr (PIPE) {
+    static_assert(HALFMODE, "32-key halves");
+    if (static_max) pipe_loop<FP8, true, POW2>(w, ring, n_half, sk, kscale, c, lane, dma_short);
+    else pipe_loop<FP8, false, POW2>(w, ring, n_half, sk, kscale, c, lane, dma_short);
+  } else if constexpr (HALFMODE) {
     const int n_iter = n_half;
     const int n_lead = sk / 32;  // leading full halves
     if (static_max) {
@@ -915,11 +977,11 @@ __device__ __forceinline__ int attn_fwd_body(const Params& p, int blk, int unit0
 
 // The block-sparse kernel and the short-key dense kernel (the block-sparse one takes its units from the work queues
 // when the launch has them: they differ in length with the tile lists on top of the XCDs' clocks).
-template <bool FP8, bool SPARSE, int WAVES, bool POW2>
-__global__ __launch_bounds__(64 * WAVES, (SPARSE ? 8 / WAVES : 3)) void attn_fwd_kernel(FwdParams p) {
-  __shared__ __attribute__((aligned(1024))) char lds_raw[fwd_lds_bytes<FP8, SPARSE, WAVES>()];
+template <bool FP8, bool SPARSE, int WAVES, bool POW2, bool PIPE = false>
+__global__ __launch_bounds__(64 * WAVES, (SPARSE ? 8 / WAVES : PIPE ? 2 : 3)) void attn_fwd_kernel(FwdParams p) {
+  __shared__ __attribute__((aligned(1024))) char lds_raw[fwd_lds_bytes<FP8, SPARSE, WAVES, PIPE>()];
   if constexpr (!SPARSE) {
-    attn_fwd_body<FP8, SPARSE, WAVES, POW2>(p, blockIdx.x, 0, p.sec_units[0], 1, 0, 0, lds_raw);
+    attn_fwd_body<FP8, SPARSE, WAVES, POW2, PIPE>(p, blockIdx.x, 0, p.sec_units[0], 1, 0, 0, lds_raw);
   } else {
     __shared__ int fetched_unit;
     int next_pos = 0;
@@ -1379,6 +1441,13 @@ static hipError_t launch_fp(FwdParams p, int cus, hipStream_t st) {
   if (form == kFormShort) {
     p.queue_next = nullptr;
     p.sec_units[0] = units(kShortWaves);
+    // Up to two workgroups per CU: the pipelined loop, which needs the registers of three waves for two.  From the third on, three
+    // to a CU overlap better (24 heads, us, plain / pipelined: 216 workgroups x 34 halves 27.8 / 22.8 and x 64 44.3 / 37.6, 168 x 25 20.5 / 18.3,
+    // 384 x 63 57.4 / 54.8, 504 x 82 78.6 / 75.2; 960 x 16 38.9 / 38.0, 2,784 x 16 94.8 / 99.1, 9,312 x 10 249 / 264; fp8 alike).
+    if (p.sec_units[0] <= 2 * cus) {
+      hipLaunchKernelGGL((attn_fwd_kernel<FP8, false, kShortWaves, POW2, true>), dim3(blocks_of(p.sec_units[0])), dim3(64 * kShortWaves), 0, st, p);
+      return hipGetLastError();
+    }
     hipLaunchKernelGGL((attn_fwd_kernel<FP8, false, kShortWaves, POW2>), dim3(blocks_of(p.sec_units[0])), dim3(64 * kShortWaves), 0, st, p);
     return hipGetLastError();
   }

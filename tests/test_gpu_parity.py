@@ -204,6 +204,24 @@ def test_kv_pass_walks_several_heads(B, H, Sk, mode, fp8, masked):
     _run_and_check(B, 40, Sk, H, seed=31 + mode, rope_mode=mode, weight_random=True, fp8=fp8, mask=mask)
 
 
+@pytest.mark.parametrize("fp8", [False, True, "pow2"])
+@pytest.mark.parametrize("std", [1.0, 8.0])   # bounded logits; logits that take the running maximum
+@pytest.mark.parametrize("Sk", [1, 32, 33, 64, 95, 128, 129, 160, 191, 225, 513])
+def test_pipelined_short_key_form_at_every_end(Sk, std, fp8):
+    """Two short-key workgroups per CU and fewer: passes work on two halves at once, the last one or two of them on what is there."""
+    import pika_h3_flex_amd as pk
+
+    H, Sq = 24, 1061
+    assert _form(1, H, Sq, Sk, fp8=fp8) == forms.SHORT
+    gen = torch.Generator().manual_seed(Sk)
+    q, k, v = (_rand((1, n, H, 128), gen, s).cuda() for n, s in ((Sq, std), (Sk, 1.0), (Sk, 1.0)))
+    got = pk.attention(q, k, v, fp8_qk=fp8).float()
+    want = pk.attention(q, k, v, fp8_qk=fp8, long_key_kernel=True).float()
+    # the same weights, rounded to bf16 at bases that may differ (2^-9 of each, in both), and both results rounded (2^-9):
+    # the weights sum to 1, so at most 4 * 2^-9 of the largest value
+    assert torch.isfinite(got).all() and (got - want).abs().max() <= 4 * 2 ** -9 * v.float().abs().max()
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("scale", [0.05, 0.2])
 def test_softmax_scale_other_than_default(scale, fp8):
