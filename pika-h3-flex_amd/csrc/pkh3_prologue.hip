@@ -259,8 +259,12 @@ hipError_t launch_kv_prologue(const QkPrologueParams& k, const VPrologueParams& 
   if (e != hipSuccess) return e;
   // Heads a workgroup walks: more of them share one read of the tables, as long as two or three workgroups of each side are
   // left per CU.  15,342 rows x 24 heads with rotation: 1 head 113 us, 2 91, 4 87, 8 85, 12 87; fp8 117, 90, 82, 76, 84.
-  const int64_t per_side = (int64_t)k.nBlk64 * k.B * k.H * 2 / (5 * max(cus, 1));
-  const int most = (int)max((int64_t)1, min(per_side, (int64_t)min(kKvMaxHeads, k.H)));
+  // Three from where single heads make more workgroups than run at once (1, 2, 3 and 4 heads, us, 24 heads with rotation:
+  // 1,000 rows 9.8, 10.1, 9.2, 10.4; 1,500 13.7, 12.5, 12.2, 13.9; 3,000 24.8, 20.8, 20.1, 22.8, fp8 25.0, 22.0, 20.4, 22.9; without rotation
+  // 1,000 rows 7.1, 7.9, 7.8, 8.9; 1,500 9.8, 9.8, 9.6, 10.9; 3,000 18.6, 17.3, 17.0, 19.2).
+  const int64_t single = (int64_t)k.nBlk64 * k.B * k.H, per_cu = max(cus, 1);
+  const int64_t per_side = max(single * 2 / (5 * per_cu), single * 4 >= 9 * per_cu ? (int64_t)3 : (int64_t)1);
+  const int most = (int)min(per_side, (int64_t)min(kKvMaxHeads, k.H));
   int groups = (k.H + most - 1) / most;
   const int n = (k.H + groups - 1) / groups;   // equal shares
   groups = (k.H + n - 1) / n;
