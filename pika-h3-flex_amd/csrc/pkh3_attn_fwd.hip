@@ -143,6 +143,9 @@ __device__ __forceinline__ void load_q_rows(QRows& r, const Params& p, const Row
   if (p.q_rope_mode != 0) load_rope_quarter(r.rope, tf, src, g);
 }
 
+// Consecutive MFMAs share an operand where they can: the two query blocks of an image come in turn (0 1, 1 0, 0 1 ..), so that only
+// one of the operands changes from one to the next.  Less toggles in the matrix unit, at a clock that is set by power: 480p 19.69 ->
+// 19.64 ms, 14,830 + 512 rows 2,142 -> 2,135 us, with the projection's GEMMs (the same) a block of them 3,153 -> 3,138.
 #define PKH3_MFMA16(A, B, C) __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, C, 0, 0, 0)
 // format codes 0/0 = e4m3 x e4m3; scale operands 0 select the unscaled form of the instruction
 #define PKH3_MFMA16_F8(A, B, C) __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(A, B, C, 0, 0, 0, 0, 0, 0)
@@ -168,7 +171,7 @@ __device__ __forceinline__ void qk_tile(WaveState<FP8>& w, const char* kbuf, con
     for (int i = 0; i < 16; ++i) {
       const int ks = (i >> 1) & 3, kb = 2 * (i >> 3) + (i & 1);
 #pragma unroll
-      for (int qb = 0; qb < 2; ++qb) w.s[kb][qb] = PKH3_MFMA16(kf[i], w.qf[qb][ks], ks == 0 ? zero : w.s[kb][qb]);
+      for (int q = 0, qb = i & 1; q < 2; ++q, qb ^= 1) w.s[kb][qb] = PKH3_MFMA16(kf[i], w.qf[qb][ks], ks == 0 ? zero : w.s[kb][qb]);
       if (i + AHEAD < 16) kf[i + AHEAD] = *(const bf16x8*)(kbuf + ((i + AHEAD) * 64 + lane) * 16);
     }
     PKH3_SGB(kSgDsRead, AHEAD);
@@ -185,7 +188,7 @@ __device__ __forceinline__ void qk_tile(WaveState<FP8>& w, const char* kbuf, con
     for (int i = 0; i < 16; ++i) {
       const int ks = (i >> 1) & 3, kb = 2 * (i >> 3) + (i & 1);
 #pragma unroll
-      for (int qb = 0; qb < 2; ++qb) w.s[kb][qb] = PKH3_MFMA16(kf[i], w.qf[qb][ks], ks == 0 ? zero : w.s[kb][qb]);
+      for (int q = 0, qb = i & 1; q < 2; ++q, qb ^= 1) w.s[kb][qb] = PKH3_MFMA16(kf[i], w.qf[qb][ks], ks == 0 ? zero : w.s[kb][qb]);
       if (i < 8)
         kf[i + 8] = *(const bf16x8*)(kbuf + ((i + 8) * 64 + lane) * 16);
       else
@@ -309,7 +312,7 @@ __device__ __forceinline__ void softmax_pv_tile(WaveState<FP8>& w, const char* v
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
 #pragma unroll
-      for (int qb = 0; qb < 2; ++qb) w.o[i & 7][qb] = PKH3_MFMA16(vg[i], pf[i >> 3][qb], w.o[i & 7][qb]);
+      for (int q = 0, qb = i & 1; q < 2; ++q, qb ^= 1) w.o[i & 7][qb] = PKH3_MFMA16(vg[i], pf[i >> 3][qb], w.o[i & 7][qb]);
       if (i + 4 < 16) vg[i + 4] = *(const bf16x8*)(vbuf + ((i + 4) * 64 + lane) * 16);
     }
   } else {
@@ -317,7 +320,7 @@ __device__ __forceinline__ void softmax_pv_tile(WaveState<FP8>& w, const char* v
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
 #pragma unroll
-      for (int qb = 0; qb < 2; ++qb) w.o[i & 7][qb] = PKH3_MFMA16(i < 8 ? w.vf[i] : vg[i - 8], pf[i >> 3][qb], w.o[i & 7][qb]);
+      for (int q = 0, qb = i & 1; q < 2; ++q, qb ^= 1) w.o[i & 7][qb] = PKH3_MFMA16(i < 8 ? w.vf[i] : vg[i - 8], pf[i >> 3][qb], w.o[i & 7][qb]);
       if (i < 8) vg[i] = *(const bf16x8*)(vbuf + ((i + 8) * 64 + lane) * 16);
     }
   }
@@ -337,7 +340,7 @@ __device__ __forceinline__ void qk_half(WaveState<FP8>& w, const char* kbuf, con
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
 #pragma unroll
-      for (int qb = 0; qb < 2; ++qb) w.s[AT + (i & 1)][qb] = PKH3_MFMA16(kf[i], w.qf[qb][i >> 1], i < 2 ? zero : w.s[AT + (i & 1)][qb]);
+      for (int q = 0, qb = i & 1; q < 2; ++q, qb ^= 1) w.s[AT + (i & 1)][qb] = PKH3_MFMA16(kf[i], w.qf[qb][i >> 1], i < 2 ? zero : w.s[AT + (i & 1)][qb]);
       if (i + 4 < 8) kf[i + 4] = *(const bf16x8*)(kbuf + ((i + 4) * 64 + lane) * 16);
     }
   } else if constexpr (!FP8) {
@@ -347,7 +350,7 @@ __device__ __forceinline__ void qk_half(WaveState<FP8>& w, const char* kbuf, con
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
 #pragma unroll
-      for (int qb = 0; qb < 2; ++qb) w.s[AT + (i & 1)][qb] = PKH3_MFMA16(kf[i], w.qf[qb][i >> 1], i < 2 ? zero : w.s[AT + (i & 1)][qb]);
+      for (int q = 0, qb = i & 1; q < 2; ++q, qb ^= 1) w.s[AT + (i & 1)][qb] = PKH3_MFMA16(kf[i], w.qf[qb][i >> 1], i < 2 ? zero : w.s[AT + (i & 1)][qb]);
       w.vf[i] = *(const bf16x8*)(vbuf + (i * 64 + lane) * 16);
     }
   } else {
@@ -387,14 +390,14 @@ __device__ __forceinline__ void softmax_pv_half(WaveState<FP8>& w, float c, int 
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
 #pragma unroll
-      for (int qb = 0; qb < 2; ++qb) w.o[i][qb] = PKH3_MFMA16(vg[i], pf[0][qb], w.o[i][qb]);
+      for (int q = 0, qb = i & 1; q < 2; ++q, qb ^= 1) w.o[i][qb] = PKH3_MFMA16(vg[i], pf[0][qb], w.o[i][qb]);
       if (i + 4 < 8) vg[i + 4] = *(const bf16x8*)(vbuf + ((i + 4) * 64 + lane) * 16);
     }
   } else {
 #pragma unroll
     for (int i = 0; i < 8; ++i)
 #pragma unroll
-      for (int qb = 0; qb < 2; ++qb) w.o[i][qb] = PKH3_MFMA16(w.vf[i], pf[0][qb], w.o[i][qb]);
+      for (int q = 0, qb = i & 1; q < 2; ++q, qb ^= 1) w.o[i][qb] = PKH3_MFMA16(w.vf[i], pf[0][qb], w.o[i][qb]);
   }
 }
 

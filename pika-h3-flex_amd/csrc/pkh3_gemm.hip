@@ -193,7 +193,8 @@ __device__ __forceinline__ void gemm_loop(const GemmParams& p, const GemmTarget&
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     static_for<8 * TB>([&](auto kc) {
-      constexpr int k = decltype(kc)::value, fb = k / TB, t = k % TB;
+      // (token blocks back and forth: from one MFMA to the next only one operand changes)
+      constexpr int k = decltype(kc)::value, fb = k / TB, t = fb & 1 ? TB - 1 - k % TB : k % TB;
       if constexpr (SWAP) mfma_acc<(TB > 4), TB == 6 && k == 8 * TB - 1>(acc[t][fb], x[t], w[fb]);
       else mfma_acc<(TB > 4), TB == 6 && k == 8 * TB - 1>(acc[t][fb], w[fb], x[t]);
       if constexpr (TB > 2) {
