@@ -124,7 +124,8 @@ WsPlan plan(const pkh3_attn_args* a, bool part_scratch = true) {
   w.split_bytes = part_wgs * 12 * (size_t)kPartialBytes;
   w.split_off = off;  off = align_up(off + w.split_bytes, 256);
   // positions of the work queues (of the fused q/k/v projection, then of a long or block-sparse attention call), then the arrival counters
-  w.split_cnt_off = off; off = align_up(off + (kQueueSlots + part_wgs * 12) * sizeof(int), 256);
+  w.n_counters = (int)(kQueueSlots + part_wgs * 12);
+  w.split_cnt_off = off; off = align_up(off + w.n_counters * sizeof(int), 256);
   w.total = off;
   return w;
 }
@@ -158,6 +159,10 @@ void build(const pkh3_attn_args* a, void* workspace, Launch& L, bool part_scratc
   k.out = ws + L.w.kv_off; k.out_bh_stride = (int64_t)L.w.nKt * L.w.kvTileBytes; k.out_blk_stride = L.w.kvTileBytes;
   k.scale_out = fp8 ? (float*)(ws + L.w.kscale_off) : nullptr; k.fp8 = fp8;
   k.fp8_pow2 = (a->flags & PKH3_FLAG_FP8_POW2_SCALES) ? 1 : 0;
+  // Long and block-sparse calls: the pass clears the attention launch's counters as well, which saves a launch of its own (390.0 -> 387.5 us
+  // for 24 heads x 6,000 rows, 271.0 -> 269.9 for 6,317 block-sparse ones).  Its workgroups are enough: 34 and more for at most 6,208 words.
+  k.clear = (unsigned*)(ws + L.w.split_cnt_off);
+  k.clear_n = a->blk_row_ptr || L.w.nKt > kShortMaxTiles ? L.w.n_counters : 0;
   k.norm_out = (float*)(ws + L.w.knorm_off); k.norm_stride = L.w.knorm_stride;
 
   VPrologueParams& v = L.vp;
@@ -190,6 +195,7 @@ void build(const pkh3_attn_args* a, void* workspace, Launch& L, bool part_scratc
   f.split_scratch_bytes = L.w.split_bytes;
   f.split_cnt = (int*)(ws + L.w.split_cnt_off) + kQueueSlots;
   f.queue_next = (int*)(ws + L.w.split_cnt_off);
+  f.counters_clear = k.clear_n > 0 && !(a->flags & PKH3_FLAG_KV_PREPARED);
 }
 
 int hip_fail(hipError_t e, const char* what) {
@@ -302,6 +308,7 @@ int prepare_call(const pkh3_attn_args* a, hipStream_t st, FwdParams* out) {
     return fail(PKH3_EWORKSPACE, "workspace too small: %zu < %zu bytes", a->workspace_bytes, L.w.total);
   if ((rc = run_prologue(a, L, st))) return rc;
   *out = L.f;
+  out->counters_clear = 0;   // the launch is repeated: it clears them itself
   g_err[0] = 0;
   return PKH3_OK;
 }

@@ -1432,7 +1432,7 @@ static hipError_t launch_fp(FwdParams p, int cus, hipStream_t st) {
     int wgs = n;
     if (p.queue_next && cus > 0 && n >= cus) {
       // at least a round of workgroups: one per CU (the LDS of the form holds no second), units from the work queues
-      hipError_t e = launch_fill_zero((unsigned*)p.queue_next, kQueues, st);
+      hipError_t e = p.counters_clear ? hipSuccess : launch_fill_zero((unsigned*)p.queue_next, kQueues, st);
       if (e != hipSuccess) return e;
       wgs = cus;
     } else {
@@ -1471,7 +1471,7 @@ static hipError_t launch_fp(FwdParams p, int cus, hipStream_t st) {
   // calls of at least one round of workgroups take their whole units from the work queues
   const bool queues = whole > 0 && !p.long_key_kernel && p.queue_next;
   if (!queues) p.queue_next = nullptr;
-  if (queues || shared > 0) {
+  if ((queues || shared > 0) && !p.counters_clear) {
     // queue positions and arrival counters start at zero (the arrival counters follow the queue slots)
     hipError_t e = launch_fill_zero((unsigned*)(p.split_cnt - kQueueSlots), kQueueSlots + shared * kDenseWaves, st);
     if (e != hipSuccess) return e;

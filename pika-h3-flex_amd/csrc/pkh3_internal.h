@@ -32,6 +32,7 @@ struct WsPlan {
   size_t kv_off, kscale_off, cnt_off, idx_off, plan_off, plan_cnt_off, knorm_off, split_off, split_cnt_off, total;
   int knorm_stride;    // floats between consecutive (b,h) at knorm_off
   size_t knorm_bytes;
+  int n_counters;      // ints at split_cnt_off
   size_t split_bytes;  // bytes at split_off: partial results of the long dense form's paired workgroups
 };
 
@@ -55,6 +56,8 @@ struct QkPrologueParams {
   float* scale_out;         // fp8: [B*H, nBlk64] dequantisation scales, else null
   int fp8;
   int fp8_pow2;             // fp8: block scales rounded up to a power of two
+  unsigned* clear;          // words the pass sets to zero besides (queue positions and arrival counters of the attention launch after it)
+  int clear_n;              // at most 256 for every workgroup of the pass
   float* norm_out;          // [B*H][norm_stride]: largest row norm (after norm and rotation) of every 32 rows written
   int norm_stride;
 };
@@ -102,6 +105,7 @@ struct FwdParams {
   float* split_scratch;
   size_t split_scratch_bytes;
   int* split_cnt;           // arrival counters; the kQueueSlots ints in front of them belong to the work queues
+  int counters_clear;       // the K/V pass of this call has cleared both
   int* queue_next;          // [kSections][kQueues] next unit of each work queue (= split_cnt - kQueueSlots), or null: fixed map
   int few_halves;           // filled per launch (narrow form with a key mask): fewer half tiles of valid keys are walked as the short-key form does
   // filled per launch: the sections of the launch.  A unit is one workgroup's block of queries; section i covers
