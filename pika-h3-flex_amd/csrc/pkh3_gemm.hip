@@ -9,7 +9,7 @@
 // l%16, elements 8*(l/16)..+7 -- the shape of the attention kernel's K images): activations as [16-token
 // block][k-step], weights as [16-feature block][k-step] (packed once when the weights are loaded).  They move
 // HBM/L2 -> LDS -> VGPR as straight 16-byte copies, like the K/V tiles of the attention kernel: direct-to-LDS loads
-// into a 3-slot ring, up to three chunks ahead, one barrier per chunk.  Since the two MFMA operands have the same register
+// into a ring of three slots (four where a launch's tiles have a CU each), as many chunks ahead, one barrier per chunk.  Since the two MFMA operands have the same register
 // form, one pair of images serves both orientations:
 //   C^T = W x^T  (features down the accumulator registers, one token per lane)   Q, K, row-major outputs
 //   C   = x W^T  (tokens down the registers, one feature per lane)               V images
@@ -36,7 +36,7 @@ namespace pkh3 {
 
 constexpr int kGemmWaves = 4;                       // two 128-feature heads x two token halves
 constexpr int kGemmFeatures = 256;                  // features per workgroup
-constexpr int kGemmRing = 3;                        // ring slots: one 32-wide k-chunk of weight and activation images each
+constexpr int kGemmRing = 3;                        // ring slots (R; see launch_gemm): one 32-wide k-chunk of weight and activation images each
 constexpr int kGemmWPieces = kGemmFeatures / 16;    // 1 KiB weight images of a chunk
 
 template <int N, int I = 0, class F>
@@ -92,11 +92,10 @@ __device__ __forceinline__ void acc_block(float (&x)[32], const f32x4 (&a)[8]) {
 }
 
 // Main loop: acc[t][fb] = the wave's 16-token block t x 16-feature block fb.  SWAP: tokens down the registers (V images).
-template <int TB, bool SWAP>
+template <int TB, int R, bool SWAP>
 __device__ __forceinline__ void gemm_loop(const GemmParams& p, const GemmTarget& tg, int m_tile, int n_tile_in_target, bool head_live,
                                           char* lds_raw, f32x4 (&acc)[TB][8]) {
   constexpr int kStage = (kGemmWPieces + 2 * TB) * 1024;
-  constexpr int R = kGemmRing;
   constexpr int kXPieces = TB / 2;                   // activation pieces of a chunk each wave copies (and 4 weight pieces)
   constexpr int PP = 4 + kXPieces;
   const int lane = threadIdx.x & 63;
@@ -482,9 +481,9 @@ __device__ __forceinline__ void epilogue_rows(const GemmParams& p, const GemmTar
   static_for<TB>([&](auto tc) { block(tc, kAhead == 2 && (decltype(tc)::value & 1) ? odd : even); });
 }
 
-template <int TB>
+template <int TB, int R>
 __global__ __launch_bounds__(64 * kGemmWaves, TB > 4 ? 1 : 2) void gemm_kernel(GemmParams p) {
-  __shared__ __attribute__((aligned(1024))) char lds_raw[kGemmRing * (kGemmWPieces + 2 * TB) * 1024];
+  __shared__ __attribute__((aligned(1024))) char lds_raw[R * (kGemmWPieces + 2 * TB) * 1024];
   // Workgroups go to the 8 XCDs round-robin; each XCD takes one contiguous run of the tile order below, in which 32
   // consecutive tiles (the workgroups the 32 CUs behind one L2 run together) form a block of 4 token tiles x 8
   // feature tiles: every activation panel is then shared by 8 and every weight panel by 4 of them.
@@ -522,13 +521,13 @@ __global__ __launch_bounds__(64 * kGemmWaves, TB > 4 ? 1 : 2) void gemm_kernel(G
   const int tok0 = (m_tile * 2 + (wave >> 1)) * (16 * TB);   // first of the wave's tokens
   f32x4 acc[TB][8];
   if (tg.epi == kEpiVImg) {
-    gemm_loop<TB, true>(p, tg, m_tile, n_tile, head_live, lds_raw, acc);
+    gemm_loop<TB, R, true>(p, tg, m_tile, n_tile, head_live, lds_raw, acc);
     // by the 64-token record, not by the wave's own tokens: with TB == 2 a wave holds half a record, and a half without tokens
     // is written as zeros (kernels that walk whole 64-key tiles multiply it by probabilities of 0)
     if (head_live && (tok0 & ~63) < p.M) epilogue_v<TB>(p, tg, head, tok0, acc);
     return;
   }
-  gemm_loop<TB, false>(p, tg, m_tile, n_tile, head_live, lds_raw, acc);
+  gemm_loop<TB, R, false>(p, tg, m_tile, n_tile, head_live, lds_raw, acc);
   if (tg.epi == kEpiKImg) {
     if (tg.rope_mode == 1) epilogue_k<TB, 1>(p, tg, head, head_live, tok0, acc);
     else if (tg.rope_mode == 2) epilogue_k<TB, 2>(p, tg, head, head_live, tok0, acc);
@@ -654,7 +653,7 @@ static int gemm_token_blocks(int tokens, int n_tiles, int cus) {
   return best;
 }
 
-template <int TB>
+template <int TB, int R = kGemmRing>
 static hipError_t launch_gemm_tb(GemmParams p, int cus, hipStream_t st) {
   p.m_tiles = (p.M + 32 * TB - 1) / (32 * TB);
   const int total = p.m_tiles * p.n_tiles;
@@ -666,7 +665,7 @@ static hipError_t launch_gemm_tb(GemmParams p, int cus, hipStream_t st) {
     if (e != hipSuccess) return e;
   }
   const int wgs = p.queue_next ? total + (total / 8 > kQueues ? total / 8 : kQueues) : total;
-  hipLaunchKernelGGL(gemm_kernel<TB>, dim3((wgs + 7) / 8 * 8), dim3(64 * kGemmWaves), 0, st, p);
+  hipLaunchKernelGGL((gemm_kernel<TB, R>), dim3((wgs + 7) / 8 * 8), dim3(64 * kGemmWaves), 0, st, p);
   return hipGetLastError();
 }
 
@@ -695,8 +694,14 @@ hipError_t launch_gemm(const GemmParams& p, hipStream_t st) {
     case 8: return launch_gemm_tb<8>(p, cus, st);
     case 6: return launch_gemm_tb<6>(p, cus, st);
     case 4: return launch_gemm_tb<4>(p, cus, st);
-    default: return launch_gemm_tb<2>(p, cus, st);
+    default: break;
   }
+  // 64 tokens with one workgroup on a CU: a chunk is done in 0.22 us, and three of them cover a copy's way where two do not.  Ring of
+  // 3 / 4, K 3,072 x 3,072 features, us: 128 tokens 29.7 / 24.6, 500 31.2 / 26.0, 1,085 32.0 / 27.2 (of 5 to 7 the same); with a dozen workgroups on
+  // the chip the way is short enough (64 tokens 23.0 / 23.6), and for few chunks the longer start costs more (K 1,024 13.4 / 12.6 and
+  // 11.7 / 12.0, 512 8.1 / 8.3).  The larger forms gain nothing from it.
+  const int64_t tiles = (int64_t)((p.M + 63) / 64) * p.n_tiles;
+  return tiles >= 24 && tiles <= cus && p.nk1 >= 48 ? launch_gemm_tb<2, 4>(p, cus, st) : launch_gemm_tb<2>(p, cus, st);
 }
 
 // ------------------------------------------------------------------------------------------------

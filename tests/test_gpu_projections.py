@@ -175,7 +175,9 @@ def test_qkv_projection_feeds_attention(S, H, variant):
     assert cos >= (0.995 if variant.startswith("fp8") else 0.9999)
 
 
-@pytest.mark.parametrize("S,N,K,lora,extras", [(300, 256, 256, True, True), (1000, 384, 256, False, True), (65, 128, 512, True, False)])
+@pytest.mark.parametrize("S,N,K,lora,extras", [(300, 256, 256, True, True), (1000, 384, 256, False, True), (65, 128, 512, True, False),
+                                                 # the ring of four slots: even and odd numbers of chunks, a last token alone in its tile
+                                                 (129, 3072, 1536, False, True), (130, 2944, 1568, True, False), (705, 1152, 1600, True, True)])
 def test_out_projection_with_gate_and_residual(S, N, K, lora, extras):
     from oracle import attention_oracle as AO
     from oracle import projection_oracle as PO
