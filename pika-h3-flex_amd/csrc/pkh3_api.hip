@@ -108,7 +108,7 @@ WsPlan plan(const pkh3_attn_args* a, bool part_scratch = true) {
   w.kscale_off = off; if (fp8) off = align_up(off + bh * w.nKt * sizeof(float), 256);
   w.cnt_off = off;    if (a->key_mask) off = align_up(off + (size_t)a->B * sizeof(int), 256);
   w.idx_off = off;    if (a->key_mask) off = align_up(off + (size_t)a->B * a->Sk * sizeof(int), 256);
-  w.knorm_stride = (2 * w.nKt + 3) / 4 * 4;
+  w.knorm_stride = kNormFirst + (2 * w.nKt + 3) / 4 * 4;
   w.knorm_bytes = align_up(bh * w.knorm_stride * sizeof(float), 256);
   w.knorm_off = off;  off += w.knorm_bytes;
   // everything above is the K/V side and depends on B, H, Sk and the K-side options only (pkh3_kv_prepare);
@@ -262,9 +262,9 @@ int check_linear(const char* name, const pkh3_linear* l) {
 // Scratch of pkh3_attn_fwd_noalloc: one array per GPU the library is loaded on, held until the process ends.
 // In host code the array's name is only a handle; each device's copy has its own address, looked up once per
 // device (with that device current) and used from then on wherever the memory itself is meant.
-// The row norms of the keys (2 floats per 64-key tile, whose record takes at least 24 KiB) don't count against the
+// The row norms of the keys (2 floats per 64-key tile, whose record takes at least 24 KiB, and at most 6 a head) don't count against the
 // advertised size but for one float a head: the array holds them besides.
-constexpr size_t kNormRoom = 65536;
+constexpr size_t kNormRoom = 131072;
 static __device__ __align__(256) unsigned char scratch[PKH3_NOALLOC_SCRATCH_BYTES + kNormRoom];
 
 size_t counted_bytes(const pkh3_attn_args* a, const WsPlan& w) {
@@ -380,6 +380,8 @@ int pkh3_kv_prepare(const pkh3_attn_args* a, void* stream) {
   if (a->workspace_bytes < L.w.total)
     return fail(PKH3_EWORKSPACE, "workspace too small: %zu < %zu bytes", a->workspace_bytes, L.w.total);
   if ((rc = run_kv_side(a, L, (hipStream_t)stream))) return rc;
+  hipError_t e = launch_fold_norms(L.kp, (hipStream_t)stream);
+  if (e != hipSuccess) return hip_fail(e, "fold_norms");
   g_err[0] = 0;
   return PKH3_OK;
 }

@@ -405,11 +405,14 @@ __device__ __forceinline__ void softmax_pv_half(WaveState<FP8>& w, float c, int 
 // time (`first`), the wave's lanes meet where the number is needed.
 template <typename Params>
 __device__ __forceinline__ f32x4 ask_key_norms(const Params& p, int bh, int lane) {
-  return *(const f32x4*)(p.knorm + (int64_t)bh * p.knorm_stride + min(4 * lane, p.knorm_stride - 4));
+  return *(const f32x4*)(p.knorm + (int64_t)bh * p.knorm_stride + min(kNormFirst + 4 * lane, p.knorm_stride - 4));
 }
 template <typename Params>
 __device__ __forceinline__ float largest_key_norm(const Params& p, int bh, int n, f32x4 first, int lane) {
   const float* norms = p.knorm + (int64_t)bh * p.knorm_stride;
+  const float known = uniform_load(norms, 0);   // prepared keys
+  if (known >= 0.f) return known;
+  norms += kNormFirst;
   float top = 0.f;
   auto take = [&](const f32x4& v, int at) {   // places past the valid keys may never have been written
 #pragma unroll
@@ -527,7 +530,9 @@ __device__ __forceinline__ int attn_fwd_body(const Params& p, int blk, int unit0
   constexpr int kHalfBytes = kTileBytes / 2;  // K and V images of 32 keys
   constexpr int kStageBytes = 32 * kD * 2;    // one wave's 32 x 128 bf16 output block, staged for the row-wise store
   char(*lds)[kTileBytes] = (char(*)[kTileBytes])lds_raw;
-  const int lane = threadIdx.x & 63;
+  int lane = threadIdx.x & 63;
+  // (what is made of the lane is made again for every unit: kept across the units, it does not fit the registers)
+  if constexpr (SPARSE) asm volatile("" : "+v"(lane));
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
   // Workgroups are handed to the 8 XCDs round-robin; give each XCD one contiguous run of

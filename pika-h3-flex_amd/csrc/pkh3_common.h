@@ -53,12 +53,6 @@ constexpr int kQ8BlkBytes = 4096;  // fp8 Q block of 32 queries
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kFp8Max = 448.0f;  // OCP e4m3fn
 
-__device__ __forceinline__ float wave_max(float x) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) x = fmaxf(x, __shfl_xor(x, o, 64));
-  return x;
-}
-
 // RMSNorm + rotation of one row: what is done to it (norm_rope_quarter below does it).
 struct RowTransform {
   const float* norm_w;  // [D] or null
@@ -82,6 +76,21 @@ __device__ __forceinline__ float max_across_groups(float x) {
   x = fmaxf(__uint_as_float(r16[0]), __uint_as_float(r16[1]));
   const auto r32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   return fmaxf(__uint_as_float(r32[0]), __uint_as_float(r32[1]));
+}
+
+// maximum over the wave, in every lane: pairs, quads and halves of the 16-lane rows by permutations that ride on the comparison,
+// then across the rows (no trip through the LDS crossbar)
+template <int CTRL>
+__device__ __forceinline__ float max_with(float x) {
+  const int v = __float_as_int(x);
+  return fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(v, v, CTRL, 0xf, 0xf, false)));
+}
+__device__ __forceinline__ float wave_max(float x) {
+  x = max_with<0xB1>(x);     // quad_perm 1 0 3 2
+  x = max_with<0x4E>(x);     // quad_perm 2 3 0 1
+  x = max_with<0x141>(x);    // row_half_mirror
+  x = max_with<0x140>(x);    // row_mirror
+  return max_across_groups(x);
 }
 
 // ---- four lanes per row: the layout of the 16x16 operand images themselves ----

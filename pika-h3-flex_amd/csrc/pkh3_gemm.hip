@@ -361,8 +361,9 @@ __device__ __forceinline__ void epilogue_k(const GemmParams& p, const GemmTarget
       nmax = fmaxf(nmax, wave_sum_groups((ssq[0] + ssq[1]) + (ssq[2] + ssq[3])));
     });
     nmax = sqrtf(wave_max(nmax));
-    float* norms = tg.norm_out + (int64_t)head * tg.norm_stride + (first >> 5);
+    float* norms = tg.norm_out + (int64_t)head * tg.norm_stride + kNormFirst + (first >> 5);
     if (lane < kTBlk / 2) norms[lane] = nmax;        // the places of the part's 32-token halves
+    if (first == 0 && lane == 0) norms[-kNormFirst] = -1.0f;
   });
   if (!tg.fp8) return;
 #pragma unroll

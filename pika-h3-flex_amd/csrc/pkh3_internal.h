@@ -21,6 +21,7 @@ constexpr int kMaxPartWorkgroups = 512;
 constexpr int kSections = 3;     // sections of a long dense launch
 constexpr int kQueueSlots = 64;  // ints set aside for their positions, in front of the arrival counters
 constexpr int kGemmQueueStride = kQueueSlots / kQueues;  // ints between the queue positions of the fused q/k/v projection, which runs before the attention call and keeps them there
+constexpr int kNormFirst = 4;   // floats in front of a head's key norms (one of them used, the others keep the norms aligned)
 constexpr int kOwnMaskKeys = 4096;  // key masks of at most this many keys are compacted by the K/V pass itself
 constexpr int kShortMaxTiles = 16;  // dense calls with at most this many key tiles never run the long-key kernel by themselves
 
@@ -58,7 +59,7 @@ struct QkPrologueParams {
   int fp8_pow2;             // fp8: block scales rounded up to a power of two
   unsigned* clear;          // words the pass sets to zero besides (queue positions and arrival counters of the attention launch after it)
   int clear_n;              // at most 256 for every workgroup of the pass
-  float* norm_out;          // [B*H][norm_stride]: largest row norm (after norm and rotation) of every 32 rows written
+  float* norm_out;          // [B*H][norm_stride]: from kNormFirst on the largest row norm (after norm and rotation) of every 32 rows written
   int norm_stride;
 };
 
@@ -95,7 +96,8 @@ struct FwdParams {
   const int* plan_cnt;      // [nQ64/kSparseRows][kSparseLists] entries per list
   int plan_stride;          // ints between consecutive workgroups' lists (kSparseLists * nKt)
   const float* kscale;      // [B*H, nKt] fp8 dequantisation scales of the K tiles
-  const float* knorm;       // [B*H][knorm_stride] largest K' row norm of every 32 keys (written for every tile that holds one)
+  const float* knorm;       // [B*H][knorm_stride] the head's largest K' row norm where a launch has taken it (else -1), then, from kNormFirst
+                            // on, that of every 32 keys (written for every tile that holds one)
   int knorm_stride;         // a multiple of 4
   int fp8;
   int fp8_pow2;         // fp8: the block scales are powers of two and ride in the scaled MFMA's operands
@@ -147,7 +149,7 @@ struct GemmTarget {
   int rope_mode;
   const float* cos_t;
   const float* sin_t;
-  float* norm_out;         // [heads][norm_stride] largest row norm of every 32 tokens
+  float* norm_out;         // [heads][norm_stride] from kNormFirst on the largest row norm of every 32 tokens
   int norm_stride;
   int fp8;
   int fp8_pow2;            // fp8: block scales rounded up to a power of two
@@ -195,6 +197,7 @@ hipError_t launch_pack_rows(const PackParams& p, hipStream_t st);
 hipError_t launch_fill_zero(unsigned* p, int n, hipStream_t st);
 
 hipError_t launch_mask_compact(const uint8_t* mask, int B, int Sk, int* idx, int* cnt, hipStream_t st);
+hipError_t launch_fold_norms(const QkPrologueParams& k, hipStream_t st);   // the largest norm of every head, for prepared keys
 hipError_t launch_kv_prologue(const QkPrologueParams& k, const VPrologueParams& v, hipStream_t st);
 hipError_t launch_attn_fwd(const FwdParams& p, hipStream_t st);
 enum AttnForm { kFormLong = 0, kFormShort = 1, kFormNarrow = 2, kFormSparse = 3 };

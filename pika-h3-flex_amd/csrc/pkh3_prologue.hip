@@ -137,7 +137,9 @@ __device__ __forceinline__ void k_tile(const QkPrologueParams& p, int tile, int 
   __syncthreads();
   if ((int)threadIdx.x < n_heads) {
     const float top = sqrtf(__uint_as_float(s_norm[threadIdx.x]));
-    *(f32x2*)(p.norm_out + (int64_t)(b * p.H + h0 + threadIdx.x) * p.norm_stride + 2 * tile) = f32x2{top, top};
+    float* row = p.norm_out + (int64_t)(b * p.H + h0 + threadIdx.x) * p.norm_stride;
+    *(f32x2*)(row + kNormFirst + 2 * tile) = f32x2{top, top};
+    if (tile == 0) row[0] = -1.0f;
   }
 }
 
@@ -273,6 +275,23 @@ hipError_t launch_kv_prologue(const QkPrologueParams& k, const VPrologueParams& 
   const dim3 grid((unsigned)(2 * groups) * k.nBlk64, k.B), block(256);
   if (k.fp8) hipLaunchKernelGGL(kv_prologue_kernel<true>, grid, block, 0, st, k, v, n, groups);
   else hipLaunchKernelGGL(kv_prologue_kernel<false>, grid, block, 0, st, k, v, n, groups);
+  return hipGetLastError();
+}
+
+// The largest norm of every head in front of its norms, for keys that many calls will use: their workgroups then read one word
+// each (24 heads x 16,366 queries against 512 prepared keys 103.2 -> 102.0 us).
+__global__ __launch_bounds__(64) void fold_norms_kernel(QkPrologueParams p) {
+  const int bh = blockIdx.x, lane = threadIdx.x;
+  const int n = ((p.row_cnt ? p.row_cnt[bh / p.H] : p.S) + 31) / 32;
+  float* row = p.norm_out + (int64_t)bh * p.norm_stride;
+  float top = 0.f;
+  for (int i = lane; i < n; i += 64) top = fmaxf(top, row[kNormFirst + i]);
+  top = wave_max(top);
+  if (lane == 0) row[0] = top;
+}
+
+hipError_t launch_fold_norms(const QkPrologueParams& k, hipStream_t st) {
+  hipLaunchKernelGGL(fold_norms_kernel, dim3((unsigned)(k.B * k.H)), dim3(64), 0, st, k);
   return hipGetLastError();
 }
 
