@@ -254,8 +254,9 @@ def test_one_key_of_a_large_norm_wherever_it_lies(H, Sq, Sk, at, sparse, long_ke
     opts = {"long_key_kernel": long_key, "fp8_qk": fp8}
     if sparse:
         opts["block_mask"] = pk.BlockMask.from_dense(torch.ones((-(-Sq // 64), -(-Sk // 64)), dtype=torch.bool), device="cuda")
-    out = pk.attention(q, k, v, **opts)
-    assert torch.equal(out, v[:, at:at + 1].expand_as(out))   # the other weights are below 2^-200 of this one
+    kv = pk.prepare_kv(k, v, fp8_qk=opts.pop("fp8_qk"), block_sparse=sparse, q_rows=Sq)
+    for out in (pk.attention(q, k, v, fp8_qk=fp8, **opts), pk.attention_prepared(q, kv, **opts)):
+        assert torch.equal(out, v[:, at:at + 1].expand_as(out))   # the other weights are below 2^-200 of this one
 
 
 @pytest.mark.parametrize("fp8", [False, True, "pow2"])
