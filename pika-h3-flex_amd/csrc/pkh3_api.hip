@@ -203,24 +203,26 @@ int hip_fail(hipError_t e, const char* what) {
 }
 
 // The K/V side of a call: key-mask compaction, then V and K into the workspace in the attention kernel's layout.
-int run_kv_side(const pkh3_attn_args* a, const Launch& L, hipStream_t st) {
+int run_kv_side(const pkh3_attn_args* a, const Launch& L, const SparsePlanParams& sparse, hipStream_t st) {
   hipError_t e;
   if (a->key_mask && !L.kp.mask && (e = launch_mask_compact(a->key_mask, a->B, a->Sk, L.idx, L.cnt, st)) != hipSuccess) return hip_fail(e, "mask_compact");
-  if ((e = launch_kv_prologue(L.kp, L.vp, st)) != hipSuccess) return hip_fail(e, "k/v pass");
+  if ((e = launch_kv_prologue(L.kp, L.vp, sparse, st)) != hipSuccess) return hip_fail(e, "k/v pass");
   return PKH3_OK;
 }
 
 int run_prologue(const pkh3_attn_args* a, const Launch& L, hipStream_t st) {
-  hipError_t e;
+  SparsePlanParams sparse{};
   if (a->blk_row_ptr) {
-    char* ws = L.ws;
-    if ((e = launch_sparse_plan(a->blk_row_ptr, a->blk_col_idx, (a->Sq + 63) / 64, L.w.nQ64, L.w.nKt, (int*)(ws + L.w.plan_off),
-                                kSparseLists * L.w.nKt, (int*)(ws + L.w.plan_cnt_off), st)) != hipSuccess)
-      return hip_fail(e, "sparse plan");
+    sparse = SparsePlanParams{a->blk_row_ptr, a->blk_col_idx, (a->Sq + 63) / 64, L.w.nKt, L.w.nQ64 / kSparseRows, (int*)(L.ws + L.w.plan_off),
+                              kSparseLists * L.w.nKt, (int*)(L.ws + L.w.plan_cnt_off)};
+    if (a->flags & PKH3_FLAG_KV_PREPARED) {
+      hipError_t e = launch_sparse_plan(sparse, st);
+      if (e != hipSuccess) return hip_fail(e, "sparse plan");
+    }
   }
   // prepared: pkh3_qkv_proj or pkh3_kv_prepare wrote K, V, the scales, the row-norm maxima and the compacted key list
   if (a->flags & PKH3_FLAG_KV_PREPARED) return PKH3_OK;
-  return run_kv_side(a, L, st);
+  return run_kv_side(a, L, sparse, st);
 }
 
 // ---- helpers of the projection entry points
@@ -379,7 +381,7 @@ int pkh3_kv_prepare(const pkh3_attn_args* a, void* stream) {
   build(a, a->workspace, L);
   if (a->workspace_bytes < L.w.total)
     return fail(PKH3_EWORKSPACE, "workspace too small: %zu < %zu bytes", a->workspace_bytes, L.w.total);
-  if ((rc = run_kv_side(a, L, (hipStream_t)stream))) return rc;
+  if ((rc = run_kv_side(a, L, SparsePlanParams{}, (hipStream_t)stream))) return rc;
   hipError_t e = launch_fold_norms(L.kp, (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(e, "fold_norms");
   g_err[0] = 0;

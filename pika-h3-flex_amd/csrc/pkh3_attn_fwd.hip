@@ -1521,64 +1521,4 @@ hipError_t launch_attn_fwd(const FwdParams& p, hipStream_t st) {
   return launch_fp<false>(p, cus, st);
 }
 
-// ------------------------------------------------------------------------------------------------
-// Block-sparse plan.  For each workgroup (kSparseRows consecutive 64-query row-blocks) 1 + kSparseRows ascending
-// tile lists, each `nKt` ints apart: [0] the key tiles every one of its row-blocks keeps (walked by all its waves
-// together), [1+r] the tiles row-block r keeps that are not in [0] (walked by that row-block's wave pair).  One
-// workgroup per attention workgroup merges the CSR rows through an LDS mask array, key tiles in chunks.
-constexpr int kPlanChunk = 8192;
-
-__global__ __launch_bounds__(256) void sparse_plan_kernel(const int* __restrict__ row_ptr, const int* __restrict__ col_idx,
-                                                          int nRow64, int nKt, int* __restrict__ plan, int plan_stride,
-                                                          int* __restrict__ plan_cnt) {
-  __shared__ unsigned char mask[kPlanChunk];
-  __shared__ int wave_tot[4];
-  __shared__ int carry[kSparseLists];
-  const int qt = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  int* out = plan + (int64_t)qt * plan_stride;
-  const int rows_here = max(0, min(kSparseRows, nRow64 - qt * kSparseRows));
-  const int full = (1 << rows_here) - 1;
-  if (tid < kSparseLists) carry[tid] = 0;
-  for (int base = 0; base < nKt; base += kPlanChunk) {
-    for (int i = tid; i < kPlanChunk; i += 256) mask[i] = 0;
-    __syncthreads();
-    for (int r = 0; r < rows_here; ++r) {
-      const int row = qt * kSparseRows + r;
-      const int beg = row_ptr[row], end = row_ptr[row + 1];
-      for (int j = beg + tid; j < end; j += 256) {
-        const int col = col_idx[j] - base;
-        // within one r two threads touch the same byte only when the row repeats a column, and then both store the
-        // same value; columns outside [0, nKt) are ignored; a row whose end lies before its start is empty
-        if (col >= 0 && col < kPlanChunk && col + base < nKt) mask[col] |= (unsigned char)(1 << r);
-      }
-      __syncthreads();
-    }
-    for (int list = 0; list < kSparseLists; ++list) {
-      for (int c0 = 0; c0 < kPlanChunk && base + c0 < nKt; c0 += 256) {
-        const int col = c0 + tid;
-        const int mk = (base + col < nKt) ? mask[col] : 0;
-        const bool take = list == 0 ? (mk == full && full != 0) : (((mk >> (list - 1)) & 1) && mk != full);
-        const unsigned long long bal = __ballot(take);
-        const int before = __popcll(bal & ((1ull << lane) - 1ull));
-        if (lane == 0) wave_tot[wave] = __popcll(bal);
-        __syncthreads();
-        int off = carry[list];
-        for (int wv = 0; wv < wave; ++wv) off += wave_tot[wv];
-        if (take) out[list * nKt + off + before] = base + col;
-        __syncthreads();
-        if (tid == 0) carry[list] += wave_tot[0] + wave_tot[1] + wave_tot[2] + wave_tot[3];
-        __syncthreads();
-      }
-    }
-  }
-  if (tid < kSparseLists) plan_cnt[qt * kSparseLists + tid] = carry[tid];
-}
-
-hipError_t launch_sparse_plan(const int* row_ptr, const int* col_idx, int nRow64, int nQ64, int nKt, int* plan,
-                              int plan_stride, int* plan_cnt, hipStream_t st) {
-  hipLaunchKernelGGL(sparse_plan_kernel, dim3(nQ64 / kSparseRows), dim3(256), 0, st, row_ptr, col_idx, nRow64, nKt, plan, plan_stride,
-                     plan_cnt);
-  return hipGetLastError();
-}
-
 }  // namespace pkh3

@@ -63,6 +63,16 @@ struct QkPrologueParams {
   int norm_stride;
 };
 
+// Block-sparse map in CSR form -> the tile lists of `n` workgroups of the attention kernel
+struct SparsePlanParams {
+  const int* row_ptr;
+  const int* col_idx;
+  int nRow64, nKt, n;
+  int* plan;                // [n] entries of kSparseLists lists, nKt ints apart
+  int plan_stride;          // ints between entries
+  int* plan_cnt;            // [n][kSparseLists]
+};
+
 struct VPrologueParams {
   const void* v;
   int64_t sb, ss, sh;
@@ -198,13 +208,12 @@ hipError_t launch_fill_zero(unsigned* p, int n, hipStream_t st);
 
 hipError_t launch_mask_compact(const uint8_t* mask, int B, int Sk, int* idx, int* cnt, hipStream_t st);
 hipError_t launch_fold_norms(const QkPrologueParams& k, hipStream_t st);   // the largest norm of every head, for prepared keys
-hipError_t launch_kv_prologue(const QkPrologueParams& k, const VPrologueParams& v, hipStream_t st);
+hipError_t launch_kv_prologue(const QkPrologueParams& k, const VPrologueParams& v, const SparsePlanParams& plan, hipStream_t st);   // plan.n may be 0
 hipError_t launch_attn_fwd(const FwdParams& p, hipStream_t st);
 enum AttnForm { kFormLong = 0, kFormShort = 1, kFormNarrow = 2, kFormSparse = 3 };
 AttnForm attn_form(const FwdParams& p, int cus);  // the form launch_attn_fwd takes on a device of `cus` CUs
 hipError_t device_cu_count(int* out);  // CUs of the current device (cached per device after the first call)
-hipError_t launch_sparse_plan(const int* row_ptr, const int* col_idx, int nRow64, int nQ64, int nKt, int* plan,
-                              int plan_stride, int* plan_cnt, hipStream_t st);
+hipError_t launch_sparse_plan(const SparsePlanParams& p, hipStream_t st);
 hipError_t launch_rope_tables(const double* pos, int S, const int* axis_dims, double theta, float* cos_out,
                               float* sin_out, hipStream_t st);
 

@@ -581,6 +581,29 @@ def test_prepared_keys_serve_several_calls(variant):
         pk.attention_prepared(_rand((B, Sq, H + 1, D), gen).to(dev), kv, **q_opts)
 
 
+@pytest.mark.parametrize("B,H,Sq,Sk,fp8", [
+    (1, 1, 64, 64, False),       # one entry beside two workgroups of tiles
+    (3, 2, 257, 190, True),       # entries ride once, not once per batch; the last one holds one row-block of four
+    (2, 1, 4097, 130, True),      # more entries than tiles
+    (1, 1, 70, 64 * 8192 + 65, False),  # key tiles past one round of the masks
+])
+def test_tile_lists_made_beside_the_kv_pass(B, H, Sq, Sk, fp8):
+    """Direct calls make the tile lists in the K/V pass's launch, calls on prepared keys in a launch of their own: the same bits."""
+    import pika_h3_flex_amd as pk
+
+    gen = torch.Generator().manual_seed(Sq + Sk)
+    q, k, v = (_rand((B, n, H, 128), gen).cuda() for n in (Sq, Sk, Sk))
+    nq, nk = -(-Sq // 64), -(-Sk // 64)
+    tiles = torch.rand((nq, nk), generator=gen) < 0.4
+    tiles[:, 0] = tiles[:, -1] = True
+    bm = pk.BlockMask.from_dense(tiles, device="cuda")
+    opts = dict(fp8_qk=fp8)
+    kv = pk.prepare_kv(k, v, q_rows=Sq, block_sparse=True, **opts)
+    want = pk.attention_prepared(q, kv, block_mask=bm)
+    assert torch.isfinite(want.float()).all()
+    assert torch.equal(pk.attention(q, k, v, block_mask=bm, **opts), want)
+
+
 def test_prepared_keys_workspace_holds_dense_and_block_sparse_calls():
     """Keys prepared with ``block_sparse=True`` at a size where long dense calls bring scratch of their own (the partial
     results of a shared last round): the workspace must hold either kind of call, and both must give the bits of the
