@@ -10,6 +10,7 @@
 #include <string.h>
 
 #include "pkh3_common.h"
+#include "pkh3_index.h"
 #include "pkh3_internal.h"
 
 using namespace pkh3;
@@ -226,7 +227,6 @@ int run_prologue(const pkh3_attn_args* a, const Launch& L, hipStream_t st) {
 }
 
 // ---- helpers of the projection entry points
-size_t padded_rows(int32_t rows) { return ((size_t)rows + 255) / 256 * 256; }
 
 int check_pack(const char* what, const void* x, int64_t row_stride, int32_t rows, int32_t K, const void* out) {
   if (!x || !out) return fail(PKH3_ENULL, "%s: NULL pointer", what);
@@ -445,7 +445,7 @@ int pkh3_rope_tables(const double* position_ids, int32_t S, const int32_t axis_d
 
 size_t pkh3_packed_bytes(int32_t rows, int32_t K) {
   if (rows < 1 || K < 32 || (K % 32) || K > 4096) return 0;
-  return padded_rows(rows) * (size_t)K * 2;
+  return (size_t)padded_rows(rows) * (size_t)K * 2;
 }
 
 int pkh3_pack_weight(const void* w, int64_t row_stride, int32_t N, int32_t K, int32_t head_perm, void* out, void* stream) {

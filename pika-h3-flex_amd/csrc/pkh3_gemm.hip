@@ -30,6 +30,7 @@
 #include <type_traits>
 
 #include "pkh3_common.h"
+#include "pkh3_index.h"
 #include "pkh3_internal.h"
 
 namespace pkh3 {
@@ -407,13 +408,15 @@ __device__ __forceinline__ void epilogue_k(const GemmParams& p, const GemmTarget
   });
 }
 
-// operand images of these GEMMs: [16-token block][k-step], this lane's piece ks at its own place in image ks
+// operand images of these GEMMs: [16-token block][k-step], this lane's piece ks at its own place in image ks; the tile's blocks past
+// the last token are zeros, where the buffer has them
 template <int TB>
 __device__ __forceinline__ void epilogue_a(const GemmParams& p, const GemmTarget& tg, int head, int tok0, const f32x4 (&acc)[TB][8]) {
   const int lane = threadIdx.x & 63, c = lane & 15;
   static_for<TB>([&](auto tc) {
     constexpr int t = decltype(tc)::value;
     const int blk = tok0 + 16 * t;
+    if (TB == 6 && !in_image_buffer(blk, p.M)) return;   // (wave-uniform)
     float x[32];
     acc_block<(TB > 4)>(x, acc[t]);
     const bool valid = blk + c < p.M;                  // rows past the end are zeros, whatever their activations held

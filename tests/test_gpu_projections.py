@@ -353,6 +353,59 @@ def test_down_projected_rows_past_the_end_are_zero(S):
     assert torch.count_nonzero(tail) == 0 and torch.isfinite(tail.float()).all()
 
 
+@pytest.mark.parametrize("S,adapters", [(16640, "shared"), (16449, "shared"), (11008, "separate"), (33280, "out")])
+def test_down_projections_of_192_token_tiles_stay_in_their_workspace(S, adapters):
+    """Calls whose down-projections take tiles of 192 tokens on 256 CUs, the last one past the padded rows of the workspace (but for
+    16,449 rows): what lies behind it is left alone, and the adapters' results are right to the last row."""
+    import ctypes as C
+
+    from pika_h3_flex_amd import _lib, ops
+    from pika_h3_flex_amd import projections as P
+
+    K, n = 64, 1 if adapters == "out" else 3
+    lins = [dict(_linear(128, K, 12 + 10 * i, bias=False), lora_scale=0.5) for i in range(n)]
+    for d in lins:
+        d["weight"] = torch.zeros_like(d["weight"])                            # the adapters alone
+    packed = [_packed(d, head_perm=i < 2) for i, d in enumerate(lins)]
+    assert adapters != "shared" or P.PackedLinear.share_adapter_buffer(*packed)
+    x = _r(S, K, seed=11).to(torch.bfloat16).cuda()
+    img = P.pack_rows(x)
+    need, guard = P.packed_bytes(S, 128 * n), 256 * 1024
+    around = torch.full((need + 2 * guard,), 0xA5, dtype=torch.uint8, device="cuda")
+    lws = around[guard:guard + need]
+    y = torch.empty((1, S, 1, D), dtype=torch.bfloat16, device="cuda")
+    stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    if n == 1:
+        a = _lib.OutArgs()
+        a.o_img, a.S, a.K, a.N = img.data_ptr(), S, K, 128
+        a.proj = packed[0].c_struct()
+        a.y, a.y_stride = y.data_ptr(), 128
+        a.lora_workspace, a.lora_workspace_bytes = lws.data_ptr(), need
+        _lib.check(_lib.load().pkh3_out_proj(C.byref(a), stream))
+    else:
+        args, keep = ops.fill_args(y, None, None, torch.empty_like(y), kv_prepared=True)
+        ws = torch.empty(ops.workspace_bytes(args), dtype=torch.uint8, device="cuda")
+        args.workspace, args.workspace_bytes = ws.data_ptr(), ws.numel()
+        a = _lib.QkvArgs()
+        a.x_img, a.S, a.K = img.data_ptr(), S, K
+        a.q, a.k, a.v = (p.c_struct() for p in packed)
+        a.lora_workspace, a.lora_workspace_bytes = lws.data_ptr(), need
+        _lib.check(_lib.load().pkh3_qkv_proj(C.byref(a), C.byref(args), stream))
+    torch.cuda.synchronize()
+    assert bool((around[:guard] == 0xA5).all()) and bool((around[guard + need:] == 0xA5).all())
+    rows = _unpack(lws, (S + 15) // 16 * 16, 128 * n).view(-1, n, 128)
+    assert torch.count_nonzero(rows[S:]) == 0
+    for i, d in enumerate(lins):
+        xa = d["lora_scale"] * (x.float() @ d["lora_a"].cuda().float().t())
+        # one rounding to bf16 (at most 2^-8 of the value) of a sum of 64 products in float32
+        assert bool(((rows[:S, i].float() - xa).abs() <= xa.abs() / 256 + 1e-5).all())
+    b = lins[0]["lora_b"].cuda().float()
+    xa = lins[0]["lora_scale"] * (x.float() @ lins[0]["lora_a"].cuda().float().t())
+    # (as in test_forms_of_the_down_projection)
+    bound = (xa @ b.t()).abs() / 256 + 6.0 / 256 * ((xa * xa) @ (b * b).t()).sqrt()
+    assert bool(((y.view(S, 128).float() - xa @ b.t()).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("S,H", [(300, 2), (1000, 3), (257, 1)])
 def test_adapters_in_one_buffer_give_the_same_bits(S, H):
     """``PackedLinear.share_adapter_buffer`` lays the three down-projection images one behind the other, and
