@@ -35,3 +35,21 @@ def test_down_projected_images_stay_in_their_buffer(tmp_path):
             CHECK(row + 16 <= padded_rows(rows), "%d rows, %d a tile: block at %d", rows, 32 * blocks, row);
         }
       }""")
+
+
+def test_words_cleared_by_the_kv_pass_are_those_of_the_list(tmp_path):
+    """Grids from the smallest that clears the longest list (6,208 words) to those of the largest calls that are accepted: the first
+    workgroups clear every word once, no index is negative and none comes twice."""
+    _run(tmp_path, """
+  struct { unsigned batches, groups; } grids[] = {{1, 34}, {17, 2}, {65535, 130}, {16, 524288}, {17, 524288}, {65535, 524288}};
+  for (auto g : grids) {
+    const int64_t all = (int64_t)g.batches * g.groups;
+    for (int64_t word = 0; word < 6208; ++word) {
+      const int64_t wg = word / 256;
+      CHECK(word_to_clear(wg / g.groups, g.groups, wg % g.groups, word % 256) == word, "word %lld", (long long)word);
+    }
+    for (int64_t wg = all > 70000 ? all - 70000 : 25; wg < all; ++wg)
+      CHECK(word_to_clear(wg / g.groups, g.groups, wg % g.groups, 0) == wg * 256, "workgroup %lld of %lld", (long long)wg, (long long)all);
+    for (int64_t wg = 25; wg < all; wg += all / 1000 + 1)
+      CHECK(word_to_clear(wg / g.groups, g.groups, wg % g.groups, 0) >= 6208, "workgroup %lld of %lld", (long long)wg, (long long)all);
+  }""")
