@@ -156,7 +156,7 @@ void build(const pkh3_attn_args* a, void* workspace, Launch& L, bool part_scratc
   k.B = a->B; k.H = a->H; k.S = a->Sk; k.nBlk64 = L.w.nKt;
   k.norm_w = a->k_norm_w; k.eps = a->norm_eps; k.rope_mode = a->rope_mode;
   k.cos_t = a->k_rope_cos; k.sin_t = a->k_rope_sin;
-  k.mask = a->Sk <= kOwnMaskKeys ? a->key_mask : nullptr; k.gather_idx = L.idx; k.row_cnt = L.cnt;
+  k.mask = a->key_mask; k.gather_idx = L.idx; k.row_cnt = L.cnt;
   k.out = ws + L.w.kv_off; k.out_bh_stride = (int64_t)L.w.nKt * L.w.kvTileBytes; k.out_blk_stride = L.w.kvTileBytes;
   k.scale_out = fp8 ? (float*)(ws + L.w.kscale_off) : nullptr; k.fp8 = fp8;
   k.fp8_pow2 = (a->flags & PKH3_FLAG_FP8_POW2_SCALES) ? 1 : 0;
@@ -204,11 +204,9 @@ int hip_fail(hipError_t e, const char* what) {
 }
 
 // The K/V side of a call: key-mask compaction, then V and K into the workspace in the attention kernel's layout.
-int run_kv_side(const pkh3_attn_args* a, const Launch& L, const SparsePlanParams& sparse, hipStream_t st) {
-  hipError_t e;
-  if (a->key_mask && !L.kp.mask && (e = launch_mask_compact(a->key_mask, a->B, a->Sk, L.idx, L.cnt, st)) != hipSuccess) return hip_fail(e, "mask_compact");
-  if ((e = launch_kv_prologue(L.kp, L.vp, sparse, st)) != hipSuccess) return hip_fail(e, "k/v pass");
-  return PKH3_OK;
+int run_kv_side(const Launch& L, const SparsePlanParams& sparse, hipStream_t st) {
+  const hipError_t e = launch_kv_prologue(L.kp, L.vp, sparse, st);
+  return e == hipSuccess ? PKH3_OK : hip_fail(e, "k/v pass");
 }
 
 int run_prologue(const pkh3_attn_args* a, const Launch& L, hipStream_t st) {
@@ -223,7 +221,7 @@ int run_prologue(const pkh3_attn_args* a, const Launch& L, hipStream_t st) {
   }
   // prepared: pkh3_qkv_proj or pkh3_kv_prepare wrote K, V, the scales, the row-norm maxima and the compacted key list
   if (a->flags & PKH3_FLAG_KV_PREPARED) return PKH3_OK;
-  return run_kv_side(a, L, sparse, st);
+  return run_kv_side(L, sparse, st);
 }
 
 // ---- helpers of the projection entry points
@@ -381,7 +379,7 @@ int pkh3_kv_prepare(const pkh3_attn_args* a, void* stream) {
   build(a, a->workspace, L);
   if (a->workspace_bytes < L.w.total)
     return fail(PKH3_EWORKSPACE, "workspace too small: %zu < %zu bytes", a->workspace_bytes, L.w.total);
-  if ((rc = run_kv_side(a, L, SparsePlanParams{}, (hipStream_t)stream))) return rc;
+  if ((rc = run_kv_side(L, SparsePlanParams{}, (hipStream_t)stream))) return rc;
   hipError_t e = launch_fold_norms(L.kp, (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(e, "fold_norms");
   g_err[0] = 0;

@@ -22,7 +22,6 @@ constexpr int kSections = 3;     // sections of a long dense launch
 constexpr int kQueueSlots = 64;  // ints set aside for their positions, in front of the arrival counters
 constexpr int kGemmQueueStride = kQueueSlots / kQueues;  // ints between the queue positions of the fused q/k/v projection, which runs before the attention call and keeps them there
 constexpr int kNormFirst = 4;   // floats in front of a head's key norms (one of them used, the others keep the norms aligned)
-constexpr int kOwnMaskKeys = 4096;  // key masks of at most this many keys are compacted by the K/V pass itself
 constexpr int kShortMaxTiles = 16;  // dense calls with at most this many key tiles never run the long-key kernel by themselves
 
 // Where each intermediate lives inside the caller's workspace (byte offsets, 256-aligned).
@@ -48,8 +47,8 @@ struct QkPrologueParams {
   int rope_mode;
   const float* cos_t;       // [S, D/2] or null
   const float* sin_t;
-  const uint8_t* mask;      // [B, S] key mask that the pass compacts itself, writing row_cnt, or null
-  const int* gather_idx;    // [B, S] compacted row -> source row, or null (read where `mask` is null)
+  const uint8_t* mask;      // [B, S] key mask, or null; the kernel gets it where it compacts the mask itself, writing row_cnt
+  int* gather_idx;          // [B, S] compacted row -> source row, or null (used where the kernel gets no mask)
   int* row_cnt;             // [B] rows that exist after compaction, or null (= S)
   char* out;                // images
   int64_t out_bh_stride;    // bytes between consecutive (b,h)
@@ -206,9 +205,8 @@ hipError_t launch_gemm(const GemmParams& p, hipStream_t st);
 hipError_t launch_pack_rows(const PackParams& p, hipStream_t st);
 hipError_t launch_fill_zero(unsigned* p, int n, hipStream_t st);
 
-hipError_t launch_mask_compact(const uint8_t* mask, int B, int Sk, int* idx, int* cnt, hipStream_t st);
 hipError_t launch_fold_norms(const QkPrologueParams& k, hipStream_t st);   // the largest norm of every head, for prepared keys
-hipError_t launch_kv_prologue(const QkPrologueParams& k, const VPrologueParams& v, const SparsePlanParams& plan, hipStream_t st);   // plan.n may be 0
+hipError_t launch_kv_prologue(QkPrologueParams k, const VPrologueParams& v, const SparsePlanParams& plan, hipStream_t st);   // plan.n may be 0
 hipError_t launch_attn_fwd(const FwdParams& p, hipStream_t st);
 enum AttnForm { kFormLong = 0, kFormShort = 1, kFormNarrow = 2, kFormSparse = 3 };
 AttnForm attn_form(const FwdParams& p, int cus);  // the form launch_attn_fwd takes on a device of `cus` CUs

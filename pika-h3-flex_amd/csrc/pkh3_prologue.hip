@@ -13,7 +13,7 @@
 namespace pkh3 {
 
 // ------------------------------------------------------------------------------------------------
-// Key-mask compaction of many keys (the K/V pass does it itself for up to kOwnMaskKeys): idx[b][slot] = key index of the slot-th valid key, cnt[b] = number of valid keys.
+// Key-mask compaction in front of the K/V pass, where the pass does not do it itself (kv_pass_reads_mask): idx[b][slot] = key index of the slot-th valid key, cnt[b] = number of valid keys.
 // One workgroup of 1024 threads per batch walks the mask in chunks, carrying the running count.
 __global__ __launch_bounds__(1024) void mask_compact_kernel(const uint8_t* __restrict__ mask, int Sk,
                                                             int* __restrict__ idx, int* __restrict__ cnt) {
@@ -46,7 +46,7 @@ __global__ __launch_bounds__(1024) void mask_compact_kernel(const uint8_t* __res
   if (tid == 0) cnt[b] = carry;
 }
 
-hipError_t launch_mask_compact(const uint8_t* mask, int B, int Sk, int* idx, int* cnt, hipStream_t st) {
+static hipError_t launch_mask_compact(const uint8_t* mask, int B, int Sk, int* idx, int* cnt, hipStream_t st) {
   hipLaunchKernelGGL(mask_compact_kernel, dim3(B), dim3(1024), 0, st, mask, Sk, idx, cnt);
   return hipGetLastError();
 }
@@ -62,7 +62,6 @@ hipError_t launch_mask_compact(const uint8_t* mask, int B, int Sk, int* idx, int
 // their way while it works on one; 16 rows per wave (a quarter of a tile) leaves the registers for three waves per SIMD.
 // Against a K and a V launch of one wave per tile and head: 48,360 rows x 24 heads 293 -> 241 us (4.9 TB/s), fp8 285 -> 215;
 // 15,342 rows 127 -> 85 us.
-constexpr int kKvMaxHeads = 8;  // heads a workgroup walks at most
 
 // K: lane (c = l%16, g = l/16) of wave kb holds the 32 elements d = 32*ks + 8*g + j of row 16*kb + c -- its own 16 bytes
 // of the block's four K images, so every load instruction reads 64 contiguous bytes of 16 rows, norm and rotation need
@@ -266,26 +265,22 @@ __global__ __launch_bounds__(256, 3) void kv_prologue_kernel(QkPrologueParams k,
   k_tile<FP8>(k, tile, b, h0, n, rows, src, s_norm, s_amax);
 }
 
-hipError_t launch_kv_prologue(const QkPrologueParams& k, const VPrologueParams& v, const SparsePlanParams& plan, hipStream_t st) {
+hipError_t launch_kv_prologue(QkPrologueParams k, const VPrologueParams& v, const SparsePlanParams& plan, hipStream_t st) {
   int cus = 0;
   hipError_t e = device_cu_count(&cus);
   if (e != hipSuccess) return e;
-  // Heads a workgroup walks: more of them share one read of the tables, as long as two or three workgroups of each side are
-  // left per CU.  15,342 rows x 24 heads with rotation: 1 head 113 us, 2 91, 4 87, 8 85, 12 87; fp8 117, 90, 82, 76, 84.
-  // Three from where single heads make more workgroups than run at once (1, 2, 3 and 4 heads, us, 24 heads with rotation:
-  // 1,000 rows 9.8, 10.1, 9.2, 10.4; 1,500 13.7, 12.5, 12.2, 13.9; 3,000 24.8, 20.8, 20.1, 22.8, fp8 25.0, 22.0, 20.4, 22.9; without rotation
-  // 1,000 rows 7.1, 7.9, 7.8, 8.9; 1,500 9.8, 9.8, 9.6, 10.9; 3,000 18.6, 17.3, 17.0, 19.2).
-  const int64_t single = (int64_t)k.nBlk64 * k.B * k.H, per_cu = max(cus, 1);
-  const int64_t per_side = max(single * 2 / (5 * per_cu), single * 4 >= 9 * per_cu ? (int64_t)3 : (int64_t)1);
-  const int most = (int)min(per_side, (int64_t)min(kKvMaxHeads, k.H));
-  int groups = (k.H + most - 1) / most;
-  const int n = (k.H + groups - 1) / groups;   // equal shares
-  groups = (k.H + n - 1) / n;
+  cus = max(cus, 1);
+  const KvSplit split = kv_split(k.nBlk64, k.B, k.H, cus);
+  const int64_t workgroups = (int64_t)2 * split.groups * k.nBlk64 * k.B;
+  if (k.mask && !kv_pass_reads_mask(k.S, workgroups, cus)) {
+    if ((e = launch_mask_compact(k.mask, k.B, k.S, k.gather_idx, k.row_cnt, st)) != hipSuccess) return e;
+    k.mask = nullptr;
+  }
   // The entries of a block-sparse plan ride in front: each is a chain of short steps, so they end under the tiles' loads.  A launch
   // of their own costs a call 3 us (4,109 tokens, 24 heads, fp8, 10 % of the tiles: 683.9 -> 680.4 us; 37,877 in bf16: 6,876 -> 6,873).
-  const dim3 grid((unsigned)(2 * groups) * k.nBlk64 + plan.n, k.B), block(256);
-  if (k.fp8) hipLaunchKernelGGL(kv_prologue_kernel<true>, grid, block, 0, st, k, v, plan, n, groups);
-  else hipLaunchKernelGGL(kv_prologue_kernel<false>, grid, block, 0, st, k, v, plan, n, groups);
+  const dim3 grid((unsigned)(2 * split.groups) * k.nBlk64 + plan.n, k.B), block(256);
+  if (k.fp8) hipLaunchKernelGGL(kv_prologue_kernel<true>, grid, block, 0, st, k, v, plan, split.heads, split.groups);
+  else hipLaunchKernelGGL(kv_prologue_kernel<false>, grid, block, 0, st, k, v, plan, split.heads, split.groups);
   return hipGetLastError();
 }
 

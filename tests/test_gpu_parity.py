@@ -375,6 +375,23 @@ def test_key_masks_compacted_by_the_kv_pass_and_before_it(Sk, dtype):
     assert (other.float() - got.float()).abs().max() <= 2 ** -7 * got.float().abs().max()   # sums in another order, rounded to bf16
 
 
+@pytest.mark.parametrize("B,H,Sk", [(15, 4, 1000), (16, 4, 1000), (40, 3, 700), (17, 8, 4096)])   # the K/V pass reads the mask in the first only
+def test_key_masks_of_many_entries(B, H, Sk):
+    """One launch makes the lists of valid keys where the K/V pass has too many workgroups to look for them itself: every entry has the
+    bits of a call of its own."""
+    import pika_h3_flex_amd as pk
+
+    gen = torch.Generator().manual_seed(B)
+    q, k, v = (_rand((B, n, H, 128), gen).cuda() for n in (33, Sk, Sk))
+    keep = (torch.rand((B, Sk), generator=gen) < torch.linspace(0.0, 1.0, B)[:, None]).cuda()   # from no key to all of them
+    k[~keep], v[~keep] = float("nan"), float("inf")
+    got = pk.attention(q, k, v, key_mask=keep, long_key_kernel=True)
+    assert torch.equal(got, pk.attention_prepared(q, pk.prepare_kv(k, v, key_mask=keep, q_rows=33), long_key_kernel=True))
+    for b in range(B):
+        own = pk.attention(*(x[b:b + 1] for x in (q, k, v)), key_mask=keep[b:b + 1], long_key_kernel=True)
+        assert torch.equal(got[b:b + 1], own) and torch.isfinite(own.float()).all()
+
+
 def test_key_mask_all_valid_equals_no_mask():
     import pika_h3_flex_amd as pk
 

@@ -53,3 +53,17 @@ def test_words_cleared_by_the_kv_pass_are_those_of_the_list(tmp_path):
     for (int64_t wg = 25; wg < all; wg += all / 1000 + 1)
       CHECK(word_to_clear(wg / g.groups, g.groups, wg % g.groups, 0) >= 6208, "workgroup %lld of %lld", (long long)wg, (long long)all);
   }""")
+
+
+def test_who_reads_the_key_mask(tmp_path):
+    """The K/V pass where its workgroups run at once (measured on 256 CUs), a launch in front of it for more of them or more keys."""
+    _run(tmp_path, """
+  struct { int keys, heads, entries; bool pass; } calls[] = {
+      {512, 24, 1, true}, {777, 8, 3, true}, {512, 24, 4, true}, {4096, 8, 2, true}, {4096, 1, 7, true},
+      {4097, 1, 1, false}, {4096, 1, 8, false}, {4096, 8, 4, false}, {1000, 4, 16, false}, {4096, 24, 16, false}, {300, 24, 64, false}};
+  for (auto c : calls) {
+    const int tiles = (c.keys + 63) / 64;
+    const KvSplit split = kv_split(tiles, c.entries, c.heads, 256);
+    CHECK(split.groups * split.heads >= c.heads && (split.groups - 1) * split.heads < c.heads, "%d heads", c.heads);
+    CHECK(kv_pass_reads_mask(c.keys, (int64_t)2 * split.groups * tiles * c.entries, 256) == c.pass, "%d keys, %d x %d", c.keys, c.entries, c.heads);
+  }""")
