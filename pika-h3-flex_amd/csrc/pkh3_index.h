@@ -24,21 +24,36 @@ constexpr int kOwnMaskKeys = 4096;    // keys whose mask a workgroup of the K/V 
 struct KvSplit {
   int heads, groups;
 };
+constexpr KvSplit kv_equal_split(int heads, int most) {
+  const int groups = (heads + most - 1) / most, n = (heads + groups - 1) / groups;
+  return KvSplit{n, (heads + n - 1) / n};
+}
 // More heads a workgroup share one read of the tables, as long as two or three workgroups of each side are left per CU.  15,342
 // rows x 24 heads with rotation: 1 head 113 us, 2 91, 4 87, 8 85, 12 87; fp8 117, 90, 82, 76, 84.
-// Three from where single heads make more workgroups than run at once (1, 2, 3 and 4 heads, us, 24 heads with rotation:
-// 1,000 rows 9.8, 10.1, 9.2, 10.4; 1,500 13.7, 12.5, 12.2, 13.9; 3,000 24.8, 20.8, 20.1, 22.8, fp8 25.0, 22.0, 20.4, 22.9; without rotation
-// 1,000 rows 7.1, 7.9, 7.8, 8.9; 1,500 9.8, 9.8, 9.6, 10.9; 3,000 18.6, 17.3, 17.0, 19.2).
-constexpr KvSplit kv_split(int tiles, int batches, int heads, int cus) {
+// In between (2.5 to about 7 workgroups of single heads a side on a CU) it is the rounds that count: three workgroups of both sides
+// run on a CU at once, and the fewest heads with which all of them do is best, if the heads in a row take no longer than the rounds
+// they replace (a workgroup of n heads n + 1/2).  With rotation, whose tables are then read less often, already from 2.25 on and with
+// up to five heads, else four; with a key mask three, as there are fewer tiles than the call says.
+// This rule / three heads throughout / the rule above alone, us: 10 heads x 9,000 rows, fp8 27.3 / 30.9 / 27.3; 16 x 5,600, fp8 25.9 /
+// 29.7 / 26.9; 24 x 3,000 20.1 / 20.1 / 24.8; 28 x 1,640 without rotation 12.8 / 14.7 / 13.8; 32 x 1,200 15.6 / 14.7 / 16.6; 4 heads x 16,384
+// 19.6 / 21.6 / 25.9.  Of 504 such calls (4 to 48 heads) none that it sends another way is more than 0.5 % behind the rule above; of 137
+// masked ones those with 10, 30, 60 and 95 % of the keys valid are 1, 2, 4 and 7 % ahead of it on average (at 10 and 30 % one in twelve
+// 3 to 25 % behind).
+constexpr KvSplit kv_split(int tiles, int batches, int heads, int cus, bool rotation, bool masked) {
   const int64_t single = (int64_t)tiles * batches * heads;
   int64_t most = single * 2 / (5 * (int64_t)cus);
-  if (most < 3 && single * 4 >= 9 * (int64_t)cus) most = 3;
   if (most > kKvMaxHeads) most = kKvMaxHeads;
   if (most > heads) most = heads;
   if (most < 1) most = 1;
-  const int groups = (heads + (int)most - 1) / (int)most;
-  const int n = (heads + groups - 1) / groups;   // equal shares
-  return KvSplit{n, (heads + n - 1) / n};
+  const KvSplit base = kv_equal_split(heads, (int)most);
+  if (single * 4 < (rotation ? 9 : 10) * (int64_t)cus) return base;
+  const int64_t side = (int64_t)tiles * batches, at_once = 3 * (int64_t)cus;
+  const int64_t rounds = (2 * base.groups * side + at_once - 1) / at_once;
+  for (int n = (int)most; n <= (masked ? 3 : rotation ? 5 : 4) && n <= heads; ++n) {
+    const KvSplit s = kv_equal_split(heads, n);
+    if (2 * s.groups * side <= at_once) return 2 * s.heads + 1 <= rounds * (2 * base.heads + 1) ? s : base;
+  }
+  return base;
 }
 
 // Whether the workgroups of the K/V pass look through the key mask themselves, each of them through all of it, or a launch of one

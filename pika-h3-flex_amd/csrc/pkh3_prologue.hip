@@ -270,7 +270,7 @@ hipError_t launch_kv_prologue(QkPrologueParams k, const VPrologueParams& v, cons
   hipError_t e = device_cu_count(&cus);
   if (e != hipSuccess) return e;
   cus = max(cus, 1);
-  const KvSplit split = kv_split(k.nBlk64, k.B, k.H, cus);
+  const KvSplit split = kv_split(k.nBlk64, k.B, k.H, cus, k.rope_mode != 0, k.mask != nullptr);
   const int64_t workgroups = (int64_t)2 * split.groups * k.nBlk64 * k.B;
   if (k.mask && !kv_pass_reads_mask(k.S, workgroups, cus)) {
     if ((e = launch_mask_compact(k.mask, k.B, k.S, k.gather_idx, k.row_cnt, st)) != hipSuccess) return e;

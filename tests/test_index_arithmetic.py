@@ -63,7 +63,26 @@ def test_who_reads_the_key_mask(tmp_path):
       {4097, 1, 1, false}, {4096, 1, 8, false}, {4096, 8, 4, false}, {1000, 4, 16, false}, {4096, 24, 16, false}, {300, 24, 64, false}};
   for (auto c : calls) {
     const int tiles = (c.keys + 63) / 64;
-    const KvSplit split = kv_split(tiles, c.entries, c.heads, 256);
+    const KvSplit split = kv_split(tiles, c.entries, c.heads, 256, false, true);
     CHECK(split.groups * split.heads >= c.heads && (split.groups - 1) * split.heads < c.heads, "%d heads", c.heads);
     CHECK(kv_pass_reads_mask(c.keys, (int64_t)2 * split.groups * tiles * c.entries, 256) == c.pass, "%d keys, %d x %d", c.keys, c.entries, c.heads);
   }""")
+
+
+def test_heads_a_workgroup_of_the_kv_pass(tmp_path):
+    """Calls that three heads a workgroup were slower for than the fewest with which all workgroups run at once, or than as many as fill
+    the CUs (measured on 256 CUs); every head is somebody's at any size."""
+    _run(tmp_path, """
+  struct { int tiles, heads; bool rotation; int want; bool masked; } calls[] = {
+      {141, 10, true, 2}, {167, 10, true, 5}, {88, 16, true, 4}, {72, 10, false, 2}, {45, 16, false, 2}, {26, 28, false, 2}, {144, 5, false, 1},
+      {50, 12, false, 1}, {47, 24, true, 3}, {47, 24, false, 3}, {16, 24, true, 1}, {240, 24, true, 8}, {8, 24, false, 1}, {256, 4, true, 4}, {256, 4, true, 1, true}, {47, 24, true, 3, true}};
+  for (auto c : calls) {
+    const KvSplit s = kv_split(c.tiles, 1, c.heads, 256, c.rotation, c.masked);
+    CHECK(s.heads == c.want, "%d tiles, %d heads: %d a workgroup", c.tiles, c.heads, s.heads);
+  }
+  for (int tiles = 1; tiles < 300; tiles += 7)
+    for (int heads = 1; heads <= 70; ++heads)
+      for (int rotation = 0; rotation < 2; ++rotation) {
+        const KvSplit s = kv_split(tiles, 1 + heads % 3, heads, 256, rotation, tiles % 2);
+        CHECK(s.heads >= 1 && s.heads <= kKvMaxHeads && s.groups * s.heads >= heads && (s.groups - 1) * s.heads < heads, "%d tiles, %d heads", tiles, heads);
+      }""")
