@@ -295,19 +295,31 @@ hipError_t launch_sparse_plan(const SparsePlanParams& p, hipStream_t st) {
 }
 
 // The largest norm of every head in front of its norms, for keys that many calls will use: their workgroups then read one word
-// each (24 heads x 16,366 queries against 512 prepared keys 103.2 -> 102.0 us).
-__global__ __launch_bounds__(64) void fold_norms_kernel(QkPrologueParams p) {
-  const int bh = blockIdx.x, lane = threadIdx.x;
+// each (24 heads x 16,366 queries against 512 prepared keys 103.2 -> 102.0 us).  A head's 4,096 norms (131,072 keys) are asked for at
+// once: bound by that one trip to memory.
+__global__ __launch_bounds__(256) void fold_norms_kernel(QkPrologueParams p) {
+  __shared__ float wave_top[4];
+  const int bh = blockIdx.x, lane = threadIdx.x & 63;
   const int n = ((p.row_cnt ? p.row_cnt[bh / p.H] : p.S) + 31) / 32;
   float* row = p.norm_out + (int64_t)bh * p.norm_stride;
   float top = 0.f;
-  for (int i = lane; i < n; i += 64) top = fmaxf(top, row[kNormFirst + i]);
+  for (int i0 = 4 * threadIdx.x; i0 < n; i0 += 4096) {
+    f32x4 v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = *(const f32x4*)(row + kNormFirst + min(i0 + 1024 * j, (n - 1) & ~3));
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) top = i0 + 1024 * j + e < n ? fmaxf(top, v[j][e]) : top;   // (places past the last may never have been written)
+  }
   top = wave_max(top);
-  if (lane == 0) row[0] = top;
+  if (lane == 0) wave_top[threadIdx.x >> 6] = top;
+  __syncthreads();
+  if (threadIdx.x == 0) row[0] = fmaxf(fmaxf(wave_top[0], wave_top[1]), fmaxf(wave_top[2], wave_top[3]));
 }
 
 hipError_t launch_fold_norms(const QkPrologueParams& k, hipStream_t st) {
-  hipLaunchKernelGGL(fold_norms_kernel, dim3((unsigned)(k.B * k.H)), dim3(64), 0, st, k);
+  hipLaunchKernelGGL(fold_norms_kernel, dim3((unsigned)(k.B * k.H)), dim3(256), 0, st, k);
   return hipGetLastError();
 }
 

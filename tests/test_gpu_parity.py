@@ -240,6 +240,8 @@ def test_softmax_scale_on_the_running_max_path():
     (24, 1085, 1085, 1084, False, False, False), (24, 1085, 1085, 33, False, False, True),   # short-key form
     (1, 400, 9000, 8193, False, True, False), (1, 64, 16500, 16499, False, True, True),      # long form
     (2, 300, 9000, 8999, True, True, False), (1, 64, 130, 129, True, False, False),          # block-sparse, 8 waves and narrow
+    (1, 33, 140001, 140000, False, False, False), (1, 33, 140001, 131071, False, False, "pow2"), (1, 33, 140001, 32769, False, False, False),
+    (2, 33, 140001, 131072, False, True, False),   # norms of more keys than one trip to memory fetches
 ])
 def test_one_key_of_a_large_norm_wherever_it_lies(H, Sq, Sk, at, sparse, long_key, fp8):
     """The softmax runs without a maximum where the largest key norm allows it: a key of a logit of 260 (base 2) anywhere, in
