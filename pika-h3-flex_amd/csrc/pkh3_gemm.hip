@@ -634,29 +634,6 @@ __global__ __launch_bounds__(64 * kThinWaves, 2) void gemm_thin_kernel(GemmParam
   *(bf16x4*)(rec + ((fb >> 1) * 64 + lane) * 16 + 8 * (fb & 1)) = o;
 }
 
-// Tokens per workgroup of a launch (16 * 2 * TB).  Time of a CU's share of the launch, in units of 100 us for K = 3,072 with an
-// adapter, from the workgroups it runs: one alone on the CU, and two (side by side for the smaller forms, one after the
-// other for TB = 8).  Measured at 1,085, 15,342 and 48,360 tokens x 9,216 and 3,072 features: TB = 8 67 us alone, 79 - 84 us
-// each in a long launch; TB = 6 53 and 104 us; TB = 4 40 us alone, 80 us for two; TB = 2 34 and 61 us.  What sets them: the smaller forms copy and
-// read more for the same MFMAs (a chunk: 64, 48 and 40 KiB read and 32, 24 and 20 KiB copied for 256, 128 and 64 MFMAs) and have
-// fewer of them between two barriers to cover a copy's way with, against how evenly their tiles fill the CUs.
-// TB = 6 is for launches of one tile a CU, where 192 tokens fill them better than 256 or 128 (us, 256 / 192 / 128 tokens: 1,085 x 9,216
-// 64.7 / 54.7 / 65.4, 3,000 x 3,072 63.9 / 52.9 / 64.8); in longer ones it is behind one of the others or the same (6,000 x 9,216 272 / 270 /
-// 251, 6,000 x 3,072 131 / 104 / 104).
-static int gemm_token_blocks(int tokens, int n_tiles, int cus) {
-  static const struct { int tb; float one, two; } kForms[4] = {{8, 0.67f, 1.55f}, {6, 0.53f, 0.f}, {4, 0.40f, 0.80f}, {2, 0.34f, 0.61f}};
-  int best = 8;
-  float best_cost = 0.f;
-  for (const auto& f : kForms) {
-    const int tiles = (tokens + 32 * f.tb - 1) / (32 * f.tb) * n_tiles;
-    const int per_cu = (tiles + cus - 1) / cus;
-    if (f.tb == 6 && per_cu > 1) continue;
-    const float cost = (per_cu / 2) * f.two + (per_cu & 1) * f.one;
-    if (f.tb == 8 || cost < best_cost) best = f.tb, best_cost = cost;
-  }
-  return best;
-}
-
 template <int TB, int R = kGemmRing>
 static hipError_t launch_gemm_tb(GemmParams p, int cus, hipStream_t st) {
   p.m_tiles = (p.M + 32 * TB - 1) / (32 * TB);
@@ -694,7 +671,7 @@ hipError_t launch_gemm(const GemmParams& p, hipStream_t st) {
       return hipGetLastError();
     }
   }
-  switch (gemm_token_blocks(p.M, p.n_tiles, cus)) {
+  switch (gemm_token_blocks(p.M, p.n_tiles, p.nk1, cus)) {
     case 8: return launch_gemm_tb<8>(p, cus, st);
     case 6: return launch_gemm_tb<6>(p, cus, st);
     case 4: return launch_gemm_tb<4>(p, cus, st);

@@ -1,4 +1,4 @@
-// Index arithmetic that kernels and host share and that a host test goes through: plain C++, no HIP.
+// Index arithmetic and rules on sizes that a host test goes through besides the kernels and their launches: plain C++, no HIP.
 #pragma once
 #include <stdint.h>
 
@@ -15,6 +15,31 @@ constexpr bool in_image_buffer(int row, int rows) { return row < padded_rows(row
 // goes that far or not.  64 bits: 2^23 workgroups (2^24 keys of 16 entries of one head) have 2^31.
 constexpr int64_t word_to_clear(unsigned batch, unsigned groups, unsigned group, unsigned thread) {
   return ((int64_t)batch * groups + group) * 256 + thread;
+}
+
+// Tokens per workgroup of a launch of gemm_kernel (16 * 2 * TB).  Time of a CU's share of the launch, in units of 100 us for K = 3,072 with an
+// adapter, from the workgroups it runs: one alone on the CU, and two (side by side for the smaller forms, one after the
+// other for TB = 8).  Measured at 1,085, 15,342 and 48,360 tokens x 9,216 and 3,072 features: TB = 8 67 us alone, 79 - 84 us
+// each in a long launch; TB = 6 53 and 104 us; TB = 4 40 us alone, 80 us for two; TB = 2 34 and 61 us.  What sets them: the smaller forms copy and
+// read more for the same MFMAs (a chunk: 64, 48 and 40 KiB read and 32, 24 and 20 KiB copied for 256, 128 and 64 MFMAs) and have
+// fewer of them between two barriers to cover a copy's way with, against how evenly their tiles fill the CUs.
+// TB = 6 is for launches of one tile a CU, where 192 tokens fill them better than 256 or 128 (us, 256 / 192 / 128 tokens: 1,085 x 9,216
+// 64.7 / 54.7 / 65.4, 3,000 x 3,072 63.9 / 52.9 / 64.8); in longer ones it is behind one of the others or the same (6,000 x 9,216 272 / 270 /
+// 251, 6,000 x 3,072 131 / 104 / 104).  Where 64-token tiles come to two a CU, its start and end (12 us against 8.5) have to be made good over
+// the chunks: from 64 of them on they are (1,305 x 6,144, K 96, 512, 1,024, 2,048 and 3,072: 192 tokens 13.1, 19.5, 26.0, 39.4 and 52.6, 64 tokens 10.0, 17.0,
+// 24.0, 40.3 and 55.2; 1,540 x 5,120, K 2,048 39.7 and 39.5).
+constexpr int gemm_token_blocks(int tokens, int n_tiles, int chunks, int cus) {
+  constexpr struct { int tb; float one, two; } kForms[4] = {{8, 0.67f, 1.55f}, {6, 0.53f, 0.f}, {4, 0.40f, 0.80f}, {2, 0.34f, 0.61f}};
+  int best = 8;
+  float best_cost = 0.f;
+  for (const auto& f : kForms) {
+    const int tiles = (tokens + 32 * f.tb - 1) / (32 * f.tb) * n_tiles;
+    const int per_cu = (tiles + cus - 1) / cus;
+    if (f.tb == 6 && (per_cu > 1 || (chunks < 64 && (tokens + 63) / 64 * n_tiles <= 2 * cus))) continue;
+    const float cost = (per_cu / 2) * f.two + (per_cu & 1) * f.one;
+    if (f.tb == 8 || cost < best_cost) best = f.tb, best_cost = cost;
+  }
+  return best;
 }
 
 constexpr int kKvMaxHeads = 8;        // heads a workgroup of the K/V pass walks at most

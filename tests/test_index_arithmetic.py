@@ -1,4 +1,4 @@
-"""Index arithmetic of the kernels at sizes and ends where it can go wrong, in a host build of the header they share: no GPU needed."""
+"""Index arithmetic and rules on sizes where they can go wrong, in a host build of the header the kernels share: no GPU needed."""
 import os
 import shutil
 import subprocess
@@ -86,3 +86,16 @@ def test_heads_a_workgroup_of_the_kv_pass(tmp_path):
         const KvSplit s = kv_split(tiles, 1 + heads % 3, heads, 256, rotation, tiles % 2);
         CHECK(s.heads >= 1 && s.heads <= kKvMaxHeads && s.groups * s.heads >= heads && (s.groups - 1) * s.heads < heads, "%d tiles, %d heads", tiles, heads);
       }""")
+
+
+def test_tokens_a_workgroup_of_the_projections(tmp_path):
+    """On 256 CUs: 192 tokens for launches of one such tile a CU, of few chunks only where 64-token tiles come to more than two."""
+    _run(tmp_path, """
+  struct { int tokens, n_tiles, chunks, want; } calls[] = {
+      {1305, 24, 3, 64}, {1305, 24, 32, 64}, {1305, 24, 64, 192}, {1305, 24, 96, 192}, {1540, 20, 16, 64}, {1352, 24, 3, 192}, {929, 36, 3, 192},
+      {1085, 36, 96, 192}, {2715, 12, 3, 192}, {31, 3, 3, 64}, {449, 9, 3, 64}, {3585, 36, 3, 128}, {1345, 36, 3, 256}, {48360, 36, 96, 256},
+      {16640, 2, 2, 192}, {16449, 2, 2, 192}, {11008, 3, 2, 192}, {33280, 1, 2, 192}};
+  for (auto c : calls) {
+    const int got = 32 * gemm_token_blocks(c.tokens, c.n_tiles, c.chunks, 256);
+    CHECK(got == c.want, "%d tokens, %d tiles, %d chunks: %d", c.tokens, c.n_tiles, c.chunks, got);
+  }""")
