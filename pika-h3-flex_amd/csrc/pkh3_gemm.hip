@@ -65,7 +65,8 @@ constexpr int waitcnt_vm_lgkm(int vm, int lgkm) { return (vm & 15) | ((vm >> 4) 
 // between the two halves of the register file inside the loop (456 moves per 128 MFMAs).  AGPR: the accumulators lie in the
 // accumulator half (TB = 8 and 6); the smaller forms keep them in the vector half, where the epilogue reads them in place.
 // WAIT: the last of a chunk with 192 accumulators.  The compiler does not know these instructions for MFMAs; where two paths join it
-// copied such an accumulator (it has registers to copy into) right behind its MFMA, before the result was there.
+// copied such an accumulator (it has registers to copy into) right behind its MFMA, before the result was there.  The other forms have been built
+// without such a copy; a host test (test_nothing_touches_a_product_before_it_is_there) looks for one in every build.
 template <bool AGPR, bool WAIT>
 __device__ __forceinline__ void mfma_acc(f32x4& c, const bf16x8& a, const bf16x8& b) {
   if constexpr (AGPR && WAIT) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\ts_nop 13" : "+a"(c) : "v"(a), "v"(b));

@@ -58,3 +58,90 @@ def test_no_load_into_registers_is_inline_assembly():
                 loads = re.findall(r"\b(?:ds_read|ds_load|global_load|buffer_load|flat_load|scratch_load|s_load)_\w+", m.group(0))
                 found += [(name, op) for op in loads if not op.startswith("global_load_lds")]
     assert not found
+
+
+OBJDUMP = shutil.which("llvm-objdump") or "/opt/rocm/llvm/bin/llvm-objdump"
+MFMA_RESULT = 12   # wait states until another instruction may touch a result of eight passes (that of a 16 x 16 x 32 product takes fewer)
+VALU_RESULT = 2    # ... until an MFMA may read what a vector instruction wrote
+
+
+def _registers(operands):
+    """The vector and accumulator registers named in operands: {("v", 7), ("a", 12), ...}."""
+    found = set()
+    for kind, one, first, last in re.findall(r"\b([va])(?:(\d+)\b|\[(\d+):(\d+)\])", operands):
+        found.update((kind, i) for i in (range(int(one), int(one) + 1) if one else range(int(first), int(last) + 1)))
+    return found
+
+
+def _hazards(listing):
+    """Instructions of one kernel's listing that come too soon after an MFMA or a vector instruction whose result they touch."""
+    code, at = [], {}
+    for line in listing.splitlines():
+        m = re.match(r"\s+(\S+)\s*(.*?)\s*// ([0-9A-F]+):(.*)", line)
+        if m:
+            at[int(m.group(3), 16)] = len(code)
+            target = re.search(r"\+0x([0-9a-f]+)>", m.group(4))
+            code.append((m.group(1), m.group(2), int(target.group(1), 16) if target else None))
+    start = min(at)
+    regs = [_registers(ops) for _, ops, _ in code]
+
+    def touched_within(i, states, touches):
+        """Whether ``touches(j)`` holds for an instruction j on a path of fewer than ``states`` wait states behind i."""
+        todo, seen = [(i + 1, 0)], set()
+        while todo:
+            j, waited = todo.pop()
+            if j >= len(code) or waited >= states or (j, waited) in seen:
+                continue
+            seen.add((j, waited))
+            if touches(j):
+                return True
+            name, ops, target = code[j]
+            waited += 1 + (int(ops) if name == "s_nop" else 0)
+            if name.startswith(("s_cbranch", "s_branch")):
+                todo.append((at[start + target], waited))
+            if name not in ("s_branch", "s_endpgm"):
+                todo.append((j + 1, waited))
+        return False
+
+    found = []
+    for i, (name, ops, _) in enumerate(code):
+        if not name.startswith("v_"):
+            continue
+        result = _registers(ops.split(",")[0])
+        mfma = name.startswith("v_mfma")
+        # (an MFMA may go on with the result of another as its own sum: the unit keeps these in order)
+        if mfma and touched_within(i, MFMA_RESULT, lambda j: result & regs[j] and not (
+                code[j][0].startswith("v_mfma") and _registers(code[j][1].split(",")[0]) == result)):
+            found.append((i, name, ops))
+        if not mfma and result and touched_within(i, VALU_RESULT, lambda j: code[j][0].startswith("v_mfma") and result & regs[j]):
+            found.append((i, name, ops))
+    return found
+
+
+@pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="llvm-objdump is not installed")
+def test_nothing_touches_a_product_before_it_is_there(tmp_path):
+    """The GEMM's MFMAs are assembly statements, behind which the compiler adds no wait states: it must not put a copy of an
+    accumulator there either.  Looked up in the listing of every form, along all branches."""
+    import __graft_entry__
+    import pika_h3_flex_amd as pk
+
+    __graft_entry__.ensure_built()
+    forms = {}
+    for i, image in enumerate(_code_objects(pk._lib.LIB_PATH)):
+        f = tmp_path / f"{i}.elf"
+        f.write_bytes(image)
+        text = subprocess.run([OBJDUMP, "-d", str(f)], check=True, capture_output=True, text=True).stdout
+        for name, listing in re.findall(r"^[0-9a-f]+ <(\S*gemm_kernel\S*)>:\n(.*?)(?=^[0-9a-f]+ <|\Z)", text, re.M | re.S):
+            forms[name] = _hazards(listing)
+            assert listing.count("v_mfma") >= 64, name
+    assert len(forms) == 5 and not {n: h[:3] for n, h in forms.items() if h}, forms
+
+
+def test_the_look_for_products_finds_what_it_looks_for():
+    mfma = "\tv_mfma_f32_16x16x32_bf16 a[0:3], v[8:11], v[4:7], a[0:3]// 000000000100: 00\n"
+    read = "\tv_accvgpr_read_b32 v0, a2                             // 000000000110: 00\n"
+    assert len(_hazards(mfma + read)) == 1
+    assert not _hazards(mfma + "\ts_nop 13                         // 000000000108: 00\n" + read)
+    assert not _hazards(mfma + mfma.replace("0100", "0108")) and not _hazards(mfma + read.replace("a2", "a4"))
+    assert len(_hazards(mfma + "\ts_branch 1                       // 000000000108: 00 <k+0x10>\n" + "\tv_mov_b32 v9, v1 // 00000000010C: 00\n" + read)) == 1
+    assert len(_hazards("\tv_mov_b32_e32 v9, v1           // 0000000000FC: 00\n" + mfma)) == 1
