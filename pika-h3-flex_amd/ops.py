@@ -181,14 +181,23 @@ def workspace_bytes(args: _lib.AttnArgs) -> int:
     return int(n)
 
 
+def _raw_stream_of_torch():
+    """The handle of a device's current stream from its index, without a ``Stream`` object made for it where this torch has such a call
+    (it is not a public one): 0.1 us instead of 1.1, on a path that small calls wait for."""
+    return getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda index: torch.cuda.current_stream(index).cuda_stream)
+
+
+_raw_stream = _raw_stream_of_torch()
+
+
 def _attn_fwd(lib, args: _lib.AttnArgs, device, workspace: Optional[torch.Tensor]) -> None:
     """Enqueues the call on the device's current stream.  ``workspace``: one that may belong to another stream than this: it must
     outlive the kernels, so it is tied to the stream.  (Memory allocated here belongs to this stream already.)"""
     if device.index == torch.cuda.current_device():
-        _lib.check(lib.pkh3_attn_fwd(C.byref(args), torch._C._cuda_getCurrentRawStream(device.index)))
+        _lib.check(lib.pkh3_attn_fwd(C.byref(args), _raw_stream(device.index)))
     else:
         with torch.cuda.device(device):
-            _lib.check(lib.pkh3_attn_fwd(C.byref(args), torch._C._cuda_getCurrentRawStream(device.index)))
+            _lib.check(lib.pkh3_attn_fwd(C.byref(args), _raw_stream(device.index)))
     if workspace is not None:
         workspace.record_stream(torch.cuda.current_stream(device))
 

@@ -143,3 +143,14 @@ def test_fp8_option_forms():
     assert fp8_mode("pow2") == "pow2"
     with pytest.raises(ValueError):
         fp8_mode("e5m2")
+
+
+def test_stream_handle_without_the_private_call(monkeypatch):
+    """A torch without it gets the handle from its public stream object."""
+    from types import SimpleNamespace
+
+    from pika_h3_flex_amd import ops
+
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda index: SimpleNamespace(cuda_stream=1000 + index))
+    assert ops._raw_stream_of_torch()(3) == 1003
