@@ -242,8 +242,10 @@ __global__ __launch_bounds__(256, 3) void kv_prologue_kernel(QkPrologueParams k,
   // head groups vary fastest across workgroups: neighbours read neighbouring pieces of the same [S, H, D] rows
   const int tile = bid / (2 * groups), in_tile = bid % (2 * groups), b = blockIdx.y;
   const int h0 = (in_tile >> 1) * heads_per_wg, n = min(heads_per_wg, k.H - h0);
-  const int64_t word = word_to_clear(blockIdx.y, gridDim.x - plan.n, bid, threadIdx.x);
-  if (word < k.clear_n) k.clear[word] = 0u;
+  if (k.clear_n > 0) {
+    const int64_t word = word_to_clear(blockIdx.y, gridDim.x - plan.n, bid, threadIdx.x);
+    if (word < k.clear_n) k.clear[word] = 0u;
+  }
   __shared__ int source[64];                            // source row of each row of the tile (key mask)
   int rows = k.S;
   if (k.row_cnt) {
