@@ -32,7 +32,8 @@
 // Block-sparse variant.  A workgroup covers 4 query row-blocks (64 queries each, a wave pair per row-block).
 // Phase 1 walks the key tiles all four row-blocks keep, exactly like the dense kernel.  Phase 2 walks the
 // remaining tiles per row-block: every iteration gives each wave pair one 32-key half of a tile of its own
-// list in its own LDS area, so all 8 waves stay busy.  The lists are built on the device by a plan kernel.
+// list in its own LDS area, so all 8 waves stay busy.  The lists are made on
+// the device by the first workgroups of the K/V pass, for calls on prepared keys by a launch of their own (pkh3_plan.h).
 #include <float.h>
 #include <limits.h>
 #include <math.h>
@@ -49,8 +50,9 @@ constexpr int kDenseWaves = 12;  // dense kernel: three waves per SIMD (<= 168 V
 constexpr int kShortWaves = 4;   // short-key dense kernel: three 4-wave workgroups per CU
 constexpr int kMaxParts = 8;     // long dense form: most workgroups a unit's key tiles are shared out among ...
 constexpr int kMinPartTiles = 24;  // ... and fewest key tiles such a workgroup is worth starting for
-constexpr int kSparseWaves = 2 * kSparseRows;  // block-sparse: a wave pair per row-block; two such workgroups share a CU
+constexpr int kSparseWaves = 2 * kSparseRows;  // block-sparse: a wave pair per row-block; one such workgroup on a CU (96 to 128 KiB of LDS)
 constexpr int kRing = 3;               // LDS ring depth (tiles)
+constexpr int kStages2 = 2;            // block-sparse phase 2: stages of row-private half tiles
 constexpr int kPipeRing = 4;           // ... of the pipelined short-key form (32-key halves)
 constexpr float kRescaleSlack = 8.0f;  // the running max is only raised when exceeded by 2^8
 // The running max before the first key.  Finite: keys whose logits are all -inf then weigh exp2(-inf - max) = 0, wherever
@@ -144,8 +146,9 @@ __device__ __forceinline__ void load_q_rows(QRows& r, const Params& p, const Row
 }
 
 // Consecutive MFMAs share an operand where they can: the two query blocks of an image come in turn (0 1, 1 0, 0 1 ..), so that only
-// one of the operands changes from one to the next.  Less toggles in the matrix unit, at a clock that is set by power: 480p 19.69 ->
-// 19.64 ms, 14,830 + 512 rows 2,142 -> 2,135 us, with the projection's GEMMs (the same) a block of them 3,153 -> 3,138.
+// one of the operands changes from one to the next.  Less toggles in the matrix unit, at a clock that is set by power: 480p 19.82 ->
+// 19.66 ms, 768p 130.1 -> 128.9, 14,830 + 512 rows 2,149 -> 2,138 us, with the projection's GEMMs (the same) a block of them 3,168 -> 3,145
+// (means of two comparisons in one box); fp8 and short calls the same.
 #define PKH3_MFMA16(A, B, C) __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, C, 0, 0, 0)
 // format codes 0/0 = e4m3 x e4m3; scale operands 0 select the unscaled form of the instruction
 #define PKH3_MFMA16_F8(A, B, C) __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(A, B, C, 0, 0, 0, 0, 0, 0)
@@ -505,15 +508,13 @@ __host__ __device__ constexpr int units_per_head(int Sq, int blocks) { return ((
 template <bool FP8, bool SPARSE, int WAVES, bool PIPE = false>
 constexpr int fwd_lds_bytes() {
   constexpr bool HALFMODE = !SPARSE && WAVES == kShortWaves;
-  constexpr int kRingT = (SPARSE && !FP8 && WAVES < 8) ? 2 : kRing;
-  constexpr int kStages2 = (SPARSE && FP8 && WAVES < 8) ? 3 : 2;
   constexpr int kTileBytes = (FP8 ? kK8TileBytes : kKTileBytes) + kVTileBytes;
   constexpr int kHalfBytes = kTileBytes / 2;
   constexpr int kStageBytes = 32 * kD * 2;    // one wave's 32 x 128 bf16 output block, staged for the row-wise store
-  // dense / phase 1: ring of kRingT whole tiles; sparse phase 2: kStages2 stages of row-private half tiles
+  // dense / phase 1: ring of kRing whole tiles; sparse phase 2: kStages2 stages of row-private half tiles
   constexpr int kPhase2Bytes = SPARSE ? kStages2 * kSparseRows * kHalfBytes : 0;
   constexpr int kRingBytes = HALFMODE ? (PIPE ? kPipeRing : kRing) * kHalfBytes
-                             : (kPhase2Bytes > kRingT * kTileBytes ? kPhase2Bytes : kRingT * kTileBytes);
+                             : (kPhase2Bytes > kRing * kTileBytes ? kPhase2Bytes : kRing * kTileBytes);
   constexpr int kAfterBytes = WAVES * kStageBytes;  // LDS use after the loops
   return kRingBytes > kAfterBytes ? kRingBytes : kAfterBytes;
 }
@@ -531,10 +532,7 @@ __device__ __forceinline__ int attn_fwd_body(const Params& p, int blk, int unit0
   static_assert(FP8 || !POW2, "power-of-two scales belong to the fp8 form");
   constexpr bool SHORT = !SPARSE && WAVES == kShortWaves;
   constexpr bool LEAN = !SPARSE;                        // dense long-key form: three waves per SIMD, lean read-ahead
-  // whole-tile ring depth: three tiles, except where two workgroups share the CU's LDS and a bf16 tile is 32 KiB
-  constexpr int kRingT = (SPARSE && !FP8 && WAVES < 8) ? 2 : kRing;
-  constexpr int kAhead = kRingT - 1;                    // tiles in flight ahead of the one being used
-  constexpr int kStages2 = (SPARSE && FP8 && WAVES < 8) ? 3 : 2;  // sparse phase 2: stages of row-private half tiles
+  constexpr int kAhead = kRing - 1;                     // tiles in flight ahead of the one being used
   constexpr bool HALFMODE = SHORT;                      // ring of 32-key half tiles
   constexpr bool PARTS = !SPARSE && !SHORT;             // the long dense form: the key tiles may be shared out (`parts`)
   constexpr int kKBytes = FP8 ? kK8TileBytes : kKTileBytes;
@@ -636,7 +634,7 @@ __device__ __forceinline__ int attn_fwd_body(const Params& p, int blk, int unit0
     if (n_mine > 1) dma_short(h_begin + 1, 1);
   } else if (t_end > t_begin) {
     dma(entry(t_begin), 0);
-    if (kAhead > 1 && t_end > t_begin + 1) dma(entry(t_begin + 1), 1);
+    if (t_end > t_begin + 1) dma(entry(t_begin + 1), 1);
   }
   // Q, fused with QK-RMSNorm, rotation and (fp8) quantisation, in the layout of the MFMA B images themselves:
   // lane (c, g) has read, for each of the wave's two 16-query blocks qb, the 32 elements d = 32*ks + 8*g + j of query
@@ -735,7 +733,7 @@ __device__ __forceinline__ int attn_fwd_body(const Params& p, int blk, int unit0
     static_max = __all(bound <= kStaticMaxLimit);
   }
 
-  int slot = 0, slot_prev = (HALFMODE ? kRing : kRingT) - 1;  // ring slots of tile i and of tile i-1 (which takes the newest copy)
+  int slot = 0, slot_prev = kRing - 1;  // ring slots of tile i and of tile i-1 (which takes the newest copy)
   // Only the last key tile can be partial.  It is peeled off the loop so that the loop body has no masking
   // branch between S^T and the softmax, which lets the numerators of the first 32 keys be scheduled under
   // the MFMAs of the second 32.
@@ -761,7 +759,7 @@ __device__ __forceinline__ int attn_fwd_body(const Params& p, int blk, int unit0
     if (POW2) dma(entry(min(i + kAhead, t_end - 1)), slot_prev);                                        \
     else if (i + kAhead < t_end) dma(entry(i + kAhead), slot_prev);                                     \
     slot_prev = slot;                                                                                   \
-    slot = slot == kRingT - 1 ? 0 : slot + 1;                                                           \
+    slot = slot == kRing - 1 ? 0 : slot + 1;                                                            \
     const float ct = (FP8 && !POW2) ? c * ks : c;                                                       \
     softmax_pv_tile<FP8, STATIC, LEAN, MASKED, POW2>(w, kbuf + kKBytes, ct, tail, lane);                \
   }
@@ -1399,7 +1397,8 @@ AttnForm attn_form(const FwdParams& p, int cus) {
   // take the narrow form where it is estimated shorter, else the short-key form.  The estimates are straight lines through
   // kernel times in microseconds (bf16; fp8 lies within a tenth of them): the narrow form, a start and a merge and 0.135 per half tile
   // for every 32-query block a CU gets; the short-key form, a half tile per 0.60 with one workgroup on a CU and per 0.87
-  // with two.  Measured (narrow / short-key / long): 240 blocks x 10 half tiles 7.9 / 11.1 / 17.2, 504 x 63 23.9 / 41.9 / 62.9,
+  // with two (the plain loop, as in the figures here; the pipelined one, which takes these calls, needs 0.48 and 0.82: the line has not been
+  // moved with it).  Measured (narrow / short-key / long): 240 blocks x 10 half tiles 7.9 / 11.1 / 17.2, 504 x 63 23.9 / 41.9 / 62.9,
   // 768 x 64 34.8 / 43.4 / 63.7, 1,256 x 157 115 / 128 / 144; on the other side of the line 456 x 4 7.9 / 7.7 / 12.6,
   // 816 x 34 27.3 / 26.3 / 38.5, 1,504 x 94 86 / 81 / 90, 1,896 x 79 95 / 73 / 78.  With three short-key workgroups per CU the
   // long form is ahead as long as its own workgroups are no more than the CUs (2,256 x 94: 114 / 94), and behind when a few

@@ -228,9 +228,9 @@ constexpr int kQueues = 8;       // work queues of a launch: one per XCD
 // (a few per cent apart), and the hardware deals workgroups to them round-robin, an eighth each whatever their speed,
 // so with a fixed workgroup -> unit map the call lasts as long as its slowest XCD needs for its eighth.  Instead every
 // XCD has a queue (a counter) over its contiguous run of units: a workgroup takes the next unit of its own XCD's queue
-// and, when that is empty, of the queue with the most units left; the launch holds an eighth more workgroups than
-// units, so an XCD that is through early keeps getting workgroups, which take units off the slower ones.  A workgroup
-// that finds every queue empty exits.  Returns the unit (index inside the section) or -1.
+// and, when that is empty, of the queue with the most units left.  Launches of a workgroup per unit hold an eighth more workgroups than
+// units, so an XCD that is through early keeps getting workgroups, which take units off the slower ones; in the block-sparse form a
+// workgroup per CU takes one unit after the other.  A workgroup that finds every queue empty exits.  Returns the unit (index inside the section) or -1.
 // `taken`: a position of the home queue that the caller has taken ahead (take_position), or -1.
 // STRIDE: ints between the queues' positions.  The accesses of all XCDs to one stretch of 32 bytes are served one after the
 // other, which is the rate of a launch of short workgroups whose positions share one (see gemm_kernel).

@@ -680,8 +680,9 @@ hipError_t launch_gemm(const GemmParams& p, hipStream_t st) {
   }
   // 64 tokens with one workgroup on a CU: a chunk is done in 0.22 us, and three of them cover a copy's way where two do not.  Ring of
   // 3 / 4, K 3,072 x 3,072 features, us: 128 tokens 29.7 / 24.6, 500 31.2 / 26.0, 1,085 32.0 / 27.2 (of 5 to 7 the same); with a dozen workgroups on
-  // the chip the way is short enough (64 tokens 23.0 / 23.6), and for few chunks the longer start costs more (K 1,024 13.4 / 12.6 and
-  // 11.7 / 12.0, 512 8.1 / 8.3).  The larger forms gain nothing from it.
+  // the chip the way is short enough (64 tokens 23.0 / 23.6), and for few chunks the longer start costs as much (K 1,024 13.4 / 12.6 and
+  // 11.7 / 12.0, 512 8.1 / 8.3).  From K 1,536 on 8 to 22 % in 53 of 56 calls of 32 to 216 tiles; 2 % slower: 44 tiles, K 1,536 13.8 / 14.1, and
+  // 32 tiles of 256 features, K 1,536 20.5 / 20.9 and 2,048 24.0 / 24.4 (with an adapter; K 3,072 36.5 / 32.7).  The larger forms gain nothing from it.
   const int64_t tiles = (int64_t)((p.M + 63) / 64) * p.n_tiles;
   return tiles >= 24 && tiles <= cus && p.nk1 >= 48 ? launch_gemm_tb<2, 4>(p, cus, st) : launch_gemm_tb<2>(p, cus, st);
 }

@@ -279,7 +279,7 @@ hipError_t launch_kv_prologue(QkPrologueParams k, const VPrologueParams& v, cons
     k.mask = nullptr;
   }
   // The entries of a block-sparse plan ride in front: each is a chain of short steps, so they end under the tiles' loads.  A launch
-  // of their own costs a call 3 us (4,109 tokens, 24 heads, fp8, 10 % of the tiles: 683.9 -> 680.4 us; 37,877 in bf16: 6,876 -> 6,873).
+  // of their own costs a call 3 us (24 heads x 14,907 rows in fp8: 683.9 -> 680.4 us; 48,360 in bf16: 6,876 -> 6,873).
   const dim3 grid((unsigned)(2 * split.groups) * k.nBlk64 + plan.n, k.B), block(256);
   if (k.fp8) hipLaunchKernelGGL(kv_prologue_kernel<true>, grid, block, 0, st, k, v, plan, split.heads, split.groups);
   else hipLaunchKernelGGL(kv_prologue_kernel<false>, grid, block, 0, st, k, v, plan, split.heads, split.groups);

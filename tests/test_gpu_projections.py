@@ -278,7 +278,7 @@ def test_qkv_projection_writes_whole_key_tiles(S, H, variant):
 @pytest.mark.parametrize("S,N", [(65, 256), (1471, 3072), (1537, 2944), (3583, 3072), (3649, 2944), (2881, 3072), (3263, 2944)])
 @pytest.mark.parametrize("gate,residual", [(True, True), (True, False), (False, True), (False, False)])
 def test_gemm_forms_of_the_out_projection(S, N, gate, residual):
-    """The three workgroup heights of the row-major epilogue with each of its four combinations, every row."""
+    """The four workgroup heights of the row-major epilogue with each of its four combinations, every row."""
     from pika_h3_flex_amd import projections as P
 
     K = 96
