@@ -148,7 +148,7 @@ __device__ __forceinline__ void load_q_rows(QRows& r, const Params& p, const Row
 // Consecutive MFMAs share an operand where they can: the two query blocks of an image come in turn (0 1, 1 0, 0 1 ..), so that only
 // one of the operands changes from one to the next.  Less toggles in the matrix unit, at a clock that is set by power: 480p 19.82 ->
 // 19.66 ms, 768p 130.1 -> 128.9, 14,830 + 512 rows 2,149 -> 2,138 us, with the projection's GEMMs (the same) a block of them 3,168 -> 3,145
-// (means of two comparisons in one box); fp8 and short calls the same.
+// (means of two comparisons on one card); fp8 and short calls the same.
 #define PKH3_MFMA16(A, B, C) __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, C, 0, 0, 0)
 // format codes 0/0 = e4m3 x e4m3; scale operands 0 select the unscaled form of the instruction
 #define PKH3_MFMA16_F8(A, B, C) __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(A, B, C, 0, 0, 0, 0, 0, 0)
