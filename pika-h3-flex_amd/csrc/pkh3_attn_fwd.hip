@@ -26,7 +26,8 @@
 //
 // Other forms of the dense kernel (see attn_fwd_body): the short-key form (few key tiles, or few queries: 4 waves per
 // workgroup, 32-key half tiles, three workgroups per CU), the narrow form (fewer queries still: one 32-query block per
-// workgroup, its waves share the keys out; attn_fwd_narrow_kernel), and the long form with the key tiles of a unit shared out
+// workgroup, its waves share the keys out; attn_fwd_narrow_kernel), the relay form (many queries, few to some dozens of key tiles: a workgroup
+// per CU goes from one block of queries to the next; attn_fwd_relay_kernel), and the long form with the key tiles of a unit shared out
 // among several workgroups that merge through global scratch, for a thinly filled last round of a long call.
 //
 // Block-sparse variant.  A workgroup covers 4 query row-blocks (64 queries each, a wave pair per row-block).
@@ -163,9 +164,17 @@ __device__ __forceinline__ void load_q_rows(QRows& r, const Params& p, const Row
 // AHEAD: images the LEAN reads run ahead (the copies of the loop that run once per workgroup take 2 and fit the registers)
 // POW2 (fp8): the block scales are powers of two and go into the MFMA as its scale operands (`ke`: exponent byte of
 // this K tile's scale), so S^T leaves the MFMA dequantised.
-template <bool FP8, bool LEAN, int AHEAD = 4, bool POW2 = false>
-__device__ __forceinline__ void qk_tile(WaveState<FP8>& w, const char* kbuf, const char* vbuf, int lane, int ke = 0) {
+// MASKED (lean bf16 form): the sums start from -inf instead of 0 for keys from `lim` on, which costs the softmax nothing.
+template <bool FP8, bool LEAN, int AHEAD = 4, bool POW2 = false, bool MASKED = false>
+__device__ __forceinline__ void qk_tile(WaveState<FP8>& w, const char* kbuf, const char* vbuf, int lane, int ke = 0, int lim = 0) {
+  static_assert(!MASKED || (!FP8 && LEAN), "the forms that ask for it");
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  if constexpr (MASKED) {
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w.s[kb][0][i] = w.s[kb][1][i] = 16 * kb + 4 * (lane >> 4) + i >= lim ? -INFINITY : 0.f;
+  }
   if constexpr (!FP8 && LEAN) {
     bf16x8 kf[16];
 #pragma unroll
@@ -174,7 +183,7 @@ __device__ __forceinline__ void qk_tile(WaveState<FP8>& w, const char* kbuf, con
     for (int i = 0; i < 16; ++i) {
       const int ks = (i >> 1) & 3, kb = 2 * (i >> 3) + (i & 1);
 #pragma unroll
-      for (int q = 0, qb = i & 1; q < 2; ++q, qb ^= 1) w.s[kb][qb] = PKH3_MFMA16(kf[i], w.qf[qb][ks], ks == 0 ? zero : w.s[kb][qb]);
+      for (int q = 0, qb = i & 1; q < 2; ++q, qb ^= 1) w.s[kb][qb] = PKH3_MFMA16(kf[i], w.qf[qb][ks], ks == 0 && !MASKED ? zero : w.s[kb][qb]);
       if (i + AHEAD < 16) kf[i + AHEAD] = *(const bf16x8*)(kbuf + ((i + AHEAD) * 64 + lane) * 16);
     }
     PKH3_SGB(kSgDsRead, AHEAD);
@@ -242,7 +251,8 @@ __device__ __forceinline__ float softmax_numerator(float s, float c, float m) {
 // STATIC: w.m is not used: every logit is bounded (|q_i| * max_j |k_j| * c), small enough that exp2(logit) is a
 // normal number; the running max, its exchange across the lane groups and the O^T rescale are then not needed at
 // all, and the numerators of the first 32 keys do not wait for the second half of S^T.
-template <bool FP8, bool STATIC, bool MASKED, int NKB, bool POW2 = false, int AT = 0>
+// FIRST: nothing has been summed up yet.
+template <bool FP8, bool STATIC, bool MASKED, int NKB, bool POW2 = false, int AT = 0, bool FIRST = false>
 __device__ __forceinline__ void softmax_blocks(WaveState<FP8>& w, bf16x8 (&pf)[NKB / 2][2], float c, int lim, int lane) {
   constexpr bool MUL = FP8 && !POW2;  // the logits still need their dequantisation scales
   const int g = lane >> 4;
@@ -270,7 +280,7 @@ __device__ __forceinline__ void softmax_blocks(WaveState<FP8>& w, bf16x8 (&pf)[N
       alpha[qb] = __builtin_amdgcn_exp2f(w.m[qb] - m_new[qb]);
       w.m[qb] = m_new[qb];
     }
-    if (__any(alpha[0] != 1.0f || alpha[1] != 1.0f)) {
+    if (!FIRST && __any(alpha[0] != 1.0f || alpha[1] != 1.0f)) {
 #pragma unroll
       for (int db = 0; db < 8; ++db)
 #pragma unroll
@@ -298,16 +308,18 @@ __device__ __forceinline__ void softmax_blocks(WaveState<FP8>& w, bf16x8 (&pf)[N
       pf[half][qb] = pk;
     }
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb) w.l[qb] = STATIC ? w.l[qb] + rsum[qb] : w.l[qb] * alpha[qb] + rsum[qb];
+  for (int qb = 0; qb < 2; ++qb) w.l[qb] = FIRST ? rsum[qb] : STATIC ? w.l[qb] + rsum[qb] : w.l[qb] * alpha[qb] + rsum[qb];
 }
 
 // Softmax of w.s, then O^T += V^T P^T for one tile: V image i is (half, db) = (i >> 3, i & 7) and feeds the two
 // query blocks, sixteen accumulators in rotation.  `c` = softmax scale * log2(e) (times the fp8 dequantisation
 // scales of this tile); `lim` = keys of this tile that exist (only read when MASKED).
-template <bool FP8, bool STATIC, bool LEAN, bool MASKED, bool POW2 = false>
+template <bool FP8, bool STATIC, bool LEAN, bool MASKED, bool POW2 = false, bool FIRST = false>
 __device__ __forceinline__ void softmax_pv_tile(WaveState<FP8>& w, const char* vbuf, float c, int lim, int lane) {
+  static_assert(!FIRST || LEAN, "the forms that ask for it");
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   bf16x8 pf[2][2];
-  softmax_blocks<FP8, STATIC, MASKED, 4, POW2>(w, pf, c, lim, lane);
+  softmax_blocks<FP8, STATIC, MASKED, 4, POW2, 0, FIRST>(w, pf, c, lim, lane);
   if constexpr (LEAN) {
     bf16x8 vg[16];
 #pragma unroll
@@ -315,7 +327,7 @@ __device__ __forceinline__ void softmax_pv_tile(WaveState<FP8>& w, const char* v
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
 #pragma unroll
-      for (int q = 0, qb = i & 1; q < 2; ++q, qb ^= 1) w.o[i & 7][qb] = PKH3_MFMA16(vg[i], pf[i >> 3][qb], w.o[i & 7][qb]);
+      for (int q = 0, qb = i & 1; q < 2; ++q, qb ^= 1) w.o[i & 7][qb] = PKH3_MFMA16(vg[i], pf[i >> 3][qb], FIRST && i < 8 ? zero : w.o[i & 7][qb]);
       if (i + 4 < 16) vg[i + 4] = *(const bf16x8*)(vbuf + ((i + 4) * 64 + lane) * 16);
     }
   } else {
@@ -437,6 +449,54 @@ __device__ __forceinline__ float largest_key_norm(const Params& p, int bh, int n
     }
   }
   return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(wave_max(top))));
+}
+
+// O = O^T * inv in bf16, out of one wave.  A lane holds 4 consecutive d of a query per accumulator, which would make 8-byte
+// stores scattered over 16 rows; instead the wave turns its 32 x 128 block around in 8 KiB of LDS of its own (`stage`;
+// 16-byte chunks XOR-swizzled by the row so both directions are conflict-free) and stores whole 256-byte rows, 16 bytes per
+// lane.  A block whose 32 rows all exist is eight stores of every lane.
+template <bool FP8, typename Params>
+__device__ __forceinline__ void store_output(const Params& p, const WaveState<FP8>& w, const float (&inv)[2], char* stage, int b, int h, int q32,
+                                             int lane) {
+  const int c16 = lane & 15, g4 = lane >> 4;
+#pragma unroll
+  for (int qb = 0; qb < 2; ++qb)
+#pragma unroll
+    for (int db = 0; db < 8; ++db) {
+      bf16x4 wv;
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) wv[rr] = (__bf16)(w.o[db][qb][rr] * inv[qb]);
+      // elements d = 16*db + 4*g .. +3 of row 16*qb + c16: 16-byte chunk 2*db + g/2, its half g%2
+      const int chunk = (2 * db + (g4 >> 1)) ^ c16;
+      *(bf16x4*)(stage + (16 * qb + c16) * 256 + chunk * 16 + 8 * (g4 & 1)) = wv;
+    }
+  // same wave wrote and reads: the LDS counter orders the two, no barrier
+  if (p.o_images) {
+    // operand images of the out-projection GEMM: image (16-row block, k-step h*4 + ks) holds, in lane (c = l % 16,
+    // g = l / 16), elements 32*ks + 8*g .. +7 of this head for row c of the block -- one 1 KiB store per image
+    if (q32 * 32 >= p.Sq) return;  // a block without rows: the buffer may end before it
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) {
+      const int r = 16 * rb + c16;
+      const bool live = q32 * 32 + r < p.Sq;
+      char* img = (char*)p.o + (int64_t)(q32 * 2 + rb) * p.o_img_blk_stride + (int64_t)h * (kD / 32) * 1024;
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        bf16x8 v = *(const bf16x8*)(stage + r * 256 + (((4 * ks + g4) ^ (r & 15)) * 16));
+        if (!live) v = bf16x8{};
+        *(bf16x8*)(img + (ks * 64 + lane) * 16) = v;
+      }
+    }
+    return;
+  }
+  __bf16* ob = (__bf16*)p.o + (int64_t)b * p.o_sb + (int64_t)h * p.o_sh;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int row = 4 * i + (lane >> 4), c = lane & 15;
+    const bf16x8 v = *(const bf16x8*)(stage + row * 256 + ((c ^ (row & 15)) * 16));
+    const int q = q32 * 32 + row;
+    if (q < p.Sq) *(bf16x8*)(ob + (int64_t)q * p.o_ss + 8 * c) = v;
+  }
 }
 
 // The loop of the pipelined short-key form.  A pass runs S^T of the next half beside the softmax of this one, for waves that
@@ -883,11 +943,6 @@ __device__ __forceinline__ int attn_fwd_body(const Params& p, int blk, int unit0
     if (p.queue_next && threadIdx.x == 0) next_pos = take_position(p.queue_next + (blockIdx.x & (kQueues - 1)));
   }
 
-  // Epilogue: O = O^T / l in bf16.  A lane holds 4 consecutive d of a query per accumulator, which would make 8-byte
-  // stores scattered over 16 rows; instead each wave turns its 32 x 128 block around in its own 8 KiB of LDS
-  // (16-byte chunks XOR-swizzled by the row so both directions are conflict-free) and stores whole 256-byte rows,
-  // 16 bytes per lane.
-  __bf16* ob = (__bf16*)p.o + (int64_t)b * p.o_sb + (int64_t)h * p.o_sh;
   __syncthreads();  // every wave is done reading K/V tiles: the LDS becomes staging space
   if constexpr (PARTS) {
     if (parts > 1) {
@@ -949,48 +1004,7 @@ __device__ __forceinline__ int attn_fwd_body(const Params& p, int blk, int unit0
     const float lt = wave_sum_groups(w.l[qb]);
     inv[qb] = lt > 0.f ? 1.0f / lt : 0.f;
   }
-  char* stage = lds_raw + wq * kStageBytes;
-  {
-    const int c16 = lane & 15, g = lane >> 4;
-#pragma unroll
-    for (int qb = 0; qb < 2; ++qb)
-#pragma unroll
-      for (int db = 0; db < 8; ++db) {
-        bf16x4 wv;
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr) wv[rr] = (__bf16)(w.o[db][qb][rr] * inv[qb]);
-        // elements d = 16*db + 4*g .. +3 of row 16*qb + c16: 16-byte chunk 2*db + g/2, its half g%2
-        const int chunk = (2 * db + (g >> 1)) ^ c16;
-        *(bf16x4*)(stage + (16 * qb + c16) * 256 + chunk * 16 + 8 * (g & 1)) = wv;
-      }
-  }
-  // same wave wrote and reads: the LDS counter orders the two, no barrier
-  if (p.o_images) {
-    // operand images of the out-projection GEMM: image (16-row block, k-step h*4 + ks) holds, in lane (c = l % 16,
-    // g = l / 16), elements 32*ks + 8*g .. +7 of this head for row c of the block -- one 1 KiB store per image
-    if (q32 * 32 >= p.Sq) return next_pos;  // a block without rows: the buffer may end before it
-    const int c16 = lane & 15, g4 = lane >> 4;
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
-      const int r = 16 * rb + c16;
-      const bool live = q32 * 32 + r < p.Sq;
-      char* img = (char*)p.o + (int64_t)(q32 * 2 + rb) * p.o_img_blk_stride + (int64_t)h * (kD / 32) * 1024;
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        bf16x8 v = *(const bf16x8*)(stage + r * 256 + (((4 * ks + g4) ^ (r & 15)) * 16));
-        if (!live) v = bf16x8{};
-        *(bf16x8*)(img + (ks * 64 + lane) * 16) = v;
-      }
-    }
-    return next_pos;
-  }
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int row = 4 * i + (lane >> 4), c = lane & 15;
-    const bf16x8 v = *(const bf16x8*)(stage + row * 256 + ((c ^ (row & 15)) * 16));
-    const int q = q32 * 32 + row;
-    if (q < p.Sq) *(bf16x8*)(ob + (int64_t)q * p.o_ss + 8 * c) = v;
-  }
+  store_output(p, w, inv, lds_raw + wq * kStageBytes, b, h, q32, lane);
   return next_pos;
 }
 
@@ -1342,6 +1356,264 @@ __global__ __launch_bounds__(64 * kNarrowWaves, 2) void attn_fwd_narrow_kernel(F
   }
 }
 
+// The relay form (bf16), for calls of many queries against few to some dozens of key tiles: one workgroup per CU for the whole call, twelve waves
+// (three groups of four) that walk the tiles of a (batch, head) round and round.  A round is three units, a unit 128 queries, a group a unit.
+// The ring of two tiles never drains: behind the last tile of a round comes the first of the next, already on its way under the
+// last one's work.  The next queries come to LDS while the tiles are walked, each wave's to a place of its own, which
+// the output goes through on its way out.
+//
+// What it is for: a workgroup of the other dense forms lasts a few tiles, and its start (the launch, keys known, queries, first tiles: one
+// trip to memory behind the other) and its end cost as much as five of them.  Here a round costs 3.9 us and 2.1 to 2.2 a tile,
+// short-key workgroups (three to a CU) 9 and 2.3, long ones 13 and 2.0.  Kernel, us, before / with it: 24 heads x 49,640 queries against
+// 302 of 512 keys 249 / 228, 1,024 keys 543 / 505; x 14,830 against 1,536 keys 242 / 228; x 9,000 against 2,048 219 / 185 (rounds of
+// long workgroups that are nearly empty at the end).  What bounds it now: the MFMAs and, between two rounds, stores and
+// queries of all CUs at once at the rate of the memory (12 KiB of each a wave: 96 KiB a CU, 14 bytes a clock).
+// Queries are copied four neighbouring lanes to 64 bytes: lanes in the order of the operand images, neighbours in different rows, keep a CU's
+// vector-memory path busy four times as long (16 against 60 bytes a clock, one workgroup alone; stores the same).
+// Measured and not kept: the three groups a third of a round apart, each handing over while the others walk tiles (302 keys 243 against
+// 237, one key tile 160 / 140: every step lasts as long as its slowest wave), and staggered CUs (1 to 2 %, as much as the stagger costs).
+constexpr int kRelayWaves = 12, kRelayGroups = 3;
+
+// The lane's number, made where it is used: kept from round to round, what is made of it does not fit the registers.
+__device__ __forceinline__ int lane_here() {
+  int l;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+  return l;
+}
+
+// `factor` times the value that lane N of this lane's row of 16 holds.  (The DPP operand must not come from the two vector instructions
+// before this one: the weights this is used for are loaded long before.)
+template <int N>
+__device__ __forceinline__ float times_row_lane(float x, float factor) {
+  float y;
+  asm("v_mul_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "=v"(y) : "v"(x), "v"(factor), "n"(N));
+  return y;
+}
+
+template <bool ROPE>
+__global__ __launch_bounds__(64 * kRelayWaves, 1) void attn_fwd_relay_kernel(FwdParams p) {
+  constexpr int kTile = kKTileBytes + kVTileBytes;
+  __shared__ __attribute__((aligned(1024))) char ring[2 * kTile];
+  __shared__ __attribute__((aligned(1024))) char rows[kRelayWaves * kQBlkBytes];   // every wave's next 32 queries
+  static_assert(sizeof(ring) + sizeof(rows) <= 163840, "all of a CU's LDS");
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int grp = wave / kShortWaves, wq = wave & (kShortWaves - 1);
+  char* own = rows + wave * kQBlkBytes;
+  const int per_head = units_per_head(p.Sq, kShortWaves), total = p.sec_units[0];
+  // a contiguous run of (batch, head, 128 queries) per XCD and workgroup
+  const int wgs = gridDim.x, rank = (blockIdx.x & 7) * (wgs >> 3) + (blockIdx.x >> 3);
+  int at = (int)((int64_t)rank * total / wgs);
+  const int end = (int)((int64_t)(rank + 1) * total / wgs);
+  unsigned long long third;                              // lanes of a tile's third copy: it is 32 KiB, for twelve waves
+  asm volatile("s_cmp_lt_i32 %1, %2\n\ts_cselect_b64 %0, -1, 0" : "=s"(third) : "s"(wave), "n"(kTile / 1024 - 2 * kRelayWaves) : "scc");
+  const unsigned rows_lds = (unsigned)(size_t)(__attribute__((address_space(3))) char*)own;
+  const unsigned ring_lds = (unsigned)(size_t)(__attribute__((address_space(3))) char*)ring;
+
+  // the norm's weights: lane (c, g) has the elements 32*(c/8) + 8*g + c%8 and those 64 further on, of which its row of lanes needs all
+  float weights[2] = {1.f, 1.f}, top_weight = 1.f;
+  if (p.q_norm_w) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) weights[i] = p.q_norm_w[64 * i + 32 * ((lane & 15) >> 3) + 8 * (lane >> 4) + (lane & 7)];
+    top_weight = wave_max(fmaxf(fabsf(weights[0]), fabsf(weights[1]))) * p.c;
+  }
+
+#pragma unroll 1
+  while (at < end) {
+    // a stretch: the units of one (batch, head), three to a round
+    WaveState<false> w;
+    const int bh = at / per_head, first = at - bh * per_head, count = min(end - at, per_head - first);
+    at += count;
+    const int b = bh / p.H, h = bh % p.H;
+    const int sk = p.row_cnt ? uniform_load(p.row_cnt, b) : p.Sk;
+    const int n = (sk + kTileKeys - 1) / kTileKeys, ring_n = max(n, 1);
+    const char* kv = p.kv + (int64_t)bh * p.kv_bh_stride + wave * 1024;
+    const int l0 = lane_here();
+    const float key_norm = n > 0 ? largest_key_norm(p, bh, (sk + 31) / 32, ask_key_norms(p, bh, l0), l0) : 0.f;
+    // a normalised row is no longer than sqrt(D) times the largest weight, whatever the queries (tables may hold what they like: a rotated
+    // one is looked at itself)
+    const bool sure = !ROPE && p.q_norm_w && __all(sqrtf((float)kD) * top_weight * key_norm * 1.01f <= kStaticMaxLimit);
+    int ahead = ring_n - 1, slot = 0;                    // the next tile to copy; slot of the tile in use (a round begins with the last tile)
+    auto copy = [&](int to) {
+      const char* g = kv + (int64_t)ahead * p.kv_tile_stride;
+      char* d = ring + to * kTile + wave * 1024;
+      lds_dma16(g, lane * 16, d);
+      lds_dma16(g + kRelayWaves * 1024, lane * 16, d + kRelayWaves * 1024);
+      asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 exec, %3\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1"
+                   :
+                   : "v"(lane * 16), "s"(g + 2 * kRelayWaves * 1024), "s"(ring_lds + to * kTile + (wave + 2 * kRelayWaves) * 1024), "s"(third)
+                   : "memory", "m0");
+      ahead = ahead + 1 == ring_n ? 0 : ahead + 1;
+    };
+    auto barrier = [&]() {
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    };
+    // 16 of a block's 32 rows of queries into `own`, four neighbouring lanes to the 64 bytes of a row: piece g of row c of image ks comes to
+    // lie at 4c + (g ^ c/4).  Rows past the end are the last one again.
+    auto ask_rows = [&](int q32, int qb) {
+      const int l = lane_here();
+      const int row0 = min(q32 * 32 + 16 * qb, p.Sq - 1);
+      const char* q = (const char*)p.q + ((int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)row0 * p.q_ss) * 2;
+      const unsigned off = (unsigned)min(l >> 2, p.Sq - 1 - row0) * ((unsigned)p.q_ss * 2) + ((l ^ (l >> 4)) & 3) * 16;
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                     :
+                     : "v"(off), "s"(q + 64 * ks), "s"(rows_lds + (4 * qb + ks) * 1024)
+                     : "memory", "m0");
+    };
+    auto q32_of = [&](int unit) { return (first + unit) * kShortWaves + wq; };
+    bool static_max = sure;
+    bf16x8 rows_now[2][4];
+    auto read_rows = [&]() {
+      const int l = lane_here(), c16 = l & 15;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) rows_now[i >> 2][i & 3] = *(const bf16x8*)(own + i * 1024 + c16 * 64 + (((l >> 4) ^ (c16 >> 2)) * 16));
+    };
+    auto prepare = [&](int q32, int q32_next) {
+      const int l = lane_here();
+      const int c16 = l & 15, g4 = l >> 4;
+      float factor[2] = {p.c, p.c};
+      if (p.q_norm_w) {
+#pragma unroll
+        for (int qb = 0; qb < 2; ++qb) {
+          float part[4];
+#pragma unroll
+          for (int ks = 0; ks < 4; ++ks) part[ks] = add_squares(rows_now[qb][ks], 0.f);
+          const float ms = wave_sum_groups((part[0] + part[1]) + (part[2] + part[3])) * (1.0f / kD) + p.q_eps;
+          factor[qb] = ms > 0.f ? rsqrtf(ms) * p.c : 0.f;
+        }
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // nothing is read from `own` any more: the next rows may come
+#pragma unroll
+      for (int qb = 0; qb < 2; ++qb) {
+        float x[32];
+        static_for<32>([&](auto ic) {
+          constexpr int i = decltype(ic)::value;
+          x[i] = times_row_lane<i & 15>(weights[i >> 4], factor[qb]);
+        });
+#pragma unroll
+        for (int i = 0; i < 32; ++i) x[i] *= (float)rows_now[qb][i >> 3][i & 7];
+        if constexpr (ROPE) {
+          const RowTransform tf{nullptr, 0.f, p.q_rope_mode, p.q_cos, p.q_sin};
+          RopeQuarter rope{};
+          load_rope_quarter(rope, tf, min(q32 * 32 + 16 * qb + c16, p.Sq - 1), g4);
+          norm_rope_quarter(x, tf, NormQuarter{}, rope, true, g4);
+        }
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+          bf16x8 q;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) q[j] = (__bf16)x[8 * ks + j];
+          w.qf[qb][ks] = q;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (!ROPE && q32_next >= 0) ask_rows(q32_next, qb);
+      }
+      // (behind the tables: the wait for those is one for everything before them)
+      if (ROPE && q32_next >= 0) ask_rows(q32_next, 0), ask_rows(q32_next, 1);
+      if (!sure) {
+        // the bound of these queries themselves
+        float n2[2][4];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) n2[i >> 2][i & 3] = add_squares(w.qf[i >> 2][i & 3], 0.f);
+        const float top = fmaxf(wave_sum_groups((n2[0][0] + n2[0][1]) + (n2[0][2] + n2[0][3])), wave_sum_groups((n2[1][0] + n2[1][1]) + (n2[1][2] + n2[1][3])));
+        static_max = __all(sqrtf(top) * key_norm * 1.01f <= kStaticMaxLimit);
+      }
+      w.m[0] = w.m[1] = kNoMax;
+    };
+    auto no_keys = [&]() {
+#pragma unroll
+      for (int db = 0; db < 8; ++db)
+#pragma unroll
+        for (int qb = 0; qb < 2; ++qb) w.o[db][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
+      w.l[0] = w.l[1] = 0.f;
+    };
+    // every wave is past the last stretch's ring, and its last copies have landed
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    barrier();
+    if (grp < count) ask_rows(q32_of(grp), 0), ask_rows(q32_of(grp), 1);
+    copy(0);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    barrier();
+    copy(1);
+    // A step: its tile is in its slot for every wave (own copies: vmcnt, the others': barrier), and every wave is past the tile before, whose
+    // slot takes the tile after this one.  The first step's tile, and the copies of the second's, were seen to at the end of the round before.
+    // The step that begins the sums takes the last tile: its keys past the end start from -inf, and O^T and the row sums from nothing.
+#define PKH3_RELAY_STEP(STATIC, FIRST, I)                                                               \
+  {                                                                                                     \
+    if (!(FIRST)) {                                                                                     \
+      if ((I) == 1 && slack) asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)" ::: "memory");               \
+      else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");                                  \
+      barrier();                                                                                        \
+    }                                                                                                   \
+    const char* kbuf = ring + slot * kTile;                                                             \
+    const int l = (FIRST) ? lane_here() : lane;                                                         \
+    qk_tile<false, true, 4, false, FIRST>(w, kbuf, kbuf + kKTileBytes, l, 0, sk - kTileKeys * (n - 1)); \
+    slot ^= 1;                                                                                          \
+    if (!(FIRST)) copy(slot);                                                                           \
+    softmax_pv_tile<false, STATIC, true, false, false, FIRST>(w, kbuf + kKTileBytes, 1.0f, 0, l);       \
+  }
+    auto round_ends = [&]() {
+      // the next round's queries and first tile are there, and its second takes the place of the last tile
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      barrier();
+      copy(slot ^ 1);
+    };
+    bool stored = false;
+    if (grp < count) read_rows();
+#pragma unroll 1
+    for (int unit = grp; unit < count; unit += kRelayGroups) {
+      const bool more = unit + kRelayGroups < count;
+      prepare(q32_of(unit), more ? q32_of(unit + kRelayGroups) : -1);
+      const bool slack = stored && more;                 // eight stores and eight loads were issued after the copies of the second tile
+      if (n == 0) {
+        no_keys();
+      } else if (static_max) {
+        PKH3_RELAY_STEP(true, true, 0)
+#pragma unroll 1
+        for (int i = 1; i < n; ++i) PKH3_RELAY_STEP(true, false, i)
+      } else {
+        PKH3_RELAY_STEP(false, true, 0)
+#pragma unroll 1
+        for (int i = 1; i < n; ++i) PKH3_RELAY_STEP(false, false, i)
+      }
+      PKH3_MFMA_DRAIN(w);
+      round_ends();
+      const int q32 = q32_of(unit);
+      float inv[2];
+#pragma unroll
+      for (int qb = 0; qb < 2; ++qb) {
+        const float lt = wave_sum_groups(w.l[qb]);
+        inv[qb] = lt > 0.f ? 1.0f / lt : 0.f;
+      }
+      read_rows();                                       // (the next unit's, if there is one) before the output takes their place
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      const int l = lane_here();
+      __builtin_amdgcn_sched_barrier(0);
+      store_output(p, w, inv, own, b, h, q32, l);
+      __builtin_amdgcn_sched_barrier(0);
+      stored = q32 * 32 + 32 <= p.Sq;
+    }
+    if (count % kRelayGroups != 0 && grp >= count % kRelayGroups) {
+      // the last round has no unit for this group: it copies and synchronises
+#pragma unroll 1
+      for (int i = 0; i < n; ++i) {
+        if (i > 0) {
+          asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+          barrier();
+        }
+        slot ^= 1;
+        if (i > 0) copy(slot);
+      }
+      round_ends();
+    }
+#undef PKH3_RELAY_STEP
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // no copy may arrive after the workgroup has given its LDS back
+}
+
 static int blocks_of(int workgroups) { return (workgroups + 7) / 8 * 8; }
 
 // How a long dense call ends.  One 12-wave workgroup per CU at a time: the call runs in rounds of `cus` workgroups, and
@@ -1422,6 +1694,19 @@ static int narrow_from(int n32, int n4, int cus) {
   return gain > 0.f ? (int)ceilf(start / gain) : INT_MAX;
 }
 
+// Whether a dense call that attn_form gives to workgroups of 128 or 384 queries runs in the relay form.  At least a round and a third per CU (with
+// fewer the other forms' rounds come out as they do), and as long as a round's start and end weigh: to 40 key tiles.  Below 17, where the
+// short-key form takes over from the long one, the gain is what the start cost: from 8 tiles on, and where the queries' tables are not read
+// besides (each wave waits for them between two rounds).  Other form / relay, us, 24 heads, without rotation, 512, 1,024, 1,536, 2,048 and 3,072
+// keys: 6,000 rows 45.0 / 43.1, 75.3 / 70.9, 115 / 99, 145 / 127, 206 / 183; 9,000 61.0 / 61.0, 105.5 / 101.7, 173 / 143, 219 / 185, 296 / 269; 14,830
+// 91.6 / 93.0, 162.5 / 159.9, 242 / 228, 304 / 296, 429 / 431; 27,000 179 / 169, 299 / 282, 427 / 398, 534 / 517, 759 / 761; 49,640 327 / 300, 543 / 505, 744 /
+// 727, 951 / 933, 1,367 / 1,361; 256 keys from 40.1 / 41.7 to 122 / 111.  With rotation: 14,830 rows 105 / 114, 175 / 178, 262 / 245, 326 / 312; 4,000 rows
+// (three units a CU) 74.7 / 77.2 against 1,536 keys.
+static bool relay_form(const FwdParams& p, int units, int cus) {
+  return !p.fp8 && !p.plan && !p.long_key_kernel && cus >= 8 && units > 4 * cus && p.nKt <= 40 && p.nKt >= (p.q_rope_mode ? kShortMaxTiles + 1 : 8) &&
+         p.q_ss <= (1 << 26);   // (16 rows of queries lie within 32 bits of each other)
+}
+
 template <bool FP8, bool POW2 = false>
 static hipError_t launch_fp(FwdParams p, int cus, hipStream_t st) {
   auto units = [&](int blocks) { return p.B * p.H * units_per_head(p.Sq, blocks); };
@@ -1457,6 +1742,16 @@ static hipError_t launch_fp(FwdParams p, int cus, hipStream_t st) {
     }
     hipLaunchKernelGGL((attn_fwd_kernel<FP8, true, kSparseWaves, POW2>), dim3(blocks_of(wgs)), dim3(64 * kSparseWaves), 0, st, p);
     return hipGetLastError();
+  }
+  if constexpr (!FP8) {
+    if (relay_form(p, units(kShortWaves), cus)) {
+      p.queue_next = nullptr;
+      p.sec_units[0] = units(kShortWaves);
+      const dim3 grid(cus / 8 * 8), block(64 * kRelayWaves);
+      if (p.q_rope_mode) hipLaunchKernelGGL(attn_fwd_relay_kernel<true>, grid, block, 0, st, p);
+      else hipLaunchKernelGGL(attn_fwd_relay_kernel<false>, grid, block, 0, st, p);
+      return hipGetLastError();
+    }
   }
   if (form == kFormShort) {
     p.queue_next = nullptr;

@@ -31,6 +31,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace pkh3 {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
@@ -42,6 +44,15 @@ typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(8))) int i32x8;
 typedef __attribute__((ext_vector_type(4))) int i32x4;
 typedef __attribute__((ext_vector_type(2))) int i32x2;
+
+// f(0) .. f(N - 1), the index as a constant
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<N, I + 1>(f);
+  }
+}
 
 constexpr int kD = 128;            // head dim (fixed)
 constexpr int kTileKeys = 64;      // keys per K/V tile, also the block-sparse tile edge
@@ -187,6 +198,16 @@ __device__ __forceinline__ void norm_rope_quarter(float (&x)[32], const RowTrans
   if (t.norm_w) load_norm_quarter(n, t, g);
   if (t.rope_mode != 0 && valid) load_rope_quarter(r, t, table_row, g);
   norm_rope_quarter(x, t, n, r, valid, g);
+}
+
+// the sum of the squares of eight bf16 values on top of `sum`
+__device__ __forceinline__ float add_squares(const bf16x8& v, float sum) {
+#pragma unroll
+  for (int j = 0; j < 8; j += 2) {
+    const bf16x2 pr = {v[j], v[j + 1]};
+    sum = __builtin_amdgcn_fdot2_f32_bf16(pr, pr, sum, false);
+  }
+  return sum;
 }
 
 // eight values -> eight fp8 e4m3 bytes

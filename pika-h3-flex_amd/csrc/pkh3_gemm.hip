@@ -40,14 +40,6 @@ constexpr int kGemmFeatures = 256;                  // features per workgroup
 constexpr int kGemmRing = 3;                        // ring slots (R; see launch_gemm): one 32-wide k-chunk of weight and activation images each
 constexpr int kGemmWPieces = kGemmFeatures / 16;    // 1 KiB weight images of a chunk
 
-template <int N, int I = 0, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for<N, I + 1>(f);
-  }
-}
-
 // The two halves of a direct-to-LDS copy (see lds_dma16 in pkh3_attn_fwd.hip: wave-uniform base address, per-lane byte
 // offset, tracked by vmcnt): where the next one goes, and the copy.  `lanes`: all or none -- past the last chunk
 // the copies are still issued, so that the waits count the same, but move nothing.

@@ -136,6 +136,62 @@ def test_short_key_form(B, H, Sq, Sk, masked, fp8):
     _run_and_check(B, Sq, Sk, H, seed=Sq + Sk, mask=mask, weight_scale=4.0, bf16_operands=not fp8, fp8=fp8, max_abs=0.35 if fp8 else MAX_ABS)
 
 
+@pytest.mark.parametrize("scale", [1.0, 6.0])
+@pytest.mark.parametrize("B,H,Sq,Sk,rope,valid", [
+    (1, 1030, 70, 449, 0, None),            # a unit a head: every round belongs to another one, one of three groups has work
+    (1, 32, 4229, 500, 0, None),            # whole rounds, some of one and two groups, a unit that holds rows of one wave only
+    (2, 22, 3072, 512, 0, None),            # nothing partial but a head's last round
+    (1, 345, 300, 1025, 1, None), (1, 516, 200, 1088, 2, None),   # 17 tiles and rotation, the last one of one key and whole
+    (3, 44, 1025, 600, 0, (0, 1, 400)),     # masked: no key, one, some
+    (6, 60, 333, 640, 0, (64, 65, 128, 129, 500, 640)),           # one to ten tiles
+])
+def test_relay_form(B, H, Sq, Sk, rope, valid, scale):
+    """Dense calls of more than four 128-query units a CU against 8 to 40 key tiles: a workgroup goes from unit to unit.  At scale 6
+    (the norm weights of the queries) the running maximum; against the oracle with operands rounded as the kernel's are.
+    Strided queries and outputs, the output in the queries' place and as operand images, and no norm at all."""
+    import pika_h3_flex_amd as pk
+    from pika_h3_flex_amd import projections as P
+
+    O = _oracle()
+    assert H * B * ((Sq + 127) // 128) > 4 * torch.cuda.get_device_properties(0).multi_processor_count
+    gen = torch.Generator(device="cuda").manual_seed(Sq + Sk)
+    rows = lambda S, std=1.0: (torch.randn((B, S, H, 128), generator=gen, device="cuda") * std).to(torch.bfloat16)
+    wide = torch.empty((B, Sq, H, 136), dtype=torch.bfloat16, device="cuda")
+    q, k, v = wide[..., :128], rows(Sk), rows(Sk)
+    q.copy_(rows(Sq))
+    w = [1.0 + 0.2 * torch.randn(128, generator=gen, device="cuda") for _ in range(2)]
+    opts = dict(q_norm_weight=w[0] * scale, k_norm_weight=w[1])
+    ref = dict(opts, bf16_operands=scale > 1)
+    if rope:
+        tabs = [O.rope_tables(torch.rand((S, 3), generator=gen, dtype=torch.float64, device="cuda") * 40) for S in (Sq, Sk)]
+        f32 = [tuple(t.float().contiguous() for t in pair) for pair in tabs]
+        opts.update(rope_mode=rope, rope_q=f32[0], rope_k=f32[1])
+        ref.update(rope_mode=rope, rope_q=tabs[0], rope_k=tabs[1])
+    if valid:
+        mask = torch.stack([torch.randperm(Sk, generator=gen, device="cuda") < n for n in valid])
+        opts.update(key_mask=mask)
+        ref.update(key_mask=mask)
+    want = torch.cat([O.reference_layer(q[:, i:i + 256], k, v, **{**ref, **({"rope_q": tuple(t[i:i + 256] for t in tabs[0])} if rope else {})})
+                      for i in range(0, Sq, 256)], dim=1)
+    out = pk.attention(q, k, v, **opts)
+    err, cos = O.max_abs_and_cosine(out, want)
+    print(f"B={B} H={H} {Sq} x {Sk} rope={rope} valid={valid} scale={scale}: max_abs={err:.3e} cos={cos:.7f}", flush=True)
+    assert err <= MAX_ABS and cos >= MIN_COS
+    if B == 1 and H <= 32:
+        img = torch.full((P.packed_bytes(Sq, H * 128),), 0xAB, dtype=torch.uint8, device="cuda")
+        pk.attention(q, k, v, out=img, out_images=True, **opts)
+        live = ((Sq + 31) // 32) * 2 * (H * 128 // 32) * 1024
+        assert torch.equal(img[:live], P.pack_rows(out.view(Sq, H * 128))[:live]) and bool((img[live:] == 0xAB).all())
+    assert torch.equal(pk.attention(q, k, v, out=q, **opts), out)
+    if scale == 1.0 and not rope:
+        del opts["q_norm_weight"], ref["q_norm_weight"]
+        ref["bf16_operands"] = True
+        q.copy_(rows(Sq, 0.5))
+        want = torch.cat([O.reference_layer(q[:, i:i + 256], k, v, **ref) for i in range(0, Sq, 256)], dim=1)
+        err, cos = O.max_abs_and_cosine(pk.attention(q, k, v, **opts), want)
+        assert err <= MAX_ABS and cos >= MIN_COS
+
+
 @pytest.mark.parametrize("valid", [0, 1, 33, 64, 230])
 def test_few_query_blocks_masked(valid):
     """Fewer valid keys than the waves of a workgroup have shares for, none among them, and running-maximum softmax with
