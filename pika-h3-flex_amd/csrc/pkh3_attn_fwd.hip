@@ -131,19 +131,31 @@ struct WaveState {
   int qe;                               // fp8 with power-of-two scales: exponent byte (E8M0) of the Q block's scale
 };
 
-// One 16-row block of raw queries with its rotation tables, as a lane group of norm_rope_quarter holds them.  Rows past the end read
-// row 0, whose place is in bounds.
+// One 16-row block of queries with its rotation tables, as they lie in memory.  Rows past the end are the last one again: what is made of
+// them is not stored, and neither the largest magnitude of their 64 queries nor any bound is another for it.
 struct QRows {
-  bf16x8 raw[4];
-  RopeQuarter rope;
+  Rows16 q, cos, sin;
 };
 template <typename Params>
-__device__ __forceinline__ void load_q_rows(QRows& r, const Params& p, const RowTransform& tf, int b, int h, int qrow, int g) {
-  const int src = qrow < p.Sq ? qrow : 0;
-  const __bf16* row = (const __bf16*)p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)src * p.q_ss + 8 * g;
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks) r.raw[ks] = *(const bf16x8*)(row + 32 * ks);
-  if (p.q_rope_mode != 0) load_rope_quarter(r.rope, tf, src, g);
+__device__ __forceinline__ void ask_q_rows(QRows& r, const Params& p, int b, int h, int first, int lane) {
+  ask_rows16(r.q, (const char*)p.q + ((int64_t)b * p.q_sb + (int64_t)h * p.q_sh) * 2, p.q_ss * 2, first, p.Sq - 1, lane);
+  if (p.q_rope_mode != 0) {
+    ask_rows16(r.cos, (const char*)p.q_cos, kD / 2 * sizeof(float), first, p.Sq - 1, lane);
+    ask_rows16(r.sin, (const char*)p.q_sin, kD / 2 * sizeof(float), first, p.Sq - 1, lane);
+  }
+}
+// RMSNorm, rotation and `factor` of such a block, through 4 KiB of LDS of the wave's own: lane (c, g) gets its 32 elements of row c
+template <typename Params>
+__device__ __forceinline__ void q_rows_ready(float (&x)[32], const QRows& r, const Params& p, const NormLanes& norm, float factor, char* lds, int lane) {
+  bf16x8 raw[4];
+  turn_elements(r.q, raw, lds, lane);
+  RopeQuarter rope;
+  if (p.q_rope_mode != 0) {
+    turn_table(r.cos, rope.c, p.q_rope_mode, lds, lane);
+    turn_table(r.sin, rope.s, p.q_rope_mode, lds, lane);
+  }
+  norm_row(x, raw, p.q_norm_w != nullptr, p.q_eps, norm, factor);
+  rope_row(x, p.q_rope_mode, rope, lane >> 4);
 }
 
 // Consecutive MFMAs share an operand where they can: the two query blocks of an image come in turn (0 1, 1 0, 0 1 ..), so that only
@@ -564,6 +576,15 @@ constexpr int kMergeBytes = kPartialBytes;  // one wave's partial result in fp32
 // workgroups of `blocks` 32-query blocks a (batch, head) needs
 __host__ __device__ constexpr int units_per_head(int Sq, int blocks) { return ((Sq + 31) / 32 + blocks - 1) / blocks; }
 
+// Where the waves turn their queries around before the loops: behind the tiles that are on their way by then, all of the ring but its last
+// slot, which is not written before every wave has its queries.
+constexpr int kTurnBytes = 16 * kD * 2;
+template <bool FP8, bool SPARSE, int WAVES, bool PIPE = false>
+constexpr int fwd_turn_offset() {
+  constexpr int kTileBytes = (FP8 ? kK8TileBytes : kKTileBytes) + kVTileBytes;
+  return !SPARSE && WAVES == kShortWaves ? ((PIPE ? kPipeRing : kRing) - 1) * (kTileBytes / 2) : (kRing - 1) * kTileBytes;
+}
+
 // bytes of LDS a form of the kernel needs
 template <bool FP8, bool SPARSE, int WAVES, bool PIPE = false>
 constexpr int fwd_lds_bytes() {
@@ -576,7 +597,9 @@ constexpr int fwd_lds_bytes() {
   constexpr int kRingBytes = HALFMODE ? (PIPE ? kPipeRing : kRing) * kHalfBytes
                              : (kPhase2Bytes > kRing * kTileBytes ? kPhase2Bytes : kRing * kTileBytes);
   constexpr int kAfterBytes = WAVES * kStageBytes;  // LDS use after the loops
-  return kRingBytes > kAfterBytes ? kRingBytes : kAfterBytes;
+  constexpr int kBeforeBytes = fwd_turn_offset<FP8, SPARSE, WAVES, PIPE>() + WAVES * kTurnBytes;   // ... and before them
+  constexpr int kBytes = kRingBytes > kAfterBytes ? kRingBytes : kAfterBytes;
+  return kBytes > kBeforeBytes ? kBytes : kBeforeBytes;
 }
 
 // POW2 (fp8 only): power-of-two block scales, applied by the scaled MFMA; softmax_scale * log2(e) rides in Q' before
@@ -594,6 +617,7 @@ __device__ __forceinline__ int attn_fwd_body(const Params& p, int blk, int unit0
   constexpr bool LEAN = !SPARSE;                        // dense long-key form: three waves per SIMD, lean read-ahead
   constexpr int kAhead = kRing - 1;                     // tiles in flight ahead of the one being used
   constexpr bool HALFMODE = SHORT;                      // ring of 32-key half tiles
+  constexpr bool kAskFirst = SPARSE || PIPE;            // (their registers hold both blocks' rows and tables)
   constexpr bool PARTS = !SPARSE && !SHORT;             // the long dense form: the key tiles may be shared out (`parts`)
   constexpr int kKBytes = FP8 ? kK8TileBytes : kKTileBytes;
   constexpr int kTileBytes = kKBytes + kVTileBytes;
@@ -625,16 +649,17 @@ __device__ __forceinline__ int attn_fwd_body(const Params& p, int blk, int unit0
   const int b = bh / p.H, h = bh % p.H;
 
   QRows q_rows[2];
-  NormQuarter q_norm;
-  const RowTransform q_tf{p.q_norm_w, p.q_eps, p.q_rope_mode, p.q_cos, p.q_sin};
+  NormLanes q_norm;
   const f32x4 first_norms = ask_key_norms(p, bh, lane);
-  auto load_q = [&](int qb) { load_q_rows(q_rows[qb], p, q_tf, b, h, q32 * 32 + 16 * qb + (lane & 15), lane >> 4); };
+  int q_lane = lane;                                      // (places in LDS that the output uses as well are not kept until then)
+  asm volatile("" : "+v"(q_lane));
+  auto load_q = [&](int qb) { ask_q_rows(q_rows[qb], p, b, h, q32 * 32 + 16 * qb, q_lane); };
   // The block-sparse form has one workgroup per CU and nothing to run beside this: rows, tables and weights are asked for before
   // anything else of the unit is known, so that they cost one trip to memory between them and the plan's look-ups and the first
-  // key copies run beside it (14,907 rows, fp8: the call 691 -> 679 us; 48,360, bf16: 6,880 -> 6,800).  Where other workgroups or
-  // a third wave per SIMD run beside it, it gave nothing.
-  if constexpr (SPARSE) load_q(0), load_q(1);
-  if (p.q_norm_w) load_norm_quarter(q_norm, q_tf, lane >> 4);
+  // key copies run beside it (14,907 rows, fp8: the call 691 -> 679 us; 48,360, bf16: 6,880 -> 6,800).  So does the pipelined short-key form.
+  // Where a third wave per SIMD runs beside it, it gave nothing.
+  if constexpr (kAskFirst) load_q(0), load_q(1);
+  load_norm_lanes(q_norm, p.q_norm_w, lane);
 
   const int sk = p.row_cnt ? uniform_load(p.row_cnt, b) : p.Sk;
   const int nkt = (sk + kTileKeys - 1) / kTileKeys;
@@ -697,40 +722,32 @@ __device__ __forceinline__ int attn_fwd_body(const Params& p, int blk, int unit0
     if (t_end > t_begin + 1) dma(entry(t_begin + 1), 1);
   }
   // Q, fused with QK-RMSNorm, rotation and (fp8) quantisation, in the layout of the MFMA B images themselves:
-  // lane (c, g) has read, for each of the wave's two 16-query blocks qb, the 32 elements d = 32*ks + 8*g + j of query
-  // row q32*32 + 16*qb + c (four lanes per row, norm_rope_quarter), so the operand images are formed in the lane
+  // lane (c, g) gets, for each of the wave's two 16-query blocks qb, the 32 elements d = 32*ks + 8*g + j of query
+  // row q32*32 + 16*qb + c (four lanes per row), so the operand images are formed in the lane
   // that uses them and Q' never exists in memory.
   float qscale = 1.0f;
-  float qn2 = 0.f;  // largest squared norm of this lane's Q' rows (bf16: before the rounding; fp8: dequantised)
+  float qn2 = 0.f;  // largest squared norm of this lane's Q' rows as the MFMAs take them
   {
     float x[2][32];
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
-      const bool valid = q32 * 32 + 16 * qb + (lane & 15) < p.Sq;
-      if constexpr (!SPARSE) load_q(qb);
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) x[qb][ks * 8 + j] = valid ? (float)q_rows[qb].raw[ks][j] : 0.f;
-      norm_rope_quarter(x[qb], q_tf, q_norm, q_rows[qb].rope, valid, lane >> 4);
+      if constexpr (!kAskFirst) load_q(qb);
+      // softmax_scale * log2(e) rides in Q' (bf16, and fp8 with power-of-two scales), so S^T comes out of the MFMAs in the log2 domain
+      q_rows_ready(x[qb], q_rows[qb], p, q_norm, FP8 && !POW2 ? 1.0f : p.c, lds_raw + fwd_turn_offset<FP8, SPARSE, WAVES, PIPE>() + wave * kTurnBytes, q_lane);
     }
     if constexpr (!FP8) {
 #pragma unroll
       for (int qb = 0; qb < 2; ++qb) {
-        float n2 = 0.f;
+        float n2[4];
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
           bf16x8 t;
 #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            // softmax_scale * log2(e) rides in Q', so S^T comes out of the MFMAs in the log2 domain
-            const float xs = x[qb][ks * 8 + j] * p.c;
-            t[j] = (__bf16)xs;
-            n2 = fmaf(xs, xs, n2);   // the norm before the rounding: the bound below carries the margin for it
-          }
+          for (int j = 0; j < 8; ++j) t[j] = (__bf16)x[qb][ks * 8 + j];
           w.qf[qb][ks] = t;
+          n2[ks] = add_squares(t, 0.f);
         }
-        qn2 = fmaxf(qn2, wave_sum_groups(n2));
+        qn2 = fmaxf(qn2, wave_sum_groups((n2[0] + n2[1]) + (n2[2] + n2[3])));
       }
     } else {
       // one absmax scale per 64-query block = this wave and its neighbour (wave ^ 1)
@@ -739,11 +756,7 @@ __device__ __forceinline__ int attn_fwd_body(const Params& p, int blk, int unit0
 #pragma unroll
       for (int qb = 0; qb < 2; ++qb)
 #pragma unroll
-        for (int i = 0; i < 32; ++i) {
-          // power-of-two scales: softmax_scale * log2(e) goes into Q' before the quantisation, as in the bf16 form
-          if constexpr (POW2) x[qb][i] *= p.c;
-          amax = fmaxf(amax, fabsf(x[qb][i]));
-        }
+        for (int i = 0; i < 32; ++i) amax = fmaxf(amax, fabsf(x[qb][i]));
       amax = wave_max(amax);
       if (lane == 0) q_amax[wave] = amax;
       __syncthreads();
@@ -787,8 +800,7 @@ __device__ __forceinline__ int attn_fwd_body(const Params& p, int blk, int unit0
   // the row sums and O^T (at most 2^bound * keys * |v|), so no running max is needed at all.
   bool static_max = false;
   if (HALFMODE ? n_half > 0 : nt > 0) {
-    // margins: Q' and K' are rounded to bf16 (relative step 2^-9 each; fp8: K' to e4m3, relative step 2^-4) after
-    // their norms were taken
+    // margins: K' is rounded to bf16 (relative step 2^-9; fp8: to e4m3, relative step 2^-4) after its norms were taken
     const float bound = sqrtf(qn2) * largest_key_norm(p, bh, n_half, first_norms, lane) * (FP8 ? (POW2 ? 1.08f : p.c * 1.08f) : 1.01f);
     static_max = __all(bound <= kStaticMaxLimit);
   }
@@ -1201,29 +1213,18 @@ __global__ __launch_bounds__(64 * kNarrowWaves, 2) void attn_fwd_narrow_kernel(F
     for (int j = 0; j < (FP8 ? 4 : 8); ++j) kf[j] = *(const i32x4*)(k + (j * 64 + lane) * 16);
   }
   const f32x4 first_norms = ask_key_norms(p, bh, lane);
-  // The queries, a 16-row block per wave for all waves (layout and arithmetic of attn_fwd_body's Q load).  fp8: one scale
+  // The queries, a 16-row block per wave for all waves (as in attn_fwd_body).  fp8: one scale
   // per 64 queries, so four waves look at the four blocks this block's 64 queries consist of, and two of them are it.
   const int mine = FP8 ? wave - 2 * (q32 & 1) : wave;      // which of the two 16-query blocks, if 0 or 1
   const bool prepares = (unsigned)mine < 2u;
   float x[32];
   float qscale = 1.0f;
   if (FP8 || prepares) {
-    const RowTransform tf{p.q_norm_w, p.q_eps, p.q_rope_mode, p.q_cos, p.q_sin};
-    const int qrow = q32 * 32 + 16 * mine + c16;
-    const bool valid = qrow < p.Sq;
-    const __bf16* row = (const __bf16*)p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)(valid ? qrow : 0) * p.q_ss + 8 * g4;
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      const bf16x8 raw = *(const bf16x8*)(row + 32 * ks);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) x[ks * 8 + j] = valid ? (float)raw[j] : 0.f;
-    }
-    norm_rope_quarter(x, tf, qrow, valid, g4);
-    // softmax_scale * log2(e) rides in Q' (bf16, and fp8 with power-of-two scales)
-    if constexpr (!FP8 || POW2) {
-#pragma unroll
-      for (int i = 0; i < 32; ++i) x[i] *= p.c;
-    }
+    QRows in;
+    NormLanes norm;
+    ask_q_rows(in, p, b, h, q32 * 32 + 16 * mine, lane);
+    load_norm_lanes(norm, p.q_norm_w, lane);
+    q_rows_ready(x, in, p, norm, FP8 && !POW2 ? 1.0f : p.c, part + wave * kSlot, lane);
     if constexpr (FP8) {
       float amax = 0.f;
 #pragma unroll
@@ -1244,10 +1245,8 @@ __global__ __launch_bounds__(64 * kNarrowWaves, 2) void attn_fwd_narrow_kernel(F
       for (int ks = 0; ks < 4; ++ks) {
         bf16x8 t;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          t[j] = (__bf16)x[ks * 8 + j];
-          n2 = fmaf(x[ks * 8 + j], x[ks * 8 + j], n2);
-        }
+        for (int j = 0; j < 8; ++j) t[j] = (__bf16)x[ks * 8 + j];
+        n2 = add_squares(t, n2);
         *(bf16x8*)(rows + ((mine * 4 + ks) * 64 + lane) * 16) = t;
       }
     } else {
@@ -1381,15 +1380,6 @@ __device__ __forceinline__ int lane_here() {
   return l;
 }
 
-// `factor` times the value that lane N of this lane's row of 16 holds.  (The DPP operand must not come from the two vector instructions
-// before this one: the weights this is used for are loaded long before.)
-template <int N>
-__device__ __forceinline__ float times_row_lane(float x, float factor) {
-  float y;
-  asm("v_mul_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "=v"(y) : "v"(x), "v"(factor), "n"(N));
-  return y;
-}
-
 template <bool ROPE>
 __global__ __launch_bounds__(64 * kRelayWaves, 1) void attn_fwd_relay_kernel(FwdParams p) {
   constexpr int kTile = kKTileBytes + kVTileBytes;
@@ -1410,13 +1400,9 @@ __global__ __launch_bounds__(64 * kRelayWaves, 1) void attn_fwd_relay_kernel(Fwd
   const unsigned rows_lds = (unsigned)(size_t)(__attribute__((address_space(3))) char*)own;
   const unsigned ring_lds = (unsigned)(size_t)(__attribute__((address_space(3))) char*)ring;
 
-  // the norm's weights: lane (c, g) has the elements 32*(c/8) + 8*g + c%8 and those 64 further on, of which its row of lanes needs all
-  float weights[2] = {1.f, 1.f}, top_weight = 1.f;
-  if (p.q_norm_w) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) weights[i] = p.q_norm_w[64 * i + 32 * ((lane & 15) >> 3) + 8 * (lane >> 4) + (lane & 7)];
-    top_weight = wave_max(fmaxf(fabsf(weights[0]), fabsf(weights[1]))) * p.c;
-  }
+  NormLanes norm;
+  load_norm_lanes(norm, p.q_norm_w, lane);
+  const float top_weight = wave_max(fmaxf(fabsf(norm.w[0]), fabsf(norm.w[1]))) * p.c;
 
 #pragma unroll 1
   while (at < end) {
@@ -1473,33 +1459,19 @@ __global__ __launch_bounds__(64 * kRelayWaves, 1) void attn_fwd_relay_kernel(Fwd
     };
     auto prepare = [&](int q32, int q32_next) {
       const int l = lane_here();
-      const int c16 = l & 15, g4 = l >> 4;
-      float factor[2] = {p.c, p.c};
-      if (p.q_norm_w) {
-#pragma unroll
-        for (int qb = 0; qb < 2; ++qb) {
-          float part[4];
-#pragma unroll
-          for (int ks = 0; ks < 4; ++ks) part[ks] = add_squares(rows_now[qb][ks], 0.f);
-          const float ms = wave_sum_groups((part[0] + part[1]) + (part[2] + part[3])) * (1.0f / kD) + p.q_eps;
-          factor[qb] = ms > 0.f ? rsqrtf(ms) * p.c : 0.f;
-        }
-      }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // nothing is read from `own` any more: the next rows may come
 #pragma unroll
       for (int qb = 0; qb < 2; ++qb) {
         float x[32];
-        static_for<32>([&](auto ic) {
-          constexpr int i = decltype(ic)::value;
-          x[i] = times_row_lane<i & 15>(weights[i >> 4], factor[qb]);
-        });
-#pragma unroll
-        for (int i = 0; i < 32; ++i) x[i] *= (float)rows_now[qb][i >> 3][i & 7];
+        norm_row(x, rows_now[qb], p.q_norm_w != nullptr, p.q_eps, norm, p.c);
         if constexpr (ROPE) {
-          const RowTransform tf{nullptr, 0.f, p.q_rope_mode, p.q_cos, p.q_sin};
-          RopeQuarter rope{};
-          load_rope_quarter(rope, tf, min(q32 * 32 + 16 * qb + c16, p.Sq - 1), g4);
-          norm_rope_quarter(x, tf, NormQuarter{}, rope, true, g4);
+          Rows16 cos, sin;
+          RopeQuarter rope;
+          ask_rows16(cos, (const char*)p.q_cos, kD / 2 * sizeof(float), q32 * 32 + 16 * qb, p.Sq - 1, l);
+          ask_rows16(sin, (const char*)p.q_sin, kD / 2 * sizeof(float), q32 * 32 + 16 * qb, p.Sq - 1, l);
+          turn_table(cos, rope.c, p.q_rope_mode, own, l);
+          turn_table(sin, rope.s, p.q_rope_mode, own, l);
+          rope_row(x, p.q_rope_mode, rope, l >> 4);
         }
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
@@ -1511,7 +1483,8 @@ __global__ __launch_bounds__(64 * kRelayWaves, 1) void attn_fwd_relay_kernel(Fwd
         __builtin_amdgcn_sched_barrier(0);
         if (!ROPE && q32_next >= 0) ask_rows(q32_next, qb);
       }
-      // (behind the tables: the wait for those is one for everything before them)
+      // (behind the tables: the wait for those is one for everything before them, and they go through `own`)
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       if (ROPE && q32_next >= 0) ask_rows(q32_next, 0), ask_rows(q32_next, 1);
       if (!sure) {
         // the bound of these queries themselves

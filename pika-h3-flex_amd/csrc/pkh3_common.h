@@ -192,14 +192,6 @@ __device__ __forceinline__ void norm_rope_quarter(float (&x)[32], const RowTrans
   }
 }
 
-__device__ __forceinline__ void norm_rope_quarter(float (&x)[32], const RowTransform& t, int64_t table_row, bool valid, int g) {
-  NormQuarter n;
-  RopeQuarter r;
-  if (t.norm_w) load_norm_quarter(n, t, g);
-  if (t.rope_mode != 0 && valid) load_rope_quarter(r, t, table_row, g);
-  norm_rope_quarter(x, t, n, r, valid, g);
-}
-
 // the sum of the squares of eight bf16 values on top of `sum`
 __device__ __forceinline__ float add_squares(const bf16x8& v, float sum) {
 #pragma unroll
@@ -208,6 +200,90 @@ __device__ __forceinline__ float add_squares(const bf16x8& v, float sum) {
     sum = __builtin_amdgcn_fdot2_f32_bf16(pr, pr, sum, false);
   }
   return sum;
+}
+
+// ---- rows on their way from memory to the layout above ----
+// Sixteen rows of 256 bytes (a block's queries or keys of a head, or its cosines, or its sines).  Loaded in the layout above, neighbouring lanes lie
+// in different rows, which keeps the CU's vector-memory path busy four times as long as whole rows do (one workgroup alone: 16
+// against 60 bytes a clock).  So they are asked for as they lie in memory, lane l the 16-byte chunk l % 16 of row 4*i + l / 16, and
+// turned around in 4 KiB of LDS of the wave's own, chunks XOR-swizzled by the row.  The start of a short-key workgroup with rotation took
+// 30 % of its 20 us, most of it these loads: 3 x 8 heads x 777 rows (the call) 32.7 -> 31.4 us; block-sparse calls, whose workgroups begin
+// anew every 70 to 350 us, 14,907 rows 658 -> 648, 4 x 24 heads x 1,000 rows with rotation 1 to 3 %.
+struct Rows16 {
+  i32x4 v[4];
+};
+// `row`: of each lane's four rows (base: the first byte of row 0 of the table or head); rows past `last` are that one again
+__device__ __forceinline__ void ask_rows16(Rows16& r, const char* base, int64_t row_bytes, int first, int last, int lane) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r.v[i] = *(const i32x4*)(base + (int64_t)min(first + 4 * i + (lane >> 4), last) * row_bytes + (lane & 15) * 16);
+}
+// chunk(j): which chunk of its row c = l % 16 the lane wants as its j-th
+template <class F>
+__device__ __forceinline__ void turn_rows16(const Rows16& r, i32x4 (&out)[4], char* lds, int lane, F&& chunk) {
+  const int c = lane & 15;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = 4 * i + (lane >> 4);
+    *(i32x4*)(lds + row * 256 + ((c ^ row) * 16)) = r.v[i];
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) out[j] = *(const i32x4*)(lds + c * 256 + ((chunk(j) ^ c) * 16));
+}
+// a row's elements, as norm_rope_row takes them
+__device__ __forceinline__ void turn_elements(const Rows16& r, bf16x8 (&raw)[4], char* lds, int lane) {
+  i32x4 out[4];
+  turn_rows16(r, out, lds, lane, [&](int j) { return 4 * j + (lane >> 4); });
+#pragma unroll
+  for (int j = 0; j < 4; ++j) raw[j] = __builtin_bit_cast(bf16x8, out[j]);
+}
+// a row's cosines or sines, as RopeQuarter holds them
+__device__ __forceinline__ void turn_table(const Rows16& r, f32x4 (&table)[4], int rope_mode, char* lds, int lane) {
+  const int g = lane >> 4;
+  i32x4 out[4];
+  turn_rows16(r, out, lds, lane, [&](int j) { return rope_mode == 1 ? 4 * j + g : 8 * (j >> 1) + 2 * g + (j & 1); });
+#pragma unroll
+  for (int j = 0; j < 4; ++j) table[j] = __builtin_bit_cast(f32x4, out[j]);
+}
+
+// The RMSNorm weights in two registers: lane (c, g) has those of the elements 32*(c/8) + 8*g + c%8 and 64 further on, of which its row of
+// 16 lanes needs all; the multiplication takes them from there.
+struct NormLanes {
+  float w[2];
+};
+__device__ __forceinline__ void load_norm_lanes(NormLanes& n, const float* norm_w, int lane) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i) n.w[i] = norm_w ? norm_w[64 * i + 32 * ((lane & 15) >> 3) + 8 * (lane >> 4) + (lane & 7)] : 1.0f;
+}
+// `factor` times the value that lane N of this lane's row of 16 holds.  (The weights must not come from the two vector instructions before
+// this one; they are loaded long before.)
+template <int N>
+__device__ __forceinline__ float times_row_lane(float x, float factor) {
+  float y;
+  asm("v_mul_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "=v"(y) : "v"(x), "v"(factor), "n"(N));
+  return y;
+}
+
+// RMSNorm (if `normed`) and `factor` of this lane's 32 elements of a row as they are in memory: the squares are summed up two at a
+// time before the elements are unpacked, and the factor (the softmax scale and log2 e of the queries) rides with the norm's.
+__device__ __forceinline__ void norm_row(float (&x)[32], const bf16x8 (&raw)[4], bool normed, float eps, const NormLanes& n, float factor) {
+  if (normed) {
+    float part[4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) part[ks] = add_squares(raw[ks], 0.f);
+    // an all-zero row with eps == 0 stays all zero instead of 0 * inf
+    const float ms = wave_sum_groups((part[0] + part[1]) + (part[2] + part[3])) * (1.0f / kD) + eps;
+    factor *= ms > 0.f ? rsqrtf(ms) : 0.f;
+  }
+  static_for<32>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    x[i] = times_row_lane<i & 15>(n.w[i >> 4], factor);
+  });
+#pragma unroll
+  for (int i = 0; i < 32; ++i) x[i] *= (float)raw[i >> 3][i & 7];
+}
+// the rotation alone
+__device__ __forceinline__ void rope_row(float (&x)[32], int rope_mode, const RopeQuarter& r, int g) {
+  norm_rope_quarter(x, RowTransform{nullptr, 0.f, rope_mode, nullptr, nullptr}, NormQuarter{}, r, true, g);
 }
 
 // eight values -> eight fp8 e4m3 bytes
