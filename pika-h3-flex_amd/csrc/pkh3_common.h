@@ -212,10 +212,15 @@ __device__ __forceinline__ float add_squares(const bf16x8& v, float sum) {
 struct Rows16 {
   i32x4 v[4];
 };
-// `row`: of each lane's four rows (base: the first byte of row 0 of the table or head); rows past `last` are that one again
+// base: the first byte of row 0 of the table or head; rows past `last` are that one again
 __device__ __forceinline__ void ask_rows16(Rows16& r, const char* base, int64_t row_bytes, int first, int last, int lane) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) r.v[i] = *(const i32x4*)(base + (int64_t)min(first + 4 * i + (lane >> 4), last) * row_bytes + (lane & 15) * 16);
+}
+// the rows src[i] of this lane
+__device__ __forceinline__ void ask_rows16(Rows16& r, const char* base, int64_t row_bytes, const int (&src)[4], int lane) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r.v[i] = *(const i32x4*)(base + (int64_t)src[i] * row_bytes + (lane & 15) * 16);
 }
 // chunk(j): which chunk of its row c = l % 16 the lane wants as its j-th
 template <class F>

@@ -63,40 +63,49 @@ static hipError_t launch_mask_compact(const uint8_t* mask, int B, int Sk, int* i
 // Against a K and a V launch of one wave per tile and head: 48,360 rows x 24 heads 293 -> 241 us (4.9 TB/s), fp8 285 -> 215;
 // 15,342 rows 127 -> 85 us.
 
-// K: lane (c = l%16, g = l/16) of wave kb holds the 32 elements d = 32*ks + 8*g + j of row 16*kb + c -- its own 16 bytes
-// of the block's four K images, so every load instruction reads 64 contiguous bytes of 16 rows, norm and rotation need
-// two cross-lane exchanges (the sum of squares), and every store instruction writes one whole 1 KiB image.
+// K: lane (c = l%16, g = l/16) of wave kb gets the 32 elements d = 32*ks + 8*g + j of row 16*kb + c -- its own 16 bytes
+// of the block's four K images, so norm and rotation need two cross-lane exchanges (the sum of squares), and every store
+// instruction writes one whole 1 KiB image.  Rows and tables are asked for as they lie in memory (four whole rows a load) and
+// turned around in 4 KiB of LDS a wave: asked for in the order of the images, 64 B of 16 rows a load, the CU's load path gives
+// a quarter of its rate.  That against this: 48,360 rows x 24 heads 218 -> 209 us, fp8 204 -> 196; 15,342 rows 70 -> 64.5;
+// 3 x 8 heads x 777 rows with a mask (with the shorter look through it below) 12.3 -> 8.6; 2 x 4 heads x 200 rows 5.0 -> 4.6.
 template <bool FP8>
 __device__ __forceinline__ void k_tile(const QkPrologueParams& p, int tile, int b, int h0, int n_heads, int rows, const int* source,
-                                       unsigned* s_norm, unsigned* s_amax) {
+                                       unsigned* s_norm, unsigned* s_amax, char* turn) {
   const int lane = threadIdx.x & 63, kb = threadIdx.x >> 6;
   const int c = lane & 15, g = lane >> 4;
-  const RowTransform tf{p.norm_w, p.eps, p.rope_mode, p.cos_t, p.sin_t};
-  const int row = tile * 64 + kb * 16 + c;
-  const bool valid = row < rows;
-  int src = 0;
-  if (valid) src = source ? source[row - tile * 64] : row;
-  const __bf16* xr = (const __bf16*)p.x + (int64_t)b * p.sb + (int64_t)src * p.ss + (int64_t)h0 * p.sh + 8 * g;
-  auto fetch = [&](bf16x8 (&raw)[4], int hi) {
+  const bool valid = tile * 64 + kb * 16 + c < rows;
+  int src[4];                                            // rows of the block as they are asked for
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) raw[ks] = *(const bf16x8*)(xr + (int64_t)hi * p.sh + 32 * ks);
-  };
-  bf16x8 next[4];
-  fetch(next, 0);
-  NormQuarter norm;
-  if (p.norm_w) load_norm_quarter(norm, tf, g);
+  for (int i = 0; i < 4; ++i) {
+    const int in_tile = kb * 16 + 4 * i + g;
+    src[i] = tile * 64 + in_tile < rows ? (source ? source[in_tile] : tile * 64 + in_tile) : 0;
+  }
+  const char* xr = (const char*)p.x + ((int64_t)b * p.sb + (int64_t)h0 * p.sh) * 2;
+  Rows16 next, cos, sin;
+  ask_rows16(next, xr, p.ss * 2, src, lane);
+  NormLanes norm;
+  load_norm_lanes(norm, p.norm_w, lane);
   RopeQuarter rope;
-  if (p.rope_mode != 0 && valid) load_rope_quarter(rope, tf, src, g);
+  if (p.rope_mode != 0) {
+    ask_rows16(cos, (const char*)p.cos_t, kD / 2 * sizeof(float), src, lane);
+    ask_rows16(sin, (const char*)p.sin_t, kD / 2 * sizeof(float), src, lane);
+    turn_table(cos, rope.c, p.rope_mode, turn, lane);
+    turn_table(sin, rope.s, p.rope_mode, turn, lane);
+  }
   char* ob = p.out + (int64_t)(b * p.H + h0) * p.out_bh_stride + (int64_t)tile * p.out_blk_stride;
 #pragma unroll 1
   for (int hi = 0; hi < n_heads; ++hi, ob += p.out_bh_stride) {
+    bf16x8 raw[4];
     float x[32];
+    turn_elements(next, raw, turn, lane);
+    if (hi + 1 < n_heads) ask_rows16(next, xr + (int64_t)(hi + 1) * p.sh * 2, p.ss * 2, src, lane);
+    norm_row(x, raw, p.norm_w != nullptr, p.eps, norm, 1.0f);
+    rope_row(x, p.rope_mode, rope, g);
+    if (tile * 64 + 64 > rows) {                         // rows past the end are zero, whatever row 0 and its rotation hold
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) x[ks * 8 + j] = valid ? (float)next[ks][j] : 0.f;
-    if (hi + 1 < n_heads) fetch(next, hi + 1);
-    norm_rope_quarter(x, tf, norm, rope, valid, g);
+      for (int i = 0; i < 32; ++i) x[i] = valid ? x[i] : 0.f;
+    }
     float part[4] = {0.f, 0.f, 0.f, 0.f};   // four running sums: one would be a chain of 32 dependent instructions
 #pragma unroll
     for (int i = 0; i < 32; ++i) part[i & 3] += x[i] * x[i];
@@ -199,8 +208,10 @@ __device__ __forceinline__ void v_tile(const VPrologueParams& p, int tile, int b
 // Key mask of one batch entry: the number of valid keys, and the source rows of this tile's 64 (where it has them) in `source`, for all
 // four waves after the next barrier.  Every workgroup looks at the whole mask: a few bytes a thread, asked for at
 // once, where a launch of its own in front of this one cost the call 3 to 4 us (3 x 8 heads x 777 rows 39.9 -> 36.5).
+// kMost: 64-key pieces of a wave.  What it costs is instructions that a wave issues one by one, so short masks take a
+// form with 4 pieces rather than 16, and a piece none of whose keys is the tile's is not placed.
+template <int kMost>
 __device__ __forceinline__ int compact_mask(const uint8_t* mask, int S, int tile, int* source) {
-  constexpr int kMost = kOwnMaskKeys / 256;             // 64-key pieces of a wave
   __shared__ int wave_tot[4];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int pieces = (S + 255) / 256;
@@ -208,12 +219,17 @@ __device__ __forceinline__ int compact_mask(const uint8_t* mask, int S, int tile
   uint8_t m[kMost];
 #pragma unroll
   for (int i = 0; i < kMost; ++i) m[i] = i < pieces && key0 + 64 * i < S ? mask[key0 + 64 * i] : 0;
+  unsigned long long on[kMost];
   int total = 0;
 #pragma unroll
-  for (int i = 0; i < kMost; ++i) total += __popcll(__ballot(m[i] != 0));
+  for (int i = 0; i < kMost; ++i) {
+    on[i] = __ballot(m[i] != 0);
+    total += __popcll(on[i]);
+  }
   if (lane == 0) wave_tot[wave] = total;
   __syncthreads();
   int at = -64 * tile, all = 0;                         // place of the next valid key, counted from the tile's first
+#pragma unroll
   for (int w = 0; w < 4; ++w) {
     const int n = wave_tot[w];
     if (w < wave) at += n;
@@ -221,10 +237,12 @@ __device__ __forceinline__ int compact_mask(const uint8_t* mask, int S, int tile
   }
 #pragma unroll
   for (int i = 0; i < kMost; ++i) {
-    const unsigned long long on = __ballot(m[i] != 0);
-    const int place = at + __popcll(on & ((1ull << lane) - 1ull));
-    if (m[i] != 0 && place >= 0 && place < 64) source[place] = key0 + 64 * i;
-    at += __popcll(on);
+    const int here = __popcll(on[i]);
+    if (at < 64 && at + here > 0) {                     // (wave-uniform) some of these 64 keys may be the tile's
+      const int place = at + __popcll(on[i] & ((1ull << lane) - 1ull));
+      if (m[i] != 0 && place >= 0 && place < 64) source[place] = key0 + 64 * i;
+    }
+    at += here;
   }
   return all;
 }
@@ -249,7 +267,8 @@ __global__ __launch_bounds__(256, 3) void kv_prologue_kernel(QkPrologueParams k,
   __shared__ int source[64];                            // source row of each row of the tile (key mask)
   int rows = k.S;
   if (k.row_cnt) {
-    rows = k.mask ? compact_mask(k.mask + (int64_t)b * k.S, k.S, tile, source) : k.row_cnt[b];
+    const uint8_t* mask = k.mask + (int64_t)b * k.S;
+    rows = !k.mask ? k.row_cnt[b] : k.S <= 1024 ? compact_mask<4>(mask, k.S, tile, source) : compact_mask<kOwnMaskKeys / 256>(mask, k.S, tile, source);
     if (k.mask && tile == 0 && in_tile == 0 && threadIdx.x == 0) k.row_cnt[b] = rows;
     if (tile * 64 >= rows) return;                      // no valid key in this tile: nothing reads its record
     if (!k.mask && threadIdx.x < 64 && tile * 64 + threadIdx.x < rows) source[threadIdx.x] = k.gather_idx[(int64_t)b * k.S + tile * 64 + threadIdx.x];
@@ -264,7 +283,7 @@ __global__ __launch_bounds__(256, 3) void kv_prologue_kernel(QkPrologueParams k,
   unsigned* s_amax = s_norm + kKvMaxHeads;
   if (threadIdx.x < 2 * kKvMaxHeads) s_norm[threadIdx.x] = 0u;
   __syncthreads();
-  k_tile<FP8>(k, tile, b, h0, n, rows, src, s_norm, s_amax);
+  k_tile<FP8>(k, tile, b, h0, n, rows, src, s_norm, s_amax, lds + 8192 + (threadIdx.x >> 6) * 4096);
 }
 
 hipError_t launch_kv_prologue(QkPrologueParams k, const VPrologueParams& v, const SparsePlanParams& plan, hipStream_t st) {
