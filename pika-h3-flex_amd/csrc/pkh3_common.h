@@ -104,6 +104,20 @@ __device__ __forceinline__ float wave_max(float x) {
   return max_across_groups(x);
 }
 
+// the sum of all lanes, the same way
+template <int CTRL>
+__device__ __forceinline__ float sum_with(float x) {
+  const int v = __float_as_int(x);
+  return x + __int_as_float(__builtin_amdgcn_update_dpp(v, v, CTRL, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float wave_sum(float x) {
+  x = sum_with<0xB1>(x);
+  x = sum_with<0x4E>(x);
+  x = sum_with<0x141>(x);
+  x = sum_with<0x140>(x);
+  return wave_sum_groups(x);
+}
+
 // ---- four lanes per row: the layout of the 16x16 operand images themselves ----
 // Lane (c = l % 16, g = l / 16) holds the pieces p8 = 4*ks + g of row c of a 16-row block, i.e. elements
 // d = 32*ks + 8*g + j at x[8*ks + j]; the three other lane groups (lanes l ^ 16, l ^ 32, l ^ 48) hold the rest of the

@@ -680,9 +680,7 @@ hipError_t launch_gemm(const GemmParams& p, hipStream_t st) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// Rows -> operand images, optionally through the AdaLN modulation of the block:
-//   y = norm(x) * (1 + scale[row_index]) + shift[row_index]
-// with norm = LayerNorm without affine parameters, RMSNorm without weight, or nothing, statistics in fp32.
+// Rows -> operand images.
 // One wave per row: lane l holds the 16-byte pieces l, l + 64, ... of the row.  Piece pc (elements 8*pc .. +7) of row r
 // belongs to image (16-row block r/16, k-step pc/4), lane 16*(pc%4) + r%16: byte ((r/16)*(K/32) + pc/4)*1024 +
 // (16*(pc%4) + r%16)*16.
@@ -693,7 +691,17 @@ constexpr int kPackMaxPieces = 8;  // 16-byte pieces per lane: rows of up to 64 
 constexpr int kPackRows = 8;                                        // rows (waves) of a workgroup
 constexpr int kPackPitch = kPackMaxPieces * 64 * 16 + 16;           // bytes between the rows staged in LDS (+16: no bank conflicts)
 
-template <int NORM>
+// the workgroup's 8 staged rows are one half of a 16-row block: piece pc of the 8 rows is 128 contiguous bytes of its image
+__device__ __forceinline__ void store_images(const PackParams& p, const char* stage, int pitch) {
+  const int row0 = blockIdx.x * kPackRows, pieces = p.K / 8;
+  char* ob = p.out + (int64_t)(row0 >> 4) * p.out_blk_stride + (row0 & 15) * 16;
+  for (int q = threadIdx.x; q < kPackRows * pieces; q += 64 * kPackRows) {
+    const int rr = q & (kPackRows - 1), pc = q / kPackRows;
+    const bf16x8 t = *(const bf16x8*)(stage + rr * pitch + pc * 16);
+    *(bf16x8*)(ob + ((int64_t)(pc >> 2) * 64 + 16 * (pc & 3) + rr) * 16) = t;
+  }
+}
+
 __global__ __launch_bounds__(64 * kPackRows) void pack_rows_kernel(PackParams p) {
   // the rows of the workgroup, as bf16 pieces, before they go out: in an image a row's pieces lie 256 bytes apart and
   // the same piece of 16 consecutive rows side by side, so whole cache lines only come from several rows together
@@ -707,83 +715,121 @@ __global__ __launch_bounds__(64 * kPackRows) void pack_rows_kernel(PackParams p)
   }
   const bool valid = src < p.rows;
   const int pieces = p.K / 8;                        // 16-byte pieces per row
-  float v[kPackMaxPieces][8];
-  float sum = 0.f;
-#pragma unroll
-  for (int c = 0; c < kPackMaxPieces; ++c) {
-    const int pc = lane + 64 * c;
-    bf16x8 t = {};
-    if (valid && pc < pieces) t = *(const bf16x8*)((const __bf16*)p.x + (int64_t)src * p.row_stride + 8 * pc);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      v[c][j] = (float)t[j];
-      sum += v[c][j];
-    }
-  }
-  if constexpr (NORM != kNormNone) {
-    // Two passes over the row held in registers: the mean first, then the sum of squared distances from it.  The
-    // one-pass form E[x^2] - mean^2 cancels when a row's mean is large against its spread.
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o, 64);
-    const float inv_k = 1.0f / (float)p.K;
-    const float mean = NORM == kNormLayer ? sum * inv_k : 0.f;
-    float ssq = 0.f;
-#pragma unroll
-    for (int c = 0; c < kPackMaxPieces; ++c) {
-      if (lane + 64 * c >= pieces) continue;  // pieces past the row's end hold zeros, not elements
-#pragma unroll
-      for (int j = 0; j < 8; ++j) ssq += (v[c][j] - mean) * (v[c][j] - mean);
-    }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) ssq += __shfl_xor(ssq, o, 64);
-    // a constant row with eps == 0 comes out as zeros (plus shift) instead of 0 * inf
-    const float ve = ssq * inv_k + p.eps;
-    const float rs = ve > 0.f ? rsqrtf(ve) : 0.f;
-    const int mrow = valid && p.row_index ? p.row_index[src] : 0;
-    const __bf16* sh = p.shift ? (const __bf16*)p.shift + (int64_t)mrow * p.table_stride : nullptr;
-    const __bf16* sc = p.scale ? (const __bf16*)p.scale + (int64_t)mrow * p.table_stride : nullptr;
-#pragma unroll
-    for (int c = 0; c < kPackMaxPieces; ++c) {
-      const int pc = lane + 64 * c;
-      if (pc >= pieces) continue;
-      bf16x8 s8 = {}, h8 = {};
-      if (sc) s8 = *(const bf16x8*)(sc + 8 * pc);
-      if (sh) h8 = *(const bf16x8*)(sh + 8 * pc);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        float y = (v[c][j] - mean) * rs;
-        if (sc) y *= 1.0f + (float)s8[j];
-        if (sh) y += (float)h8[j];
-        v[c][j] = valid ? y : 0.f;
-      }
-    }
-  }
 #pragma unroll
   for (int c = 0; c < kPackMaxPieces; ++c) {
     const int pc = lane + 64 * c;
     if (pc >= pieces) continue;
-    bf16x8 t;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) t[j] = (__bf16)v[c][j];
+    bf16x8 t = {};
+    if (valid) t = *(const bf16x8*)((const __bf16*)p.x + (int64_t)src * p.row_stride + 8 * pc);
     *(bf16x8*)(stage + wave * kPackPitch + pc * 16) = t;
   }
   __syncthreads();
-  // the workgroup's 8 rows are one half of a 16-row block: piece pc of the 8 rows is 128 contiguous bytes of its image
-  const int row0 = blockIdx.x * kPackRows;
-  char* ob = p.out + (int64_t)(row0 >> 4) * p.out_blk_stride + (row0 & 15) * 16;
-  for (int q = threadIdx.x; q < kPackRows * pieces; q += 64 * kPackRows) {
-    const int rr = q & (kPackRows - 1), pc = q / kPackRows;
-    const bf16x8 t = *(const bf16x8*)(stage + rr * kPackPitch + pc * 16);
-    *(bf16x8*)(ob + ((int64_t)(pc >> 2) * 64 + 16 * (pc & 3) + rr) * 16) = t;
+  store_images(p, stage, kPackPitch);
+}
+
+// Rows -> operand images through the AdaLN modulation of the block:
+//   y = norm(x) * (1 + scale[row_index]) + shift[row_index]
+// with norm = LayerNorm without affine parameters or RMSNorm without weight, statistics in fp32.  Rows, pieces and staging as
+// above; NP: pieces of a lane, of which only the last may lie past the row's end (lanes there read the row's last piece and take zeros for it).
+// Bound by the memory from some thousand rows on (2 bytes in and out per element: 48,360 x 3,072 at 5.5 TB/s), below by a row's chain of trips to
+// memory (row, its table row's number, tables) and its two sums across the wave, with four waves a SIMD beside it.  So the tables' pieces are asked for all
+// at once and before the sums.  Asked for piece by piece where they were used, behind a test each, with 1.6 times the instructions (what may
+// not be there was looked after element by element) and sums through the LDS crossbar, us, before / now: K 3,072: 1,085 rows 8.0 / 6.4, 4,000
+// 17.6 / 11.4, 15,342 57.0 / 36.2, 48,360 160.7 / 108.9; K 512: 128 rows 4.4 / 3.0, 15,342 23.9 / 9.4; K 4,096: 15,342 79.9 / 45.2.
+template <int NORM, int NP>
+__global__ __launch_bounds__(64 * kPackRows, 4) void modulate_rows_kernel(PackParams p) {
+  constexpr int kPitch = NP * 1024 + 16;
+  __shared__ __attribute__((aligned(16))) char stage[kPackRows * kPitch];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row = blockIdx.x * kPackRows + wave;
+  const int last = p.K / 8 - 1;                      // the row's last piece
+  char* mine = stage + wave * kPitch;
+  auto piece = [&](int c) { return c < NP - 1 ? lane + 64 * c : min(lane + 64 * c, last); };
+  if (row < p.rows) {                                // (wave-uniform)
+    bf16x8 x[NP], scale[NP], shift[NP];
+    const __bf16* src = (const __bf16*)p.x + (int64_t)row * p.row_stride;
+#pragma unroll
+    for (int c = 0; c < NP; ++c) x[c] = *(const bf16x8*)(src + 8 * piece(c));
+    const int64_t table = (p.row_index ? p.row_index[row] : 0) * p.table_stride;
+    // (in the place of a table that is not there the row itself: no branches between these loads and the wait for those above)
+    const __bf16* scale_row = p.scale ? (const __bf16*)p.scale + table : src;
+    const __bf16* shift_row = p.shift ? (const __bf16*)p.shift + table : src;
+#pragma unroll
+    for (int c = 0; c < NP; ++c) {
+      scale[c] = *(const bf16x8*)(scale_row + 8 * piece(c));
+      shift[c] = *(const bf16x8*)(shift_row + 8 * piece(c));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // the row's values are formed anew for every pass where they do not fit the registers beside the tables
+    auto anew = [&]() {
+      if constexpr (NP > 6)
+#pragma unroll
+        for (int c = 0; c < NP; ++c) {
+          i32x4 v = __builtin_bit_cast(i32x4, x[c]);
+          asm volatile("" : "+v"(v));
+          x[c] = __builtin_bit_cast(bf16x8, v);
+        }
+    };
+    const bool there = lane + 64 * (NP - 1) <= last;
+    // Two passes over the row held in registers: the mean first, then the sum of squared distances from it.  The
+    // one-pass form E[x^2] - mean^2 cancels when a row's mean is large against its spread.
+    const float inv_k = 1.0f / (float)p.K;
+    float mean = 0.f;
+    if constexpr (NORM == kNormLayer) {
+      float sum[8] = {};
+#pragma unroll
+      for (int c = 0; c < NP; ++c)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) sum[j] += c < NP - 1 || there ? (float)x[c][j] : 0.f;
+      mean = wave_sum(((sum[0] + sum[1]) + (sum[2] + sum[3])) + ((sum[4] + sum[5]) + (sum[6] + sum[7]))) * inv_k;
+      asm volatile("" : "+v"(mean));                 // rounded: as part of a fused x - sum / K it leaves a constant row something
+    }
+    anew();
+    float ssq[8] = {};
+#pragma unroll
+    for (int c = 0; c < NP; ++c)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float d = c < NP - 1 || there ? (float)x[c][j] - mean : 0.f;
+        ssq[j] = fmaf(d, d, ssq[j]);
+      }
+    // a constant row with eps == 0 comes out as zeros (plus shift) instead of 0 * inf
+    const float ve = wave_sum(((ssq[0] + ssq[1]) + (ssq[2] + ssq[3])) + ((ssq[4] + ssq[5]) + (ssq[6] + ssq[7]))) * inv_k + p.eps;
+    const float rs = ve > 0.f ? rsqrtf(ve) : 0.f;
+    anew();
+    if (!p.scale)
+#pragma unroll
+      for (int c = 0; c < NP; ++c) scale[c] = bf16x8{};
+    if (!p.shift)
+#pragma unroll
+      for (int c = 0; c < NP; ++c) shift[c] = bf16x8{};
+#pragma unroll
+    for (int c = 0; c < NP; ++c) {
+      bf16x8 t;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) t[j] = (__bf16)fmaf(((float)x[c][j] - mean) * rs, 1.0f + (float)scale[c][j], (float)shift[c][j]);
+      *(bf16x8*)(mine + (lane + 64 * c) * 16) = t;   // (what lies past the row's end is not read again)
+    }
+  } else {
+#pragma unroll
+    for (int c = 0; c < NP; ++c) *(bf16x8*)(mine + (lane + 64 * c) * 16) = bf16x8{};
   }
+  __syncthreads();
+  store_images(p, stage, kPitch);
+}
+
+template <int NORM, int NP = 1>
+static void launch_modulate(const PackParams& p, hipStream_t st) {
+  if constexpr (NP < kPackMaxPieces)
+    if (p.K > NP * 512) return launch_modulate<NORM, NP + 1>(p, st);
+  hipLaunchKernelGGL((modulate_rows_kernel<NORM, NP>), dim3(p.rows_padded / kPackRows), dim3(64 * kPackRows), 0, st, p);
 }
 
 hipError_t launch_pack_rows(const PackParams& p, hipStream_t st) {
-  const dim3 grid(p.rows_padded / kPackRows), block(64 * kPackRows);
   switch (p.norm) {
-    case kNormLayer: hipLaunchKernelGGL(pack_rows_kernel<kNormLayer>, grid, block, 0, st, p); break;
-    case kNormRms: hipLaunchKernelGGL(pack_rows_kernel<kNormRms>, grid, block, 0, st, p); break;
-    default: hipLaunchKernelGGL(pack_rows_kernel<kNormNone>, grid, block, 0, st, p); break;
+    case kNormLayer: launch_modulate<kNormLayer>(p, st); break;
+    case kNormRms: launch_modulate<kNormRms>(p, st); break;
+    default: hipLaunchKernelGGL(pack_rows_kernel, dim3(p.rows_padded / kPackRows), dim3(64 * kPackRows), 0, st, p); break;
   }
   return hipGetLastError();
 }

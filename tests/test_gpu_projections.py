@@ -76,6 +76,28 @@ def test_adaln_modulate_matches_oracle(norm):
     assert AO.max_abs_and_cosine(row0, PO.adaln_modulate(x, shift=shift, scale=scale, norm=norm))[1] >= 0.99999
 
 
+@pytest.mark.parametrize("norm", ["layer", "rms"])
+@pytest.mark.parametrize("S,K", [(1, 32), (16, 512), (9, 544), (17, 1024), (24, 1056), (40, 1536), (23, 1568), (8, 2048), (31, 2080), (33, 2560), (15, 2592),
+                                 (48, 3104), (7, 3584), (25, 3616), (64, 4064), (39, 4096)])
+def test_adaln_modulate_of_every_row_length(S, K, norm):
+    """A wave holds one to eight pieces a lane, the last of them partly or wholly there; rows up to the next 16 are zeros.  Either table
+    may be missing.  One bf16 rounding of the value (2^-9 of it) and float32 statistics: 2^-8 covers both."""
+    from oracle import projection_oracle as PO
+    from pika_h3_flex_amd import projections as P
+
+    x = (_r(S, K, seed=21) * 2 + 0.3).to(torch.bfloat16)
+    tables = dict(shift=_r(3, K, seed=22, std=0.3).to(torch.bfloat16), scale=_r(3, K, seed=23, std=0.3).to(torch.bfloat16))
+    idx = torch.arange(S).remainder(3).to(torch.int32)
+    padded = -(-S // 16) * 16
+    for names in ((), ("shift",), ("scale",), ("shift", "scale")):
+        opts = {n: tables[n] for n in names}
+        img = P.adaln_modulate(x.cuda(), **{n: t.cuda() for n, t in opts.items()}, **(dict(row_index=idx.cuda()) if names else {}), norm=norm)
+        got = _unpack(img, padded, K).cpu()
+        ref = PO.adaln_modulate(x, **opts, **(dict(row_index=idx) if names else {}), norm=norm)
+        assert float(((got[:S].double() - ref).abs() / (ref.abs() + 1.0)).max()) <= 2.0 ** -8
+        assert torch.count_nonzero(got[S:]) == 0
+
+
 def test_adaln_layer_norm_of_rows_with_a_large_common_offset():
     """Rows whose mean is large against their spread (massive-activation channels): the variance must come from the
     distances to the mean, not from E[x^2] - mean^2, which cancels in float32.  x = 0.25 * randn + 50 (bf16 grid step
