@@ -155,7 +155,7 @@ __device__ __forceinline__ void q_rows_ready(float (&x)[32], const QRows& r, con
     turn_table(r.sin, rope.s, p.q_rope_mode, lds, lane);
   }
   norm_row(x, raw, p.q_norm_w != nullptr, p.q_eps, norm, factor);
-  rope_row(x, p.q_rope_mode, rope, lane >> 4);
+  rope_row(x, p.q_rope_mode, rope);
 }
 
 // Consecutive MFMAs share an operand where they can: the two query blocks of an image come in turn (0 1, 1 0, 0 1 ..), so that only
@@ -1471,7 +1471,7 @@ __global__ __launch_bounds__(64 * kRelayWaves, 1) void attn_fwd_relay_kernel(Fwd
           ask_rows16(sin, (const char*)p.q_sin, kD / 2 * sizeof(float), q32 * 32 + 16 * qb, p.Sq - 1, l);
           turn_table(cos, rope.c, p.q_rope_mode, own, l);
           turn_table(sin, rope.s, p.q_rope_mode, own, l);
-          rope_row(x, p.q_rope_mode, rope, l >> 4);
+          rope_row(x, p.q_rope_mode, rope);
         }
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {

@@ -25,7 +25,7 @@
 //       contraction needs.
 //
 // Rows are prepared (RMSNorm, rotation, quantisation) in the layout of the images themselves, four lanes per row
-// (norm_rope_quarter below): by the K prologue, by the K epilogue of the projection GEMM and by the attention
+// (norm_row and rope_row below): by the K prologue, by the K epilogue of the projection GEMM and by the attention
 // kernel's Q load.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -63,15 +63,6 @@ constexpr int kQBlkBytes = 8192;   // bf16 Q block of 32 queries
 constexpr int kQ8BlkBytes = 4096;  // fp8 Q block of 32 queries
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kFp8Max = 448.0f;  // OCP e4m3fn
-
-// RMSNorm + rotation of one row: what is done to it (norm_rope_quarter below does it).
-struct RowTransform {
-  const float* norm_w;  // [D] or null
-  float eps;
-  int rope_mode;        // 0 none, 1 interleaved, 2 half-split
-  const float* cos_t;   // [rows, D/2]
-  const float* sin_t;
-};
 
 __device__ __forceinline__ float wave_sum_groups(float x) {
   // sum over the four lanes l % 16 == const (one per 16-lane group): two row swaps, no trip through the LDS crossbar
@@ -133,58 +124,9 @@ struct RopeQuarter {
   f32x4 c[4], s[4];
 };
 
-__device__ __forceinline__ void load_rope_quarter(RopeQuarter& r, const RowTransform& t, int64_t table_row, int g) {
-  const float* ct = t.cos_t + table_row * (kD / 2);
-  const float* st = t.sin_t + table_row * (kD / 2);
-  if (t.rope_mode == 1) {
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      r.c[ks] = *(const f32x4*)(ct + 16 * ks + 4 * g);
-      r.s[ks] = *(const f32x4*)(st + 16 * ks + 4 * g);
-    }
-  } else if (t.rope_mode == 2) {
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      r.c[2 * ks] = *(const f32x4*)(ct + 32 * ks + 8 * g), r.c[2 * ks + 1] = *(const f32x4*)(ct + 32 * ks + 8 * g + 4);
-      r.s[2 * ks] = *(const f32x4*)(st + 32 * ks + 8 * g), r.s[2 * ks + 1] = *(const f32x4*)(st + 32 * ks + 8 * g + 4);
-    }
-  }
-}
-
-// The RMSNorm weights of this lane's 32 elements: w[2*ks], w[2*ks + 1] = weights 32*ks + 8*g .. +7
-struct NormQuarter {
-  f32x4 w[8];
-};
-
-__device__ __forceinline__ void load_norm_quarter(NormQuarter& n, const RowTransform& t, int g) {
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks) {
-    n.w[2 * ks] = *(const f32x4*)(t.norm_w + 32 * ks + 8 * g);
-    n.w[2 * ks + 1] = *(const f32x4*)(t.norm_w + 32 * ks + 8 * g + 4);
-  }
-}
-
-// RMSNorm and rotation of this lane's 32 elements of a row, with the weights and the row's tables already in registers
-__device__ __forceinline__ void norm_rope_quarter(float (&x)[32], const RowTransform& t, const NormQuarter& n, const RopeQuarter& r,
-                                                  bool valid, int g) {
-  if (t.norm_w) {
-    // four running sums: one would be a chain of 32 dependent instructions
-    float part[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int i = 0; i < 32; ++i) part[i & 3] += x[i] * x[i];
-    const float ssq = wave_sum_groups((part[0] + part[1]) + (part[2] + part[3]));
-    // an all-zero row with eps == 0 stays all zero instead of 0 * inf
-    const float ms = ssq * (1.0f / kD) + t.eps;
-    const float rs = ms > 0.f ? rsqrtf(ms) : 0.f;
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        x[ks * 8 + j] *= rs * n.w[2 * ks][j];
-        x[ks * 8 + 4 + j] *= rs * n.w[2 * ks + 1][j];
-      }
-  }
-  if (t.rope_mode == 1 && valid) {
+// the rotation of this lane's 32 elements of a row, with the row's tables already in registers
+__device__ __forceinline__ void rope_row(float (&x)[32], int rope_mode, const RopeQuarter& r) {
+  if (rope_mode == 1) {
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
@@ -193,7 +135,7 @@ __device__ __forceinline__ void norm_rope_quarter(float (&x)[32], const RowTrans
         x[ks * 8 + 2 * jj] = a0 * r.c[ks][jj] - a1 * r.s[ks][jj];
         x[ks * 8 + 2 * jj + 1] = a1 * r.c[ks][jj] + a0 * r.s[ks][jj];
       }
-  } else if (t.rope_mode == 2 && valid) {
+  } else if (rope_mode == 2) {
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
@@ -300,9 +242,19 @@ __device__ __forceinline__ void norm_row(float (&x)[32], const bf16x8 (&raw)[4],
 #pragma unroll
   for (int i = 0; i < 32; ++i) x[i] *= (float)raw[i >> 3][i & 7];
 }
-// the rotation alone
-__device__ __forceinline__ void rope_row(float (&x)[32], int rope_mode, const RopeQuarter& r, int g) {
-  norm_rope_quarter(x, RowTransform{nullptr, 0.f, rope_mode, nullptr, nullptr}, NormQuarter{}, r, true, g);
+// RMSNorm of this lane's 32 elements of a row
+__device__ __forceinline__ void norm_lanes(float (&x)[32], float eps, NormLanes& n) {
+  float part[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 32; ++i) part[i & 3] += x[i] * x[i];
+  // an all-zero row with eps == 0 stays all zero instead of 0 * inf
+  const float ms = wave_sum_groups((part[0] + part[1]) + (part[2] + part[3])) * (1.0f / kD) + eps;
+  const float rs = ms > 0.f ? rsqrtf(ms) : 0.f;
+  asm volatile("s_nop 1" : "+v"(n.w[0]), "+v"(n.w[1]));   // (where the weights were kept elsewhere, they have been back for as long as it takes)
+  static_for<32>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    x[i] *= times_row_lane<i & 15>(n.w[i >> 4], rs);
+  });
 }
 
 // eight values -> eight fp8 e4m3 bytes

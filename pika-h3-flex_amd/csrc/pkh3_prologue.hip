@@ -101,7 +101,7 @@ __device__ __forceinline__ void k_tile(const QkPrologueParams& p, int tile, int 
     turn_elements(next, raw, turn, lane);
     if (hi + 1 < n_heads) ask_rows16(next, xr + (int64_t)(hi + 1) * p.sh * 2, p.ss * 2, src, lane);
     norm_row(x, raw, p.norm_w != nullptr, p.eps, norm, 1.0f);
-    rope_row(x, p.rope_mode, rope, g);
+    rope_row(x, p.rope_mode, rope);
     if (tile * 64 + 64 > rows) {                         // rows past the end are zero, whatever row 0 and its rotation hold
 #pragma unroll
       for (int i = 0; i < 32; ++i) x[i] = valid ? x[i] : 0.f;
