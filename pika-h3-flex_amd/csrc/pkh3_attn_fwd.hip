@@ -43,6 +43,7 @@
 #include <type_traits>
 
 #include "pkh3_common.h"
+#include "pkh3_index.h"
 #include "pkh3_internal.h"
 
 namespace pkh3 {
@@ -1380,6 +1381,47 @@ __device__ __forceinline__ int lane_here() {
   return l;
 }
 
+// The units [at, end) of this workgroup: equal shares of all units or, where a key mask leaves the entries of a batch unequal keys (which the
+// device alone knows), of their weights (relay_weight): in equal shares half of the CUs may have the short entry and wait for the other
+// half.  us, long form (whose queues even this out) / equal counts / by weight: 2 x 24 heads x 20,000 queries against 2,500 keys, 64 and 2,500 of
+// them valid, 849 / 934 / 536, 625 and 2,500 852 / 937 / 629, all 961 / 958 / 950; x 14,830 against 1,500, 64 and 1,500 424 / 443 / 273; 8 x 12 x 4,000
+// against 2,000, 250 to 2,000 290 / 339 / 227; x 49,640 against 512, 64 and 512 598 (short-key form) / 544 / 425.
+struct RelayRun {
+  int at, end;
+};
+__device__ __forceinline__ RelayRun relay_run(const FwdParams& p, int per_head) {
+  const int wgs = gridDim.x, rank = (blockIdx.x & 7) * (wgs >> 3) + (blockIdx.x >> 3);   // a contiguous run per XCD and workgroup
+  const int per_entry = p.H * per_head, all = p.B * per_entry;
+  if (!p.row_cnt || p.B == 1) return {(int)((int64_t)rank * all / wgs), (int)((int64_t)(rank + 1) * all / wgs)};
+  const int lane = threadIdx.x & 63;
+  auto weight = [&](int b) { return b < p.B ? relay_weight(p.row_cnt[b]) : 0; };
+  auto sum_up = [&](int x) {                             // over this lane and those before it
+#pragma unroll
+    for (int d = 1; d < 64; d *= 2) {
+      const int y = __shfl_up(x, d, 64);
+      if (lane >= d) x += y;
+    }
+    return x;
+  };
+  int total = 0;
+  for (int b0 = 0; b0 < p.B; b0 += 64) total += __builtin_amdgcn_readlane(sum_up(weight(b0 + lane)), 63);
+  RelayRun run{all, all};                                // (no entry holds the end of the last run)
+  for (int b0 = 0, before = 0; b0 < p.B; b0 += 64) {
+    const int w = weight(b0 + lane), sum = sum_up(w);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int64_t into = (int64_t)(rank + i) * total - (int64_t)(before + sum - w) * wgs;   // (in 1 / wgs of a weight)
+      const unsigned long long here = __ballot(into >= 0 && into < (int64_t)w * wgs);
+      if (here) {                                        // (one lane at most, in one turn of the loop)
+        const int unit = (b0 + lane) * per_entry + (int)relay_unit(into, w, wgs, per_entry);
+        (i ? run.end : run.at) = __builtin_amdgcn_readlane(unit, __builtin_ctzll(here));
+      }
+    }
+    before += __builtin_amdgcn_readlane(sum, 63);
+  }
+  return run;
+}
+
 template <bool ROPE>
 __global__ __launch_bounds__(64 * kRelayWaves, 1) void attn_fwd_relay_kernel(FwdParams p) {
   constexpr int kTile = kKTileBytes + kVTileBytes;
@@ -1390,11 +1432,8 @@ __global__ __launch_bounds__(64 * kRelayWaves, 1) void attn_fwd_relay_kernel(Fwd
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int grp = wave / kShortWaves, wq = wave & (kShortWaves - 1);
   char* own = rows + wave * kQBlkBytes;
-  const int per_head = units_per_head(p.Sq, kShortWaves), total = p.sec_units[0];
-  // a contiguous run of (batch, head, 128 queries) per XCD and workgroup
-  const int wgs = gridDim.x, rank = (blockIdx.x & 7) * (wgs >> 3) + (blockIdx.x >> 3);
-  int at = (int)((int64_t)rank * total / wgs);
-  const int end = (int)((int64_t)(rank + 1) * total / wgs);
+  const int per_head = units_per_head(p.Sq, kShortWaves);
+  RelayRun run = relay_run(p, per_head);
   unsigned long long third;                              // lanes of a tile's third copy: it is 32 KiB, for twelve waves
   asm volatile("s_cmp_lt_i32 %1, %2\n\ts_cselect_b64 %0, -1, 0" : "=s"(third) : "s"(wave), "n"(kTile / 1024 - 2 * kRelayWaves) : "scc");
   const unsigned rows_lds = (unsigned)(size_t)(__attribute__((address_space(3))) char*)own;
@@ -1405,11 +1444,11 @@ __global__ __launch_bounds__(64 * kRelayWaves, 1) void attn_fwd_relay_kernel(Fwd
   const float top_weight = wave_max(fmaxf(fabsf(norm.w[0]), fabsf(norm.w[1]))) * p.c;
 
 #pragma unroll 1
-  while (at < end) {
+  while (run.at < run.end) {
     // a stretch: the units of one (batch, head), three to a round
     WaveState<false> w;
-    const int bh = at / per_head, first = at - bh * per_head, count = min(end - at, per_head - first);
-    at += count;
+    const int bh = run.at / per_head, first = run.at - bh * per_head, count = min(run.end - run.at, per_head - first);
+    run.at += count;
     const int b = bh / p.H, h = bh % p.H;
     const int sk = p.row_cnt ? uniform_load(p.row_cnt, b) : p.Sk;
     const int n = (sk + kTileKeys - 1) / kTileKeys, ring_n = max(n, 1);
@@ -1719,7 +1758,6 @@ static hipError_t launch_fp(FwdParams p, int cus, hipStream_t st) {
   if constexpr (!FP8) {
     if (relay_form(p, units(kShortWaves), cus)) {
       p.queue_next = nullptr;
-      p.sec_units[0] = units(kShortWaves);
       const dim3 grid(cus / 8 * 8), block(64 * kRelayWaves);
       if (p.q_rope_mode) hipLaunchKernelGGL(attn_fwd_relay_kernel<true>, grid, block, 0, st, p);
       else hipLaunchKernelGGL(attn_fwd_relay_kernel<false>, grid, block, 0, st, p);

@@ -42,6 +42,12 @@ constexpr int gemm_token_blocks(int tokens, int n_tiles, int chunks, int cus) {
   return best;
 }
 
+// The relay form of the attention kernel shares the units of a call out by weight.  One of a batch entry takes as long as a third of a round,
+// 3.9 us for its start and end and 2.1 to 2.2 for every key tile: two tiles' time besides the tiles.
+constexpr int relay_weight(int valid_keys) { return (valid_keys + 63) / 64 + 2; }
+// The unit of an entry of `units` units and weight `weight` that a workgroup begins with whose share begins into / wgs of a weight into it
+constexpr int64_t relay_unit(int64_t into, int weight, int wgs, int units) { return into * units / ((int64_t)weight * wgs); }
+
 constexpr int kKvMaxHeads = 8;        // heads a workgroup of the K/V pass walks at most
 constexpr int kOwnMaskKeys = 4096;    // keys whose mask a workgroup of the K/V pass can look through
 

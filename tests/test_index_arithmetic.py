@@ -99,3 +99,41 @@ def test_tokens_a_workgroup_of_the_projections(tmp_path):
     const int got = 32 * gemm_token_blocks(c.tokens, c.n_tiles, c.chunks, 256);
     CHECK(got == c.want, "%d tokens, %d tiles, %d chunks: %d", c.tokens, c.n_tiles, c.chunks, got);
   }""")
+
+
+def test_relay_shares_go_by_the_work_of_the_entries(tmp_path):
+    """Entries of unequal valid keys, none to 40 tiles of them, shared out among 8 to 304 workgroups: the runs follow each other without a gap from
+    the first unit to the last, and no run is longer than the mean by more than two of the longest units (one at either end)."""
+    _run(tmp_path, """
+  const int tiles[][6] = {{1, 40}, {40, 1}, {5, 5}, {0, 40}, {0, 0}, {1, 2, 4, 8, 16, 40}, {40, 40, 1, 1, 0, 40}, {0, 0, 0, 0, 0, 1}};
+  const int entries[] = {2, 6, 70}, workgroups[] = {8, 104, 256, 304}, sizes[] = {1, 3, 24 * 116, 2 * 388, 1030, 16777216};
+  for (auto& t : tiles)
+    for (int B : entries)
+      for (int wgs : workgroups)
+        for (int units : sizes) {                                         // of an entry
+          auto weight = [&](int b) { return relay_weight(t[b % (B == 2 ? 2 : 6)] * 64); };
+          int64_t total = 0, longest = 0;
+          for (int b = 0; b < B; ++b) {
+            total += weight(b);
+            if (weight(b) > longest) longest = weight(b);
+          }
+          int64_t at = 0;                                                 // units in front of the run
+          double done = 0;                                                // ... and their weight, a unit of an entry counting weight(b)
+          for (int rank = 0; rank < wgs; ++rank) {
+            int64_t end = (int64_t)B * units, before = 0;
+            for (int b = 0; b < B; before += weight(b++)) {
+              const int64_t into = (int64_t)(rank + 1) * total - before * wgs;
+              if (into >= 0 && into < (int64_t)weight(b) * wgs) end = (int64_t)b * units + relay_unit(into, weight(b), wgs, units);
+            }
+            CHECK(end >= at && end <= (int64_t)B * units, "%d entries x %d units, workgroup %d of %d: [%lld, %lld)", B, units, rank, wgs, (long long)at, (long long)end);
+            double run = 0;
+            for (int b = 0; b < B; ++b) {
+              const int64_t from = at > (int64_t)b * units ? at : (int64_t)b * units, to = end < (int64_t)(b + 1) * units ? end : (int64_t)(b + 1) * units;
+              if (to > from) run += (double)(to - from) * weight(b);
+            }
+            CHECK(run <= (double)total * units / wgs + 2 * longest, "%d entries x %d units: workgroup %d of %d has %g of %g", B, units, rank, wgs, run,
+                  (double)total * units);
+            done += run, at = end;
+          }
+          CHECK(at == (int64_t)B * units && done == (double)total * units, "%d entries x %d units: %lld", B, units, (long long)at);
+        }""")
