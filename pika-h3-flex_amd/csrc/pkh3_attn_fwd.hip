@@ -1389,10 +1389,11 @@ __device__ __forceinline__ int lane_here() {
 struct RelayRun {
   int at, end;
 };
+template <bool ROPE>
 __device__ __forceinline__ RelayRun relay_run(const FwdParams& p, int per_head) {
   const int wgs = gridDim.x, rank = (blockIdx.x & 7) * (wgs >> 3) + (blockIdx.x >> 3);   // a contiguous run per XCD and workgroup
   const int per_entry = p.H * per_head, all = p.B * per_entry;
-  if (!p.row_cnt || p.B == 1) return {(int)((int64_t)rank * all / wgs), (int)((int64_t)(rank + 1) * all / wgs)};
+  if (!p.row_cnt || p.B == 1) return {relay_cut(rank, all, per_head, wgs, !ROPE), relay_cut(rank + 1, all, per_head, wgs, !ROPE)};
   const int lane = threadIdx.x & 63;
   auto weight = [&](int b) { return b < p.B ? relay_weight(p.row_cnt[b]) : 0; };
   auto sum_up = [&](int x) {                             // over this lane and those before it
@@ -1433,7 +1434,7 @@ __global__ __launch_bounds__(64 * kRelayWaves, 1) void attn_fwd_relay_kernel(Fwd
   const int grp = wave / kShortWaves, wq = wave & (kShortWaves - 1);
   char* own = rows + wave * kQBlkBytes;
   const int per_head = units_per_head(p.Sq, kShortWaves);
-  RelayRun run = relay_run(p, per_head);
+  RelayRun run = relay_run<ROPE>(p, per_head);
   unsigned long long third;                              // lanes of a tile's third copy: it is 32 KiB, for twelve waves
   asm volatile("s_cmp_lt_i32 %1, %2\n\ts_cselect_b64 %0, -1, 0" : "=s"(third) : "s"(wave), "n"(kTile / 1024 - 2 * kRelayWaves) : "scc");
   const unsigned rows_lds = (unsigned)(size_t)(__attribute__((address_space(3))) char*)own;

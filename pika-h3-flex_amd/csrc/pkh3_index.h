@@ -42,7 +42,28 @@ constexpr int gemm_token_blocks(int tokens, int n_tiles, int chunks, int cus) {
   return best;
 }
 
-// The relay form of the attention kernel shares the units of a call out by weight.  One of a batch entry takes as long as a third of a round,
+// The relay form of the attention kernel gives every workgroup a run of units, 128 queries each of one head after the other, and walks three
+// units of a head in a round.  Units in front of the run of workgroup `rank`, in equal shares:
+constexpr int relay_even_cut(int rank, int units, int wgs) { return rank * (units / wgs) + rank * (units % wgs) / wgs; }
+constexpr int relay_rounds(int units) { return (units + 2) / 3; }
+// ... and with a unit moved to the run before where that saves a round.  A run that crosses the end of a head has rounds of fewer than three
+// units on both sides of it: eight of 256 workgroups took a round more than the others, which the call waits for, and a round is
+// what the form gains.  24 heads, us, form in its place before / equal shares / now: 6,500 rows (51 units a head) x 512 keys 50.2 / 54.0 / 50.2,
+// x 1,024 82.6 / 88.3 / 80.9; 14,830 (116) x 1,024 167 / 164.5 / 162.3; with rotation 3 x 24 x 2,000 (16) x 2,000 179 / 168 / 154.
+// `fills`: also where the last round of the run before becomes one of three units.  With rotation, whose partial rounds are cheaper beside whole ones
+// (waiting for the tables is the same), that lost what it saved: 14,830 x 1,088 189 -> 193, x 1,536 246.5 -> 250.
+// (Runs of whole rounds throughout were worse, 49.5 -> 53.3 for 6,000 rows: a round of one unit takes 0.6 of one of three.)
+constexpr int relay_cut(int rank, int units, int per_head, int wgs, bool fills) {
+  const int at = relay_even_cut(rank, units, wgs);
+  if (rank == 0 || rank >= wgs) return at;
+  const int before = relay_even_cut(rank - 1, units, wgs), end = relay_even_cut(rank + 1, units, wgs);
+  const int head = at / per_head * per_head, next = head + per_head;
+  const bool crosses = before >= head && end > next && end <= next + per_head;   // one head's end, and the run before none
+  const int most = relay_rounds((units + wgs - 1) / wgs), over = (at - before) % 3;
+  if (!crosses || (next - at) % 3 != 1 || relay_rounds(next - at) + relay_rounds(end - next) <= most) return at;
+  return over == 1 || (over == 2 && fills) ? at + 1 : at;                        // (the run before has no more rounds for it)
+}
+// Where the entries of a batch keep unequal keys, they are shared out by weight.  One of a batch entry takes as long as a third of a round,
 // 3.9 us for its start and end and 2.1 to 2.2 for every key tile: two tiles' time besides the tiles.
 constexpr int relay_weight(int valid_keys) { return (valid_keys + 63) / 64 + 2; }
 // The unit of an entry of `units` units and weight `weight` that a workgroup begins with whose share begins into / wgs of a weight into it

@@ -101,6 +101,40 @@ def test_tokens_a_workgroup_of_the_projections(tmp_path):
   }""")
 
 
+def test_relay_runs_make_no_round_too_many(tmp_path):
+    """Runs follow each other without a gap, are as long as equal shares to a unit, and the longest has no more rounds than of equal shares; where
+    those cross a head's end with one unit over on either side (51, 116 and 149 units a head), as many as its units need."""
+    _run(tmp_path, """
+  for (int wgs = 8; wgs <= 304; wgs += 8)
+    for (int heads = 1; heads <= 96; heads += heads < 8 ? 1 : 8)
+      for (int per_head = 1; per_head <= 400; per_head += per_head < 160 ? 1 : 17) {
+        const int units = heads * per_head;
+        if (units <= 4 * wgs) continue;
+        for (int fills = 0; fills < 2; ++fills) {
+          int most[2] = {0, 0}, at = 0;
+          for (int rank = 0; rank < wgs; ++rank) {
+            const int begin = relay_cut(rank, units, per_head, wgs, fills), end = relay_cut(rank + 1, units, per_head, wgs, fills);
+            CHECK(begin == at && end >= begin && end <= units, "%d x %d units, workgroup %d of %d: [%d, %d)", heads, per_head, rank, wgs, begin, end);
+            CHECK(end - begin <= units / wgs + 2 && end - begin >= units / wgs - 1, "%d x %d units, workgroup %d of %d: [%d, %d)", heads, per_head, rank, wgs, begin, end);
+            at = end;
+            for (int even = 0; even < 2; ++even) {
+              int a = even ? (int)((int64_t)rank * units / wgs) : begin, rounds = 0;
+              const int b = even ? (int)((int64_t)(rank + 1) * units / wgs) : end;
+              for (int part; a < b; a += part) {
+                part = (a / per_head + 1) * per_head < b ? (a / per_head + 1) * per_head - a : b - a;
+                rounds += relay_rounds(part);
+              }
+              if (rounds > most[even]) most[even] = rounds;
+            }
+          }
+          CHECK(at == units && most[0] <= most[1], "%d x %d units on %d: %d rounds, %d in equal shares", heads, per_head, wgs, most[0], most[1]);
+          if (fills && wgs == 256 && heads == 24 && (per_head == 51 || per_head == 116 || per_head == 149))
+            CHECK(most[0] == relay_rounds((units + 255) / 256) && most[1] == most[0] + 1, "%d units: %d and %d rounds", per_head, most[0], most[1]);
+          if (!fills && wgs == 256 && heads == 72 && per_head == 16) CHECK(most[0] == 2 && most[1] == 3, "%d and %d rounds", most[0], most[1]);
+        }
+      }""")
+
+
 def test_relay_shares_go_by_the_work_of_the_entries(tmp_path):
     """Entries of unequal valid keys, none to 40 tiles of them, shared out among 8 to 304 workgroups: the runs follow each other without a gap from
     the first unit to the last, and no run is longer than the mean by more than two of the longest units (one at either end)."""
