@@ -24,7 +24,8 @@ enum {
   PKH3_FORM_LONG = 0,   /* dense, 12 waves of 32 queries per workgroup */
   PKH3_FORM_SHORT = 1,  /* dense, 4 waves of 32 queries, half tiles of 32 keys */
   PKH3_FORM_NARROW = 2, /* dense or block-sparse, one block of 32 queries, 4 waves share its keys out */
-  PKH3_FORM_SPARSE = 3  /* block-sparse, 8 waves of 32 queries */
+  PKH3_FORM_SPARSE = 3, /* block-sparse, 8 waves of 32 queries */
+  PKH3_FORM_RELAY = 4   /* dense bf16, a workgroup of 12 waves per CU that goes from one 128 queries to the next */
 };
 int pkh3_attn_form(const pkh3_attn_args* a, int cus);
 

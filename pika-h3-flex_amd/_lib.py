@@ -171,7 +171,7 @@ def load() -> C.CDLL:
 
 BENCH_LIB_PATH = os.path.join(os.path.dirname(LIB_PATH), "libpkh3attn_bench.so")
 BENCH_EXPORTS = ("pkh3_attn_time_kernel", "pkh3_attn_form")   # include/pkh3_attn_bench.h
-FORM_LONG, FORM_SHORT, FORM_NARROW, FORM_SPARSE = 0, 1, 2, 3    # results of pkh3_attn_form
+FORM_LONG, FORM_SHORT, FORM_NARROW, FORM_SPARSE, FORM_RELAY = 0, 1, 2, 3, 4    # results of pkh3_attn_form
 _bench = None
 
 

@@ -1659,6 +1659,29 @@ static TailPlan plan_tail(int rest, int cus, int n_tiles, int64_t max_workgroups
   return best;
 }
 
+// Whether a dense call runs in the relay form.  At least a round and a third per CU (with fewer the other forms' rounds come out as they do), and
+// as long as a round's start and end weigh: to 40 key tiles.  Below 17, where the short-key form takes over from the long one, the gain is what
+// the start cost: from 8 tiles on, and where the queries' tables are not read besides (each wave waits for them between two rounds).  Other form /
+// relay, us, 24 heads, without rotation, 512, 1,024, 1,536, 2,048 and 3,072 keys: 6,000 rows 45.0 / 43.1, 75.3 / 70.9, 115 / 99, 145 / 127,
+// 206 / 183; 9,000 61.0 / 61.0, 105.5 / 101.7, 173 / 143, 219 / 185, 296 / 269; 27,000 179 / 169, 299 / 282, 427 / 398, 534 / 517, 759 / 761; 49,640
+// 327 / 300, 543 / 505, 744 / 727, 951 / 933, 1,367 / 1,361; 256 keys from 40.1 / 41.7 to 122 / 111.  With rotation: 14,830 rows
+// 105 / 114 (512 keys), 175 / 178 (1,024), 262 / 245, 326 / 312; 4,000 rows (three units a CU) 74.7 / 77.2 against 1,536 keys.
+// What the figures leave out, from 600 calls of other sizes (whole calls, us):
+// - against the short-key form, about five units a CU where an XCD does not have whole heads (31 heads of 41 units x 896 keys 79 / 84, 33 of 40 x 704 71
+//   / 76, 54 of 25 x 640 69 / 72.5, 45 of 34 x 640 71 / 74; 48 of 31 x 832 89 / 83, 24 of 51 to 63 0.98 to 1.05 times as fast, and from 6.5 units a CU on
+//   0.98 to 1.07, whatever the heads), and heads of no more than eight units with fewer than ten a CU (210 of 6 x 512 63 / 69, 516 of 4 x 1,024
+//   245 / 252; 400 of 7 x 838, eleven a CU, 233 / 227): of 354 calls that come here against few tiles, 6 are more than 2 % behind and 256 ahead;
+// - against the long form, the keys of all heads being walked at once: where they do not fit the 256 MB cache behind the L2s and that form's
+//   blocks of 384 rows are full (tiles of all heads, us: 7,696 561 / 588, 7,956 744 / 779, 10,791 592 / 626; 7,068 529 / 515, 5,874 615 / 603; blocks
+//   full to 0.87 7,099 451 / 416, 7,917 522 / 486).
+static bool relay_form(const FwdParams& p, int cus) {
+  const int64_t per_head = units_per_head(p.Sq, kShortWaves), units = p.B * p.H * per_head;
+  if (p.fp8 || p.plan || cus < 8 || units <= 4 * cus || p.nKt > 40 || p.q_ss > (1 << 26)) return false;   // (16 rows of queries lie within 32 bits of each other)
+  if (p.nKt > kShortMaxTiles) return (int64_t)p.B * p.H * p.nKt <= 7168 || 10 * per_head < 27 * units_per_head(p.Sq, kDenseWaves);
+  if (p.nKt < 8 || p.q_rope_mode) return false;
+  return per_head > 8 ? 2 * units > 13 * (int64_t)cus || (p.B * p.H) % 8 == 0 : units > 10 * cus;
+}
+
 // Which form of the kernel a call takes.
 AttnForm attn_form(const FwdParams& p, int cus) {
   if (p.long_key_kernel) return p.plan ? kFormSparse : kFormLong;
@@ -1689,6 +1712,7 @@ AttnForm attn_form(const FwdParams& p, int cus) {
   // long form is ahead as long as its own workgroups are no more than the CUs (2,256 x 94: 114 / 94), and behind when a few
   // are left over for a second round (3,000 x 125: 165 / 218).
   if (narrow && per_cu <= 2 && 3.2f + (n32 + cus - 1) / cus * (0.135f * n_half + 2.7f) < 5.0f + (per_cu == 1 ? 0.60f : 0.87f) * n_half) return kFormNarrow;
+  if (relay_form(p, cus)) return kFormRelay;
   const bool few = per_cu <= 2 || (per_cu == 3 && units(kDenseWaves) > cus);
   return few || p.nKt <= kShortMaxTiles ? kFormShort : kFormLong;
 }
@@ -1705,19 +1729,6 @@ static int narrow_from(int n32, int n4, int cus) {
   const float start = (per_cu == 1 ? 5.9f : 2.6f + 4.2f * rounds) - (one ? 5.5f : 8.0f);
   const float gain = (one ? 0.585f : 0.80f) - 0.125f * per_cu;   // per half tile
   return gain > 0.f ? (int)ceilf(start / gain) : INT_MAX;
-}
-
-// Whether a dense call that attn_form gives to workgroups of 128 or 384 queries runs in the relay form.  At least a round and a third per CU (with
-// fewer the other forms' rounds come out as they do), and as long as a round's start and end weigh: to 40 key tiles.  Below 17, where the
-// short-key form takes over from the long one, the gain is what the start cost: from 8 tiles on, and where the queries' tables are not read
-// besides (each wave waits for them between two rounds).  Other form / relay, us, 24 heads, without rotation, 512, 1,024, 1,536, 2,048 and 3,072
-// keys: 6,000 rows 45.0 / 43.1, 75.3 / 70.9, 115 / 99, 145 / 127, 206 / 183; 9,000 61.0 / 61.0, 105.5 / 101.7, 173 / 143, 219 / 185, 296 / 269; 14,830
-// 91.6 / 93.0, 162.5 / 159.9, 242 / 228, 304 / 296, 429 / 431; 27,000 179 / 169, 299 / 282, 427 / 398, 534 / 517, 759 / 761; 49,640 327 / 300, 543 / 505, 744 /
-// 727, 951 / 933, 1,367 / 1,361; 256 keys from 40.1 / 41.7 to 122 / 111.  With rotation: 14,830 rows 105 / 114, 175 / 178, 262 / 245, 326 / 312; 4,000 rows
-// (three units a CU) 74.7 / 77.2 against 1,536 keys.
-static bool relay_form(const FwdParams& p, int units, int cus) {
-  return !p.fp8 && !p.plan && !p.long_key_kernel && cus >= 8 && units > 4 * cus && p.nKt <= 40 && p.nKt >= (p.q_rope_mode ? kShortMaxTiles + 1 : 8) &&
-         p.q_ss <= (1 << 26);   // (16 rows of queries lie within 32 bits of each other)
 }
 
 template <bool FP8, bool POW2 = false>
@@ -1757,7 +1768,7 @@ static hipError_t launch_fp(FwdParams p, int cus, hipStream_t st) {
     return hipGetLastError();
   }
   if constexpr (!FP8) {
-    if (relay_form(p, units(kShortWaves), cus)) {
+    if (form == kFormRelay) {
       p.queue_next = nullptr;
       const dim3 grid(cus / 8 * 8), block(64 * kRelayWaves);
       if (p.q_rope_mode) hipLaunchKernelGGL(attn_fwd_relay_kernel<true>, grid, block, 0, st, p);

@@ -208,7 +208,7 @@ hipError_t launch_fill_zero(unsigned* p, int n, hipStream_t st);
 hipError_t launch_fold_norms(const QkPrologueParams& k, hipStream_t st);   // the largest norm of every head, for prepared keys
 hipError_t launch_kv_prologue(QkPrologueParams k, const VPrologueParams& v, const SparsePlanParams& plan, hipStream_t st);   // plan.n may be 0
 hipError_t launch_attn_fwd(const FwdParams& p, hipStream_t st);
-enum AttnForm { kFormLong = 0, kFormShort = 1, kFormNarrow = 2, kFormSparse = 3 };
+enum AttnForm { kFormLong = 0, kFormShort = 1, kFormNarrow = 2, kFormSparse = 3, kFormRelay = 4 };
 AttnForm attn_form(const FwdParams& p, int cus);  // the form launch_attn_fwd takes on a device of `cus` CUs
 hipError_t device_cu_count(int* out);  // CUs of the current device (cached per device after the first call)
 hipError_t launch_sparse_plan(const SparsePlanParams& p, hipStream_t st);
