@@ -1671,6 +1671,9 @@ static TailPlan plan_tail(int rest, int cus, int n_tiles, int64_t max_workgroups
 //   / 76, 54 of 25 x 640 69 / 72.5, 45 of 34 x 640 71 / 74; 48 of 31 x 832 89 / 83, 24 of 51 to 63 0.98 to 1.05 times as fast, and from 6.5 units a CU on
 //   0.98 to 1.07, whatever the heads), and heads of no more than eight units with fewer than ten a CU (210 of 6 x 512 63 / 69, 516 of 4 x 1,024
 //   245 / 252; 400 of 7 x 838, eleven a CU, 233 / 227): of 354 calls that come here against few tiles, 6 are more than 2 % behind and 256 ahead;
+// - with a key mask, which may leave one or two tiles of the few (24 heads, 512 keys, valid 64, 100, 190 and 302: 6,500 rows 25.7 / 28.1, 29.1 / 31.4, 32.4
+//   / 34.8, 40.1 / 42.7; 14,830 41.1 / 43.1, 47.9 / 49.4, 56.3 / 56.6, 72.5 / 73.1; from 14 units a CU on only a single tile is behind: 49,640
+//   143 / 147, 169 / 152, 197 / 173, 250 / 225);
 // - against the long form, the keys of all heads being walked at once: where they do not fit the 256 MB cache behind the L2s and that form's
 //   blocks of 384 rows are full (tiles of all heads, us: 7,696 561 / 588, 7,956 744 / 779, 10,791 592 / 626; 7,068 529 / 515, 5,874 615 / 603; blocks
 //   full to 0.87 7,099 451 / 416, 7,917 522 / 486).
@@ -1678,7 +1681,7 @@ static bool relay_form(const FwdParams& p, int cus) {
   const int64_t per_head = units_per_head(p.Sq, kShortWaves), units = p.B * p.H * per_head;
   if (p.fp8 || p.plan || cus < 8 || units <= 4 * cus || p.nKt > 40 || p.q_ss > (1 << 26)) return false;   // (16 rows of queries lie within 32 bits of each other)
   if (p.nKt > kShortMaxTiles) return (int64_t)p.B * p.H * p.nKt <= 7168 || 10 * per_head < 27 * units_per_head(p.Sq, kDenseWaves);
-  if (p.nKt < 8 || p.q_rope_mode) return false;
+  if (p.nKt < 8 || p.q_rope_mode || (p.row_cnt && units <= 14 * cus)) return false;
   return per_head > 8 ? 2 * units > 13 * (int64_t)cus || (p.B * p.H) % 8 == 0 : units > 10 * cus;
 }
 

@@ -70,6 +70,7 @@ def test_dense_calls_go_by_their_workgroups_and_keys(B, H, Sq, Sk, want):
     (1, 24, 49640, 448, SHORT, SHORT), (1, 24, 49640, 449, RELAY, SHORT), (1, 24, 49640, 1024, RELAY, SHORT),   # 7 | 8 .. 16 | 17 .. 40 | 41 tiles
     (1, 24, 49640, 1025, RELAY, RELAY), (1, 24, 49640, 2560, RELAY, RELAY), (1, 24, 49640, 2561, LONG, LONG),
     (1, 32, 4096, 1024, SHORT, SHORT), (1, 32, 4096, 1025, LONG, LONG), (1, 33, 4096, 1025, RELAY, RELAY),       # four units a CU and 32 more
+    (1, 28, 16384, 1024, RELAY, SHORT), (1, 28, 16385, 1024, RELAY, SHORT),                                       # (masked: 14 units a CU and 28 more)
     (1, 24, 6500, 512, RELAY, SHORT), (4, 2, 18000, 1024, RELAY, SHORT),                                          # whole heads for eight XCDs
     (1, 31, 5248, 832, SHORT, SHORT), (1, 31, 5248, 1088, RELAY, RELAY), (1, 31, 6912, 1024, RELAY, SHORT),       # ... and not, below and above 6.5 a CU
     (1, 208, 1024, 1024, SHORT, SHORT), (1, 319, 1024, 1024, SHORT, SHORT), (1, 321, 1024, 1024, RELAY, SHORT),   # heads of eight units: ten a CU
@@ -78,7 +79,9 @@ def test_dense_calls_go_by_their_workgroups_and_keys(B, H, Sq, Sk, want):
     (1, 256, 1280, 1793, RELAY, RELAY), (4, 100, 396, 1395, RELAY, RELAY),                                        # ... and blocks of 384 rows not full
 ])
 def test_calls_of_the_relay_form(B, H, Sq, Sk, want, rotated):
-    assert form(B, H, Sq, Sk) == form(B, H, Sq, Sk, masked=True) == form(B, H, Sq, Sk, in_place=True) == want
+    few = Sk <= 1024 and B * H * ((Sq + 127) // 128) <= 14 * 256
+    assert form(B, H, Sq, Sk) == form(B, H, Sq, Sk, in_place=True) == want
+    assert form(B, H, Sq, Sk, masked=True) == (SHORT if few else want)
     assert form(B, H, Sq, Sk, rope=1) == form(B, H, Sq, Sk, rope=2) == rotated
     assert form(B, H, Sq, Sk, fp8=True) in (SHORT, LONG) and form(B, H, Sq, Sk, fp8="pow2") in (SHORT, LONG)
     assert form(B, H, Sq, Sk, long_key_kernel=True) == LONG and form(B, H, Sq, Sk, sparse=True) == SPARSE
