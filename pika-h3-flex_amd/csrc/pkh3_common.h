@@ -215,8 +215,8 @@ __device__ __forceinline__ void load_norm_lanes(NormLanes& n, const float* norm_
 #pragma unroll
   for (int i = 0; i < 2; ++i) n.w[i] = norm_w ? norm_w[64 * i + 32 * ((lane & 15) >> 3) + 8 * (lane >> 4) + (lane & 7)] : 1.0f;
 }
-// `factor` times the value that lane N of this lane's row of 16 holds.  (The weights must not come from the two vector instructions before
-// this one; they are loaded long before.)
+// `factor` times the value that lane N of this lane's row of 16 holds.  (`x` must not come from the two vector instructions before this one, and the
+// compiler puts no wait states in front of assembly: see settle.)
 template <int N>
 __device__ __forceinline__ float times_row_lane(float x, float factor) {
   float y;
@@ -224,9 +224,12 @@ __device__ __forceinline__ float times_row_lane(float x, float factor) {
   return y;
 }
 
+// where the weights were kept elsewhere, they have been back for as long as it takes
+__device__ __forceinline__ void settle(NormLanes& n) { asm volatile("s_nop 1" : "+v"(n.w[0]), "+v"(n.w[1])); }
+
 // RMSNorm (if `normed`) and `factor` of this lane's 32 elements of a row as they are in memory: the squares are summed up two at a
 // time before the elements are unpacked, and the factor (the softmax scale and log2 e of the queries) rides with the norm's.
-__device__ __forceinline__ void norm_row(float (&x)[32], const bf16x8 (&raw)[4], bool normed, float eps, const NormLanes& n, float factor) {
+__device__ __forceinline__ void norm_row(float (&x)[32], const bf16x8 (&raw)[4], bool normed, float eps, NormLanes n, float factor) {
   if (normed) {
     float part[4];
 #pragma unroll
@@ -235,6 +238,7 @@ __device__ __forceinline__ void norm_row(float (&x)[32], const bf16x8 (&raw)[4],
     const float ms = wave_sum_groups((part[0] + part[1]) + (part[2] + part[3])) * (1.0f / kD) + eps;
     factor *= ms > 0.f ? rsqrtf(ms) : 0.f;
   }
+  settle(n);
   static_for<32>([&](auto ic) {
     constexpr int i = decltype(ic)::value;
     x[i] = times_row_lane<i & 15>(n.w[i >> 4], factor);
@@ -250,7 +254,7 @@ __device__ __forceinline__ void norm_lanes(float (&x)[32], float eps, NormLanes&
   // an all-zero row with eps == 0 stays all zero instead of 0 * inf
   const float ms = wave_sum_groups((part[0] + part[1]) + (part[2] + part[3])) * (1.0f / kD) + eps;
   const float rs = ms > 0.f ? rsqrtf(ms) : 0.f;
-  asm volatile("s_nop 1" : "+v"(n.w[0]), "+v"(n.w[1]));   // (where the weights were kept elsewhere, they have been back for as long as it takes)
+  settle(n);
   static_for<32>([&](auto ic) {
     constexpr int i = decltype(ic)::value;
     x[i] *= times_row_lane<i & 15>(n.w[i >> 4], rs);

@@ -62,7 +62,8 @@ def test_no_load_into_registers_is_inline_assembly():
 
 OBJDUMP = shutil.which("llvm-objdump") or "/opt/rocm/llvm/bin/llvm-objdump"
 MFMA_RESULT = 12   # wait states until another instruction may touch a result of eight passes (that of a 16 x 16 x 32 product takes fewer)
-VALU_RESULT = 2    # ... until an MFMA may read what a vector instruction wrote
+VALU_RESULT = 2    # ... until an MFMA, or the lane-crossing operand of another vector instruction, may read what a vector instruction wrote
+SCALAR_RESULT = 5  # ... until a memory instruction may take a scalar register that a vector instruction wrote
 
 
 def _registers(operands):
@@ -73,8 +74,26 @@ def _registers(operands):
     return found
 
 
+def _scalar_registers(operands):
+    """The scalar registers named in operands: {7, 8, ...}."""
+    found = set()
+    for one, first, last in re.findall(r"\bs(?:(\d+)\b|\[(\d+):(\d+)\])", operands):
+        found.update(range(int(one), int(one) + 1) if one else range(int(first), int(last) + 1))
+    return found
+
+
 def _hazards(listing):
     """Instructions of one kernel's listing that come too soon after an MFMA or a vector instruction whose result they touch."""
+    return _look(listing)[0]
+
+
+def _operand_hazards(listing):
+    """Vector instructions of one kernel's listing whose result is taken too soon by the lane-crossing operand of another, or as the scalar address of a
+    memory instruction: what the compiler sees to, but not in front of assembly statements."""
+    return _look(listing)[1]
+
+
+def _look(listing):
     code, at = [], {}
     for line in listing.splitlines():
         m = re.match(r"\s+(\S+)\s*(.*?)\s*// ([0-9A-F]+):(.*)", line)
@@ -103,10 +122,18 @@ def _hazards(listing):
                 todo.append((j + 1, waited))
         return False
 
-    found = []
+    found, operands = [], []
+    crossing = [_registers(ops.split(",")[1]) if re.search(r"\b(?:quad_perm|row_\w+|wave_\w+):?", ops) else set() for _, ops, _ in code]
+    address = [_scalar_registers(ops) if name.startswith(("global_", "buffer_", "scratch_", "flat_")) else set() for name, ops, _ in code]
     for i, (name, ops, _) in enumerate(code):
         if not name.startswith("v_"):
             continue
+        scalars = _scalar_registers(" ".join(ops.split(",")[:2 if "_co_" in name else 1]))
+        if scalars and touched_within(i, SCALAR_RESULT, lambda j: scalars & address[j]):
+            operands.append((i, name, ops))
+        if not name.startswith(("v_mfma", "v_cmp", "v_readlane", "v_readfirstlane")) and (_registers(ops.split(",")[0]) and touched_within(
+                i, VALU_RESULT, lambda j: _registers(ops.split(",")[0]) & crossing[j])):
+            operands.append((i, name, ops))
         result = _registers(ops.split(",")[0])
         mfma = name.startswith("v_mfma")
         # (an MFMA may go on with the result of another as its own sum: the unit keeps these in order)
@@ -115,7 +142,7 @@ def _hazards(listing):
             found.append((i, name, ops))
         if not mfma and result and touched_within(i, VALU_RESULT, lambda j: code[j][0].startswith("v_mfma") and result & regs[j]):
             found.append((i, name, ops))
-    return found
+    return found, operands
 
 
 @pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="llvm-objdump is not installed")
@@ -135,6 +162,40 @@ def test_nothing_touches_a_product_before_it_is_there(tmp_path):
             forms[name] = _hazards(listing)
             assert listing.count("v_mfma") >= 64, name
     assert len(forms) == 5 and not {n: h[:3] for n, h in forms.items() if h}, forms
+
+
+@pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="llvm-objdump is not installed")
+def test_no_operand_of_an_assembly_statement_is_too_young(tmp_path):
+    """Multiplications that take an operand from another lane, and copies from memory to LDS whose address is scalar (some of those registers are
+    kept in lanes of vector registers and come back from there), are assembly statements: the compiler puts no wait states in
+    front of them.  Looked up in the listing of every kernel, along all branches."""
+    import __graft_entry__
+    import pika_h3_flex_amd as pk
+
+    __graft_entry__.ensure_built()
+    kernels, crossings, copies = {}, 0, 0
+    for i, image in enumerate(_code_objects(pk._lib.LIB_PATH)):
+        f = tmp_path / f"{i}.elf"
+        f.write_bytes(image)
+        text = subprocess.run([OBJDUMP, "-d", str(f)], check=True, capture_output=True, text=True).stdout
+        for name, listing in re.findall(r"^[0-9a-f]+ <(\S+)>:\n(.*?)(?=^[0-9a-f]+ <|\Z)", text, re.M | re.S):
+            kernels[name] = _operand_hazards(listing)
+            crossings += listing.count("row_newbcast")
+            copies += listing.count("global_load_lds_dwordx4")
+    assert crossings > 500 and copies > 100 and any("relay" in n for n in kernels), (crossings, copies, sorted(kernels))
+    assert not {n: h[:3] for n, h in kernels.items() if h}
+
+
+def test_the_look_for_young_operands_finds_what_it_looks_for():
+    write = "\tv_mov_b32_e32 v9, v1           // 0000000000F0: 00\n"
+    cross = "\tv_mul_f32_dpp v3, v9, v4 row_newbcast:5 row_mask:0xf bank_mask:0xf // 0000000000FC: 00\n"
+    lane = "\tv_readlane_b32 s12, v40, 3    // 0000000000F0: 00\n"
+    copy = "\tglobal_load_lds_dwordx4 v5, s[12:13] // 000000000108: 00\n"
+    move = "\ts_mov_b32 m0, s7 // 0000000000F4: 00\n"
+    assert len(_operand_hazards(write + cross)) == 1 and len(_operand_hazards(lane + move + copy)) == 1
+    assert not _operand_hazards(write + "\ts_nop 1 // 0000000000F4: 00\n" + cross) and not _operand_hazards(write.replace("v9", "v4") + cross)
+    assert not _operand_hazards(lane + "\ts_nop 4 // 0000000000F8: 00\n" + copy) and not _operand_hazards(lane.replace("s12", "s14") + copy)
+    assert len(_operand_hazards(lane + "\ts_nop 3 // 0000000000F8: 00\n" + copy)) == 1
 
 
 def test_the_look_for_products_finds_what_it_looks_for():
