@@ -249,6 +249,29 @@ def test_runs_of_keys_with_logits_of_minus_infinity(first, last, sparse, H):
         assert err <= MAX_ABS and cos >= MIN_COS
 
 
+@pytest.mark.parametrize("first,last", [(448, 512), (384, 512), (500, 505), (0, 64), (96, 160), (0, 448)])
+@pytest.mark.parametrize("Sk", [505, 512])
+def test_runs_of_keys_with_logits_of_minus_infinity_in_the_relay_form(first, last, Sk):
+    """As above where a workgroup goes from unit to unit: it takes a head's last tile first (with fewer keys than the tile has places, or all),
+    so that runs which end there leave the first sums without a finite logit."""
+    import pika_h3_flex_amd as pk
+
+    O = _oracle()
+    H, Sq, last = 24, 5600, min(last, Sk)
+    assert _form(1, H, Sq, Sk) == forms.RELAY
+    gen = torch.Generator(device="cuda").manual_seed(first + Sk)
+    q, k, v = (torch.randn((1, S, H, 128), generator=gen, device="cuda").to(torch.bfloat16) for S in (Sq, Sk, Sk))
+    q[..., 0] = q[..., 0].abs() + 0.5
+    k[:, first:last, :, 0] = -math.inf
+    mask = torch.ones((1, Sk), dtype=torch.bool, device="cuda")
+    mask[:, first:last] = False
+    out = pk.attention(q, k, v)
+    assert torch.isfinite(out.float()).all()
+    want = torch.cat([O.reference_layer(q[:, i:i + 256], torch.nan_to_num(k, neginf=0.0), v, key_mask=mask) for i in range(0, Sq, 256)], dim=1)
+    err, cos = O.max_abs_and_cosine(out, want)
+    assert err <= MAX_ABS and cos >= MIN_COS
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("mode", [1, 2])
 @pytest.mark.parametrize("Sq,Sk", [(5, 300), (300, 5), (513, 129), (200, 2100)])
