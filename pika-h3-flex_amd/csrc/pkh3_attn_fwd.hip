@@ -1393,32 +1393,33 @@ template <bool ROPE>
 __device__ __forceinline__ RelayRun relay_run(const FwdParams& p, int per_head) {
   const int wgs = gridDim.x, rank = (blockIdx.x & 7) * (wgs >> 3) + (blockIdx.x >> 3);   // a contiguous run per XCD and workgroup
   const int per_entry = p.H * per_head, all = p.B * per_entry;
-  if (!p.row_cnt || p.B == 1) return {relay_cut(rank, all, per_head, wgs, !ROPE), relay_cut(rank + 1, all, per_head, wgs, !ROPE)};
-  const int lane = threadIdx.x & 63;
-  auto weight = [&](int b) { return b < p.B ? relay_weight(p.row_cnt[b]) : 0; };
-  auto sum_up = [&](int x) {                             // over this lane and those before it
+  // (entries of fewer than four units: every run has some, and looking at all of them costs as much as it evens out)
+  if (!p.row_cnt || p.B == 1 || per_entry < 4) return {relay_cut(rank, all, per_head, wgs, !ROPE), relay_cut(rank + 1, all, per_head, wgs, !ROPE)};
+  // Every lane has B / 64 entries.  (64 at a time, with a prefix sum for each, took 4 us for 300 entries, 21 for 1,500.)
+  const int lane = threadIdx.x & 63, each = (p.B + 63) / 64, first = min(lane * each, p.B), last = min(first + each, p.B);
+  int w = 0;
+  for (int b = first; b < last; ++b) w += relay_weight(p.row_cnt[b]);
+  int sum = w;                                           // over this lane and those before it
 #pragma unroll
-    for (int d = 1; d < 64; d *= 2) {
-      const int y = __shfl_up(x, d, 64);
-      if (lane >= d) x += y;
-    }
-    return x;
-  };
-  int total = 0;
-  for (int b0 = 0; b0 < p.B; b0 += 64) total += __builtin_amdgcn_readlane(sum_up(weight(b0 + lane)), 63);
+  for (int d = 1; d < 64; d *= 2) {
+    const int x = __shfl_up(sum, d, 64);
+    if (lane >= d) sum += x;
+  }
+  const int total = __builtin_amdgcn_readlane(sum, 63);
   RelayRun run{all, all};                                // (no entry holds the end of the last run)
-  for (int b0 = 0, before = 0; b0 < p.B; b0 += 64) {
-    const int w = weight(b0 + lane), sum = sum_up(w);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int64_t into = (int64_t)(rank + i) * total - (int64_t)(before + sum - w) * wgs;   // (in 1 / wgs of a weight)
-      const unsigned long long here = __ballot(into >= 0 && into < (int64_t)w * wgs);
-      if (here) {                                        // (one lane at most, in one turn of the loop)
-        const int unit = (b0 + lane) * per_entry + (int)relay_unit(into, w, wgs, per_entry);
-        (i ? run.end : run.at) = __builtin_amdgcn_readlane(unit, __builtin_ctzll(here));
+  for (int i = 0; i < 2; ++i) {
+    int into = (rank + i) * total - (sum - w) * wgs;     // (in 1 / wgs of a weight; 65,535 entries of at most 42 each)
+    const unsigned long long here = __ballot(into >= 0 && into < w * wgs);
+    if (here) {                                          // (one lane)
+      int b = first, entry = 0;
+      for (; b < last; ++b, into -= entry * wgs) {
+        entry = each == 1 ? w : relay_weight(p.row_cnt[b]);
+        if (into < entry * wgs) break;
       }
+      const int unit = b * per_entry + relay_unit(into, max(entry, 1), wgs, per_entry);
+      (i ? run.end : run.at) = __builtin_amdgcn_readlane(unit, __builtin_ctzll(here));
     }
-    before += __builtin_amdgcn_readlane(sum, 63);
   }
   return run;
 }

@@ -146,7 +146,7 @@ def test_short_key_form(B, H, Sq, Sk, masked, fp8):
     (1, 345, 300, 1025, 1, None), (1, 516, 200, 1088, 2, None),   # 17 tiles and rotation, the last one of one key and whole
     (3, 144, 1025, 600, 0, (0, 1, 400)),    # masked: no key, one, some
     (6, 60, 1250, 640, 0, (64, 65, 128, 129, 500, 640)),          # one to ten tiles
-    (70, 4, 500, 1100, 0, tuple(75 * i % 1101 for i in range(70))), (2, 24, 2900, 2500, 1, (64, 2500)),   # shared out by the entries' keys
+    (70, 4, 500, 1100, 0, tuple(75 * i % 1101 for i in range(70))), (530, 1, 200, 1100, 0, tuple(75 * i % 1101 for i in range(530))), (2, 24, 2900, 2500, 1, (64, 2500)),   # shared out by the entries' keys
 ])
 def test_relay_form(B, H, Sq, Sk, rope, valid, scale):
     """Dense calls of more than four 128-query units a CU against 8 to 40 key tiles: a workgroup goes from unit to unit.  At scale 6

@@ -157,7 +157,10 @@ def test_relay_shares_go_by_the_work_of_the_entries(tmp_path):
             int64_t end = (int64_t)B * units, before = 0;
             for (int b = 0; b < B; before += weight(b++)) {
               const int64_t into = (int64_t)(rank + 1) * total - before * wgs;
-              if (into >= 0 && into < (int64_t)weight(b) * wgs) end = (int64_t)b * units + relay_unit(into, weight(b), wgs, units);
+              if (into < 0 || into >= (int64_t)weight(b) * wgs) continue;
+              const int unit = relay_unit((int)into, weight(b), wgs, units);
+              CHECK(unit >= 0 && unit < units, "unit %d of %d", unit, units);
+              end = (int64_t)b * units + unit;
             }
             CHECK(end >= at && end <= (int64_t)B * units, "%d entries x %d units, workgroup %d of %d: [%lld, %lld)", B, units, rank, wgs, (long long)at, (long long)end);
             double run = 0;
