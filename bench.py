@@ -42,7 +42,7 @@ MEASURED_TRAFFIC = {
     "480p-sparse-fp8": (2.129e10, "profiles/attn_fwd_kernel_480p_sparse_fp8.md"),
     "768p": (2.33e10, "profiles/attn_fwd_dense_kernel_768p_bf16.md"),
     "joint": (4.55e9, "profiles/attn_fwd_dense_kernel_joint_bf16.md"),
-    "cross": (6.15e8, "profiles/attn_fwd_kernel_cross_short_key.md"),
+    "cross": (6.46e8, "profiles/attn_fwd_relay_kernel_cross.md"),
 }
 GEMM_TRAFFIC = (8.28e9, "profiles/gemm_kernel_480p_block.md")  # to_q/to_k/to_v launch of the 480p block
 

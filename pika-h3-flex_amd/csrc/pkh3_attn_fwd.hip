@@ -658,7 +658,8 @@ __device__ __forceinline__ int attn_fwd_body(const Params& p, int blk, int unit0
   // The block-sparse form has one workgroup per CU and nothing to run beside this: rows, tables and weights are asked for before
   // anything else of the unit is known, so that they cost one trip to memory between them and the plan's look-ups and the first
   // key copies run beside it (14,907 rows, fp8: the call 691 -> 679 us; 48,360, bf16: 6,880 -> 6,800).  So does the pipelined short-key form.
-  // Where a third wave per SIMD runs beside it, it gave nothing.
+  // Where a third wave per SIMD runs beside it, it gave nothing.  (The turn through LDS did: against loads in the order of the images in the long form
+  // alone, 124,992 rows 128.74 -> 127.18 ms, 48,360 19.68 -> 19.54, 15,342 2.093 -> 2.078, 48,360 in fp8 the same.)
   if constexpr (kAskFirst) load_q(0), load_q(1);
   load_norm_lanes(q_norm, p.q_norm_w, lane);
 
@@ -1366,8 +1367,9 @@ __global__ __launch_bounds__(64 * kNarrowWaves, 2) void attn_fwd_narrow_kernel(F
 // trip to memory behind the other) and its end cost as much as five of them.  Here a round costs 3.9 us and 2.1 to 2.2 a tile,
 // short-key workgroups (three to a CU) 9 and 2.3, long ones 13 and 2.0.  Kernel, us, before / with it: 24 heads x 49,640 queries against
 // 302 of 512 keys 249 / 228, 1,024 keys 543 / 505; x 14,830 against 1,536 keys 242 / 228; x 9,000 against 2,048 219 / 185 (rounds of
-// long workgroups that are nearly empty at the end).  What bounds it now: the MFMAs and, between two rounds, stores and
-// queries of all CUs at once at the rate of the memory (12 KiB of each a wave: 96 KiB a CU, 14 bytes a clock).
+// long workgroups that are nearly empty at the end).  What bounds it now, by counters of 49,640 x 302: vector work.  A SIMD's MFMAs take 46 % of the
+// cycles and its other vector instructions 54 %, at the same time 11 %; memory alone would take half of the time.  Between two rounds stores and
+// queries of all CUs (8 KiB of each a wave: 96 KiB a CU) come at once.
 // Queries are copied four neighbouring lanes to 64 bytes: lanes in the order of the operand images, neighbours in different rows, keep a CU's
 // vector-memory path busy four times as long (16 against 60 bytes a clock, one workgroup alone; stores the same).
 // Measured and not kept: the three groups a third of a round apart, each handing over while the others walk tiles (302 keys 243 against

@@ -190,7 +190,7 @@ __device__ __forceinline__ void turn_rows16(const Rows16& r, i32x4 (&out)[4], ch
 #pragma unroll
   for (int j = 0; j < 4; ++j) out[j] = *(const i32x4*)(lds + c * 256 + ((chunk(j) ^ c) * 16));
 }
-// a row's elements, as norm_rope_row takes them
+// a row's elements, as norm_row takes them
 __device__ __forceinline__ void turn_elements(const Rows16& r, bf16x8 (&raw)[4], char* lds, int lane) {
   i32x4 out[4];
   turn_rows16(r, out, lds, lane, [&](int j) { return 4 * j + (lane >> 4); });
